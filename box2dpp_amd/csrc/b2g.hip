@@ -5465,6 +5465,45 @@ __global__ __launch_bounds__(256) void k_toi_append(WorldView w, ToiState* st, u
     }
 }
 
+// b2g_body_state rows of bodies [first, first + n) written straight into
+// pinned host memory. Bound by round trips when small and by the bus when
+// large: a body's state lies in ten arrays, and reading it back array by array
+// took ten blocking copies into pageable memory. Here each lane gathers one body and puts its row
+// together in LDS, and the workgroup writes the rows out as consecutive
+// 16-byte words. A
+// call takes 15 us for 211 bodies (168 before), 55 us for 9974 (279) and
+// 324 us for 100 001 (1189, now 32 GB/s through the bus and the host's copy).
+constexpr int kReadBlock = 256;
+constexpr int kBodyWords = (int)(sizeof(b2g_body_state) / 4);
+static_assert(kBodyWords == 26 && sizeof(b2g_body_state) == 104, "row layout of k_read_bodies");
+__global__ void __launch_bounds__(kReadBlock) k_read_bodies(WorldView w, int first, int n, uint4* out) {
+    __shared__ uint4 stage[kReadBlock * kBodyWords / 4];
+    const int base = blockIdx.x * kReadBlock;
+    const int rows = min(kReadBlock, n - base);
+    if ((int)threadIdx.x < rows) {
+        const int b = first + base + (int)threadIdx.x;
+        const float4 xf = w.xf[b], c0 = w.pos0[b], c = w.pos[b], v = w.vel[b], f = w.force[b], m = w.mass[b];
+        const float2 lc = w.lcenter[b], gs = w.gsleep[b];
+        int* i = (int*)stage + threadIdx.x * kBodyWords;
+        float* o = (float*)i;
+        i[0] = w.btype[b];
+        i[1] = w.bflags[b];
+        o[2] = xf.x; o[3] = xf.y; o[4] = xf.z; o[5] = xf.w;
+        o[6] = lc.x; o[7] = lc.y;
+        o[8] = c0.x; o[9] = c0.y; o[10] = c0.z;
+        o[11] = c.x; o[12] = c.y; o[13] = c.z;
+        o[14] = v.x; o[15] = v.y; o[16] = v.z;
+        o[17] = f.x; o[18] = f.y; o[19] = f.z;
+        o[20] = m.x; o[21] = m.y; o[22] = m.z; o[23] = m.w;
+        o[24] = gs.x; o[25] = gs.y;
+    }
+    __syncthreads();
+    // the staging buffer holds whole 16-byte words past the last row
+    const int words = (rows * kBodyWords + 3) / 4;
+    uint4* dst = out + (size_t)base * kBodyWords / 4;
+    for (int k = threadIdx.x; k < words; k += kReadBlock) dst[k] = stage[k];
+}
+
 inline int blocks(int n, int bs = 256) { return (n + bs - 1) / bs; }
 
 }  // namespace
@@ -5559,6 +5598,10 @@ struct b2g_context {
     Counters* cnt = nullptr;       // device
     Counters* hcnt = nullptr;      // pinned host mirror
     double* penAcc = nullptr;
+    // body readback: pinned rows of up to kReadSlots chunks in flight
+    b2g_body_state* readRows = nullptr;
+    int readCap = 0;               // bodies the rows hold
+    hipEvent_t readDone[4] = {};
 
     // world switches
     V2 gravity = mk(0.0f, -10.0f);
@@ -7684,6 +7727,60 @@ int uploadBodies(b2g_context* ctx, int first, int count, const b2g_body_state* b
     return B2G_OK;
 }
 
+// Bodies to the host (k_read_bodies) in chunks, a ring of kReadSlots of them
+// in flight, so the host copies one chunk to the caller while the next ones
+// cross the bus. Chunks of 8192 bodies (852 KB): about 20 us of bus time
+// each, against about 5 us to launch one and wait for it.
+constexpr int kReadChunk = 8192;
+constexpr int kReadSlots = 4;
+static_assert(kReadChunk % kReadBlock == 0, "a chunk is whole workgroups");
+
+int ensureReadRows(b2g_context* ctx, int count) {
+    const int need = std::min(count, kReadSlots * kReadChunk);
+    if (need <= ctx->readCap) return B2G_OK;
+    const int cap = std::min(std::max(ctx->capBodies, need), kReadSlots * kReadChunk);
+    if (ctx->readRows) (void)hipHostFree(ctx->readRows);
+    ctx->readRows = nullptr;
+    ctx->readCap = 0;
+    HIPCHK(ctx, hipHostMalloc((void**)&ctx->readRows, sizeof(b2g_body_state) * (size_t)cap + sizeof(uint4),
+                              hipHostMallocDefault));
+    for (hipEvent_t& e : ctx->readDone)
+        if (!e) HIPCHK(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    ctx->readCap = cap;
+    return B2G_OK;
+}
+
+int readBodies(b2g_context* ctx, int first, int count, b2g_body_state* out) {
+    (void)hipSetDevice(ctx->device);
+    const int rc = ensureReadRows(ctx, count);
+    if (rc != B2G_OK) return rc;
+    hipStream_t s = ctx->stream;
+    const WorldView w = ctx->view();
+    const int chunks = (count + kReadChunk - 1) / kReadChunk;
+    auto rows = [&](int i) { return ctx->readRows + (size_t)(i % kReadSlots) * kReadChunk; };
+    auto size = [&](int i) { return std::min(kReadChunk, count - i * kReadChunk); };
+    auto launch = [&](int i) -> int {
+        hipLaunchKernelGGL(k_read_bodies, dim3(blocks(size(i), kReadBlock)), dim3(kReadBlock), 0, s, w,
+                           first + i * kReadChunk, size(i), (uint4*)rows(i));
+        LAUNCHCHK(ctx);
+        HIPCHK(ctx, hipEventRecord(ctx->readDone[i % kReadSlots], s));
+        return B2G_OK;
+    };
+    for (int i = 0; i < std::min(chunks, kReadSlots); ++i) {
+        const int lrc = launch(i);
+        if (lrc != B2G_OK) return lrc;
+    }
+    for (int i = 0; i < chunks; ++i) {
+        HIPCHK(ctx, hipEventSynchronize(ctx->readDone[i % kReadSlots]));
+        memcpy(out + (size_t)i * kReadChunk, rows(i), sizeof(b2g_body_state) * (size_t)size(i));
+        if (i + kReadSlots < chunks) {
+            const int lrc = launch(i + kReadSlots);
+            if (lrc != B2G_OK) return lrc;
+        }
+    }
+    return B2G_OK;
+}
+
 }  // namespace
 
 // ====================================================================
@@ -7777,6 +7874,9 @@ int b2g_destroy(b2g_context* ctx) {
     if (ctx->cnt) (void)hipFree(ctx->cnt);
     if (ctx->penAcc) (void)hipFree(ctx->penAcc);
     if (ctx->hcnt) (void)hipHostFree(ctx->hcnt);
+    if (ctx->readRows) (void)hipHostFree(ctx->readRows);
+    for (hipEvent_t e : ctx->readDone)
+        if (e) (void)hipEventDestroy(e);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return B2G_OK;
@@ -7829,35 +7929,7 @@ int b2g_set_bodies(b2g_context* ctx, int first, int count, const b2g_body_state*
 int b2g_get_bodies(b2g_context* ctx, int first, int count, b2g_body_state* out) {
     if (!ctx || first < 0 || count < 0 || first + count > ctx->nBodies || (count > 0 && !out)) return B2G_ERR_ARG;
     if (count == 0) return B2G_OK;
-    std::vector<int> type(count), flags(count);
-    std::vector<float4> xf(count), pos(count), pos0(count), vel(count), force(count), mass(count);
-    std::vector<float2> lc(count), gs(count);
-    hipStream_t s = ctx->stream;
-    HIPCHK(ctx, hipMemcpyAsync(type.data(), ctx->btype + first, sizeof(int) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(flags.data(), ctx->bflags + first, sizeof(int) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(xf.data(), ctx->xf + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(pos.data(), ctx->pos + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(pos0.data(), ctx->pos0 + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(vel.data(), ctx->vel + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(force.data(), ctx->force + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(mass.data(), ctx->mass + first, sizeof(float4) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(lc.data(), ctx->lcenter + first, sizeof(float2) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipMemcpyAsync(gs.data(), ctx->gsleep + first, sizeof(float2) * count, hipMemcpyDeviceToHost, s));
-    HIPCHK(ctx, hipStreamSynchronize(s));
-    for (int i = 0; i < count; ++i) {
-        b2g_body_state& b = out[i];
-        b.type = type[i];
-        b.flags = flags[i];
-        b.xf[0] = xf[i].x; b.xf[1] = xf[i].y; b.xf[2] = xf[i].z; b.xf[3] = xf[i].w;
-        b.lc[0] = lc[i].x; b.lc[1] = lc[i].y;
-        b.c0[0] = pos0[i].x; b.c0[1] = pos0[i].y; b.a0 = pos0[i].z;
-        b.c[0] = pos[i].x; b.c[1] = pos[i].y; b.a = pos[i].z;
-        b.v[0] = vel[i].x; b.v[1] = vel[i].y; b.w = vel[i].z;
-        b.force[0] = force[i].x; b.force[1] = force[i].y; b.torque = force[i].z;
-        b.invMass = mass[i].x; b.invI = mass[i].y; b.linearDamping = mass[i].z; b.angularDamping = mass[i].w;
-        b.gravityScale = gs[i].x; b.sleepTime = gs[i].y;
-    }
-    return B2G_OK;
+    return readBodies(ctx, first, count, out);
 }
 
 }  // extern "C"
