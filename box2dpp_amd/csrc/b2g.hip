@@ -303,24 +303,27 @@ __device__ inline int waveAppend(int* counter, bool want) {
     return want ? base + __popcll(mask & ((1ull << lane) - 1ull)) : -1;
 }
 
+// Impulses of the old manifold carried over by feature id, the first match
+// winning (REF/Dynamics/Contacts/b2Contact.cpp:190-205); unrolled, so both
+// manifolds stay in registers.
+__device__ inline void carryImpulses(b2g_manifold& m, const b2g_manifold& old) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const bool match0 = i < m.pointCount && old.pointCount > 0 && old.points[0].id == m.points[i].id;
+        const bool match1 = i < m.pointCount && old.pointCount > 1 && old.points[1].id == m.points[i].id;
+        const float n1 = match1 ? old.points[1].normalImpulse : 0.0f, t1 = match1 ? old.points[1].tangentImpulse : 0.0f;
+        m.points[i].normalImpulse = match0 ? old.points[0].normalImpulse : n1;
+        m.points[i].tangentImpulse = match0 ? old.points[0].tangentImpulse : t1;
+    }
+}
+
 // b2Contact::Update after the manifold is known: impulses carried over by
 // feature id, touching flag, wakes and begin/end counts.
 __device__ inline void collideFinish(const WorldView& w, Counters* cnt, int c, int flags, b2g_manifold& m,
                                      const b2g_manifold& old, int bA, int bB) {
     const bool wasTouching = (flags & CF_TOUCHING) != 0;
     const bool touching = m.pointCount > 0;
-    for (int i = 0; i < 2; ++i) {
-        m.points[i].normalImpulse = 0.0f;
-        m.points[i].tangentImpulse = 0.0f;
-        if (i >= m.pointCount) continue;
-        for (int j = 0; j < old.pointCount; ++j) {
-            if (old.points[j].id == m.points[i].id) {
-                m.points[i].normalImpulse = old.points[j].normalImpulse;
-                m.points[i].tangentImpulse = old.points[j].tangentImpulse;
-                break;
-            }
-        }
-    }
+    carryImpulses(m, old);
     if (touching != wasTouching) {
         wakeBody(w, bA);
         wakeBody(w, bB);
@@ -460,7 +463,7 @@ __device__ inline void stageShapes(b2g_shape* dst, const b2g_shape& a, const b2g
 // in LDS; the workgroups walk the list in steps of their tile count.
 constexpr int kTileBlock = 64;
 __global__ void __launch_bounds__(kTileBlock) k_collide_tiles(WorldView w, Counters* cnt, const int* tiles) {
-    __shared__ b2g_shape sh[kTileBlock / kTileLanes][2];
+    __shared__ __align__(16) b2g_shape sh[kTileBlock / kTileLanes][2];
     const int grp = threadIdx.x / kTileLanes, lane = threadIdx.x % kTileLanes;
     const int perBlock = kTileBlock / kTileLanes;
     const int n = cnt->nTiles;
@@ -884,7 +887,9 @@ __device__ inline void initConstraintOne(const WorldView& w, const ConView& cv, 
     float nm[2] = {0.0f, 0.0f}, tm[2] = {0.0f, 0.0f}, vb[2] = {0.0f, 0.0f};
     V2 rA[2] = {mk(0.0f, 0.0f), mk(0.0f, 0.0f)}, rB[2] = {mk(0.0f, 0.0f), mk(0.0f, 0.0f)};
     float ni[2] = {0.0f, 0.0f}, ti[2] = {0.0f, 0.0f};
-    for (int j = 0; j < pc; ++j) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        if (j >= pc) continue;
         if (warm) {
             ni[j] = dtRatio * m.points[j].normalImpulse;
             ti[j] = dtRatio * m.points[j].tangentImpulse;
@@ -947,7 +952,9 @@ __device__ inline void initConstraintOne(const WorldView& w, const ConView& cv, 
         // the carried normal and tangent impulse instead, in velocity-change
         // units (impulse over the point's normal or tangent mass).
         int fm = 0;
-        for (int j = 0; j < vpc; ++j) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            if (j >= vpc) continue;
             if (fv.scope == 0 && (ni[j] != 0.0f || ti[j] != 0.0f)) continue;
             fm |= 1 << j;
             const V2 dv = vB + cross(wB, rB[j]) - vA - cross(wA, rA[j]);
@@ -4419,15 +4426,7 @@ __global__ void k_collide_serial(WorldView w, RefView r, Counters* cnt) {
         b2g_manifold m = r.tmpMan[c];
         const bool wasTouching = (flags & CF_TOUCHING) != 0;
         const bool touching = m.pointCount > 0;
-        for (int i = 0; i < m.pointCount; ++i) {
-            for (int j = 0; j < old.pointCount; ++j) {
-                if (old.points[j].id == m.points[i].id) {
-                    m.points[i].normalImpulse = old.points[j].normalImpulse;
-                    m.points[i].tangentImpulse = old.points[j].tangentImpulse;
-                    break;
-                }
-            }
-        }
+        carryImpulses(m, old);
         if (touching != wasTouching) { wakeBody(w, bA); wakeBody(w, bB); }
         flags |= CF_ENABLED | CF_UPDATED;
         if (touching) flags |= CF_TOUCHING;
@@ -4738,7 +4737,7 @@ __global__ void k_collide_batch(const b2g_shape* A, const b2g_transform* xa, con
 __global__ void __launch_bounds__(kTileBlock) k_collide_batch_tiles(const b2g_shape* A, const b2g_transform* xa,
                                                                     const b2g_shape* B, const b2g_transform* xb, int n,
                                                                     b2g_manifold* out) {
-    __shared__ b2g_shape sh[kTileBlock / kTileLanes][2];
+    __shared__ __align__(16) b2g_shape sh[kTileBlock / kTileLanes][2];
     const int grp = threadIdx.x / kTileLanes, lane = threadIdx.x % kTileLanes;
     const int i = blockIdx.x * (kTileBlock / kTileLanes) + grp;
     const bool mine = i < n && A[i].type == B2G_POLYGON && B[i].type == B2G_POLYGON;
@@ -4924,17 +4923,7 @@ __device__ inline void toiUpdateContact(const WorldView& w, int c) {
     b2g_manifold m;
     zeroManifold(m);
     collideShapes(m, w.shape[fA], xfOf(w.xf[bA]), w.shape[fB], xfOf(w.xf[bB]));
-    for (int i = 0; i < m.pointCount; ++i) {
-        m.points[i].normalImpulse = 0.0f;
-        m.points[i].tangentImpulse = 0.0f;
-        for (int j = 0; j < old.pointCount; ++j) {
-            if (old.points[j].id == m.points[i].id) {
-                m.points[i].normalImpulse = old.points[j].normalImpulse;
-                m.points[i].tangentImpulse = old.points[j].tangentImpulse;
-                break;
-            }
-        }
-    }
+    carryImpulses(m, old);
     const bool wasTouching = (flags & CF_TOUCHING) != 0;
     const bool touching = m.pointCount > 0;
     if (touching != wasTouching) {
@@ -5231,17 +5220,7 @@ __global__ void k_toi_prep(WorldView w, ToiState* st, const unsigned long long* 
     b2g_manifold m;
     zeroManifold(m);
     collideShapes(m, w.shape[fA], xfX, w.shape[fB], xfY);
-    for (int p = 0; p < m.pointCount; ++p) {
-        m.points[p].normalImpulse = 0.0f;
-        m.points[p].tangentImpulse = 0.0f;
-        for (int j = 0; j < old.pointCount; ++j) {
-            if (old.points[j].id == m.points[p].id) {
-                m.points[p].normalImpulse = old.points[j].normalImpulse;
-                m.points[p].tangentImpulse = old.points[j].tangentImpulse;
-                break;
-            }
-        }
-    }
+    carryImpulses(m, old);
     const int slot = (int)(key & ((1u << kGatherSlotBits) - 1));
     man[slot] = m;
     touching[slot] = m.pointCount > 0 ? 1 : 0;
@@ -5468,11 +5447,11 @@ __global__ __launch_bounds__(256) void k_toi_append(WorldView w, ToiState* st, u
 // b2g_body_state rows of bodies [first, first + n) written straight into
 // pinned host memory. Bound by round trips when small and by the bus when
 // large: a body's state lies in ten arrays, and reading it back array by array
-// took ten blocking copies into pageable memory. Here each lane gathers one body and puts its row
-// together in LDS, and the workgroup writes the rows out as consecutive
-// 16-byte words. A
-// call takes 15 us for 211 bodies (168 before), 55 us for 9974 (279) and
-// 324 us for 100 001 (1189, now 32 GB/s through the bus and the host's copy).
+// took ten blocking copies into pageable memory. Here each lane gathers one
+// body and puts its row together in LDS, and the workgroup writes the rows out
+// as consecutive 16-byte words. A call takes 15 us for 211 bodies (168 before),
+// 55 us for 9974 (279) and 324 us for 100 001 (1189; now 32 GB/s through the
+// bus and the host's copy).
 constexpr int kReadBlock = 256;
 constexpr int kBodyWords = (int)(sizeof(b2g_body_state) / 4);
 static_assert(kBodyWords == 26 && sizeof(b2g_body_state) == 104, "row layout of k_read_bodies");
