@@ -855,8 +855,8 @@ struct FreshView {
 
 // b2ContactSolver ctor + InitializeVelocityConstraints,
 // REF/Dynamics/Contacts/b2ContactSolver.cpp:52-252.
-__device__ inline void initConstraintOne(const WorldView& w, const ConView& cv, int k, int c, float dtRatio, int warm,
-                                         Counters* cnt, const FreshView& fv) {
+__device__ inline int initConstraintOne(const WorldView& w, const ConView& cv, int k, int c, float dtRatio, int warm,
+                                        const FreshView& fv) {
     const int fA = w.cfA[c], fB = w.cfB[c];
     const int bA = w.fbody[fA], bB = w.fbody[fB];
     const b2g_manifold& m = w.cman[c];
@@ -872,11 +872,9 @@ __device__ inline void initConstraintOne(const WorldView& w, const ConView& cv, 
     const float wA = vA4.z, wB = vB4.z;
     const float2 mat = w.cmat[c];
     const int pc = m.pointCount;
-    atomicAdd(&cnt->points, pc);
 
     Xf xfA, xfB;
-    xfA.q = rotOf(pA.z);
-    xfB.q = rotOf(pB.z);
+    rotOf2(pA.z, pB.z, xfA.q, xfB.q);
     xfA.p = cA - mul(xfA.q, lcA);
     xfB.p = cB - mul(xfB.q, lcB);
     WorldManifold wm;
@@ -969,13 +967,21 @@ __device__ inline void initConstraintOne(const WorldView& w, const ConView& cv, 
         fv.mask[k] = fm;
         fv.num[k] = __popc(fm);
     }
+    return pc;
+}
+
+// Manifold points of the step: one add per wavefront (an atomic add of a
+// value per lane becomes a loop over the lanes).
+__device__ inline void countPoints(Counters* cnt, int pc) {
+    const int n = __popcll(__ballot(pc > 0)) + __popcll(__ballot(pc > 1));
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x && n > 0) atomicAdd(&cnt->points, n);
 }
 
 __global__ void k_init_constraints(WorldView w, ConView cv, const int* order, int n, float dtRatio, int warm,
                                    Counters* cnt, FreshView fv) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
-    initConstraintOne(w, cv, k, order[k], dtRatio, warm, cnt, fv);
+    countPoints(cnt, initConstraintOne(w, cv, k, order[k], dtRatio, warm, fv));
 }
 
 // Compacts the fresh points in constraint order: ref = (k << 1) | j.
@@ -1321,51 +1327,74 @@ __global__ void k_integrate_positions(WorldView w, float h) {
     integratePositionOne(w, b, h);
 }
 
+// A position constraint's row in registers. A pass over a colour is bound by
+// the latency of its reads, each kernel starting with cold caches, so every
+// array of the row is read at once, and only the bodies' rows and the
+// island's flag, whose addresses it holds, wait for it: two trips to memory
+// where testing the flag before reading on took four.
+struct PosRow {
+    int2 bodies;
+    int info, island;
+    float4 mass, lc, lp, lnp;
+    float2 rad;
+};
+
+__device__ inline PosRow loadPosRow(const ConView& cv, int k) {
+    PosRow r;
+    r.bodies = cv.bodies[k];
+    r.island = cv.island[k];
+    r.info = cv.info[k];
+    r.mass = cv.mass[k];
+    r.lc = cv.lc[k];
+    r.lp = cv.lp[k];
+    r.lnp = cv.lnp[k];
+    r.rad = cv.rad[k];
+    return r;
+}
+
 // b2ContactSolver::SolvePositionConstraints with b2PositionSolverManifold,
-// REF/Dynamics/Contacts/b2ContactSolver.cpp:614-744. Skips itself when the
-// previous iteration already met the early-exit test of b2Island::Solve.
-__device__ inline float solvePositionCore(const ConView& cv, int k, int info, float4& pA, float4& pB) {
-    const float4 ms = cv.mass[k];
-    const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
-    const int pc = (info >> 2) & 3;
-    const int type = (info >> 8) & 3;
-    const float4 lc = cv.lc[k];
-    const V2 lcA = mk(lc.x, lc.y), lcB = mk(lc.z, lc.w);
-    const float4 lp = cv.lp[k];
-    const float4 lnp = cv.lnp[k];
-    const float2 rad = cv.rad[k];
+// REF/Dynamics/Contacts/b2ContactSolver.cpp:614-744, one constraint: the
+// bodies' positions are passed in and returned (w = 0).
+__device__ inline float solvePositionRow(const PosRow& r, float4& pA, float4& pB) {
+    const float mA = r.mass.x, iA = r.mass.y, mB = r.mass.z, iB = r.mass.w;
+    const int pc = (r.info >> 2) & 3;
+    const int type = (r.info >> 8) & 3;
+    const bool circles = type == B2G_MANIFOLD_CIRCLES, faceB = type == B2G_MANIFOLD_FACE_B;
     V2 cA = mk(pA.x, pA.y), cB = mk(pB.x, pB.y);
     float aA = pA.z, aB = pB.z;
     float minSep = 0.0f;
+    // The three manifold types share one path: the reference point (a face's
+    // plane point, or the first circle's centre) on body 1, the other point on
+    // body 2, where face B swaps the bodies. With three paths, which a mixed
+    // wavefront runs one after another, a peeled first iteration and four
+    // copies of the library's sine the kernel had 1624 instructions instead of
+    // 736 and took 7.8 us instead of 7.4 us over 3000 constraints.
+#pragma clang loop unroll(disable)
     for (int j = 0; j < pc; ++j) {
         Xf xfA, xfB;
-        xfA.q = rotOf(aA);
-        xfB.q = rotOf(aB);
-        xfA.p = cA - mul(xfA.q, lcA);
-        xfB.p = cB - mul(xfB.q, lcB);
-        V2 normal, point;
-        float separation;
-        if (type == B2G_MANIFOLD_CIRCLES) {
-            const V2 pointA = mul(xfA, mk(lnp.z, lnp.w));
-            const V2 pointB = mul(xfB, mk(lp.x, lp.y));
-            normal = pointB - pointA;
+        rotOf2(aA, aB, xfA.q, xfB.q);
+        xfA.p = cA - mul(xfA.q, mk(r.lc.x, r.lc.y));
+        xfB.p = cB - mul(xfB.q, mk(r.lc.z, r.lc.w));
+        Xf xf1, xf2;
+        xf1.p.x = faceB ? xfB.p.x : xfA.p.x;
+        xf1.p.y = faceB ? xfB.p.y : xfA.p.y;
+        xf1.q.s = faceB ? xfB.q.s : xfA.q.s;
+        xf1.q.c = faceB ? xfB.q.c : xfA.q.c;
+        xf2.p.x = faceB ? xfA.p.x : xfB.p.x;
+        xf2.p.y = faceB ? xfA.p.y : xfB.p.y;
+        xf2.q.s = faceB ? xfA.q.s : xfB.q.s;
+        xf2.q.c = faceB ? xfA.q.c : xfB.q.c;
+        const V2 reference = mul(xf1, mk(r.lnp.z, r.lnp.w));
+        const V2 other = mul(xf2, j == 0 ? mk(r.lp.x, r.lp.y) : mk(r.lp.z, r.lp.w));
+        V2 normal = mul(xf1.q, mk(r.lnp.x, r.lnp.y));
+        V2 point = other;
+        if (circles) {
+            normal = other - reference;
             normalizeV(normal);
-            point = 0.5f * (pointA + pointB);
-            separation = dot(pointB - pointA, normal) - rad.x - rad.y;
-        } else if (type == B2G_MANIFOLD_FACE_A) {
-            normal = mul(xfA.q, mk(lnp.x, lnp.y));
-            const V2 planePoint = mul(xfA, mk(lnp.z, lnp.w));
-            const V2 clipPoint = mul(xfB, j == 0 ? mk(lp.x, lp.y) : mk(lp.z, lp.w));
-            separation = dot(clipPoint - planePoint, normal) - rad.x - rad.y;
-            point = clipPoint;
-        } else {
-            normal = mul(xfB.q, mk(lnp.x, lnp.y));
-            const V2 planePoint = mul(xfB, mk(lnp.z, lnp.w));
-            const V2 clipPoint = mul(xfA, j == 0 ? mk(lp.x, lp.y) : mk(lp.z, lp.w));
-            separation = dot(clipPoint - planePoint, normal) - rad.x - rad.y;
-            point = clipPoint;
-            normal = -normal;
+            point = 0.5f * (reference + other);
         }
+        const float separation = dot(other - reference, normal) - r.rad.x - r.rad.y;
+        if (faceB) normal = -normal;
         const V2 rA = point - cA;
         const V2 rB = point - cB;
         minSep = fminB(minSep, separation);
@@ -1386,69 +1415,78 @@ __device__ inline float solvePositionCore(const ConView& cv, int k, int info, fl
 }
 
 __device__ inline float solvePositionOne(const WorldView& w, const ConView& cv, int k) {
-    const int2 bi = cv.bodies[k];
-    const int info = cv.info[k];
-    float4 pA = w.pos[bi.x], pB = w.pos[bi.y];
-    const float minSep = solvePositionCore(cv, k, info, pA, pB);
-    if (info & 16) w.pos[bi.x] = pA;
-    if (info & 32) w.pos[bi.y] = pB;
+    const PosRow r = loadPosRow(cv, k);
+    float4 pA = w.pos[r.bodies.x], pB = w.pos[r.bodies.y];
+    const float minSep = solvePositionRow(r, pA, pB);
+    if (r.info & 16) w.pos[r.bodies.x] = pA;
+    if (r.info & 32) w.pos[r.bodies.y] = pB;
     return minSep;
 }
 
 // Early exit per island (b2Island::Solve, REF/Dynamics/b2Island.cpp:310-328):
 // a pass leaves an island solved when none of its points is deeper than
-// 3 * linearSlop, so per island and pass one "failed" flag suffices. Lanes
-// set it only while it is still clear, which keeps the writes to a large
-// island's flag few.
-__global__ void k_solve_position(WorldView w, ConView cv, int begin, int end, Counters* cnt, int it) {
-    __shared__ int blockMin;
-    if (threadIdx.x == 0) blockMin = 0;
-    __syncthreads();
-    const int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < end) {
-        const int root = cv.island[k];
-        const bool done = it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0;
-        if (!done) {
-            const float minSep = solvePositionOne(w, cv, k);
-            if (minSep < -3.0f * kLinearSlop) {
-                int* f = &w.islandMinSep[it * w.nBodies + root];
-                if (*f == 0) *f = 1;
-            }
-            if (minSep < 0.0f) atomicMin(&blockMin, encodeOrdered(minSep));
-        }
+// 3 * linearSlop, so per island and pass one "failed" flag suffices, and a
+// constraint of an island that the previous pass left solved is passed over.
+// Returns the separation (0: passed over). Of a wavefront's failing lanes only
+// the first stores the flag for those of its island, which keeps the writes
+// to a large island's flag few without reading it.
+__device__ inline float solvePositionStep(const WorldView& w, const ConView& cv, int k, int it) {
+    const PosRow r = loadPosRow(cv, k);
+    float4 pA = w.pos[r.bodies.x], pB = w.pos[r.bodies.y];
+    if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + r.island] == 0) return 0.0f;
+    const float minSep = solvePositionRow(r, pA, pB);
+    if (r.info & 16) w.pos[r.bodies.x] = pA;
+    if (r.info & 32) w.pos[r.bodies.y] = pB;
+    if (minSep < -3.0f * kLinearSlop) {
+        const int first = __builtin_amdgcn_readfirstlane(r.island);
+        const bool leader = __builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x;
+        if (leader || r.island != first) w.islandMinSep[it * w.nBodies + r.island] = 1;
     }
-    __syncthreads();
-    if (threadIdx.x == 0 && blockMin < 0) atomicMin(&cnt->minSep[it], blockMin);
+    return minSep;
+}
+
+__device__ inline int waveMin(int v) {
+    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
+    return v;
+}
+
+// The pass's minimum separation, over the wavefronts that lower it: `seen` is
+// an earlier reading of the counter, which only ever falls, so a wavefront
+// that has nothing below it has nothing to report. Called by whole
+// wavefronts. (An atomic minimum of every lane's value, in LDS or not, becomes
+// a loop over the lanes: k_solve_position over 3000 constraints took 7.4 us
+// with one, and takes 5.4 us; over 20 000, 9.1 and 7.2 us.)
+__device__ inline void recordMinSep(Counters* cnt, int it, int seen, float minSep) {
+    const int enc = minSep < 0.0f ? encodeOrdered(minSep) : 0;
+    if (!__any(enc < seen)) return;
+    const int lowest = waveMin(enc);
+    if (__lane_id() == 0) atomicMin(&cnt->minSep[it], lowest);
+}
+
+__global__ void k_solve_position(WorldView w, ConView cv, int begin, int end, Counters* cnt, int it) {
+    const int k = begin + blockIdx.x * blockDim.x + threadIdx.x;
+    int seen = 0;
+    float minSep = 0.0f;
+    if (k < end) {
+        seen = cnt->minSep[it];
+        minSep = solvePositionStep(w, cv, k, it);
+    }
+    recordMinSep(cnt, it, seen, minSep);
 }
 
 __global__ void k_solve_position_r(WorldView w, ConView cv, const int* ranges, int c, Counters* cnt, int it) {
-    __shared__ int blockMin;
-    if (threadIdx.x == 0) blockMin = 0;
-    __syncthreads();
     const int b1 = ranges[c + 1];
-    int lowest = 0;
-    for (int k = ranges[c] + blockIdx.x * blockDim.x + threadIdx.x; k < b1; k += gridDim.x * blockDim.x) {
-        const int root = cv.island[k];
-        if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) continue;
-        const float minSep = solvePositionOne(w, cv, k);
-        if (minSep < -3.0f * kLinearSlop) {
-            int* f = &w.islandMinSep[it * w.nBodies + root];
-            if (*f == 0) *f = 1;
-        }
-        if (minSep < 0.0f) lowest = min(lowest, encodeOrdered(minSep));
-    }
-    if (lowest < 0) atomicMin(&blockMin, lowest);
-    __syncthreads();
-    if (threadIdx.x == 0 && blockMin < 0) atomicMin(&cnt->minSep[it], blockMin);
+    const int seen = cnt->minSep[it];
+    float lowest = 0.0f;
+    for (int k = ranges[c] + blockIdx.x * blockDim.x + threadIdx.x; k < b1; k += gridDim.x * blockDim.x)
+        lowest = fminB(lowest, solvePositionStep(w, cv, k, it));
+    recordMinSep(cnt, it, seen, lowest);
 }
 
 __global__ void k_solve_position_serial_r(WorldView w, ConView cv, const int* ranges, int c, Counters* cnt, int it) {
     int lowest = 0;
     for (int k = ranges[c]; k < ranges[c + 1]; ++k) {
-        const int root = cv.island[k];
-        if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) continue;
-        const float minSep = solvePositionOne(w, cv, k);
-        if (minSep < -3.0f * kLinearSlop) w.islandMinSep[it * w.nBodies + root] = 1;
+        const float minSep = solvePositionStep(w, cv, k, it);
         if (minSep < 0.0f) lowest = min(lowest, encodeOrdered(minSep));
     }
     if (lowest < 0) atomicMin(&cnt->minSep[it], lowest);
@@ -1488,29 +1526,17 @@ __global__ void k_solve_velocity_tail(WorldView w, ConView cv, ColourRanges r, i
 
 __global__ void k_solve_position_tail(WorldView w, ConView cv, ColourRanges r, int c0, int c1, Counters* cnt,
                                       int it) {
-    __shared__ int blockMin;
-    if (threadIdx.x == 0) blockMin = 0;
-    __syncthreads();
-    int lowest = 0;
+    const int seen = cnt->minSep[it];
+    float lowest = 0.0f;
     for (int c = c0; c < c1; ++c) {
         const bool serial = c == kOverflowColour;
         if (!serial || threadIdx.x == 0) {
-            for (int k = r.s[c] + (serial ? 0 : threadIdx.x); k < r.s[c + 1]; k += serial ? 1 : blockDim.x) {
-                const int root = cv.island[k];
-                if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) continue;
-                const float minSep = solvePositionOne(w, cv, k);
-                if (minSep < -3.0f * kLinearSlop) {
-                    int* f = &w.islandMinSep[it * w.nBodies + root];
-                    if (*f == 0) *f = 1;
-                }
-                if (minSep < 0.0f) lowest = min(lowest, encodeOrdered(minSep));
-            }
+            for (int k = r.s[c] + (serial ? 0 : threadIdx.x); k < r.s[c + 1]; k += serial ? 1 : blockDim.x)
+                lowest = fminB(lowest, solvePositionStep(w, cv, k, it));
         }
         __syncthreads();
     }
-    if (lowest < 0) atomicMin(&blockMin, lowest);
-    __syncthreads();
-    if (threadIdx.x == 0 && blockMin < 0) atomicMin(&cnt->minSep[it], blockMin);
+    recordMinSep(cnt, it, seen, lowest);
 }
 
 // ====================================================================
@@ -1715,13 +1741,12 @@ __global__ void k_solve_position_cluster(WorldView w, ConView cv, ClusterView cl
     clusterColours(rs, [&](int k) {
         const int root = cv.island[k];
         if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) return;
-        const int2 bi = cv.bodies[k];
+        const PosRow row = loadPosRow(cv, k);
         const int2 sl = cv.slot[k];
-        const int info = cv.info[k];
-        float4 pA = stagedRow(st, w.pos, sl.x, bi.x), pB = stagedRow(st, w.pos, sl.y, bi.y);
-        const float minSep = solvePositionCore(cv, k, info, pA, pB);
-        if ((info & 16) && sl.x >= 0) st[sl.x] = pA;
-        if ((info & 32) && sl.y >= 0) st[sl.y] = pB;
+        float4 pA = stagedRow(st, w.pos, sl.x, row.bodies.x), pB = stagedRow(st, w.pos, sl.y, row.bodies.y);
+        const float minSep = solvePositionRow(row, pA, pB);
+        if ((row.info & 16) && sl.x >= 0) st[sl.x] = pA;
+        if ((row.info & 32) && sl.y >= 0) st[sl.y] = pB;
         if (minSep < -3.0f * kLinearSlop) {
             int* f = &w.islandMinSep[it * w.nBodies + root];
             if (*f == 0) *f = 1;
@@ -1736,10 +1761,7 @@ __global__ void k_solve_position_cluster(WorldView w, ConView cv, ClusterView cl
 __global__ void k_solve_position_serial(WorldView w, ConView cv, int begin, int end, Counters* cnt, int it) {
     int lowest = 0;
     for (int k = begin; k < end; ++k) {
-        const int root = cv.island[k];
-        if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) continue;
-        const float minSep = solvePositionOne(w, cv, k);
-        if (minSep < -3.0f * kLinearSlop) w.islandMinSep[it * w.nBodies + root] = 1;
+        const float minSep = solvePositionStep(w, cv, k, it);
         if (minSep < 0.0f) lowest = min(lowest, encodeOrdered(minSep));
     }
     if (lowest < 0) atomicMin(&cnt->minSep[it], lowest);
@@ -3629,11 +3651,6 @@ __device__ inline void gridBarrier(Counters* cnt) {
     __syncthreads();
 }
 
-__device__ inline int waveMin(int v) {
-    for (int o = 32; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o));
-    return v;
-}
-
 // kJoints: the joint passes are compiled in (worlds with joints), with at
 // most kPersistJointBlock lanes per workgroup so the joint code keeps its
 // registers; without them the kernel keeps the contact passes' budget.
@@ -3709,13 +3726,7 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
     for (int it = 0; it < p.posIters; ++it) {
         int lowest = 0;
         contactColours([&](int k) {
-            const int root = cv.island[k];
-            if (it > 0 && w.islandMinSep[(it - 1) * w.nBodies + root] == 0) return;
-            const float minSep = solvePositionOne(w, cv, k);
-            if (minSep < -3.0f * kLinearSlop) {
-                int* f = &w.islandMinSep[it * w.nBodies + root];
-                if (*f == 0) *f = 1;
-            }
+            const float minSep = solvePositionStep(w, cv, k, it);
             if (minSep < 0.0f) lowest = min(lowest, encodeOrdered(minSep));
         });
         lowest = waveMin(lowest);
@@ -4586,7 +4597,7 @@ __global__ void k_island_solve(WorldView w, ConView cv, JointView jv, RefView r,
     __syncthreads();
     const FreshView noFresh{nullptr, nullptr, nullptr};
     for (int k = k0 + tid; k < k1; k += nt)
-        initConstraintOne(w, cv, k, r.islandContacts[k], dtRatio, warm, cnt, noFresh);
+        countPoints(cnt, initConstraintOne(w, cv, k, r.islandContacts[k], dtRatio, warm, noFresh));
     __syncthreads();
     if (tid == 0) {
         if (warm)
@@ -4845,7 +4856,6 @@ struct ToiState {
     float4 backup[4];           // pos0 / pos of body A and B before the advance
     int movedList[kToiMovedCap];
     unsigned long long newKeys[kToiNewCap];
-    Counters scratch;           // counters the constraint set-up writes
 };
 constexpr size_t kToiReadback = offsetof(ToiState, bodyA);
 
@@ -4958,8 +4968,7 @@ __device__ inline float solveTOIPositionOne(const WorldView& w, const ConView& c
     float minSep = 0.0f;
     for (int j = 0; j < pc; ++j) {
         Xf xfA, xfB;
-        xfA.q = rotOf(aA);
-        xfB.q = rotOf(aB);
+        rotOf2(aA, aB, xfA.q, xfB.q);
         xfA.p = cA - mul(xfA.q, lcA);
         xfB.p = cB - mul(xfB.q, lcB);
         V2 normal, point;
@@ -5314,7 +5323,7 @@ __global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, Toi
     // b2Island::SolveTOI
     const FreshView noFresh{nullptr, nullptr, nullptr, 0};
     const int ncons = st->nContacts;
-    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, &st->scratch, noFresh);
+    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, noFresh);
     for (int it = 0; it < 20; ++it) {
         float minSep = 0.0f;
         for (int k = 0; k < ncons; ++k) minSep = fminB(minSep, solveTOIPositionOne(w, cv, k, bA, bB));
@@ -5323,7 +5332,7 @@ __global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, Toi
     const float4 pa = w.pos[bA], pb = w.pos[bB];
     w.pos0[bA] = make_float4(pa.x, pa.y, pa.z, w.pos0[bA].w);
     w.pos0[bB] = make_float4(pb.x, pb.y, pb.z, w.pos0[bB].w);
-    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, &st->scratch, noFresh);
+    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, noFresh);
     for (int it = 0; it < velIters; ++it)
         for (int k = 0; k < ncons; ++k) solveVelocityOne(w, cv, k);
     const float h = (1.0f - st->alpha) * dt;
