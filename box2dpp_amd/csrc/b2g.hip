@@ -853,10 +853,53 @@ struct FreshView {
     int scope;    // 0: fresh points; 1: every solved point, carried impulse as input
 };
 
+// A velocity constraint's row in registers. The block matrix of two points is
+// read as soon as the point count is there, together with the bodies' rows.
+struct VelRow {
+    int2 bodies;
+    int info;
+    float4 mass, normal, r0, r1, pmass, imp, K, NM;
+    float2 bias;
+};
+
+__device__ inline VelRow loadVelRow(const ConView& cv, int k) {
+    VelRow r;
+    r.bodies = cv.bodies[k];
+    r.info = cv.info[k];
+    r.mass = cv.mass[k];
+    r.normal = cv.normal[k];
+    r.r0 = cv.r0[k];
+    r.r1 = cv.r1[k];
+    r.pmass = cv.pmass[k];
+    r.imp = cv.imp[k];
+    r.bias = cv.bias[k];
+    r.K = r.NM = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if ((r.info & 3) == 2) {
+        r.K = cv.K[k];
+        r.NM = cv.NM[k];
+    }
+    return r;
+}
+
+__device__ inline void storeVelRow(const ConView& cv, int k, const VelRow& r) {
+    cv.info[k] = r.info;
+    cv.mass[k] = r.mass;
+    cv.normal[k] = r.normal;
+    cv.r0[k] = r.r0;
+    cv.r1[k] = r.r1;
+    cv.pmass[k] = r.pmass;
+    cv.bias[k] = r.bias;
+    cv.imp[k] = r.imp;
+    cv.K[k] = r.K;
+    cv.NM[k] = r.NM;
+}
+
 // b2ContactSolver ctor + InitializeVelocityConstraints,
 // REF/Dynamics/Contacts/b2ContactSolver.cpp:52-252.
-__device__ inline int initConstraintOne(const WorldView& w, const ConView& cv, int k, int c, float dtRatio, int warm,
-                                        const FreshView& fv) {
+// Returns the point count; the velocity row goes to v, the rest of the
+// constraint to the arrays.
+__device__ inline int initConstraintRow(const WorldView& w, const ConView& cv, int k, int c, float dtRatio, int warm,
+                                        const FreshView& fv, VelRow& v) {
     const int fA = w.cfA[c], fB = w.cfB[c];
     const int bA = w.fbody[fA], bB = w.fbody[fB];
     const b2g_manifold& m = w.cman[c];
@@ -926,16 +969,17 @@ __device__ inline int initConstraintOne(const WorldView& w, const ConView& cv, i
     const bool dynA = w.btype[bA] == BT_DYNAMIC, dynB = w.btype[bB] == BT_DYNAMIC;
     cv.contact[k] = c;
     cv.bodies[k] = make_int2(bA, bB);
-    cv.mass[k] = make_float4(mA, iA, mB, iB);
-    cv.normal[k] = make_float4(normal.x, normal.y, mat.x, w.ctan[c]);
-    cv.r0[k] = make_float4(rA[0].x, rA[0].y, rB[0].x, rB[0].y);
-    cv.r1[k] = make_float4(rA[1].x, rA[1].y, rB[1].x, rB[1].y);
-    cv.pmass[k] = make_float4(nm[0], tm[0], nm[1], tm[1]);
-    cv.bias[k] = make_float2(vb[0], vb[1]);
-    cv.imp[k] = make_float4(ni[0], ti[0], ni[1], ti[1]);
-    cv.K[k] = K;
-    cv.NM[k] = NM;
-    cv.info[k] = vpc | (pc << 2) | (dynA ? 16 : 0) | (dynB ? 32 : 0) | (m.type << 8);
+    v.bodies = make_int2(bA, bB);
+    v.mass = make_float4(mA, iA, mB, iB);
+    v.normal = make_float4(normal.x, normal.y, mat.x, w.ctan[c]);
+    v.r0 = make_float4(rA[0].x, rA[0].y, rB[0].x, rB[0].y);
+    v.r1 = make_float4(rA[1].x, rA[1].y, rB[1].x, rB[1].y);
+    v.pmass = make_float4(nm[0], tm[0], nm[1], tm[1]);
+    v.bias = make_float2(vb[0], vb[1]);
+    v.imp = make_float4(ni[0], ti[0], ni[1], ti[1]);
+    v.K = K;
+    v.NM = NM;
+    v.info = vpc | (pc << 2) | (dynA ? 16 : 0) | (dynB ? 32 : 0) | (m.type << 8);
     cv.lp[k] = make_float4(m.points[0].localPoint.x, m.points[0].localPoint.y, m.points[1].localPoint.x,
                            m.points[1].localPoint.y);
     cv.lnp[k] = make_float4(m.localNormal.x, m.localNormal.y, m.localPoint.x, m.localPoint.y);
@@ -967,6 +1011,14 @@ __device__ inline int initConstraintOne(const WorldView& w, const ConView& cv, i
         fv.mask[k] = fm;
         fv.num[k] = __popc(fm);
     }
+    return pc;
+}
+
+__device__ inline int initConstraintOne(const WorldView& w, const ConView& cv, int k, int c, float dtRatio, int warm,
+                                        const FreshView& fv) {
+    VelRow v;
+    const int pc = initConstraintRow(w, cv, k, c, dtRatio, warm, fv, v);
+    storeVelRow(cv, k, v);
     return pc;
 }
 
@@ -1065,16 +1117,13 @@ __global__ void k_residual(WorldView w, ConView cv, int n, Counters* cnt) {
 // b2ContactSolver::WarmStart, REF/Dynamics/Contacts/b2ContactSolver.cpp:254-292.
 // The body velocities are passed in and returned (w = 0), so the same
 // arithmetic serves global and LDS-staged bodies.
-__device__ inline void warmStartCore(const ConView& cv, int k, int info, float4& va, float4& vbv) {
-    const float4 ms = cv.mass[k];
+__device__ inline void warmStartRow(int info, const float4& ms, const float4& nf, const float4& imp, const float4& r0,
+                                    const float4& r1, float4& va, float4& vbv) {
     const int pc = info & 3;
     V2 vA = mk(va.x, va.y), vB = mk(vbv.x, vbv.y);
     float wA = va.z, wB = vbv.z;
-    const float4 nf = cv.normal[k];
     const V2 normal = mk(nf.x, nf.y);
     const V2 tangent = cross(normal, 1.0f);
-    const float4 imp = cv.imp[k];
-    const float4 r0 = cv.r0[k], r1 = cv.r1[k];
     for (int j = 0; j < pc; ++j) {
         const float ni = j == 0 ? imp.x : imp.z;
         const float ti = j == 0 ? imp.y : imp.w;
@@ -1087,6 +1136,10 @@ __device__ inline void warmStartCore(const ConView& cv, int k, int info, float4&
     }
     va = make_float4(vA.x, vA.y, wA, 0.0f);
     vbv = make_float4(vB.x, vB.y, wB, 0.0f);
+}
+
+__device__ inline void warmStartCore(const ConView& cv, int k, int info, float4& va, float4& vbv) {
+    warmStartRow(info, cv.mass[k], cv.normal[k], cv.imp[k], cv.r0[k], cv.r1[k], va, vbv);
 }
 
 __device__ inline void warmStartOne(const WorldView& w, const ConView& cv, int k) {
@@ -1113,20 +1166,20 @@ __global__ void k_warm_start_serial(WorldView w, ConView cv, int begin, int end)
 // b2ContactSolver::SolveVelocityConstraints, REF/Dynamics/Contacts/b2ContactSolver.cpp:294-597:
 // friction per point clamped to the friction cone, then the normal impulse,
 // by a 2x2 linear complementarity solve (total enumeration) for two points.
-__device__ inline void solveVelocityCore(const ConView& cv, int k, int info, float4& va, float4& vbv) {
-    const float4 ms = cv.mass[k];
+__device__ inline void solveVelocityRow(VelRow& r, float4& va, float4& vbv) {
+    const float4 ms = r.mass;
     const float mA = ms.x, iA = ms.y, mB = ms.z, iB = ms.w;
-    const int pc = info & 3;
+    const int pc = r.info & 3;
     V2 vA = mk(va.x, va.y), vB = mk(vbv.x, vbv.y);
     float wA = va.z, wB = vbv.z;
-    const float4 nf = cv.normal[k];
+    const float4 nf = r.normal;
     const V2 normal = mk(nf.x, nf.y);
     const V2 tangent = cross(normal, 1.0f);
     const float friction = nf.z;
     const float tangentSpeed = nf.w;
-    float4 imp = cv.imp[k];
-    const float4 pm = cv.pmass[k];
-    const float4 r0 = cv.r0[k], r1 = cv.r1[k];
+    float4 imp = r.imp;
+    const float4 pm = r.pmass;
+    const float4 r0 = r.r0, r1 = r.r1;
     const V2 rA0 = mk(r0.x, r0.y), rB0 = mk(r0.z, r0.w);
     const V2 rA1 = mk(r1.x, r1.y), rB1 = mk(r1.z, r1.w);
 
@@ -1163,7 +1216,7 @@ __device__ inline void solveVelocityCore(const ConView& cv, int k, int info, flo
     if (pc == 1) {
         const V2 dv = vB + cross(wB, rB0) - vA - cross(wA, rA0);
         const float vn = dot(dv, normal);
-        float lambda = -pm.x * (vn - cv.bias[k].x);
+        float lambda = -pm.x * (vn - r.bias.x);
         const float ni = fmaxB(imp.x + lambda, 0.0f);
         lambda = ni - imp.x;
         imp.x = ni;
@@ -1173,8 +1226,8 @@ __device__ inline void solveVelocityCore(const ConView& cv, int k, int info, flo
         vB += mB * P;
         wB += iB * cross(rB0, P);
     } else {
-        const float2 vbias = cv.bias[k];
-        const float4 K = cv.K[k], NM = cv.NM[k];
+        const float2 vbias = r.bias;
+        const float4 K = r.K, NM = r.NM;
         const V2 a = mk(imp.x, imp.z);
         const V2 dv1 = vB + cross(wB, rB0) - vA - cross(wA, rA0);
         const V2 dv2 = vB + cross(wB, rB1) - vA - cross(wA, rA1);
@@ -1224,18 +1277,18 @@ __device__ inline void solveVelocityCore(const ConView& cv, int k, int info, flo
             imp.z = x.y;
         }
     }
-    cv.imp[k] = imp;
+    r.imp = imp;
     va = make_float4(vA.x, vA.y, wA, 0.0f);
     vbv = make_float4(vB.x, vB.y, wB, 0.0f);
 }
 
 __device__ inline void solveVelocityOne(const WorldView& w, const ConView& cv, int k) {
-    const int2 bi = cv.bodies[k];
-    const int info = cv.info[k];
-    float4 va = w.vel[bi.x], vb = w.vel[bi.y];
-    solveVelocityCore(cv, k, info, va, vb);
-    if (info & 16) w.vel[bi.x] = va;
-    if (info & 32) w.vel[bi.y] = vb;
+    VelRow r = loadVelRow(cv, k);
+    float4 va = w.vel[r.bodies.x], vb = w.vel[r.bodies.y];
+    solveVelocityRow(r, va, vb);
+    cv.imp[k] = r.imp;
+    if (r.info & 16) w.vel[r.bodies.x] = va;
+    if (r.info & 32) w.vel[r.bodies.y] = vb;
 }
 
 __global__ void k_solve_velocity(WorldView w, ConView cv, int begin, int end) {
@@ -1249,16 +1302,17 @@ __global__ void k_solve_velocity_serial(WorldView w, ConView cv, int begin, int 
 }
 
 // b2ContactSolver::StoreImpulses, REF/Dynamics/Contacts/b2ContactSolver.cpp:599-612.
-__device__ inline void storeImpulsesOne(const WorldView& w, const ConView& cv, int k) {
-    const int c = cv.contact[k];
-    const int vpc = cv.info[k] & 3;
-    const float4 imp = cv.imp[k];
+__device__ inline void storeImpulsesTo(const WorldView& w, int c, int vpc, const float4& imp) {
     w.cman[c].points[0].normalImpulse = imp.x;
     w.cman[c].points[0].tangentImpulse = imp.y;
     if (vpc == 2) {
         w.cman[c].points[1].normalImpulse = imp.z;
         w.cman[c].points[1].tangentImpulse = imp.w;
     }
+}
+
+__device__ inline void storeImpulsesOne(const WorldView& w, const ConView& cv, int k) {
+    storeImpulsesTo(w, cv.contact[k], cv.info[k] & 3, cv.imp[k]);
 }
 
 __global__ void k_store_impulses(WorldView w, ConView cv, int n) {
@@ -1423,13 +1477,22 @@ __device__ inline float solvePositionOne(const WorldView& w, const ConView& cv, 
     return minSep;
 }
 
+// Flags an island that this pass has not left solved. Of a wavefront's
+// failing lanes only the first stores the flag for those of its island, which
+// keeps the writes to a large island's flag few without reading it.
+__device__ inline void failIsland(const WorldView& w, int island, int it, float minSep) {
+    if (minSep < -3.0f * kLinearSlop) {
+        const int first = __builtin_amdgcn_readfirstlane(island);
+        const bool leader = __builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x;
+        if (leader || island != first) w.islandMinSep[it * w.nBodies + island] = 1;
+    }
+}
+
 // Early exit per island (b2Island::Solve, REF/Dynamics/b2Island.cpp:310-328):
 // a pass leaves an island solved when none of its points is deeper than
 // 3 * linearSlop, so per island and pass one "failed" flag suffices, and a
 // constraint of an island that the previous pass left solved is passed over.
-// Returns the separation (0: passed over). Of a wavefront's failing lanes only
-// the first stores the flag for those of its island, which keeps the writes
-// to a large island's flag few without reading it.
+// Returns the separation (0: passed over).
 __device__ inline float solvePositionStep(const WorldView& w, const ConView& cv, int k, int it) {
     const PosRow r = loadPosRow(cv, k);
     float4 pA = w.pos[r.bodies.x], pB = w.pos[r.bodies.y];
@@ -1437,11 +1500,7 @@ __device__ inline float solvePositionStep(const WorldView& w, const ConView& cv,
     const float minSep = solvePositionRow(r, pA, pB);
     if (r.info & 16) w.pos[r.bodies.x] = pA;
     if (r.info & 32) w.pos[r.bodies.y] = pB;
-    if (minSep < -3.0f * kLinearSlop) {
-        const int first = __builtin_amdgcn_readfirstlane(r.island);
-        const bool leader = __builtin_amdgcn_readfirstlane(threadIdx.x) == threadIdx.x;
-        if (leader || r.island != first) w.islandMinSep[it * w.nBodies + r.island] = 1;
-    }
+    failIsland(w, r.island, it, minSep);
     return minSep;
 }
 
@@ -1718,13 +1777,13 @@ __global__ void k_solve_velocity_cluster(WorldView w, ConView cv, ClusterView cl
     const int nb = stageCluster(cl, w.vel, st, rs);
     if (nb < 0) return;
     clusterColours(rs, [&](int k) {
-        const int2 bi = cv.bodies[k];
+        VelRow row = loadVelRow(cv, k);
         const int2 sl = cv.slot[k];
-        const int info = cv.info[k];
-        float4 va = stagedRow(st, w.vel, sl.x, bi.x), vb = stagedRow(st, w.vel, sl.y, bi.y);
-        solveVelocityCore(cv, k, info, va, vb);
-        if ((info & 16) && sl.x >= 0) st[sl.x] = va;
-        if ((info & 32) && sl.y >= 0) st[sl.y] = vb;
+        float4 va = stagedRow(st, w.vel, sl.x, row.bodies.x), vb = stagedRow(st, w.vel, sl.y, row.bodies.y);
+        solveVelocityRow(row, va, vb);
+        cv.imp[k] = row.imp;
+        if ((row.info & 16) && sl.x >= 0) st[sl.x] = va;
+        if ((row.info & 32) && sl.y >= 0) st[sl.y] = vb;
     });
     unstageCluster(cl, w.vel, st, nb);
 }
@@ -3735,6 +3794,183 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
     }
     for (int b = t; b < w.nBodies; b += stride)
         if (islandBody(w, b)) syncTransformOne(w, b);
+}
+
+// ====================================================================
+// Block solve: the whole island solve of a small world (or of a group of
+// sub-worlds) by one workgroup in one launch. A per-colour launch costs 4 to
+// 5 us however few constraints it has: dispatch, cold caches, two trips to
+// memory. Here the bodies' rows stay in LDS, the first kBlockRows *
+// blockDim.x constraints' rows in registers from the first velocity pass to
+// the last, and colours are a workgroup barrier apart, so a colour costs its
+// arithmetic and two LDS reads. Constraints beyond the registers' reach are
+// read row by row from memory (L2) in every pass.
+//
+// Lane t holds constraints t, t + blockDim.x, ... in colour order, so a
+// colour's constraints lie on neighbouring lanes and a wavefront without any
+// of them passes it over. Each constraint goes through the per-colour
+// kernels' functions in the same order of colours, so the results are theirs
+// bit for bit. The overflow colour, whose constraints share bodies, is left
+// to the per-colour kernels (blockSolveFits). What bounds it is one
+// wavefront's arithmetic: a colour's velocity pass is some 300 instructions,
+// of which a wavefront issues one in four cycles. The solve of a 210-box
+// pyramid (400 constraints, 5 colours, 8/3 iterations) takes 75 us, that of a
+// 1493-body pile (2650 constraints, 7 colours) 153 us, in place of 16
+// launches with 110 and 210 us of kernel time.
+// ====================================================================
+constexpr int kBlockBodies = 4096;       // body rows in LDS: 64 KB
+constexpr int kBlockConstraints = 8192;  // most constraints (blockSolveFits)
+constexpr int kBlockJointed = 4096;      // most constraints, and most joints, with joints
+constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane, whose rows take most of them
+template <bool kJoints>
+constexpr int kBlockRows = kJoints ? 3 : 4;  // constraint rows a lane holds
+
+struct BlockPlan {
+    SolvePlan solve;
+    V2 gravity;
+    int initHere;   // integrate the velocities and set up the constraints, too
+};
+
+template <bool kJoints>
+__global__ void __launch_bounds__(kBlockLanes)
+    k_solve_block(WorldView w, ConView cv, JointView jv, const int* order, BlockPlan plan, Counters* cnt) {
+    extern __shared__ float4 rows[];  // velocities, then positions, of the bodies
+    constexpr int R = kBlockRows<kJoints>;
+    const SolvePlan& p = plan.solve;
+    const int t = threadIdx.x, T = blockDim.x;
+    const int nb = w.nBodies;
+    WorldView wl = w;  // the bodies' rows in LDS for the functions that take a world
+    wl.vel = rows;
+
+    for (int b = t; b < nb; b += T) {
+        rows[b] = w.vel[b];
+        if (plan.initHere && islandBody(w, b)) integrateVelocityOne(wl, b, plan.gravity, p.h);
+    }
+    __syncthreads();
+
+    // The rows: set up here (every constraint then has a register row) or read.
+    VelRow row[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = t + r * T;
+        row[r].info = 0;
+        int pc = 0;
+        if (k < p.nCons) {
+            if (plan.initHere)
+                pc = initConstraintRow(wl, cv, k, order[k], p.dtRatio, p.jointWarm, FreshView{}, row[r]);
+            else
+                row[r] = loadVelRow(cv, k);
+        }
+        if (plan.initHere) countPoints(cnt, pc);
+    }
+    if (plan.initHere) __syncthreads();  // the set-up reads the velocities that the warm start changes
+
+    // reg(row) over the constraints in registers, mem(k) over the others,
+    // colour after colour.
+    auto colours = [&](auto reg, auto mem) {
+        for (int c = 0; c < p.nColours; ++c) {
+            const int b0 = p.cs[c], b1 = p.cs[c + 1];
+            if (b1 <= b0) continue;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int k = t + r * T;
+                if (k >= b0 && k < b1) reg(r);
+            }
+            for (int k = max(b0, R * T) + t; k < b1; k += T) mem(k);
+            __syncthreads();
+        }
+    };
+    auto jointColours = [&](auto one) {
+        if (!kJoints) return;
+        for (int c = 0; c < p.nJointColours; ++c) {
+            const int b0 = p.js[c], b1 = p.js[c + 1];
+            if (b1 <= b0) continue;
+            for (int k = b0 + t; k < b1; k += T) one(jv.order[k]);
+            __syncthreads();
+        }
+    };
+    auto keep = [&](int info, int2 bodies, const float4& a, const float4& b) {
+        if (info & 16) rows[bodies.x] = a;
+        if (info & 32) rows[bodies.y] = b;
+    };
+    // b2Island::Solve, REF/Dynamics/b2Island.cpp:246-270
+    if (p.contactWarm)
+        colours(
+            [&](int r) {
+                float4 va = rows[row[r].bodies.x], vb = rows[row[r].bodies.y];
+                warmStartRow(row[r].info, row[r].mass, row[r].normal, row[r].imp, row[r].r0, row[r].r1, va, vb);
+                keep(row[r].info, row[r].bodies, va, vb);
+            },
+            [&](int k) { warmStartOne(wl, cv, k); });
+    jointColours([&](int j) { jointInitOne(wl, jv, j, p.dtRatio, p.jointWarm); });
+    for (int it = 0; it < p.velIters; ++it) {
+        jointColours([&](int j) { jointSolveVelocityOne(wl, jv, j, p.h); });
+        colours(
+            [&](int r) {
+                float4 va = rows[row[r].bodies.x], vb = rows[row[r].bodies.y];
+                solveVelocityRow(row[r], va, vb);
+                keep(row[r].info, row[r].bodies, va, vb);
+            },
+            [&](int k) { solveVelocityOne(wl, cv, k); });
+    }
+    // StoreImpulses and the position integration (b2Island.cpp:272-306); a
+    // body's row in LDS goes from velocity to position in its own lane.
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = t + r * T;
+        if (k < p.nCons) storeImpulsesTo(w, cv.contact[k], row[r].info & 3, row[r].imp);
+    }
+    for (int k = R * T + t; k < p.nCons; k += T) storeImpulsesOne(w, cv, k);
+    for (int b = t; b < nb; b += T) {
+        if (islandBody(w, b)) {
+            integratePositionOne(wl, b, p.h);
+            w.vel[b] = rows[b];
+        }
+        rows[b] = w.pos[b];
+    }
+    wl = w;
+    wl.pos = rows;
+    // Position iterations: contacts, then joints (b2Island.cpp:310-328), each
+    // skipped for islands the previous pass left solved.
+    PosRow prow[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = t + r * T;
+        if (k >= p.nCons) continue;
+        prow[r].bodies = row[r].bodies;
+        prow[r].info = row[r].info;
+        prow[r].mass = row[r].mass;
+        prow[r].island = cv.island[k];
+        prow[r].lc = cv.lc[k];
+        prow[r].lp = cv.lp[k];
+        prow[r].lnp = cv.lnp[k];
+        prow[r].rad = cv.rad[k];
+    }
+    __syncthreads();
+    for (int it = 0; it < p.posIters; ++it) {
+        float lowest = 0.0f;
+        bool done[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+            done[r] = t + r * T < p.nCons && it > 0 && w.islandMinSep[(it - 1) * nb + prow[r].island] == 0;
+        colours(
+            [&](int r) {
+                if (done[r]) return;
+                float4 pA = rows[prow[r].bodies.x], pB = rows[prow[r].bodies.y];
+                const float minSep = solvePositionRow(prow[r], pA, pB);
+                keep(prow[r].info, prow[r].bodies, pA, pB);
+                failIsland(w, prow[r].island, it, minSep);
+                lowest = fminB(lowest, minSep);
+            },
+            [&](int k) { lowest = fminB(lowest, solvePositionStep(wl, cv, k, it)); });
+        recordMinSep(cnt, it, 0, lowest);
+        jointColours([&](int j) { jointSolvePositionOne(wl, jv, j, it); });
+    }
+    for (int b = t; b < nb; b += T)
+        if (islandBody(w, b)) {
+            w.pos[b] = rows[b];
+            syncTransformOne(w, b);
+        }
 }
 
 // Sleep (b2Island::Solve, REF/Dynamics/b2Island.cpp:345-382): per island,
@@ -6700,6 +6936,33 @@ int labelIslands(b2g_context* ctx, const WorldView& w) {
     return B2G_OK;
 }
 
+// Whether the step's solve goes to the block solve (k_solve_block): the bodies
+// fit its LDS rows, the constraints its reach, no colour is the overflow one,
+// and nothing has to look in between the passes (residual check, trace, log)
+// or asks for another way of running them (captured, clustered, one-launch or
+// per-colour solve: tailColours 0). Settled piles, a step per colour against
+// the block solve: 433 constraints 357 -> 297 us, 2868 463 -> 401 us, 6010
+// 624 -> 521 us, 8145 672 -> 600 us; beyond its registers the one compute
+// unit is left behind by the whole chip somewhere above that. With joints,
+// whose passes read memory: 1558 constraints and 620 joints 597 -> 501 us,
+// 3607 703 -> 643 us, but 4831 689 -> 718 us.
+bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, const int* colourStart, int nCons) {
+    if (ctx->nBodies > kBlockBodies || nCons == 0 || nCons > kBlockConstraints) return false;
+    if (colourStart[kOverflowColour + 1] > colourStart[kOverflowColour]) return false;
+    if (ctx->nJoints > 0) {
+        if (nCons > kBlockJointed || ctx->nJoints > kBlockJointed) return false;
+        if (ctx->jointColourStart[kOverflowColour + 1] > ctx->jointColourStart[kOverflowColour]) return false;
+    }
+    if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->graphs) return false;
+    if (ctx->traceIters > 0 || ctx->logCap > 0) return false;
+    return !(p->learnedWarmStart && p->residualThreshold > 0.0f);
+}
+
+int blockSolveLanes(const b2g_context* ctx, int nCons) {
+    const int rows = ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>;
+    return 256 * rows < nCons ? kBlockLanes : 256;
+}
+
 // First half of a coloured step: counters, pending broad-phase, and the
 // narrowphase over the contact table (b2ContactManager::Collide's Update of
 // every contact, REF/Dynamics/b2ContactManager.cpp:107-175). The table still
@@ -6941,10 +7204,18 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const bool wantFresh = nCons > 0 && (learned || ctx->logCap > 0 || ctx->traceIters > 0);
         if (wantFresh && (rc = ensureFresh(ctx)) != B2G_OK) return rc;
         const FreshView fv{wantFresh ? ctx->freshMask : nullptr, ctx->freshNum, ctx->freshAll, ctx->learnedScope};
-        int pe = profStart(ctx);
-        hipLaunchKernelGGL(k_integrate_velocities, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w, ctx->gravity, dt);
-        profEnd(ctx, PH_INTEGRATE_V, pe);
-        if (nCons > 0) {
+        const bool block = !clustered && blockSolveFits(ctx, p, colourStart, nCons);
+        const int blockLanes = block ? blockSolveLanes(ctx, nCons) : 0;
+        const bool blockInit = block && !wantFresh &&
+                               nCons <= blockLanes * (ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>);
+        int pe = -1;
+        if (!blockInit) {
+            pe = profStart(ctx);
+            hipLaunchKernelGGL(k_integrate_velocities, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w, ctx->gravity,
+                               dt);
+            profEnd(ctx, PH_INTEGRATE_V, pe);
+        }
+        if (nCons > 0 && !blockInit) {
             pe = profStart(ctx);
             hipLaunchKernelGGL(k_init_constraints, dim3(blocks(nCons)), dim3(256), 0, s, w, ctx->cv, ctx->consOrder,
                                nCons, dtRatio, ctx->warmStarting ? 1 : 0, ctx->cnt, fv);
@@ -7101,7 +7372,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         // and the position passes (the residual fallback, the impulse log).
         const bool persist = ctx->sched.persistentSolve > 0 && !clusterLaunch && ctx->traceIters == 0 &&
                              (nCons > 0 || ctx->nJoints > 0);
-        auto persistentLaunch = [&](int stages, bool contactWarm) -> int {
+        auto solvePlan = [&](int stages, bool contactWarm) {
             SolvePlan plan;
             memset(&plan, 0, sizeof(plan));
             memcpy(plan.cs, colourStart, sizeof(plan.cs));
@@ -7119,6 +7390,10 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             plan.velIters = p->velocityIterations;
             plan.posIters = posIters;
             plan.nCons = nCons;
+            return plan;
+        };
+        auto persistentLaunch = [&](int stages, bool contactWarm) -> int {
+            SolvePlan plan = solvePlan(stages, contactWarm);
             int nb = 0;
             const int pb = ctx->nJoints > 0 ? std::min(sb, kPersistJointBlock) : sb;
             const int brc = persistentBlocks(ctx, pb, &nb);
@@ -7172,7 +7447,14 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         // passes, the one-launch solve runs them all in one launch below.
         const bool velocityDeferred = persist && !checkResidual && ctx->logCap == 0;
         const bool contactWarm = nCons > 0 && (ctx->warmStarting || usePrediction);
-        if (!persist) {
+        if (block) {
+            BlockPlan plan{solvePlan(SP_WARM | SP_VELOCITY | SP_POSITION, contactWarm), ctx->gravity, blockInit ? 1 : 0};
+            pe = profStart(ctx);
+            hipLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(blockLanes),
+                               sizeof(float4) * (size_t)ctx->nBodies, s, w, ctx->cv, jv, (const int*)ctx->consOrder, plan,
+                               ctx->cnt);
+            profEnd(ctx, PH_SOLVE_V, pe);
+        } else if (!persist) {
             startSolve(contactWarm);
             solveVelocity(p->velocityIterations);
         } else if (!velocityDeferred && (rc = persistentLaunch(SP_WARM | SP_VELOCITY, contactWarm)) != B2G_OK) {
@@ -7208,7 +7490,9 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             LAUNCHCHK(ctx);
             ctx->logCount = std::min(ctx->logCap, ctx->logCount + nFresh);
         }
-        if (persist) {
+        if (block) {
+            // done in the one launch
+        } else if (persist) {
             // store, integrate, position passes and transforms (and the
             // velocity passes when deferred) in one launch
             const int stages = SP_POSITION | (velocityDeferred ? SP_WARM | SP_VELOCITY : 0);
@@ -7262,7 +7546,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         }  // !persist
         }  // !graphRan
         pe = profStart(ctx);
-        if (!graphRan && !persist) hipLaunchKernelGGL(k_sync_transforms, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w);
+        if (!graphRan && !persist && !block) hipLaunchKernelGGL(k_sync_transforms, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w);
         if (ctx->allowSleep) {
             hipLaunchKernelGGL(k_sleep_accum, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w, dt);
         }
