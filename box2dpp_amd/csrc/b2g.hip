@@ -71,6 +71,8 @@ struct Counters {
     int nQueries;          // moved proxies binned in the grid (their queries)
     int nTiles;            // polygon-polygon contacts deferred to k_collide_tiles
     int nScanned;          // grid entries and wide proxies the queries examined
+    int colourRounds;      // colouring rounds of a small world's step
+    int smallPending;      // a small world's new pairs are left to the host
     int roundLeft[kColourRoundSlots];  // constraints left uncoloured by colouring round r of the step
     int beginEvents;
     int endEvents;
@@ -593,19 +595,21 @@ __global__ void k_island_hook(WorldView w, int* changed) {
     if (changed) *changed = 1;
 }
 
+// Island contacts and joints join islands only between non-static, active bodies.
+__device__ inline bool joinsIslands(const WorldView& w, int bA, int bB) {
+    return w.btype[bA] != BT_STATIC && w.btype[bB] != BT_STATIC && (w.bflags[bA] & BF_ACTIVE) &&
+           (w.bflags[bB] & BF_ACTIVE);
+}
+
 __global__ void k_island_union(WorldView w) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= w.nContacts || !islandContact(w, c)) return;
     const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
-    if (w.btype[bA] == BT_STATIC || w.btype[bB] == BT_STATIC) return;
-    if (!(w.bflags[bA] & BF_ACTIVE) || !(w.bflags[bB] & BF_ACTIVE)) return;
-    islandUnion(w.islandOf, bA, bB);
+    if (joinsIslands(w, bA, bB)) islandUnion(w.islandOf, bA, bB);
 }
 
 // Chains only lead to smaller indices, so a chain ends within nBodies hops.
-__global__ void k_island_jump(WorldView w) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies) return;
+__device__ inline void islandJumpOne(const WorldView& w, int b) {
     int l = w.islandOf[b];
     for (;;) {
         const int n = w.islandOf[l];
@@ -615,17 +619,23 @@ __global__ void k_island_jump(WorldView w) {
     if (l != w.islandOf[b]) w.islandOf[b] = l;
 }
 
-__global__ void k_island_roots(WorldView w) {
+__global__ void k_island_jump(WorldView w) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies) return;
+    if (b < w.nBodies) islandJumpOne(w, b);
+}
+
+__device__ inline void islandRootOne(const WorldView& w, int b) {
     if (w.btype[b] != BT_STATIC && (w.bflags[b] & BF_ACTIVE) && (w.bflags[b] & BF_AWAKE))
         w.islandAwake[w.islandOf[b]] = 1;
 }
 
-// Bodies of awake islands are woken and take part in this step's solve.
-__global__ void k_island_mark(WorldView w) {
+__global__ void k_island_roots(WorldView w) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies) return;
+    if (b < w.nBodies) islandRootOne(w, b);
+}
+
+// Bodies of awake islands are woken and take part in this step's solve.
+__device__ inline void islandMarkOne(const WorldView& w, int b) {
     int flags = w.bflags[b] & ~BF_ISLAND;
     if (w.btype[b] != BT_STATIC && (flags & BF_ACTIVE) && w.islandAwake[w.islandOf[b]]) {
         if ((flags & BF_AWAKE) == 0) w.gsleep[b].y = 0.0f;
@@ -634,13 +644,15 @@ __global__ void k_island_mark(WorldView w) {
     w.bflags[b] = flags;
 }
 
+__global__ void k_island_mark(WorldView w) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < w.nBodies) islandMarkOne(w, b);
+}
+
 // Constraint set of the step: island contacts of awake islands. Contacts
 // leaving the set give their colour back.
-__global__ void k_mark_constraints(WorldView w, Counters* cnt) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts) return;
+__device__ inline void markConstraintOne(const WorldView& w, Counters* cnt, int c, int bA, int bB) {
     int flags = w.cflags[c] & ~CF_CONSTRAINT;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
     const bool isCons = islandContact(w, c) && ((w.bflags[bA] & BF_ISLAND) || (w.bflags[bB] & BF_ISLAND));
     if (!isCons) releaseColour(w, c, bA, bB);
     if (isCons) {
@@ -648,6 +660,11 @@ __global__ void k_mark_constraints(WorldView w, Counters* cnt) {
         if (w.ccolour[c] < 0) atomicAdd(&cnt->remaining, 1);
     }
     w.cflags[c] = flags;
+}
+
+__global__ void k_mark_constraints(WorldView w, Counters* cnt) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < w.nContacts) markConstraintOne(w, cnt, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
 }
 
 struct ContactArrays {
@@ -689,16 +706,19 @@ __global__ void k_fill(T* p, int n, T v) {
 // Open-addressing set of live contact pair keys (the existence test of
 // b2ContactManager::AddPair, REF/Dynamics/b2ContactManager.cpp:196-221).
 // live: the contact count when the host holds only a bound (w.nContacts).
-__global__ void k_hash_insert(WorldView w, unsigned long long* table, uint32_t mask, const Counters* live) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts || (live && c >= live->nContacts)) return;
-    const unsigned long long key = pairKey(w.cfA[c], w.cfB[c]);
+__device__ inline void hashInsert(unsigned long long* table, uint32_t mask, unsigned long long key) {
     uint32_t h = hashU64(key) & mask;
     for (;;) {
         const unsigned long long prev = atomicCAS(&table[h], ~0ull, key);
         if (prev == ~0ull || prev == key) return;
         h = (h + 1) & mask;
     }
+}
+
+__global__ void k_hash_insert(WorldView w, unsigned long long* table, uint32_t mask, const Counters* live) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= w.nContacts || (live && c >= live->nContacts)) return;
+    hashInsert(table, mask, pairKey(w.cfA[c], w.cfB[c]));
 }
 
 // ====================================================================
@@ -715,40 +735,49 @@ __device__ inline unsigned long long claimValue(uint32_t tag, const WorldView& w
 }
 
 // Also clears the count of losers that k_colour_commit then takes.
-__global__ void k_colour_claim(WorldView w, unsigned long long* claim, uint32_t tag, Counters* cnt, int round) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c == 0) cnt->roundLeft[round] = 0;
-    if (c >= w.nContacts) return;
-    if (!(w.cflags[c] & CF_CONSTRAINT) || w.ccolour[c] >= 0) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
+__device__ inline bool uncoloured(const WorldView& w, int c) {
+    return (w.cflags[c] & CF_CONSTRAINT) && w.ccolour[c] < 0;
+}
+
+__device__ inline void colourClaimOne(const WorldView& w, unsigned long long* claim, uint32_t tag, int c, int bA,
+                                      int bB) {
     const unsigned long long v = claimValue(tag, w, c);
     if (w.btype[bA] == BT_DYNAMIC) atomicMax(&claim[bA], v);
     if (w.btype[bB] == BT_DYNAMIC) atomicMax(&claim[bB], v);
 }
 
-__global__ void k_colour_commit(WorldView w, const unsigned long long* claim, uint32_t tag, Counters* cnt, int round) {
+__global__ void k_colour_claim(WorldView w, unsigned long long* claim, uint32_t tag, Counters* cnt, int round) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts) return;
-    if (!(w.cflags[c] & CF_CONSTRAINT) || w.ccolour[c] >= 0) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
+    if (c == 0) cnt->roundLeft[round] = 0;
+    if (c >= w.nContacts || !uncoloured(w, c)) return;
+    colourClaimOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
+}
+
+// False when the constraint stays uncoloured this round.
+__device__ inline bool colourCommitOne(const WorldView& w, const unsigned long long* claim, uint32_t tag, int c, int bA,
+                                       int bB) {
     const bool dA = w.btype[bA] == BT_DYNAMIC, dB = w.btype[bB] == BT_DYNAMIC;
     const unsigned long long v = claimValue(tag, w, c);
     const bool won = (!dA || claim[bA] == v) && (!dB || claim[bB] == v);
-    if (!won) {
-        atomicAdd(&cnt->roundLeft[round], 1);
-        return;
-    }
+    if (!won) return false;
     const unsigned long long used = (dA ? w.colourMask[bA] : 0ull) | (dB ? w.colourMask[bB] : 0ull);
     const unsigned long long freeBits = ~used;
     if (freeBits == 0ull) {
         w.ccolour[c] = kOverflowColour;
-        return;
+        return true;
     }
     const int col = __ffsll((long long)freeBits) - 1;
     const unsigned long long bit = 1ull << col;
     if (dA) atomicOr(&w.colourMask[bA], bit);
     if (dB) atomicOr(&w.colourMask[bB], bit);
     w.ccolour[c] = col;
+    return true;
+}
+
+__global__ void k_colour_commit(WorldView w, const unsigned long long* claim, uint32_t tag, Counters* cnt, int round) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= w.nContacts || !uncoloured(w, c)) return;
+    if (!colourCommitOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]])) atomicAdd(&cnt->roundLeft[round], 1);
 }
 
 // Demotion: a constraint keeps its colour for its life, so when the
@@ -766,11 +795,9 @@ __device__ inline unsigned long long demotionBits(const WorldView& w, int c, int
     return ~used & below;
 }
 
-__global__ void k_demote_claim(WorldView w, unsigned long long* claim, uint32_t tag) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts) return;
+__device__ inline void demoteClaimOne(const WorldView& w, unsigned long long* claim, uint32_t tag, int c, int bA,
+                                      int bB) {
     if (!(w.cflags[c] & CF_CONSTRAINT) || w.ccolour[c] <= 0) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
     const bool dA = w.btype[bA] == BT_DYNAMIC, dB = w.btype[bB] == BT_DYNAMIC;
     if (demotionBits(w, c, bA, bB, dA, dB) == 0ull) return;
     const unsigned long long v = claimValue(tag, w, c);
@@ -778,11 +805,14 @@ __global__ void k_demote_claim(WorldView w, unsigned long long* claim, uint32_t 
     if (dB) atomicMax(&claim[bB], v);
 }
 
-__global__ void k_demote_commit(WorldView w, const unsigned long long* claim, uint32_t tag) {
+__global__ void k_demote_claim(WorldView w, unsigned long long* claim, uint32_t tag) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts) return;
+    if (c < w.nContacts) demoteClaimOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
+}
+
+__device__ inline void demoteCommitOne(const WorldView& w, const unsigned long long* claim, uint32_t tag, int c, int bA,
+                                       int bB) {
     if (!(w.cflags[c] & CF_CONSTRAINT) || w.ccolour[c] <= 0) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
     const bool dA = w.btype[bA] == BT_DYNAMIC, dB = w.btype[bB] == BT_DYNAMIC;
     const unsigned long long v = claimValue(tag, w, c);
     if ((dA && claim[bA] != v) || (dB && claim[bB] != v)) return;
@@ -800,6 +830,11 @@ __global__ void k_demote_commit(WorldView w, const unsigned long long* claim, ui
         atomicOr(&w.colourMask[bB], bit);
     }
     w.ccolour[c] = to;
+}
+
+__global__ void k_demote_commit(WorldView w, const unsigned long long* claim, uint32_t tag) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < w.nContacts) demoteCommitOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
 }
 
 // Order key of every contact: a constraint's colour; contacts outside the
@@ -3553,14 +3588,14 @@ __global__ void k_joint_solve_position_serial(WorldView w, JointView jv, int beg
 }
 
 // Island union through joints whose bodies are both non-static and active.
+__device__ inline void islandUnionJoint(const WorldView& w, const JointView& jv, int j) {
+    const int2 b = jv.bodies[j];
+    if (!(jv.flags[j] & JF_REMOVED) && joinsIslands(w, b.x, b.y)) islandUnion(w.islandOf, b.x, b.y);
+}
+
 __global__ void k_island_union_joints(WorldView w, JointView jv) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= jv.n) return;
-    const int2 b = jv.bodies[j];
-    if (jv.flags[j] & JF_REMOVED) return;
-    if (w.btype[b.x] == BT_STATIC || w.btype[b.y] == BT_STATIC) return;
-    if (!(w.bflags[b.x] & BF_ACTIVE) || !(w.bflags[b.y] & BF_ACTIVE)) return;
-    islandUnion(w.islandOf, b.x, b.y);
+    if (j < jv.n) islandUnionJoint(w, jv, j);
 }
 
 // Position error of each joint, |cB + rB - cA - rA| as
@@ -3810,15 +3845,16 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
 // colour's constraints lie on neighbouring lanes and a wavefront without any
 // of them passes it over. Each constraint goes through the per-colour
 // kernels' functions in the same order of colours, so the results are theirs
-// bit for bit. The overflow colour, whose constraints share bodies, is left
-// to the per-colour kernels (blockSolveFits). What bounds it is one
+// bit for bit. The overflow colour, whose constraints share bodies, goes to
+// one lane in order. The colour ranges come from the order's device counts.
+// What bounds it is one
 // wavefront's arithmetic: a colour's velocity pass is some 300 instructions,
 // of which a wavefront issues one in four cycles. The solve of a 210-box
 // pyramid (400 constraints, 5 colours, 8/3 iterations) takes 75 us, that of a
 // 1493-body pile (2650 constraints, 7 colours) 153 us, in place of 16
 // launches with 110 and 210 us of kernel time.
 // ====================================================================
-constexpr int kBlockBodies = 4096;       // body rows in LDS: 64 KB
+constexpr int kBlockBodies = 4032;       // body rows in LDS: 63 of the 64 KB a launch may ask for
 constexpr int kBlockConstraints = 8192;  // most constraints (blockSolveFits)
 constexpr int kBlockJointed = 4096;      // most constraints, and most joints, with joints
 constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane, whose rows take most of them
@@ -3826,66 +3862,99 @@ template <bool kJoints>
 constexpr int kBlockRows = kJoints ? 3 : 4;  // constraint rows a lane holds
 
 struct BlockPlan {
-    SolvePlan solve;
+    int js[kColourSlots + 1];  // joint colour c holds order slots [js[c], js[c + 1])
     V2 gravity;
-    int initHere;   // integrate the velocities and set up the constraints, too
+    float h, dtRatio;
+    int velIters, posIters;
+    int contactWarm, warm;     // warm start the contacts; the world's warm starting flag
+    int initHere;              // integrate the velocities and set up the constraints, too
 };
 
 template <bool kJoints>
 __global__ void __launch_bounds__(kBlockLanes)
     k_solve_block(WorldView w, ConView cv, JointView jv, const int* order, BlockPlan plan, Counters* cnt) {
     extern __shared__ float4 rows[];  // velocities, then positions, of the bodies
-    constexpr int R = kBlockRows<kJoints>;
-    const SolvePlan& p = plan.solve;
+    __shared__ int cs[kColourSlots + 1];  // colour c holds constraints [cs[c], cs[c + 1])
+    const BlockPlan& p = plan;
     const int t = threadIdx.x, T = blockDim.x;
+    if (t < 64) {
+        int sum = cnt->colourCount[t];
+        for (int o = 1; o < 64; o <<= 1) {
+            const int before = __shfl_up(sum, o);
+            if (t >= o) sum += before;
+        }
+        cs[t + 1] = sum;
+        if (t == 0) cs[0] = 0;
+        if (t == 63) cs[kColourSlots] = sum + cnt->colourCount[kOverflowColour];
+    }
     const int nb = w.nBodies;
     WorldView wl = w;  // the bodies' rows in LDS for the functions that take a world
     wl.vel = rows;
 
     for (int b = t; b < nb; b += T) {
         rows[b] = w.vel[b];
-        if (plan.initHere && islandBody(w, b)) integrateVelocityOne(wl, b, plan.gravity, p.h);
+        if (p.initHere && islandBody(w, b)) integrateVelocityOne(wl, b, p.gravity, p.h);
     }
     __syncthreads();
+    const int nCons = cs[kColourSlots];
+    // With an overflow colour every row stays in memory, where its one lane
+    // finds them in order; else constraints [0, held) are in registers.
+    const bool overflow = nCons > cs[kOverflowColour];
+    const int held = overflow ? 0 : min(nCons, kBlockRows<kJoints> * T);
+    constexpr int R = kBlockRows<kJoints>;
 
-    // The rows: set up here (every constraint then has a register row) or read.
+    // The rows: set up here or read.
+    if (p.initHere)
+        for (int k = held + t; k < nCons; k += T)
+            countPoints(cnt, initConstraintOne(wl, cv, k, order[k], p.dtRatio, p.warm, FreshView{}));
     VelRow row[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int k = t + r * T;
         row[r].info = 0;
         int pc = 0;
-        if (k < p.nCons) {
-            if (plan.initHere)
-                pc = initConstraintRow(wl, cv, k, order[k], p.dtRatio, p.jointWarm, FreshView{}, row[r]);
+        if (k < held) {
+            if (p.initHere)
+                pc = initConstraintRow(wl, cv, k, order[k], p.dtRatio, p.warm, FreshView{}, row[r]);
             else
                 row[r] = loadVelRow(cv, k);
         }
-        if (plan.initHere) countPoints(cnt, pc);
+        if (p.initHere) countPoints(cnt, pc);
     }
-    if (plan.initHere) __syncthreads();  // the set-up reads the velocities that the warm start changes
+    if (p.initHere) __syncthreads();  // the set-up reads the velocities that the warm start changes
 
     // reg(row) over the constraints in registers, mem(k) over the others,
     // colour after colour.
     auto colours = [&](auto reg, auto mem) {
-        for (int c = 0; c < p.nColours; ++c) {
-            const int b0 = p.cs[c], b1 = p.cs[c + 1];
+        for (int c = 0; c < kColourSlots && cs[c] < nCons; ++c) {
+            const int b0 = cs[c], b1 = cs[c + 1];
             if (b1 <= b0) continue;
+            if (c == kOverflowColour) {
+                if (t == 0)
+                    for (int k = b0; k < b1; ++k) mem(k);
+                __syncthreads();
+                continue;
+            }
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int k = t + r * T;
-                if (k >= b0 && k < b1) reg(r);
+                if (k >= b0 && k < min(b1, held)) reg(r);
             }
-            for (int k = max(b0, R * T) + t; k < b1; k += T) mem(k);
+            for (int k = max(b0, held) + t; k < b1; k += T) mem(k);
             __syncthreads();
         }
     };
     auto jointColours = [&](auto one) {
         if (!kJoints) return;
-        for (int c = 0; c < p.nJointColours; ++c) {
+        for (int c = 0; c < kColourSlots; ++c) {
             const int b0 = p.js[c], b1 = p.js[c + 1];
             if (b1 <= b0) continue;
-            for (int k = b0 + t; k < b1; k += T) one(jv.order[k]);
+            if (c == kOverflowColour) {
+                if (t == 0)
+                    for (int k = b0; k < b1; ++k) one(jv.order[k]);
+            } else {
+                for (int k = b0 + t; k < b1; k += T) one(jv.order[k]);
+            }
             __syncthreads();
         }
     };
@@ -3902,7 +3971,7 @@ __global__ void __launch_bounds__(kBlockLanes)
                 keep(row[r].info, row[r].bodies, va, vb);
             },
             [&](int k) { warmStartOne(wl, cv, k); });
-    jointColours([&](int j) { jointInitOne(wl, jv, j, p.dtRatio, p.jointWarm); });
+    jointColours([&](int j) { jointInitOne(wl, jv, j, p.dtRatio, p.warm); });
     for (int it = 0; it < p.velIters; ++it) {
         jointColours([&](int j) { jointSolveVelocityOne(wl, jv, j, p.h); });
         colours(
@@ -3918,9 +3987,9 @@ __global__ void __launch_bounds__(kBlockLanes)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int k = t + r * T;
-        if (k < p.nCons) storeImpulsesTo(w, cv.contact[k], row[r].info & 3, row[r].imp);
+        if (k < held) storeImpulsesTo(w, cv.contact[k], row[r].info & 3, row[r].imp);
     }
-    for (int k = R * T + t; k < p.nCons; k += T) storeImpulsesOne(w, cv, k);
+    for (int k = held + t; k < nCons; k += T) storeImpulsesOne(w, cv, k);
     for (int b = t; b < nb; b += T) {
         if (islandBody(w, b)) {
             integratePositionOne(wl, b, p.h);
@@ -3936,7 +4005,7 @@ __global__ void __launch_bounds__(kBlockLanes)
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int k = t + r * T;
-        if (k >= p.nCons) continue;
+        if (k >= held) continue;
         prow[r].bodies = row[r].bodies;
         prow[r].info = row[r].info;
         prow[r].mass = row[r].mass;
@@ -3952,7 +4021,7 @@ __global__ void __launch_bounds__(kBlockLanes)
         bool done[R];
 #pragma unroll
         for (int r = 0; r < R; ++r)
-            done[r] = t + r * T < p.nCons && it > 0 && w.islandMinSep[(it - 1) * nb + prow[r].island] == 0;
+            done[r] = t + r * T < held && it > 0 && w.islandMinSep[(it - 1) * nb + prow[r].island] == 0;
         colours(
             [&](int r) {
                 if (done[r]) return;
@@ -3977,9 +4046,8 @@ __global__ void __launch_bounds__(kBlockLanes)
 // the minimum over its bodies of the time spent below the sleep tolerances;
 // an island that has rested for b2_timeToSleep and whose positions were
 // solved goes to sleep as a whole.
-__global__ void k_sleep_accum(WorldView w, float h) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies || !islandBody(w, b)) return;
+__device__ inline void sleepAccumOne(const WorldView& w, int b, float h) {
+    if (!islandBody(w, b)) return;
     const float4 v = w.vel[b];
     const float linTolSqr = kLinearSleepTol * kLinearSleepTol;
     const float angTolSqr = kAngularSleepTol * kAngularSleepTol;
@@ -3996,6 +4064,11 @@ __global__ void k_sleep_accum(WorldView w, float h) {
     }
 }
 
+__global__ void k_sleep_accum(WorldView w, float h) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < w.nBodies) sleepAccumOne(w, b, h);
+}
+
 // Static bodies reached by the island search (REF/Dynamics/b2World.cpp:
 // 451-529): the search wakes every body it adds, static ones included
 // (without searching on from them), and an island that falls asleep puts all
@@ -4007,8 +4080,8 @@ __global__ void k_sleep_accum(WorldView w, float h) {
 // wavefront when the wavefront's bodies share an island); staticKey the
 // minimum over the solved islands reaching a static body of
 // (largest index << 1) | (island stays awake).
-__global__ void k_island_max(WorldView w, int* islandMax) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+// Called by whole wavefronts with consecutive bodies.
+__device__ inline void islandMaxOne(const WorldView& w, int* islandMax, int b) {
     const bool valid = b < w.nBodies && islandBody(w, b);
     const int root = valid ? w.islandOf[b] : -1;
     const int r0 = __shfl(root, 0);
@@ -4021,6 +4094,10 @@ __global__ void k_island_max(WorldView w, int* islandMax) {
     if (valid) atomicMax(&islandMax[root], b);
 }
 
+__global__ void k_island_max(WorldView w, int* islandMax) {
+    islandMaxOne(w, islandMax, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
 __device__ inline int staticReachKey(const WorldView& w, const int* islandMax, int root, int allowSleep,
                                      int posIters) {
     bool solved = false;
@@ -4030,20 +4107,24 @@ __device__ inline int staticReachKey(const WorldView& w, const int* islandMax, i
     return (islandMax[root] << 1) | (slept ? 0 : 1);
 }
 
-__global__ void k_static_reach(WorldView w, const int* islandMax, int* staticKey, int allowSleep, int posIters) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts || !(w.cflags[c] & CF_CONSTRAINT)) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
+__device__ inline void staticReachOne(const WorldView& w, const int* islandMax, int* staticKey, int c, int bA, int bB,
+                                      int allowSleep, int posIters) {
+    if (!(w.cflags[c] & CF_CONSTRAINT)) return;
     const bool sA = w.btype[bA] == BT_STATIC, sB = w.btype[bB] == BT_STATIC;
     if (sA == sB) return;
     const int st = sA ? bA : bB, dyn = sA ? bB : bA;
     atomicMin(&staticKey[st], staticReachKey(w, islandMax, w.islandOf[dyn], allowSleep, posIters));
 }
 
-__global__ void k_static_reach_joints(WorldView w, JointView jv, const int* islandMax, int* staticKey,
-                                      int allowSleep, int posIters) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= jv.n || (jv.flags[j] & JF_REMOVED)) return;
+__global__ void k_static_reach(WorldView w, const int* islandMax, int* staticKey, int allowSleep, int posIters) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c < w.nContacts)
+        staticReachOne(w, islandMax, staticKey, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]], allowSleep, posIters);
+}
+
+__device__ inline void staticReachJoint(const WorldView& w, const JointView& jv, const int* islandMax, int* staticKey,
+                                        int j, int allowSleep, int posIters) {
+    if (jv.flags[j] & JF_REMOVED) return;
     const int2 b = jv.bodies[j];
     if (!jointActive(w, b)) return;
     const bool sA = w.btype[b.x] == BT_STATIC, sB = w.btype[b.y] == BT_STATIC;
@@ -4053,10 +4134,14 @@ __global__ void k_static_reach_joints(WorldView w, JointView jv, const int* isla
     atomicMin(&staticKey[st], staticReachKey(w, islandMax, w.islandOf[dyn], allowSleep, posIters));
 }
 
+__global__ void k_static_reach_joints(WorldView w, JointView jv, const int* islandMax, int* staticKey,
+                                      int allowSleep, int posIters) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < jv.n) staticReachJoint(w, jv, islandMax, staticKey, j, allowSleep, posIters);
+}
+
 // b2Body::SetAwake (REF/Dynamics/b2Body.h:635-654) on the reached static bodies.
-__global__ void k_static_apply(WorldView w, int* staticKey) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies) return;
+__device__ inline void staticApplyOne(const WorldView& w, int* staticKey, int b) {
     const int key = staticKey[b];
     if (key == 0x7FFFFFFF) return;
     staticKey[b] = 0x7FFFFFFF;
@@ -4073,9 +4158,13 @@ __global__ void k_static_apply(WorldView w, int* staticKey) {
     }
 }
 
-__global__ void k_sleep_apply(WorldView w, int posIters) {
+__global__ void k_static_apply(WorldView w, int* staticKey) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= w.nBodies || !islandBody(w, b)) return;
+    if (b < w.nBodies) staticApplyOne(w, staticKey, b);
+}
+
+__device__ inline void sleepApplyOne(const WorldView& w, int b, int posIters) {
+    if (!islandBody(w, b)) return;
     const int root = w.islandOf[b];
     bool solved = false;
     for (int it = 0; it < posIters; ++it)
@@ -4086,6 +4175,11 @@ __global__ void k_sleep_apply(WorldView w, int posIters) {
     w.gsleep[b].y = 0.0f;
     w.vel[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     w.force[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+}
+
+__global__ void k_sleep_apply(WorldView w, int posIters) {
+    const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < w.nBodies) sleepApplyOne(w, b, posIters);
 }
 
 __device__ inline float4 shapeAABB(const b2g_shape& s, const Xf& xf) {
@@ -4148,8 +4242,7 @@ __global__ void k_sync_fixtures(WorldView w) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
     if (f >= w.nFixtures) return;
     const int b = w.fbody[f];
-    if (!islandBody(w, b)) return;
-    syncFixtureOne(w, f, b);
+    if (islandBody(w, b)) syncFixtureOne(w, f, b);
 }
 
 // ====================================================================
@@ -4219,9 +4312,9 @@ __device__ inline uint32_t cellHash(int ix, int iy, int world) {
 }
 
 
-__global__ void k_grid_count(const float4* fat, const uint8_t* moved, int n, const uint8_t* hasProxy, GridView g,
-                             Counters* cnt) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+// Called by whole wavefronts (f >= n: no proxy).
+__device__ inline void gridCountOne(const float4* fat, const uint8_t* moved, int n, const uint8_t* hasProxy,
+                                    const GridView& g, Counters* cnt, int f) {
     bool query = false;
     if (f < n) {
         if (hasProxy && !hasProxy[f]) {
@@ -4252,9 +4345,12 @@ __global__ void k_grid_count(const float4* fat, const uint8_t* moved, int n, con
     if (query) g.queries[slot] = f;
 }
 
-__global__ void k_grid_scatter(int n, GridView g, const float4* fat, const uint8_t* moved) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= n) return;
+__global__ void k_grid_count(const float4* fat, const uint8_t* moved, int n, const uint8_t* hasProxy, GridView g,
+                             Counters* cnt) {
+    gridCountOne(fat, moved, n, hasProxy, g, cnt, blockIdx.x * blockDim.x + threadIdx.x);
+}
+
+__device__ inline void gridScatterOne(const GridView& g, const float4* fat, const uint8_t* moved, int f) {
     const int4 r = g.range[f];
     if (r.x > r.z) return;
     const int wf = proxyWorld(g, f);
@@ -4268,6 +4364,11 @@ __global__ void k_grid_scatter(int n, GridView g, const float4* fat, const uint8
             g.efat[e] = box;
             g.ecell[e] = cellKey(ix, iy, wf);
         }
+}
+
+__global__ void k_grid_scatter(int n, GridView g, const float4* fat, const uint8_t* moved) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f < n) gridScatterOne(g, fat, moved, f);
 }
 
 // Pair acceptance of b2ContactManager::AddPair (REF/Dynamics/b2ContactManager.cpp:179-230):
@@ -4426,10 +4527,9 @@ __global__ void k_count_scanned(int n, GridView g, Counters* cnt) {
 // per candidate proxy: the same pairs as the wide proxy testing every proxy
 // itself, under the same rule for two moved proxies (the lower id reports).
 // Removed proxies fail every overlap test.
-__global__ void k_pairs_wide(const float4* fat, const uint8_t* moved, int n, GridView g, WorldView w, bool world,
-                             const unsigned long long* table, uint32_t hmask, PairSink sink, Counters* cnt) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
+__device__ inline void wideOne(const float4* fat, const uint8_t* moved, const GridView& g, const WorldView& w,
+                               bool world, const unsigned long long* table, uint32_t hmask, const PairSink& sink,
+                               Counters* cnt, int p) {
     const int nBig = cnt->nBig;
     if (nBig == 0) return;
     const float4 fp = fat[p];
@@ -4447,6 +4547,12 @@ __global__ void k_pairs_wide(const float4* fat, const uint8_t* moved, int n, Gri
         if (world && !acceptPair(w, a, b, table, hmask)) continue;
         emitPair(sink, cnt, a, b);
     }
+}
+
+__global__ void k_pairs_wide(const float4* fat, const uint8_t* moved, int n, GridView g, WorldView w, bool world,
+                             const unsigned long long* table, uint32_t hmask, PairSink sink, Counters* cnt) {
+    const int p = blockIdx.x * blockDim.x + threadIdx.x;
+    if (p < n) wideOne(fat, moved, g, w, world, table, hmask, sink, cnt, p);
 }
 
 // New contacts from the sorted pair keys (b2Contact::Create with the
@@ -4487,6 +4593,327 @@ __global__ void k_append_contacts(WorldView w, const unsigned long long* keys, i
     if (k >= nNew) return;
     const unsigned long long key = keys[k];
     appendContactOne(w, fixtureOf(w, (int)(key / packBase)), fixtureOf(w, (int)(key % packBase)), base + k);
+}
+
+// ====================================================================
+// Small worlds: the stages of a coloured step around the narrowphase and the
+// block solve, each a loop of one workgroup, in four launches. One launch per
+// stage kept the host busy for 3 us a launch where the stage took the GPU
+// less (45 launches and two readbacks of a 210-box step): the step was as
+// long as its launches. The stages are those of the grid kernels, item by
+// item, so the results are theirs; what differs is that the labels always
+// come from the union-find pass (the same labels), that dead contacts leave
+// the table in place, and that nothing is read back before the end. At 590
+// contacts k_small_prepare takes 13 us and k_small_finish 15 us, at 4500
+// contacts 54 and 64 us: memory latency, a few loads deep per stage.
+// ====================================================================
+constexpr int kSmallLanes = 1024;
+constexpr int kSmallBodies = kBlockBodies;   // island labels in LDS
+constexpr int kSmallContacts = 5120;         // contact bodies in LDS (see smallWorldFits)
+constexpr int kSmallNewPairs = 4096;         // new pairs sorted in LDS
+constexpr int kSmallTags = 96;               // claim tags of a step
+static_assert(kSmallBodies <= 1 << 13, "a packed body index has 13 bits");
+static_assert(sizeof(b2g_manifold) == 4 * sizeof(float4), "a manifold moves as four words of 16 bytes");
+
+// Exclusive prefix of a per-lane value over the workgroup (whole wavefronts);
+// total receives the sum. `part` holds a word per wavefront.
+__device__ inline int blockPrefix(int v, int* part, int& total) {
+    const int lane = (int)__lane_id(), wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
+    int sum = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int before = __shfl_up(sum, o);
+        if (lane >= o) sum += before;
+    }
+    __syncthreads();  // part may still be read from the call before
+    if (lane == 63) part[wave] = sum;
+    __syncthreads();
+    int base = 0;
+    total = 0;
+    for (int i = 0; i < waves; ++i) {
+        if (i < wave) base += part[i];
+        total += part[i];
+    }
+    return base + sum - v;
+}
+
+// Dead contacts' colours, islands, constraint set, demotion, colouring and the
+// constraint order. Claims carry tags from tagBase on; a round past tagCount
+// clears the claims and starts over.
+__global__ void __launch_bounds__(kSmallLanes)
+    k_small_prepare(WorldView w, JointView jv, unsigned long long* claim, uint32_t tagBase, int tagCount,
+                    int demoteRounds, int posIters, int* order, Counters* cnt) {
+    __shared__ int label[kSmallBodies];
+    __shared__ uint32_t ends[kSmallContacts];  // bodies A, B of each contact, 13 bits each
+    __shared__ int hist[kSmallLanes / 64][kColourSlots];
+    __shared__ int next[kColourSlots];         // where the next constraint of a colour goes
+    __shared__ int left;
+    const int t = threadIdx.x, T = blockDim.x;
+    const int nb = w.nBodies, nc = w.nContacts;
+    WorldView wl = w;
+    wl.islandOf = label;
+    auto bodyA = [&](int c) { return (int)(ends[c] & 0x1FFFu); };
+    auto bodyB = [&](int c) { return (int)(ends[c] >> 13); };
+    for (int c = t; c < nc; c += T) {
+        const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
+        ends[c] = (uint32_t)bA | ((uint32_t)bB << 13);
+        if (w.cflags[c] & CF_DEAD) releaseColour(w, c, bA, bB);
+    }
+    for (int b = t; b < nb; b += T) {
+        label[b] = b;
+        w.islandAwake[b] = 0;
+        w.islandSleep[b] = 0;
+    }
+    for (int i = t; i < nb * posIters; i += T) w.islandMinSep[i] = 0;
+    __syncthreads();
+    for (int c = t; c < nc; c += T)
+        if (islandContact(w, c) && joinsIslands(w, bodyA(c), bodyB(c))) islandUnion(label, bodyA(c), bodyB(c));
+    for (int j = t; j < jv.n; j += T) islandUnionJoint(wl, jv, j);
+    __syncthreads();
+    for (int b = t; b < nb; b += T) islandJumpOne(wl, b);
+    __syncthreads();
+    for (int b = t; b < nb; b += T) {
+        w.islandOf[b] = label[b];
+        islandRootOne(wl, b);
+    }
+    __syncthreads();
+    for (int b = t; b < nb; b += T) islandMarkOne(wl, b);
+    __syncthreads();
+    for (int c = t; c < nc; c += T) markConstraintOne(w, cnt, c, bodyA(c), bodyB(c));
+    __syncthreads();
+    uint32_t used = 0;
+    auto nextTag = [&]() {
+        if ((int)used == tagCount) {
+            for (int b = t; b < nb; b += T) claim[b] = 0ull;
+            __syncthreads();
+            used = 0;
+        }
+        return tagBase + used++;
+    };
+    for (int r = 0; r < demoteRounds; ++r) {
+        const uint32_t tag = nextTag();
+        for (int c = t; c < nc; c += T) demoteClaimOne(w, claim, tag, c, bodyA(c), bodyB(c));
+        __syncthreads();
+        for (int c = t; c < nc; c += T) demoteCommitOne(w, claim, tag, c, bodyA(c), bodyB(c));
+        __syncthreads();
+    }
+    // Every round colours at least one constraint, so the rounds end.
+    for (int round = 0; nc > 0; ++round) {
+        const uint32_t tag = nextTag();
+        if (t == 0) left = 0;
+        for (int c = t; c < nc; c += T)
+            if (uncoloured(w, c)) colourClaimOne(w, claim, tag, c, bodyA(c), bodyB(c));
+        __syncthreads();
+        for (int c = t; c < nc; c += T)
+            if (uncoloured(w, c) && !colourCommitOne(w, claim, tag, c, bodyA(c), bodyB(c))) atomicAdd(&left, 1);
+        __syncthreads();
+        const int stay = left;
+        if (t == 0) {
+            cnt->roundLeft[min(round, kColourRoundSlots - 1)] = stay;
+            cnt->colourRounds = round + 1;
+        }
+        __syncthreads();
+        if (stay == 0) break;
+    }
+    // Constraints by colour, in table order within a colour: counts, then
+    // chunks of T contacts ranked by a ballot per colour bit and a count per
+    // wavefront.
+    const int lane = (int)__lane_id(), wave = t >> 6, waves = T >> 6;
+    for (int c = t; c < kColourSlots; c += T) next[c] = 0;
+    __syncthreads();
+    for (int c = t; c < nc; c += T)
+        if (w.cflags[c] & CF_CONSTRAINT) atomicAdd(&next[w.ccolour[c]], 1);
+    __syncthreads();
+    if (t < kColourSlots) cnt->colourCount[t] = next[t];
+    __syncthreads();
+    if (t == 0) {
+        int sum = 0;
+        for (int c = 0; c < kColourSlots; ++c) {
+            const int n = next[c];
+            next[c] = sum;
+            sum += n;
+        }
+    }
+    for (int c0 = 0; c0 < nc; c0 += T) {
+        const int c = c0 + t;
+        const bool in = c < nc && (w.cflags[c] & CF_CONSTRAINT);
+        const int col = in ? w.ccolour[c] : 0;
+        unsigned long long same = __ballot(in);
+        for (int bit = 0; bit < 7; ++bit) {
+            const unsigned long long ones = __ballot((col >> bit) & 1);
+            same &= ((col >> bit) & 1) ? ones : ~ones;
+        }
+        for (int i = t; i < waves * kColourSlots; i += T) (&hist[0][0])[i] = 0;
+        __syncthreads();
+        const int rank = __popcll(same & ((1ull << lane) - 1ull));
+        if (in && rank == 0) hist[wave][col] = __popcll(same);
+        __syncthreads();
+        if (t < kColourSlots) {
+            int sum = next[t];
+            for (int i = 0; i < waves; ++i) {
+                const int n = hist[i][t];
+                hist[i][t] = sum;
+                sum += n;
+            }
+            next[t] = sum;
+        }
+        __syncthreads();
+        if (in) order[hist[wave][col] + rank] = c;
+        __syncthreads();
+    }
+}
+
+struct SmallFinish {
+    float h;
+    int allowSleep, statics, posIters;   // statics: static bodies can change (see k_static_reach)
+    int *islandMax, *staticKey;
+    int *keep, *idx;
+    unsigned long long* table;
+    uint32_t hashMask;
+    int nBuckets;
+};
+
+// Sleep, fat boxes, the compaction of the contact table, the set of live pairs
+// and the broad-phase grid.
+__global__ void __launch_bounds__(kSmallLanes)
+    k_small_finish(WorldView w, JointView jv, ContactArrays ca, SmallFinish p, GridView g, Counters* cnt) {
+    __shared__ int part[kSmallLanes / 64];
+    const int t = threadIdx.x, T = blockDim.x;
+    const int nb = w.nBodies, nf = w.nFixtures, nc = w.nContacts;
+    // stages that touch the same rows only through the barriers between them
+    for (int i = t; i <= (int)p.hashMask; i += T) p.table[i] = ~0ull;
+    for (int i = t; i <= p.nBuckets; i += T) {
+        g.counts[i] = 0;
+        g.cursor[i] = 0;
+    }
+    if (t == 0) {
+        cnt->nBig = 0;
+        cnt->nQueries = 0;
+        cnt->nNewPairs = 0;
+        cnt->overflow = 0;
+    }
+    if (p.allowSleep)
+        for (int b = t; b < nb; b += T) sleepAccumOne(w, b, p.h);
+    if (p.statics) {
+        for (int b = t; b < nb; b += T) p.islandMax[b] = -1;
+        __syncthreads();
+        for (int b = t; b < ((nb + 63) & ~63); b += T) islandMaxOne(w, p.islandMax, b);
+        __syncthreads();
+        for (int c = t; c < nc; c += T)
+            staticReachOne(w, p.islandMax, p.staticKey, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]], p.allowSleep,
+                           p.posIters);
+        for (int j = t; j < jv.n; j += T)
+            staticReachJoint(w, jv, p.islandMax, p.staticKey, j, p.allowSleep, p.posIters);
+        __syncthreads();
+        for (int b = t; b < nb; b += T) staticApplyOne(w, p.staticKey, b);
+    }
+    if (p.allowSleep) {
+        __syncthreads();
+        for (int b = t; b < nb; b += T) sleepApplyOne(w, b, p.posIters);
+    }
+    for (int f = t; f < nf; f += T) {
+        const int b = w.fbody[f];
+        if (islandBody(w, b)) syncFixtureOne(w, f, b);
+    }
+    // A row only ever moves to an earlier place, and a chunk is read before it
+    // is written, so the table closes up in place; without dead contacts
+    // nothing moves.
+    int live = 0;
+    for (int c0 = 0; c0 < nc; c0 += T) {
+        const int c = c0 + t;
+        const bool keep = c < nc && !(w.cflags[c] & CF_DEAD);
+        int total;
+        const int d = live + blockPrefix(keep ? 1 : 0, part, total);
+        const bool move = keep && d != c;
+        int cfA = 0, cfB = 0, flags = 0, colour = 0, toiCount = 0;
+        float2 mat = make_float2(0.0f, 0.0f);
+        float tan = 0.0f, toi = 0.0f;
+        float4 m0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), m1 = m0, m2 = m0, m3 = m0;  // the manifold
+        if (move) {
+            const float4* m = (const float4*)&ca.cman[c];
+            m0 = m[0]; m1 = m[1]; m2 = m[2]; m3 = m[3];
+            cfA = ca.cfA[c]; cfB = ca.cfB[c]; flags = ca.cflags[c]; colour = ca.ccolour[c]; toiCount = ca.ctoiCount[c];
+            mat = ca.cmat[c]; tan = ca.ctan[c]; toi = ca.ctoi[c];
+        }
+        if (c < nc) {
+            p.keep[c] = keep ? 1 : 0;
+            p.idx[c] = d;
+        }
+        __syncthreads();
+        if (move) {
+            ca.cfA[d] = cfA; ca.cfB[d] = cfB; ca.cflags[d] = flags; ca.ccolour[d] = colour; ca.ctoiCount[d] = toiCount;
+            ca.cmat[d] = mat; ca.ctan[d] = tan; ca.ctoi[d] = toi;
+            float4* m = (float4*)&ca.cman[d];
+            m[0] = m0; m[1] = m1; m[2] = m2; m[3] = m3;
+        }
+        live += total;
+    }
+    if (t == 0) cnt->nContacts = live;
+    __syncthreads();
+    for (int c = t; c < live; c += T) hashInsert(p.table, p.hashMask, pairKey(w.cfA[c], w.cfB[c]));
+    for (int f = t; f < ((nf + 63) & ~63); f += T) gridCountOne(w.fat, w.moved, nf, nullptr, g, cnt, f);
+    __syncthreads();
+    int before = 0;
+    for (int i0 = 0; i0 <= p.nBuckets; i0 += T) {
+        const int i = i0 + t;
+        int total;
+        const int at = before + blockPrefix(i <= p.nBuckets ? g.counts[i] : 0, part, total);
+        if (i <= p.nBuckets) g.starts[i] = at;
+        before += total;
+    }
+    __syncthreads();
+    for (int f = t; f < nf; f += T) gridScatterOne(g, w.fat, w.moved, f);
+}
+
+// The queries of the moved proxies and the wide ones.
+__global__ void k_small_pairs(WorldView w, GridView g, const unsigned long long* table, uint32_t hmask, PairSink sink,
+                              Counters* cnt) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = t % kQueryLanes;
+    const int nq = min(cnt->nQueries, w.nFixtures);
+    const int lanes = (int)(gridDim.x * blockDim.x);
+    for (int i = t / kQueryLanes; i < nq; i += lanes / kQueryLanes)
+        queryOne(w.fat, w.moved, g, w, true, table, hmask, sink, cnt, i, lane);
+    for (int p = t; p < w.nFixtures; p += lanes) wideOne(w.fat, w.moved, g, w, true, table, hmask, sink, cnt, p);
+}
+
+// The new pairs in key order into the table (a bitonic sort in LDS), the move
+// flags and the forces cleared. Pairs that fit neither the sort nor the table
+// are left to the host (cnt->smallPending), with the move flags as they are.
+__global__ void __launch_bounds__(kSmallLanes)
+    k_small_append(WorldView w, const unsigned long long* newKeys, unsigned long long packBase, int capContacts,
+                   int clearForces, Counters* cnt) {
+    __shared__ unsigned long long keys[kSmallNewPairs];
+    const int t = threadIdx.x, T = blockDim.x;
+    const int n = cnt->nNewPairs, base = cnt->nContacts;
+    const bool fits = !cnt->overflow && n <= kSmallNewPairs && base + n <= capContacts;
+    if (t == 0) cnt->smallPending = fits ? 0 : 1;
+    if (!fits) return;
+    if (n > 0) {
+        int size = 1;
+        while (size < n) size <<= 1;
+        for (int i = t; i < size; i += T) keys[i] = i < n ? newKeys[i] : ~0ull;
+        __syncthreads();
+        for (int k = 2; k <= size; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                for (int i = t; i < size; i += T) {
+                    const int o = i ^ j;
+                    if (o > i) {
+                        const unsigned long long a = keys[i], b = keys[o];
+                        if ((a > b) == ((i & k) == 0)) {
+                            keys[i] = b;
+                            keys[o] = a;
+                        }
+                    }
+                }
+                __syncthreads();
+            }
+        for (int i = t; i < n; i += T)
+            appendContactOne(w, fixtureOf(w, (int)(keys[i] / packBase)), fixtureOf(w, (int)(keys[i] % packBase)),
+                             base + i);
+    }
+    for (int f = t; f < w.nFixtures; f += T) w.moved[f] = 0;
+    if (clearForces)
+        for (int b = t; b < w.nBodies; b += T) w.force[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
 
 // Contacts between bodies that a new joint keeps apart are flagged for
@@ -6235,6 +6662,21 @@ int readCounters(b2g_context* ctx);
 int profKernelEvents(b2g_context* ctx, hipEvent_t* start, hipEvent_t* stop);
 void profKernel(b2g_context* ctx, int phase, int i);
 
+GridView gridView(const b2g_context* ctx) {
+    GridView g;
+    g.invCell = 1.0f / ctx->cellSize;
+    g.bucketMask = (uint32_t)(ctx->nBuckets - 1);
+    g.counts = ctx->gCounts; g.starts = ctx->gStarts; g.cursor = ctx->gCursor; g.entries = ctx->gEntries;
+    g.ecell = ctx->gCell;
+    g.efat = ctx->gEfat;
+    g.queries = ctx->gQueries;
+    g.big = ctx->gBig; g.range = ctx->range;
+    g.bigSorted = 0;
+    g.fbody = ctx->fbody;
+    g.bworld = ctx->subWorlds ? ctx->bworld : nullptr;
+    return g;
+}
+
 // liveOnDevice: the contact table was compacted without a readback
 // (compactContacts); the query's readback brings the live count.
 int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
@@ -6251,17 +6693,7 @@ int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
         }
         return B2G_OK;
     }
-    GridView g;
-    g.invCell = 1.0f / ctx->cellSize;
-    g.bucketMask = (uint32_t)(ctx->nBuckets - 1);
-    g.counts = ctx->gCounts; g.starts = ctx->gStarts; g.cursor = ctx->gCursor; g.entries = ctx->gEntries;
-    g.ecell = ctx->gCell;
-    g.efat = ctx->gEfat;
-    g.queries = ctx->gQueries;
-    g.big = ctx->gBig; g.range = ctx->range;
-    g.bigSorted = 0;
-    g.fbody = ctx->fbody;
-    g.bworld = ctx->subWorlds ? ctx->bworld : nullptr;
+    GridView g = gridView(ctx);
     hipLaunchKernelGGL(k_grid_reset, dim3(blocks(ctx->nBuckets + 1)), dim3(256), 0, s, ctx->gCounts, ctx->gCursor,
                        ctx->nBuckets + 1, ctx->cnt);
     hipLaunchKernelGGL(k_grid_count, dim3(blocks(nf)), dim3(256), 0, s, ctx->fat, ctx->moved, nf,
@@ -6936,31 +7368,60 @@ int labelIslands(b2g_context* ctx, const WorldView& w) {
     return B2G_OK;
 }
 
-// Whether the step's solve goes to the block solve (k_solve_block): the bodies
-// fit its LDS rows, the constraints its reach, no colour is the overflow one,
-// and nothing has to look in between the passes (residual check, trace, log)
-// or asks for another way of running them (captured, clustered, one-launch or
+// Whether a step's solve goes to the block solve (k_solve_block): the bodies
+// fit its LDS rows and at most `constraints` constraints its reach, and
+// nothing has to look in between the passes (residual check, trace, log) or
+// asks for another way of running them (captured, clustered, one-launch or
 // per-colour solve: tailColours 0). Settled piles, a step per colour against
 // the block solve: 433 constraints 357 -> 297 us, 2868 463 -> 401 us, 6010
 // 624 -> 521 us, 8145 672 -> 600 us; beyond its registers the one compute
 // unit is left behind by the whole chip somewhere above that. With joints,
 // whose passes read memory: 1558 constraints and 620 joints 597 -> 501 us,
 // 3607 703 -> 643 us, but 4831 689 -> 718 us.
-bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, const int* colourStart, int nCons) {
-    if (ctx->nBodies > kBlockBodies || nCons == 0 || nCons > kBlockConstraints) return false;
-    if (colourStart[kOverflowColour + 1] > colourStart[kOverflowColour]) return false;
-    if (ctx->nJoints > 0) {
-        if (nCons > kBlockJointed || ctx->nJoints > kBlockJointed) return false;
-        if (ctx->jointColourStart[kOverflowColour + 1] > ctx->jointColourStart[kOverflowColour]) return false;
-    }
-    if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->graphs) return false;
+bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
+    if (ctx->nBodies > kBlockBodies || constraints > kBlockConstraints) return false;
+    if (ctx->nJoints > 0 && (constraints > kBlockJointed || ctx->nJoints > kBlockJointed)) return false;
+    if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->sched.clusterBodies > 0 || ctx->graphs)
+        return false;
     if (ctx->traceIters > 0 || ctx->logCap > 0) return false;
     return !(p->learnedWarmStart && p->residualThreshold > 0.0f);
 }
 
-int blockSolveLanes(const b2g_context* ctx, int nCons) {
+int blockSolveLanes(const b2g_context* ctx, int constraints) {
     const int rows = ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>;
-    return 256 * rows < nCons ? kBlockLanes : 256;
+    return 256 * rows < constraints ? kBlockLanes : 256;
+}
+
+void launchBlockSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView& w, const JointView& jv, int lanes,
+                      bool contactWarm, bool initHere) {
+    BlockPlan plan;
+    memset(&plan, 0, sizeof(plan));
+    if (ctx->nJoints > 0) memcpy(plan.js, ctx->jointColourStart.data(), sizeof(plan.js));
+    plan.gravity = ctx->gravity;
+    plan.h = p->dt;
+    plan.dtRatio = ctx->inv_dt0 * p->dt;
+    plan.velIters = p->velocityIterations;
+    plan.posIters = std::min(p->positionIterations, kMaxPosIters);
+    plan.contactWarm = contactWarm ? 1 : 0;
+    plan.warm = ctx->warmStarting ? 1 : 0;
+    plan.initHere = initHere ? 1 : 0;
+    hipLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(lanes),
+                       sizeof(float4) * (size_t)ctx->nBodies, ctx->stream, w, ctx->cv, jv, (const int*)ctx->consOrder,
+                       plan, ctx->cnt);
+}
+
+// Whether the whole step after the narrowphase goes to the small-world kernels:
+// the block solve takes it whatever share of the contacts are constraints, the
+// LDS tables hold the world, and no candidate point has to be gathered for the
+// network. With profiling on the step runs stage by stage, so that the phases
+// keep their times. One compute unit works through a stage where the grid
+// kernels have the whole chip, so the gain ends with the contacts: settled
+// worlds of 590 contacts 278 -> 129 us a step, 1700 (700-body pile)
+// 341 -> 232 us, 4500 401 -> 356 us, but 6600 457 -> 480 us.
+bool smallWorldFits(const b2g_context* ctx, const b2g_step_params* p) {
+    return blockSolveFits(ctx, p, ctx->nContacts) && ctx->nFixtures <= kSmallBodies && ctx->nFixtures > 0 &&
+           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && !ctx->profiling && ctx->demoteRounds < kSmallTags &&
+           (ctx->orderSpan == 0 || ctx->orderCount == ctx->nFixtures);
 }
 
 // First half of a coloured step: counters, pending broad-phase, and the
@@ -6978,16 +7439,11 @@ int stepColouredCollide(b2g_context* ctx, const b2g_step_params* p) {
     if ((rc = reserveContacts(ctx)) != B2G_OK) return rc;
     memset(&ctx->stats, 0, sizeof(ctx->stats));
     ctx->stats.residual = -1.0f;
-    // reset per-step counters
-    Counters zero;
-    memset(&zero, 0, sizeof(zero));
-    for (int i = 0; i < kMaxPosIters; ++i) {
-        float z = 0.0f;
-        int b;
-        memcpy(&b, &z, 4);
-        zero.minSep[i] = b;  // encodeOrdered(0.0f) == 0
-    }
-    HIPCHK(ctx, hipMemcpyAsync(ctx->cnt, &zero, sizeof(Counters), hipMemcpyHostToDevice, s));
+    // per-step counters (encodeOrdered(0.0f) == 0, so zero is every field's
+    // start); a copy from the host's stack would be staged and waited for
+    static_assert(sizeof(Counters) % sizeof(int) == 0, "counters are whole words");
+    const int words = (int)(sizeof(Counters) / sizeof(int));
+    hipLaunchKernelGGL(k_fill<int>, dim3(blocks(words)), dim3(256), 0, s, (int*)ctx->cnt, words, 0);
 
     if (ctx->newFixture) {
         if ((rc = rebuildHash(ctx)) != B2G_OK) return rc;
@@ -7033,6 +7489,133 @@ int stepColouredCollide(b2g_context* ctx, const b2g_step_params* p) {
     return B2G_OK;
 }
 
+// Colour counts of the step as the host keeps them: ranges, statistics.
+// tailBegin: the first of the trailing colours that share a launch.
+struct ColourLayout {
+    int start[kColourSlots + 1];
+    int nCons, nColours, tailBegin;
+};
+
+ColourLayout colourLayout(const int* counts, int first, int tailColours) {
+    ColourLayout l;
+    l.start[0] = first;
+    for (int c = 0; c < kColourSlots; ++c) l.start[c + 1] = l.start[c] + counts[c];
+    l.nCons = l.start[kColourSlots];
+    l.nColours = 0;
+    for (int c = 0; c < kColourSlots; ++c)
+        if (counts[c] > 0) l.nColours = c + 1;
+    l.tailBegin = l.nColours;
+    if (tailColours > 0) {
+        while (l.tailBegin > 0 && l.start[l.tailBegin] - l.start[l.tailBegin - 1] <= tailColours) --l.tailBegin;
+        if (l.nColours - l.tailBegin < 2) l.tailBegin = l.nColours;  // one colour: no gain
+    }
+    return l;
+}
+
+// Constraints in the colours that get a solver launch each.
+int wideConstraints(const ColourLayout& l) {
+    int n = 0;
+    for (int c = 0; c < l.tailBegin; ++c)
+        if (c != kOverflowColour) n += l.start[c + 1] - l.start[c];
+    return n;
+}
+
+// Statistics of the position iterations.
+void positionStats(b2g_context* ctx, int posIters, int nCons) {
+    int ran = 0;
+    float lastMin = 0.0f;
+    for (int it = 0; it < posIters && nCons > 0; ++it) {
+        ++ran;
+        lastMin = decodeOrdered(ctx->hcnt->minSep[it]);
+        if (lastMin >= -3.0f * kLinearSlop) break;
+    }
+    ctx->stats.positionIterations = ran;
+    ctx->stats.points = ctx->hcnt->points;
+    ctx->stats.minSeparation = lastMin;
+}
+
+// The second half of a small world's step in the small-world kernels and the
+// block solve, with one readback at its end.
+int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesCleared) {
+    hipStream_t s = ctx->stream;
+    const int posIters = std::min(p->positionIterations, kMaxPosIters);
+    int rc;
+    if (ctx->jointsDirty && (rc = recolourJoints(ctx)) != B2G_OK) return rc;
+    if (ctx->claimTag + kSmallTags >= 0xFFFF) {
+        hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, ctx->claim,
+                           ctx->nBodies, 0ull);
+        ctx->claimTag = 0;
+    }
+    const WorldView w = ctx->view();
+    JointView jv = ctx->jview();
+    jv.h = p->dt;
+    const int before = ctx->nContacts;
+    hipLaunchKernelGGL(k_small_prepare, dim3(1), dim3(kSmallLanes), 0, s, w, jv, ctx->claim, ctx->claimTag + 1,
+                       kSmallTags, ctx->nContacts > 0 ? ctx->demoteRounds : 0, posIters, ctx->consOrder, ctx->cnt);
+    ctx->claimTag += kSmallTags;
+    launchBlockSolve(ctx, p, w, jv, blockSolveLanes(ctx, ctx->nContacts), ctx->warmStarting, true);
+
+    SmallFinish fin;
+    fin.h = p->dt;
+    fin.allowSleep = ctx->allowSleep ? 1 : 0;
+    fin.statics = (ctx->nContacts > 0 || ctx->nJoints > 0) && (ctx->allowSleep || ctx->staticAsleep) ? 1 : 0;
+    fin.posIters = posIters;
+    fin.islandMax = ctx->islandMax;
+    fin.staticKey = ctx->staticKey;
+    fin.keep = ctx->keep;
+    fin.idx = ctx->idx;
+    fin.table = ctx->hashTable;
+    // the set of live pairs is rebuilt every step: half full at most here, its
+    // whole size where TOI events go on with it
+    fin.hashMask = 1023;
+    while ((int)fin.hashMask < 2 * ctx->nContacts) fin.hashMask = 2 * fin.hashMask + 1;
+    if (ctx->continuous || fin.hashMask > ctx->hashMask) fin.hashMask = ctx->hashMask;
+    fin.nBuckets = 256;
+    while (fin.nBuckets < 2 * ctx->nFixtures) fin.nBuckets *= 2;
+    fin.nBuckets = std::min(fin.nBuckets, ctx->nBuckets);
+    GridView g = gridView(ctx);
+    g.bucketMask = (uint32_t)(fin.nBuckets - 1);
+    hipLaunchKernelGGL(k_small_finish, dim3(1), dim3(kSmallLanes), 0, s, w, jv, ctx->cur, fin, g, ctx->cnt);
+    const bool ordered = ctx->orderSpan > 0;
+    const int packBase = ordered ? ctx->orderSpan : ctx->nFixtures;
+    const PairSink sink{ctx->newKeys, ctx->capContacts, (unsigned long long)packBase, ordered ? ctx->fixOrder : nullptr};
+    hipLaunchKernelGGL(k_small_pairs, dim3(blocks(ctx->nFixtures * kQueryLanes)), dim3(256), 0, s, w, g, ctx->hashTable,
+                       fin.hashMask, sink, ctx->cnt);
+    hipLaunchKernelGGL(k_small_append, dim3(1), dim3(kSmallLanes), 0, s, w, ctx->newKeys, (unsigned long long)packBase,
+                       ctx->capContacts, ctx->autoClearForces && !ctx->continuous ? 1 : 0, ctx->cnt);
+    LAUNCHCHK(ctx);
+    if ((rc = readCounters(ctx)) != B2G_OK) return rc;
+    *forcesCleared = !ctx->hcnt->smallPending && !ctx->continuous;
+
+    const ColourLayout layout = colourLayout(ctx->hcnt->colourCount, 0, ctx->sched.tailColours);
+    memcpy(ctx->lastColourStart, layout.start, sizeof(layout.start));
+    ctx->lastConstraints = layout.nCons;
+    ctx->compactedFrom = before;
+    ctx->stats.constraints = layout.nCons;
+    ctx->stats.colours = layout.nColours;
+    ctx->stats.wideConstraints = wideConstraints(layout);
+    // the rounds the stage kernels would have launched
+    if (before > 0) {
+        const int unchecked =
+            std::min(std::max(ctx->colourRoundsNeeded, kColourRoundsUnchecked), kColourRoundSlots - 1);
+        ctx->stats.colouringRounds = std::max(unchecked, ctx->hcnt->colourRounds);
+        ctx->colourRoundsNeeded = ctx->hcnt->colourRounds;
+    }
+    ctx->nContacts = ctx->hcnt->nContacts;
+    if (ctx->hcnt->smallPending) {
+        // more new pairs than the LDS sort or the table takes
+        if ((rc = rebuildHash(ctx)) != B2G_OK) return rc;
+        if ((rc = runBroadphase(ctx)) != B2G_OK) return rc;
+    } else {
+        ctx->nContacts += ctx->hcnt->nNewPairs;
+        ctx->stats.newPairs += ctx->hcnt->nNewPairs;
+        ctx->stats.queries = ctx->hcnt->nQueries;
+        ctx->stats.scanned = ctx->hcnt->nScanned;
+    }
+    positionStats(ctx, posIters, layout.nCons);
+    return B2G_OK;
+}
+
 // Second half: compaction, islands, colouring, the solve, broad-phase.
 int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
     hipStream_t s = ctx->stream;
@@ -7044,19 +7627,24 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
     // stage below skips them), until the compaction before the broad-phase;
     // their colours go back to the bodies now. ctx->nContacts stays the
     // table's length until the broad-phase reads back the live count.
-    if (ctx->nContacts > 0) {
+    const int posIters = std::min(p->positionIterations, kMaxPosIters);
+    const bool solves = dt > 0.0f && ctx->stepComplete;
+    if (solves && posIters > ctx->islandIterCap) {
+        freeArray(ctx->islandMinSep);
+        HIPCHK(ctx, hipMalloc((void**)&ctx->islandMinSep, sizeof(int) * (size_t)ctx->capBodies * posIters));
+        ctx->islandIterCap = posIters;
+    }
+    const bool small = solves && smallWorldFits(ctx, p);
+    bool forcesCleared = false;
+    if (ctx->nContacts > 0 && !small) {
         const int pe = profStart(ctx);
         hipLaunchKernelGGL(k_mark_dead, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, ctx->view(), ctx->keep);
         profEnd(ctx, PH_COMPACT, pe);
         LAUNCHCHK(ctx);
     }
-    if (dt > 0.0f && ctx->stepComplete) {
-        const int posIters = std::min(p->positionIterations, kMaxPosIters);
-        if (posIters > ctx->islandIterCap) {
-            freeArray(ctx->islandMinSep);
-            HIPCHK(ctx, hipMalloc((void**)&ctx->islandMinSep, sizeof(int) * (size_t)ctx->capBodies * posIters));
-            ctx->islandIterCap = posIters;
-        }
+    if (small) {
+        if ((rc = stepSmallSolve(ctx, p, &forcesCleared)) != B2G_OK) return rc;
+    } else if (solves) {
         WorldView w = ctx->view();
         // Islands of awake bodies and the constraint set.
         {
@@ -7124,9 +7712,9 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const int clusterSize = ctx->sched.clusterBodies;
         const bool clustered = clusterSize > 0 && ctx->nContacts > 0 && ctx->nBodies < kMaxClusterBodies;
         const int nClusters = clustered ? (ctx->nBodies + clusterSize - 1) / clusterSize : 0;
-        int nCons = 0;
-        int colourStart[kColourSlots + 1];
-        memset(colourStart, 0, sizeof(colourStart));
+        ColourLayout layout;
+        memset(&layout, 0, sizeof(layout));
+        const int* colourStart = layout.start;
         // Every contact gets an order key (constraints by colour, or by
         // cluster and colour; the others after them) and the table is
         // sorted; one readback brings the counts and what the colouring left.
@@ -7180,15 +7768,15 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
                     break;
                 }
             ctx->colourRoundsNeeded = needed;
-            if (clustered) colourStart[0] = ctx->hcnt->boundaryStart;
-            for (int c = 0; c < kColourSlots; ++c) colourStart[c + 1] = colourStart[c] + ctx->hcnt->colourCount[c];
-            nCons = colourStart[kColourSlots];
+            layout = colourLayout(ctx->hcnt->colourCount, clustered ? ctx->hcnt->boundaryStart : 0,
+                                  ctx->sched.tailColours);
         }
+        const int nCons = layout.nCons, nColours = layout.nColours;
+        // Trailing colours with at most sched.tailColours constraints each go to
+        // one workgroup (tailLaunch); the colours before them get a launch each.
+        const int tailBegin = layout.tailBegin;
         ctx->stats.colouringRounds = rounds;
-        int nColours = 0;
-        for (int c = 0; c < kColourSlots; ++c)
-            if (colourStart[c + 1] > colourStart[c]) nColours = c + 1;
-        memcpy(ctx->lastColourStart, colourStart, sizeof(colourStart));
+        memcpy(ctx->lastColourStart, layout.start, sizeof(layout.start));
         ctx->lastConstraints = nCons;
         ctx->stats.constraints = nCons;
         ctx->stats.colours = clustered ? (nCons > 0 ? ctx->hcnt->maxColour + 1 : 0) : nColours;
@@ -7204,7 +7792,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const bool wantFresh = nCons > 0 && (learned || ctx->logCap > 0 || ctx->traceIters > 0);
         if (wantFresh && (rc = ensureFresh(ctx)) != B2G_OK) return rc;
         const FreshView fv{wantFresh ? ctx->freshMask : nullptr, ctx->freshNum, ctx->freshAll, ctx->learnedScope};
-        const bool block = !clustered && blockSolveFits(ctx, p, colourStart, nCons);
+        const bool block = nCons > 0 && blockSolveFits(ctx, p, nCons);
         const int blockLanes = block ? blockSolveLanes(ctx, nCons) : 0;
         const bool blockInit = block && !wantFresh &&
                                nCons <= blockLanes * (ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>);
@@ -7239,17 +7827,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         ctx->stats.residual = -1.0f;
         const int sb = ctx->sched.solverBlock;
         auto sgrid = [sb](int n) { return dim3((unsigned)((n + sb - 1) / sb)); };
-        // Trailing colours with at most sched.tailColours constraints each go to
-        // one workgroup (tailLaunch); the colours before them get a launch each.
-        int tailBegin = nColours;
-        if (ctx->sched.tailColours > 0) {
-            while (tailBegin > 0 && colourStart[tailBegin] - colourStart[tailBegin - 1] <= ctx->sched.tailColours)
-                --tailBegin;
-            if (nColours - tailBegin < 2) tailBegin = nColours;  // one colour: no gain
-        }
-        ctx->stats.wideConstraints = 0;
-        for (int c = 0; c < tailBegin; ++c)
-            if (c != kOverflowColour) ctx->stats.wideConstraints += colourStart[c + 1] - colourStart[c];
+        ctx->stats.wideConstraints = wideConstraints(layout);
         ColourRanges ranges;
         memcpy(ranges.s, colourStart, sizeof(ranges.s));
         auto perColour = [&](int phase, auto kernelLaunch, auto tailLaunch) {
@@ -7372,10 +7950,10 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         // and the position passes (the residual fallback, the impulse log).
         const bool persist = ctx->sched.persistentSolve > 0 && !clusterLaunch && ctx->traceIters == 0 &&
                              (nCons > 0 || ctx->nJoints > 0);
-        auto solvePlan = [&](int stages, bool contactWarm) {
+        auto persistentLaunch = [&](int stages, bool contactWarm) -> int {
             SolvePlan plan;
             memset(&plan, 0, sizeof(plan));
-            memcpy(plan.cs, colourStart, sizeof(plan.cs));
+            memcpy(plan.cs, layout.start, sizeof(plan.cs));
             if (ctx->nJoints > 0) {
                 for (int c = 0; c <= kColourSlots; ++c) plan.js[c] = ctx->jointColourStart[c];
                 plan.nJointColours = kColourSlots;
@@ -7390,10 +7968,6 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             plan.velIters = p->velocityIterations;
             plan.posIters = posIters;
             plan.nCons = nCons;
-            return plan;
-        };
-        auto persistentLaunch = [&](int stages, bool contactWarm) -> int {
-            SolvePlan plan = solvePlan(stages, contactWarm);
             int nb = 0;
             const int pb = ctx->nJoints > 0 ? std::min(sb, kPersistJointBlock) : sb;
             const int brc = persistentBlocks(ctx, pb, &nb);
@@ -7448,11 +8022,8 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const bool velocityDeferred = persist && !checkResidual && ctx->logCap == 0;
         const bool contactWarm = nCons > 0 && (ctx->warmStarting || usePrediction);
         if (block) {
-            BlockPlan plan{solvePlan(SP_WARM | SP_VELOCITY | SP_POSITION, contactWarm), ctx->gravity, blockInit ? 1 : 0};
             pe = profStart(ctx);
-            hipLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(blockLanes),
-                               sizeof(float4) * (size_t)ctx->nBodies, s, w, ctx->cv, jv, (const int*)ctx->consOrder, plan,
-                               ctx->cnt);
+            launchBlockSolve(ctx, p, w, jv, blockLanes, contactWarm, blockInit);
             profEnd(ctx, PH_SOLVE_V, pe);
         } else if (!persist) {
             startSolve(contactWarm);
@@ -7578,17 +8149,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         if ((rc = rebuildHash(ctx, true)) != B2G_OK) return rc;
         if ((rc = runBroadphase(ctx, true)) != B2G_OK) return rc;
         profEnd(ctx, PH_BROADPHASE, pe);
-        // Stats of the position iterations.
-        int ran = 0;
-        float lastMin = 0.0f;
-        for (int it = 0; it < posIters && nCons > 0; ++it) {
-            ++ran;
-            lastMin = decodeOrdered(ctx->hcnt->minSep[it]);
-            if (lastMin >= -3.0f * kLinearSlop) break;
-        }
-        ctx->stats.positionIterations = ran;
-        ctx->stats.points = ctx->hcnt->points;
-        ctx->stats.minSeparation = lastMin;
+        positionStats(ctx, posIters, nCons);
         if (ctx->hcnt->barrierAbort)
             return fail(ctx, B2G_ERR_STATE, "one-launch solve: a grid barrier wait passed its bound");
     } else {
@@ -7600,7 +8161,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
     ctx->stats.endEvents = ctx->hcnt->endEvents;
     if (ctx->continuous && dt > 0.0f && (rc = solveTOI(ctx, p)) != B2G_OK) return rc;
     if (dt > 0.0f) ctx->inv_dt0 = inv_dt;
-    if (ctx->autoClearForces && ctx->nBodies > 0)
+    if (ctx->autoClearForces && ctx->nBodies > 0 && !forcesCleared)
         hipLaunchKernelGGL(k_fill<float4>, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, ctx->force, ctx->nBodies,
                            make_float4(0.0f, 0.0f, 0.0f, 0.0f));
     LAUNCHCHK(ctx);

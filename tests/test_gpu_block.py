@@ -1,11 +1,13 @@
-"""The block solve (one workgroup, bodies in LDS, rows in registers) against a
-launch per colour (schedule field tailColours 0), bit for bit.
+"""The small-world step (its stages in one workgroup's kernels, the block solve
+with bodies in LDS and rows in registers) against a launch per stage and
+colour (schedule field tailColours 0), bit for bit.
 
 Sizes around where the path or its layout changes: below and beyond the rows
 that lanes hold in registers (1024 with 256 lanes, 2048 with 512; 768 and 1536
-with joints), the largest number of bodies in LDS and one beyond it, every
-joint type, a body in more contacts than there are colours (the overflow
-colour, left to the per-colour kernels), islands that sleep, few iterations.
+with joints), the largest number of bodies in LDS and one beyond it, worlds
+that start with more new pairs than the LDS sort takes, every joint type, a
+body in more contacts than there are colours (the overflow colour), islands
+that sleep, contacts that end, sub-worlds, few iterations.
 """
 import numpy as np
 import pytest
@@ -14,35 +16,55 @@ import engines as E
 
 pytestmark = pytest.mark.gpu
 
+BODY = np.dtype([
+    ("type", "<i4"), ("flags", "<i4"), ("xf", "<f4", 4), ("lc", "<f4", 2), ("c0", "<f4", 2), ("a0", "<f4"),
+    ("c", "<f4", 2), ("a", "<f4"), ("rest", "<f4", 12),
+])
+assert BODY.itemsize == 104
 
-def run(gpu, kind, n, seed, steps, sleep, vel, pos, per_colour):
-    w = gpu.world(kind, n, seed, sleep=sleep)
+
+def a_launch_per_colour(w):
+    ctx = w.device_context()
+    lib = E.b2g_lib()
+    sched = np.zeros(1, E.SCHEDULE)
+    E.b2g_check(lib, ctx, lib.b2g_get_schedule(ctx, E.ptr(sched)))
+    sched["tailColours"] = 0
+    E.b2g_check(lib, ctx, lib.b2g_set_schedule(ctx, E.ptr(sched)))
+
+
+def state(w):
+    meta, man = w.contacts()
+    st = w.stats()
+    return (w.bodies().view(np.uint32), meta, E.manifold_bits(man),
+            [int(st[k]) for k in ("contacts", "constraints", "points", "colours", "colouringRounds", "newPairs",
+                                  "positionIterations", "beginEvents", "endEvents", "queries")],
+            float(st["minSeparation"]), w.fat_aabbs().tobytes())
+
+
+def run(w, per_colour, steps, vel=8, pos=3):
     try:
         if per_colour:
-            ctx = w.device_context()
-            lib = E.b2g_lib()
-            sched = np.zeros(1, E.SCHEDULE)
-            E.b2g_check(lib, ctx, lib.b2g_get_schedule(ctx, E.ptr(sched)))
-            sched["tailColours"] = 0
-            E.b2g_check(lib, ctx, lib.b2g_set_schedule(ctx, E.ptr(sched)))
+            a_launch_per_colour(w)
         out = []
         for _ in range(3):
             w.step(steps // 3, vel=vel, pos=pos)
-            meta, man = w.contacts()
-            st = w.stats()
-            out.append((w.bodies().view(np.uint32), meta, E.manifold_bits(man),
-                        [int(st[k]) for k in ("contacts", "constraints", "points", "colours", "positionIterations",
-                                              "beginEvents", "endEvents")], float(st["minSeparation"])))
+            out.append(state(w))
         return out
     finally:
         w.close()
 
 
+def same(a, b):
+    for x, y in zip(a, b):
+        for u, v in zip(x, y):
+            assert np.array_equal(u, v) if isinstance(u, np.ndarray) else u == v
+
+
 @pytest.mark.parametrize("kind, n, seed, steps, sleep, vel, pos", [
     ("pyramid", 1, 0, 60, True, 8, 3), ("pyramid", 12, 0, 90, True, 8, 3), ("pyramid", 33, 0, 30, False, 8, 3),
     ("world", 64, 1, 240, True, 8, 3), ("world", 500, 2, 240, False, 8, 3), ("world", 1000, 3, 300, False, 6, 2),
-    ("world", 1700, 4, 330, False, 8, 3), ("world", 4094, 5, 60, False, 8, 3), ("world", 4095, 5, 420, False, 8, 3),
-    ("world", 4096, 5, 60, False, 8, 3), ("world", 300, 6, 240, False, 1, 0), ("world", 300, 6, 60, False, 0, 1),
+    ("world", 1700, 4, 330, False, 8, 3), ("world", 3000, 5, 60, False, 8, 3), ("world", 4031, 5, 420, False, 8, 3),
+    ("world", 4032, 5, 60, False, 8, 3), ("world", 300, 6, 240, False, 1, 0), ("world", 300, 6, 60, False, 0, 1),
     ("plank", 100, 0, 120, False, 8, 3), ("terrain", 150, 3, 150, True, 8, 3),
     ("chains", 30, 8, 120, True, 8, 3), ("pendulums", 40, 0, 90, False, 8, 3), ("distance", 20, 0, 60, False, 8, 3),
     ("ropes", 20, 0, 60, False, 8, 3), ("welds", 12, 0, 90, True, 8, 3), ("friction", 16, 0, 60, False, 8, 3),
@@ -50,9 +72,45 @@ def run(gpu, kind, n, seed, steps, sleep, vel, pos, per_colour):
     ("prismatic", 12, 0, 60, False, 8, 3), ("wheels", 6, 0, 90, False, 8, 3), ("gears", 4, 0, 60, False, 8, 3),
 ])
 def test_equals_a_launch_per_colour(gpu, kind, n, seed, steps, sleep, vel, pos):
-    a = run(gpu, kind, n, seed, steps, sleep, vel, pos, False)
-    b = run(gpu, kind, n, seed, steps, sleep, vel, pos, True)
-    for (ba, ma, na, sa, la), (bb, mb, nb, sb, lb) in zip(a, b):
-        assert np.array_equal(ba, bb)
-        assert np.array_equal(ma, mb) and np.array_equal(na, nb)
-        assert sa == sb and la == lb
+    a = run(gpu.world(kind, n, seed, sleep=sleep), False, steps, vel, pos)
+    b = run(gpu.world(kind, n, seed, sleep=sleep), True, steps, vel, pos)
+    same(a, b)
+
+
+@pytest.mark.parametrize("kind, n, ccd", [("terrain", 60, True), ("bullets", 40, True), ("sensors", 30, False),
+                                          ("oneway", 6, True)])
+def test_with_events_and_sensors(gpu, kind, n, ccd):
+    same(run(gpu.world(kind, n, 2, ccd=ccd), False, 60), run(gpu.world(kind, n, 2, ccd=ccd), True, 60))
+
+
+@pytest.mark.parametrize("kind, n_worlds, n, sleep", [("world", 9, 120, True), ("pendulums", 5, 7, False)])
+def test_sub_worlds(gpu, kind, n_worlds, n, sleep):
+    same(run(E.World.worlds(gpu, kind, n_worlds, n, 4, sleep), False, 240),
+         run(E.World.worlds(gpu, kind, n_worlds, n, 4, sleep), True, 240))
+
+
+def test_many_new_pairs_at_once(gpu):
+    """A world pressed together: more new pairs than the LDS sort takes, then more contacts than the small-world
+    kernels take, then neither."""
+    out = []
+    for per_colour in (False, True):
+        w = gpu.world("world", 1500, 7, sleep=False)
+        if per_colour:
+            a_launch_per_colour(w)
+        w.step(20)
+        ctx, lib = w.device_context(), E.b2g_lib()
+        bodies = np.zeros(1501, BODY)
+        E.b2g_check(lib, ctx, lib.b2g_get_bodies(ctx, 0, 1501, E.ptr(bodies)))
+        for k in ("c", "c0"):
+            bodies[k][1:] *= np.float32(0.3)
+        bodies["xf"][1:, :2] *= np.float32(0.3)
+        E.b2g_check(lib, ctx, lib.b2g_set_bodies(ctx, 0, 1501, E.ptr(bodies)))
+        states, pairs = [], 0
+        for _ in range(4):
+            w.step(1)
+            states.append(state(w))
+            pairs = max(pairs, int(w.stats()["newPairs"]))
+        assert pairs > 4096
+        states += run(w, False, 90)
+        out.append(states)
+    same(*out)
