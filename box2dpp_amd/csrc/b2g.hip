@@ -60,6 +60,8 @@ constexpr int kMaxCellsPerProxy = 16;
 constexpr int kColourRoundsUnchecked = 2;  // fewest colouring rounds launched before the first readback
 constexpr int kColourRoundSlots = 16;      // rounds whose leftovers are recorded (later rounds share the last)
 constexpr uint32_t kNotConstraintKey = 0x7Fu;  // order key of a contact outside the constraint set
+constexpr int kOrderKeys = 127;                // order keys of the constraint set
+constexpr int kSplitColours = 62;              // colours whose two-point constraints have a key of their own
 
 struct Counters {
     int nContacts;
@@ -83,7 +85,8 @@ struct Counters {
     int nFresh;            // fresh contact points of the step (learned warm start, log, trace)
     int residualPoints;
     float residualSum;     // sum of squared complementarity residuals (k_residual)
-    int colourCount[kColourSlots + 3];
+    int colourCount[kColourSlots + 3];  // constraints per colour (clustered solve: of the boundary set)
+    int orderCount[kOrderKeys + 1];     // constraints per order key (orderKey)
     int minSep[kMaxPosIters];
     int nClustered;        // bodies placed in clusters (clustered solve)
     int boundaryStart;     // first constraint between clusters (clustered solve)
@@ -335,6 +338,8 @@ __device__ inline void collideFinish(const WorldView& w, Counters* cnt, int c, i
     else flags &= ~CF_TOUCHING;
     if (wasTouching) flags |= CF_WAS_TOUCHING;
     else flags &= ~CF_WAS_TOUCHING;
+    if (m.pointCount == 2) flags |= CF_TWO_POINTS;
+    else flags &= ~CF_TWO_POINTS;
     if (!wasTouching && touching) atomicAdd(&cnt->beginEvents, 1);
     if (wasTouching && !touching) atomicAdd(&cnt->endEvents, 1);
     w.cman[c] = m;
@@ -837,14 +842,35 @@ __global__ void k_demote_commit(WorldView w, const unsigned long long* claim, ui
     if (c < w.nContacts) demoteCommitOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
 }
 
-// Order key of every contact: a constraint's colour; contacts outside the
-// constraint set sort after every colour.
-// Also clears the colour counts that the order's counting sort then takes.
-__global__ void k_cons_keys(WorldView w, uint32_t* keys, int* vals, Counters* cnt) {
+// Order key of a constraint: its colour and, with `split`, its point count.
+// The constraints of a colour may come in any order, and a wavefront with one
+// two-point constraint in it pays for the 2x2 block solve and a second
+// position point: in a pile of circles and polygons one constraint in ten has
+// two points, so that unsplit nearly every wavefront does. The keys have 7
+// bits, so colours 62 and 63, if it comes to them, stay whole, as does the
+// overflow colour, whose order counts. k_solve_velocity over 3000 constraints
+// of a pile 4.2 -> 3.7 us, over 20 000 5.95 -> 5.2 us; k_solve_position
+// 5.4 -> 4.7 and 7.15 -> 6.8 us.
+__host__ __device__ inline int orderKey(int colour, bool twoPoints, bool split) {
+    if (colour >= kSplitColours) return kSplitColours + colour;
+    return 2 * colour + (split && twoPoints ? 1 : 0);
+}
+static_assert(kSplitColours + kOverflowColour == kOrderKeys - 1, "order keys up to the overflow colour's");
+
+__host__ __device__ inline int colourCountOf(const int* orderCount, int colour) {
+    if (colour >= kSplitColours) return orderCount[kSplitColours + colour];
+    return orderCount[2 * colour] + orderCount[2 * colour + 1];
+}
+
+// Order key of every contact; contacts outside the constraint set sort after
+// every colour. Also clears the counts that the order's counting sort takes.
+__global__ void k_cons_keys(WorldView w, uint32_t* keys, int* vals, int split, Counters* cnt) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < kColourSlots + 3) cnt->colourCount[c] = 0;
+    if (c < kOrderKeys) cnt->orderCount[c] = 0;
     if (c >= w.nContacts) return;
-    keys[c] = (w.cflags[c] & CF_CONSTRAINT) ? (uint32_t)w.ccolour[c] : kNotConstraintKey;
+    const int flags = w.cflags[c];
+    keys[c] = (flags & CF_CONSTRAINT) ? (uint32_t)orderKey(w.ccolour[c], (flags & CF_TWO_POINTS) != 0, split != 0)
+                                      : kNotConstraintKey;
     vals[c] = c;
 }
 
@@ -3878,14 +3904,14 @@ __global__ void __launch_bounds__(kBlockLanes)
     const BlockPlan& p = plan;
     const int t = threadIdx.x, T = blockDim.x;
     if (t < 64) {
-        int sum = cnt->colourCount[t];
+        int sum = colourCountOf(cnt->orderCount, t);
         for (int o = 1; o < 64; o <<= 1) {
             const int before = __shfl_up(sum, o);
             if (t >= o) sum += before;
         }
         cs[t + 1] = sum;
         if (t == 0) cs[0] = 0;
-        if (t == 63) cs[kColourSlots] = sum + cnt->colourCount[kOverflowColour];
+        if (t == 63) cs[kColourSlots] = sum + colourCountOf(cnt->orderCount, kOverflowColour);
     }
     const int nb = w.nBodies;
     WorldView wl = w;  // the bodies' rows in LDS for the functions that take a world
@@ -4644,8 +4670,8 @@ __global__ void __launch_bounds__(kSmallLanes)
                     int demoteRounds, int posIters, int* order, Counters* cnt) {
     __shared__ int label[kSmallBodies];
     __shared__ uint32_t ends[kSmallContacts];  // bodies A, B of each contact, 13 bits each
-    __shared__ int hist[kSmallLanes / 64][kColourSlots];
-    __shared__ int next[kColourSlots];         // where the next constraint of a colour goes
+    __shared__ int hist[kSmallLanes / 64][kOrderKeys];
+    __shared__ int next[kOrderKeys];           // where the next constraint of a key goes
     __shared__ int left;
     const int t = threadIdx.x, T = blockDim.x;
     const int nb = w.nBodies, nc = w.nContacts;
@@ -4714,40 +4740,41 @@ __global__ void __launch_bounds__(kSmallLanes)
         __syncthreads();
         if (stay == 0) break;
     }
-    // Constraints by colour, in table order within a colour: counts, then
-    // chunks of T contacts ranked by a ballot per colour bit and a count per
+    // Constraints by order key, in table order within a key: counts, then
+    // chunks of T contacts ranked by a ballot per key bit and a count per
     // wavefront.
     const int lane = (int)__lane_id(), wave = t >> 6, waves = T >> 6;
-    for (int c = t; c < kColourSlots; c += T) next[c] = 0;
+    auto keyOf = [&](int c) { return orderKey(w.ccolour[c], (w.cflags[c] & CF_TWO_POINTS) != 0, true); };
+    for (int k = t; k < kOrderKeys; k += T) next[k] = 0;
     __syncthreads();
     for (int c = t; c < nc; c += T)
-        if (w.cflags[c] & CF_CONSTRAINT) atomicAdd(&next[w.ccolour[c]], 1);
+        if (w.cflags[c] & CF_CONSTRAINT) atomicAdd(&next[keyOf(c)], 1);
     __syncthreads();
-    if (t < kColourSlots) cnt->colourCount[t] = next[t];
+    if (t < kOrderKeys) cnt->orderCount[t] = next[t];
     __syncthreads();
     if (t == 0) {
         int sum = 0;
-        for (int c = 0; c < kColourSlots; ++c) {
-            const int n = next[c];
-            next[c] = sum;
+        for (int k = 0; k < kOrderKeys; ++k) {
+            const int n = next[k];
+            next[k] = sum;
             sum += n;
         }
     }
     for (int c0 = 0; c0 < nc; c0 += T) {
         const int c = c0 + t;
         const bool in = c < nc && (w.cflags[c] & CF_CONSTRAINT);
-        const int col = in ? w.ccolour[c] : 0;
+        const int key = in ? keyOf(c) : 0;
         unsigned long long same = __ballot(in);
         for (int bit = 0; bit < 7; ++bit) {
-            const unsigned long long ones = __ballot((col >> bit) & 1);
-            same &= ((col >> bit) & 1) ? ones : ~ones;
+            const unsigned long long ones = __ballot((key >> bit) & 1);
+            same &= ((key >> bit) & 1) ? ones : ~ones;
         }
-        for (int i = t; i < waves * kColourSlots; i += T) (&hist[0][0])[i] = 0;
+        for (int i = t; i < waves * kOrderKeys; i += T) (&hist[0][0])[i] = 0;
         __syncthreads();
         const int rank = __popcll(same & ((1ull << lane) - 1ull));
-        if (in && rank == 0) hist[wave][col] = __popcll(same);
+        if (in && rank == 0) hist[wave][key] = __popcll(same);
         __syncthreads();
-        if (t < kColourSlots) {
+        if (t < kOrderKeys) {
             int sum = next[t];
             for (int i = 0; i < waves; ++i) {
                 const int n = hist[i][t];
@@ -4757,7 +4784,7 @@ __global__ void __launch_bounds__(kSmallLanes)
             next[t] = sum;
         }
         __syncthreads();
-        if (in) order[hist[wave][col] + rank] = c;
+        if (in) order[hist[wave][key] + rank] = c;
         __syncthreads();
     }
 }
@@ -7496,6 +7523,10 @@ struct ColourLayout {
     int nCons, nColours, tailBegin;
 };
 
+void coloursFromKeys(const int* orderCount, int* colourCount) {
+    for (int c = 0; c < kColourSlots; ++c) colourCount[c] = colourCountOf(orderCount, c);
+}
+
 ColourLayout colourLayout(const int* counts, int first, int tailColours) {
     ColourLayout l;
     l.start[0] = first;
@@ -7587,6 +7618,7 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     if ((rc = readCounters(ctx)) != B2G_OK) return rc;
     *forcesCleared = !ctx->hcnt->smallPending && !ctx->continuous;
 
+    coloursFromKeys(ctx->hcnt->orderCount, ctx->hcnt->colourCount);
     const ColourLayout layout = colourLayout(ctx->hcnt->colourCount, 0, ctx->sched.tailColours);
     memcpy(ctx->lastColourStart, layout.start, sizeof(layout.start));
     ctx->lastConstraints = layout.nCons;
@@ -7733,8 +7765,10 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
                 hipLaunchKernelGGL(k_cons_keys_clustered, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w,
                                    ctx->bodyCluster, ctx->consKeys, ctx->consVals, ctx->cnt);
             } else {
+                // the log and the trace take their points in table order
+                const int split = ctx->logCap == 0 && ctx->traceIters == 0 ? 1 : 0;
                 hipLaunchKernelGGL(k_cons_keys, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w, ctx->consKeys,
-                                   ctx->consVals, ctx->cnt);
+                                   ctx->consVals, split, ctx->cnt);
             }
             if (clustered) {
                 HIPCHK(ctx, prims_sort_pairs_u32(ctx->scratch, ctx->scratchBytes, ctx->consKeys, ctx->consKeysSorted,
@@ -7742,14 +7776,16 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
                 hipLaunchKernelGGL(k_cluster_ranges, dim3(blocks((nClusters + 1) * (kColourSlots + 1))), dim3(256), 0,
                                    s, ctx->consKeysSorted, ctx->nContacts, nClusters, ctx->clusterStart, ctx->cnt);
             } else {
-                // colours and the key of the contacts outside the set fit 7 bits
+                // the order keys and that of the contacts outside the set fit 7 bits
                 HIPCHK(ctx, prims_count_sort_pairs(ctx->scratch, ctx->scratchBytes, ctx->consKeys, ctx->consKeysSorted,
                                                    ctx->consVals, ctx->consOrder, ctx->nContacts,
-                                                   ctx->cnt->colourCount, kColourSlots, s));
+                                                   ctx->cnt->orderCount, kOrderKeys, s));
             }
             profEnd(ctx, PH_ORDER, pe);
             LAUNCHCHK(ctx);
-            return readCounters(ctx);
+            const int orc = readCounters(ctx);
+            if (orc == B2G_OK && !clustered) coloursFromKeys(ctx->hcnt->orderCount, ctx->hcnt->colourCount);
+            return orc;
         };
         if (ctx->nContacts > 0) {
             if ((rc = order()) != B2G_OK) return rc;
