@@ -93,7 +93,13 @@ struct Counters {
     int maxColour;         // highest constraint colour of the step
     unsigned barrierCount; // one-launch solve: workgroups arrived at the grid barrier
     unsigned barrierGen;   // one-launch solve: barrier generation
-    int barrierAbort;      // one-launch solve: a barrier wait passed its bound
+    int barrierAbort;      // one-launch and team solve: a barrier wait passed its bound
+    unsigned teamXcc;      // team solve: the team's XCD, plus one
+    unsigned teamJoined;   // team solve: workgroups that joined, with kTeamClosed once that is settled
+    unsigned teamSize;     // team solve: members (0: not settled yet)
+    int pad0[29];
+    unsigned teamArrived;  // team solve: arrivals at its barriers, on a cache line of its own
+    int pad1[31];
 };
 
 // Constraint arrays (b2ContactVelocityConstraint / b2ContactPositionConstraint,
@@ -1413,9 +1419,7 @@ __global__ void k_store_impulses_r(WorldView w, ConView cv, const int* ranges) {
 
 // Position integration with translation and rotation clamps,
 // REF/Dynamics/b2Island.cpp:276-306.
-__device__ inline void integratePositionOne(const WorldView& w, int b, float h) {
-    float4 p = w.pos[b];
-    const float4 vv = w.vel[b];
+__device__ inline void integratePosition(float4& p, float4& vv, float h) {
     V2 c = mk(p.x, p.y);
     float a = p.z;
     V2 v = mk(vv.x, vv.y);
@@ -1432,8 +1436,15 @@ __device__ inline void integratePositionOne(const WorldView& w, int b, float h) 
     }
     c += h * v;
     a += h * wv;
-    w.pos[b] = make_float4(c.x, c.y, a, 0.0f);
-    w.vel[b] = make_float4(v.x, v.y, wv, 0.0f);
+    p = make_float4(c.x, c.y, a, 0.0f);
+    vv = make_float4(v.x, v.y, wv, 0.0f);
+}
+
+__device__ inline void integratePositionOne(const WorldView& w, int b, float h) {
+    float4 p = w.pos[b], v = w.vel[b];
+    integratePosition(p, v, h);
+    w.pos[b] = p;
+    w.vel[b] = v;
 }
 
 __global__ void k_integrate_positions(WorldView w, float h) {
@@ -3694,14 +3705,15 @@ __global__ void k_body_energy(WorldView w, V2 g, double2* out) {
 // Copy-back transform of every solved body (b2Body::SynchronizeTransform,
 // REF/Dynamics/b2Body.h:836-840). Static bodies keep their creation-time
 // transform, which the reference's recomputation reproduces exactly.
-__device__ inline void syncTransformOne(const WorldView& w, int b) {
-    const float4 p = w.pos[b];
+__device__ inline void syncTransformFrom(const WorldView& w, int b, const float4& p) {
     const float2 lc = w.lcenter[b];
     Xf xf;
     xf.q = rotOf(p.z);
     xf.p = mk(p.x, p.y) - mul(xf.q, mk(lc.x, lc.y));
     w.xf[b] = f4(xf);
 }
+
+__device__ inline void syncTransformOne(const WorldView& w, int b) { syncTransformFrom(w, b, w.pos[b]); }
 
 __global__ void k_sync_transforms(WorldView w) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
@@ -3887,6 +3899,19 @@ constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane,
 template <bool kJoints>
 constexpr int kBlockRows = kJoints ? 3 : 4;  // constraint rows a lane holds
 
+// The colours' ranges from the order's counts, by one whole wavefront.
+__device__ inline void colourStarts(const Counters* cnt, int* cs) {
+    const int c = (int)__lane_id();
+    int sum = colourCountOf(cnt->orderCount, c);
+    for (int o = 1; o < 64; o <<= 1) {
+        const int before = __shfl_up(sum, o);
+        if (c >= o) sum += before;
+    }
+    cs[c + 1] = sum;
+    if (c == 0) cs[0] = 0;
+    if (c == 63) cs[kColourSlots] = sum + colourCountOf(cnt->orderCount, kOverflowColour);
+}
+
 struct BlockPlan {
     int js[kColourSlots + 1];  // joint colour c holds order slots [js[c], js[c + 1])
     V2 gravity;
@@ -3903,16 +3928,7 @@ __global__ void __launch_bounds__(kBlockLanes)
     __shared__ int cs[kColourSlots + 1];  // colour c holds constraints [cs[c], cs[c + 1])
     const BlockPlan& p = plan;
     const int t = threadIdx.x, T = blockDim.x;
-    if (t < 64) {
-        int sum = colourCountOf(cnt->orderCount, t);
-        for (int o = 1; o < 64; o <<= 1) {
-            const int before = __shfl_up(sum, o);
-            if (t >= o) sum += before;
-        }
-        cs[t + 1] = sum;
-        if (t == 0) cs[0] = 0;
-        if (t == 63) cs[kColourSlots] = sum + colourCountOf(cnt->orderCount, kOverflowColour);
-    }
+    if (t < 64) colourStarts(cnt, cs);
     const int nb = w.nBodies;
     WorldView wl = w;  // the bodies' rows in LDS for the functions that take a world
     wl.vel = rows;
@@ -4066,6 +4082,226 @@ __global__ void __launch_bounds__(kBlockLanes)
             w.pos[b] = rows[b];
             syncTransformOne(w, b);
         }
+}
+
+// ====================================================================
+// Team solve: the island solve of a mid-sized world in one launch by the
+// workgroups of one XCD. Between the reach of a single workgroup and the size
+// where a colour fills the chip, a launch per colour is mostly launch: 3.7 us
+// for 3000 constraints whose two trips to memory and arithmetic take half of
+// it, and over a grid barrier of all XCDs the caches have to be written back
+// and invalidated (see k_solve_persistent). The 32 compute units of one XCD
+// share an L2, so data handed on through it needs neither: a body's row is
+// stored as it is (a compute unit's cache writes through), every lane waits
+// for its stores, the barrier is one counter, and rows are read with
+// agent-scope relaxed loads, which pass the compute unit's cache by. Measured per barrier (16 workgroups, 256 lanes): 0.71 us,
+// 1.0 us with a row read, a row written and the wait for it; with an
+// agent-scope acquire fence in its place 5.1 us.
+//
+// The team is whoever got there: the grid is eight times the workgroups
+// wanted, each asks for its XCD, the first one settles which XCD it is and
+// closes the list when the wanted number has joined or 20 us have passed, and
+// everybody else leaves at once. Members are running by definition, so no
+// barrier waits for a workgroup that has no place on the chip; the waits are
+// bounded all the same (barrierAbort).
+//
+// A constraint belongs to one lane for the whole solve, which holds its row in
+// registers as in the block solve. Every constraint goes through the
+// per-colour kernels' functions, colour after colour, so the results are
+// theirs bit for bit. A colour takes 2.5 us at 20 000 constraints: the
+// barrier, and then one wavefront per SIMD, which waits for its own results
+// between instructions. (32 workgroups are as fast there and slower below;
+// rows read from memory ahead of the barrier instead of kept 3.0 us.)
+// ====================================================================
+constexpr unsigned kTeamClosed = 0x80000000u;
+constexpr int kTeamLanes = 256;
+constexpr int kTeamConstraints = 24576;        // most constraints (teamSolveFits)
+constexpr int kTeamSize = 16;                  // workgroups wanted, half an XCD's compute units
+constexpr long long kTeamJoinTicks = 2000;     // of the 100 MHz wall clock
+
+__device__ inline unsigned teamLoad(const unsigned* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// A row that other members write: two 8-byte accesses, which no store
+// overlaps (a colour writes only rows that no other constraint of it reads).
+__device__ inline float4 teamRow(const float4* p) {
+    const unsigned long long* q = (const unsigned long long*)p;
+    const unsigned long long a = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned long long b = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return make_float4(__uint_as_float((unsigned)a), __uint_as_float((unsigned)(a >> 32)), __uint_as_float((unsigned)b),
+                       __uint_as_float((unsigned)(b >> 32)));
+}
+// False for a workgroup that is not in the team. `shared` holds two words.
+__device__ inline bool teamJoin(Counters* cnt, unsigned wanted, unsigned* shared, unsigned& rank, unsigned& size) {
+    if (threadIdx.x == 0) {
+        unsigned xcc;
+        asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
+        shared[0] = shared[1] = 0u;
+        const unsigned first = atomicCAS(&cnt->teamXcc, 0u, xcc + 1u);
+        if (first == 0u || first == xcc + 1u) {
+            const unsigned r = atomicAdd(&cnt->teamJoined, 1u);
+            const long long t0 = wall_clock64();
+            if (r == 0u) {
+                while (teamLoad(&cnt->teamJoined) < wanted && wall_clock64() - t0 < kTeamJoinTicks) {
+                }
+                const unsigned n = atomicOr(&cnt->teamJoined, kTeamClosed);
+                __hip_atomic_store(&cnt->teamSize, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                shared[1] = n;
+            } else if (!(r & kTeamClosed)) {
+                unsigned n = 0u;
+                while ((n = teamLoad(&cnt->teamSize)) == 0u && wall_clock64() - t0 < kBarrierSpinTicks) {
+                }
+                if (n == 0u) __hip_atomic_store(&cnt->barrierAbort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                shared[0] = r;
+                shared[1] = n;
+            }
+        }
+    }
+    __syncthreads();
+    rank = shared[0];
+    size = shared[1];
+    return size != 0u;
+}
+
+// `phase` counts the barriers. Every lane waits for its own stores first, so
+// they are in the shared L2 before the workgroup arrives.
+__device__ inline void teamBarrier(Counters* cnt, unsigned size, unsigned& phase) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    ++phase;
+    if (threadIdx.x == 0 && __hip_atomic_load(&cnt->barrierAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
+        const unsigned all = size * phase;
+        unsigned n = __hip_atomic_fetch_add(&cnt->teamArrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+        const long long t0 = wall_clock64();
+        for (int turn = 1; n < all; ++turn) {
+            n = teamLoad(&cnt->teamArrived);
+            if ((turn & 1023) == 0 && wall_clock64() - t0 > kBarrierSpinTicks) {
+                __hip_atomic_store(&cnt->barrierAbort, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+        }
+    }
+    __syncthreads();
+}
+
+struct TeamPlan {
+    float h;
+    int velIters, posIters, contactWarm;
+    unsigned wanted;
+};
+
+// R: constraint rows a lane holds.
+template <int R>
+__global__ void __launch_bounds__(kTeamLanes) k_solve_team(WorldView w, ConView cv, TeamPlan p, Counters* cnt) {
+    __shared__ unsigned shared[2];
+    __shared__ int cs[kColourSlots + 1];  // colour c holds constraints [cs[c], cs[c + 1])
+    unsigned rank, size, phase = 0;
+    if (!teamJoin(cnt, p.wanted, shared, rank, size)) return;
+    if (threadIdx.x < 64) colourStarts(cnt, cs);
+    __syncthreads();
+    const int nCons = cs[kColourSlots], nb = w.nBodies;
+    // lanes by wavefront across the members, so a colour spreads over the compute units
+    const int lane = ((int)(threadIdx.x >> 6) * (int)size + (int)rank) * 64 + (int)(threadIdx.x & 63);
+    const int lanes = (int)size * kTeamLanes;
+    // Constraint lane + r * lanes in row r; those beyond (a team smaller than
+    // wanted) and all of them with an overflow colour, which one lane solves
+    // in order, are read in every pass.
+    const int held = nCons > cs[kOverflowColour] ? 0 : min(nCons, R * lanes);
+    VelRow row[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (lane + r * lanes < held) row[r] = loadVelRow(cv, lane + r * lanes);
+
+    // reg(r) over the constraints in registers, mem(k) over the others, colour
+    // after colour.
+    auto colours = [&](auto reg, auto mem) {
+        for (int c = 0; c < kColourSlots && cs[c] < nCons; ++c) {
+            const int b0 = cs[c], b1 = cs[c + 1];
+            if (b1 <= b0) continue;
+            if (c == kOverflowColour) {
+                if (lane == 0)
+                    for (int k = b0; k < b1; ++k) mem(k);
+            } else {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const int k = lane + r * lanes;
+                    if (k >= b0 && k < min(b1, held)) reg(r);
+                }
+                for (int k = max(b0, held) + lane; k < b1; k += lanes) mem(k);
+            }
+            teamBarrier(cnt, size, phase);
+        }
+    };
+    auto keep = [&](float4* rows, int info, int2 bodies, const float4& a, const float4& b) {
+        if (info & 16) rows[bodies.x] = a;
+        if (info & 32) rows[bodies.y] = b;
+    };
+    // b2Island::Solve, REF/Dynamics/b2Island.cpp:246-270
+    auto warm = [&](VelRow& r) {
+        float4 va = teamRow(w.vel + r.bodies.x), vb = teamRow(w.vel + r.bodies.y);
+        warmStartRow(r.info, r.mass, r.normal, r.imp, r.r0, r.r1, va, vb);
+        keep(w.vel, r.info, r.bodies, va, vb);
+    };
+    auto solve = [&](VelRow& r) {
+        float4 va = teamRow(w.vel + r.bodies.x), vb = teamRow(w.vel + r.bodies.y);
+        solveVelocityRow(r, va, vb);
+        keep(w.vel, r.info, r.bodies, va, vb);
+    };
+    if (p.contactWarm)
+        colours([&](int r) { warm(row[r]); },
+                [&](int k) {
+                    VelRow m = loadVelRow(cv, k);
+                    warm(m);
+                });
+    for (int it = 0; it < p.velIters; ++it)
+        colours([&](int r) { solve(row[r]); },
+                [&](int k) {
+                    VelRow m = loadVelRow(cv, k);
+                    solve(m);
+                    cv.imp[k] = m.imp;
+                });
+    // StoreImpulses by the lanes that hold them, and the position integration
+    // (b2Island.cpp:272-306).
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int k = lane + r * lanes;
+        if (k < held) storeImpulsesTo(w, cv.contact[k], row[r].info & 3, row[r].imp);
+    }
+    for (int c = 0; c < kColourSlots; ++c) {
+        const bool serial = c == kOverflowColour;
+        if (serial && lane != 0) continue;
+        for (int k = max(cs[c], held) + (serial ? 0 : lane); k < cs[c + 1]; k += serial ? 1 : lanes)
+            storeImpulsesOne(w, cv, k);
+    }
+    for (int b = lane; b < nb; b += lanes) {
+        if (!islandBody(w, b)) continue;
+        float4 pos = w.pos[b], v = teamRow(w.vel + b);
+        integratePosition(pos, v, p.h);
+        w.vel[b] = v;
+        w.pos[b] = pos;
+    }
+    PosRow prow[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (lane + r * lanes < held) prow[r] = loadPosRow(cv, lane + r * lanes);
+    teamBarrier(cnt, size, phase);
+    // Position iterations (b2Island.cpp:310-328), constraints of islands that
+    // the previous pass left solved passed over.
+    for (int it = 0; it < p.posIters; ++it) {
+        float lowest = 0.0f;
+        auto correct = [&](const PosRow& r) {
+            float4 pA = teamRow(w.pos + r.bodies.x), pB = teamRow(w.pos + r.bodies.y);
+            if (it > 0 && teamLoad((const unsigned*)&w.islandMinSep[(it - 1) * nb + r.island]) == 0u) return;
+            const float minSep = solvePositionRow(r, pA, pB);
+            keep(w.pos, r.info, r.bodies, pA, pB);
+            failIsland(w, r.island, it, minSep);
+            lowest = fminB(lowest, minSep);
+        };
+        colours([&](int r) { correct(prow[r]); }, [&](int k) { correct(loadPosRow(cv, k)); });
+        recordMinSep(cnt, it, 0, lowest);
+    }
+    for (int b = lane; b < nb; b += lanes)
+        if (islandBody(w, b)) syncTransformFrom(w, b, teamRow(w.pos + b));
 }
 
 // Sleep (b2Island::Solve, REF/Dynamics/b2Island.cpp:345-382): per island,
@@ -7395,6 +7631,41 @@ int labelIslands(b2g_context* ctx, const WorldView& w) {
     return B2G_OK;
 }
 
+// Colour counts of the step as the host keeps them: ranges, statistics.
+// tailBegin: the first of the trailing colours that share a launch.
+struct ColourLayout {
+    int start[kColourSlots + 1];
+    int nCons, nColours, tailBegin;
+};
+
+void coloursFromKeys(const int* orderCount, int* colourCount) {
+    for (int c = 0; c < kColourSlots; ++c) colourCount[c] = colourCountOf(orderCount, c);
+}
+
+ColourLayout colourLayout(const int* counts, int first, int tailColours) {
+    ColourLayout l;
+    l.start[0] = first;
+    for (int c = 0; c < kColourSlots; ++c) l.start[c + 1] = l.start[c] + counts[c];
+    l.nCons = l.start[kColourSlots];
+    l.nColours = 0;
+    for (int c = 0; c < kColourSlots; ++c)
+        if (counts[c] > 0) l.nColours = c + 1;
+    l.tailBegin = l.nColours;
+    if (tailColours > 0) {
+        while (l.tailBegin > 0 && l.start[l.tailBegin] - l.start[l.tailBegin - 1] <= tailColours) --l.tailBegin;
+        if (l.nColours - l.tailBegin < 2) l.tailBegin = l.nColours;  // one colour: no gain
+    }
+    return l;
+}
+
+// Constraints in the colours that get a solver launch each.
+int wideConstraints(const ColourLayout& l) {
+    int n = 0;
+    for (int c = 0; c < l.tailBegin; ++c)
+        if (c != kOverflowColour) n += l.start[c + 1] - l.start[c];
+    return n;
+}
+
 // Whether a step's solve goes to the block solve (k_solve_block): the bodies
 // fit its LDS rows and at most `constraints` constraints its reach, and
 // nothing has to look in between the passes (residual check, trace, log) or
@@ -7435,6 +7706,31 @@ void launchBlockSolve(b2g_context* ctx, const b2g_step_params* p, const WorldVie
     hipLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(lanes),
                        sizeof(float4) * (size_t)ctx->nBodies, ctx->stream, w, ctx->cv, jv, (const int*)ctx->consOrder,
                        plan, ctx->cnt);
+}
+
+// Whether a step's solve goes to the team solve (k_solve_team) when the block
+// solve does not take it. Settled piles, launches per colour against the team:
+// 8355 constraints 630 -> 450 us a step, 12 576 590 -> 500 us, 21 885
+// 633 -> 590 us, 33 886 658 -> 660 us (and 32 batched worlds of 14 700 in all
+// 515 -> 455 us): by then a colour has work enough for the whole chip.
+bool teamSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
+    if (ctx->nJoints > 0 || constraints == 0 || constraints > kTeamConstraints) return false;
+    if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->sched.clusterBodies > 0 || ctx->graphs)
+        return false;
+    if (ctx->traceIters > 0 || ctx->logCap > 0) return false;
+    return !(p->learnedWarmStart && p->residualThreshold > 0.0f);
+}
+
+void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView& w, int constraints,
+                     bool contactWarm) {
+    TeamPlan plan;
+    plan.h = p->dt;
+    plan.velIters = p->velocityIterations;
+    plan.posIters = std::min(p->positionIterations, kMaxPosIters);
+    plan.contactWarm = contactWarm ? 1 : 0;
+    plan.wanted = kTeamSize;
+    hipLaunchKernelGGL(constraints <= 4 * kTeamSize * kTeamLanes ? k_solve_team<4> : k_solve_team<8>,
+                       dim3(8 * kTeamSize), dim3(kTeamLanes), 0, ctx->stream, w, ctx->cv, plan, ctx->cnt);
 }
 
 // Whether the whole step after the narrowphase goes to the small-world kernels:
@@ -7514,41 +7810,6 @@ int stepColouredCollide(b2g_context* ctx, const b2g_step_params* p) {
         LAUNCHCHK(ctx);
     }
     return B2G_OK;
-}
-
-// Colour counts of the step as the host keeps them: ranges, statistics.
-// tailBegin: the first of the trailing colours that share a launch.
-struct ColourLayout {
-    int start[kColourSlots + 1];
-    int nCons, nColours, tailBegin;
-};
-
-void coloursFromKeys(const int* orderCount, int* colourCount) {
-    for (int c = 0; c < kColourSlots; ++c) colourCount[c] = colourCountOf(orderCount, c);
-}
-
-ColourLayout colourLayout(const int* counts, int first, int tailColours) {
-    ColourLayout l;
-    l.start[0] = first;
-    for (int c = 0; c < kColourSlots; ++c) l.start[c + 1] = l.start[c] + counts[c];
-    l.nCons = l.start[kColourSlots];
-    l.nColours = 0;
-    for (int c = 0; c < kColourSlots; ++c)
-        if (counts[c] > 0) l.nColours = c + 1;
-    l.tailBegin = l.nColours;
-    if (tailColours > 0) {
-        while (l.tailBegin > 0 && l.start[l.tailBegin] - l.start[l.tailBegin - 1] <= tailColours) --l.tailBegin;
-        if (l.nColours - l.tailBegin < 2) l.tailBegin = l.nColours;  // one colour: no gain
-    }
-    return l;
-}
-
-// Constraints in the colours that get a solver launch each.
-int wideConstraints(const ColourLayout& l) {
-    int n = 0;
-    for (int c = 0; c < l.tailBegin; ++c)
-        if (c != kOverflowColour) n += l.start[c + 1] - l.start[c];
-    return n;
 }
 
 // Statistics of the position iterations.
@@ -7829,6 +8090,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         if (wantFresh && (rc = ensureFresh(ctx)) != B2G_OK) return rc;
         const FreshView fv{wantFresh ? ctx->freshMask : nullptr, ctx->freshNum, ctx->freshAll, ctx->learnedScope};
         const bool block = nCons > 0 && blockSolveFits(ctx, p, nCons);
+        const bool team = !block && teamSolveFits(ctx, p, nCons);
         const int blockLanes = block ? blockSolveLanes(ctx, nCons) : 0;
         const bool blockInit = block && !wantFresh &&
                                nCons <= blockLanes * (ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>);
@@ -8061,6 +8323,10 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             pe = profStart(ctx);
             launchBlockSolve(ctx, p, w, jv, blockLanes, contactWarm, blockInit);
             profEnd(ctx, PH_SOLVE_V, pe);
+        } else if (team) {
+            pe = profStart(ctx);
+            launchTeamSolve(ctx, p, w, nCons, contactWarm);
+            profEnd(ctx, PH_SOLVE_V, pe);
         } else if (!persist) {
             startSolve(contactWarm);
             solveVelocity(p->velocityIterations);
@@ -8097,7 +8363,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             LAUNCHCHK(ctx);
             ctx->logCount = std::min(ctx->logCap, ctx->logCount + nFresh);
         }
-        if (block) {
+        if (block || team) {
             // done in the one launch
         } else if (persist) {
             // store, integrate, position passes and transforms (and the
@@ -8153,7 +8419,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         }  // !persist
         }  // !graphRan
         pe = profStart(ctx);
-        if (!graphRan && !persist && !block) hipLaunchKernelGGL(k_sync_transforms, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w);
+        if (!graphRan && !persist && !block && !team) hipLaunchKernelGGL(k_sync_transforms, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w);
         if (ctx->allowSleep) {
             hipLaunchKernelGGL(k_sleep_accum, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w, dt);
         }
@@ -8187,7 +8453,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         profEnd(ctx, PH_BROADPHASE, pe);
         positionStats(ctx, posIters, nCons);
         if (ctx->hcnt->barrierAbort)
-            return fail(ctx, B2G_ERR_STATE, "one-launch solve: a grid barrier wait passed its bound");
+            return fail(ctx, B2G_ERR_STATE, "one-launch solve: a barrier wait passed its bound");
     } else {
         if ((rc = compactContacts(ctx)) != B2G_OK) return rc;
         if ((rc = readCounters(ctx)) != B2G_OK) return rc;

@@ -7,7 +7,8 @@ that lanes hold in registers (1024 with 256 lanes, 2048 with 512; 768 and 1536
 with joints), the largest number of bodies in LDS and one beyond it, worlds
 that start with more new pairs than the LDS sort takes, every joint type, a
 body in more contacts than there are colours (the overflow colour), islands
-that sleep, contacts that end, sub-worlds, few iterations.
+that sleep, contacts that end, sub-worlds, few iterations. Larger worlds go to
+the team solve (the workgroups of one XCD with a barrier between colours).
 """
 import numpy as np
 import pytest
@@ -70,6 +71,9 @@ def same(a, b):
     ("ropes", 20, 0, 60, False, 8, 3), ("welds", 12, 0, 90, True, 8, 3), ("friction", 16, 0, 60, False, 8, 3),
     ("motor", 12, 0, 60, False, 8, 3), ("pulley", 8, 0, 60, False, 8, 3), ("mouse", 8, 0, 60, False, 8, 3),
     ("prismatic", 12, 0, 60, False, 8, 3), ("wheels", 6, 0, 90, False, 8, 3), ("gears", 4, 0, 60, False, 8, 3),
+    # the team solve
+    ("world", 4033, 8, 420, True, 8, 3), ("world", 6000, 9, 300, False, 6, 2), ("world", 13000, 10, 480, False, 8, 3),
+    ("world", 5000, 11, 240, False, 2, 0), ("world", 5000, 11, 240, False, 0, 2), ("plank", 4100, 0, 9, False, 8, 3),
 ])
 def test_equals_a_launch_per_colour(gpu, kind, n, seed, steps, sleep, vel, pos):
     a = run(gpu.world(kind, n, seed, sleep=sleep), False, steps, vel, pos)
