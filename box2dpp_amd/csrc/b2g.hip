@@ -57,7 +57,6 @@ constexpr int kOverflowColour = 64;   // solved serially when masks are full
 constexpr int kColourSlots = 65;
 constexpr int kMaxPosIters = 32;
 constexpr int kMaxCellsPerProxy = 16;
-constexpr int kColourRoundsUnchecked = 2;  // fewest colouring rounds launched before the first readback
 constexpr int kColourRoundSlots = 16;      // rounds whose leftovers are recorded (later rounds share the last)
 constexpr uint32_t kNotConstraintKey = 0x7Fu;  // order key of a contact outside the constraint set
 constexpr int kOrderKeys = 127;                // order keys of the constraint set
@@ -73,15 +72,15 @@ struct Counters {
     int nQueries;          // moved proxies binned in the grid (their queries)
     int nTiles;            // polygon-polygon contacts deferred to k_collide_tiles
     int nScanned;          // grid entries and wide proxies the queries examined
-    int colourRounds;      // colouring rounds of a small world's step
-    int smallPending;      // a small world's new pairs are left to the host
+    int colourRounds;      // rounds of the one-workgroup colouring
+    int colourLeft;        // constraints it left to rounds over the table
+    int appendPending;     // k_append_sorted left the new pairs to the host
     int roundLeft[kColourRoundSlots];  // constraints left uncoloured by colouring round r of the step
     int beginEvents;
     int endEvents;
     int points;
     int nEdges;
     int nIslands;
-    int islandChanged;     // set by a propagation round that lowered a label
     int nFresh;            // fresh contact points of the step (learned warm start, log, trace)
     int residualPoints;
     float residualSum;     // sum of squared complementarity residuals (k_residual)
@@ -558,8 +557,9 @@ __device__ inline bool islandContact(const WorldView& w, int c) {
 //    such an ancestor, so it keeps every invariant above.
 // Roots only ever move under smaller indices, so each component ends up
 // labelled with its smallest body index, for any thread schedule.
-__global__ void k_island_init(WorldView w) {
+__global__ void k_island_init(WorldView w, int posIters) {
     const int b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < w.nBodies * posIters) w.islandMinSep[b] = 0;
     if (b >= w.nBodies) return;
     w.islandOf[b] = b;
     w.islandAwake[b] = 0;
@@ -592,24 +592,22 @@ __device__ inline void islandUnion(int* L, int a, int b) {
     }
 }
 
-// A propagation round: each island contact lowers the larger of its
-// bodies' labels to the smaller (atomicMin only).
-__global__ void k_island_hook(WorldView w, int* changed) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= w.nContacts || !islandContact(w, c)) return;
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
-    if (w.btype[bA] == BT_STATIC || w.btype[bB] == BT_STATIC) return;
-    if (!(w.bflags[bA] & BF_ACTIVE) || !(w.bflags[bB] & BF_ACTIVE)) return;
-    const int la = w.islandOf[bA], lb = w.islandOf[bB];
-    if (la == lb) return;
-    atomicMin(&w.islandOf[la > lb ? la : lb], la < lb ? la : lb);
-    if (changed) *changed = 1;
-}
-
 // Island contacts and joints join islands only between non-static, active bodies.
 __device__ inline bool joinsIslands(const WorldView& w, int bA, int bB) {
     return w.btype[bA] != BT_STATIC && w.btype[bB] != BT_STATIC && (w.bflags[bA] & BF_ACTIVE) &&
            (w.bflags[bB] & BF_ACTIVE);
+}
+
+// A propagation round: each island contact lowers the larger of its
+// bodies' labels to the smaller (atomicMin only).
+__global__ void k_island_hook(WorldView w) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= w.nContacts || !islandContact(w, c)) return;
+    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
+    if (!joinsIslands(w, bA, bB)) return;
+    const int la = w.islandOf[bA], lb = w.islandOf[bB];
+    if (la == lb) return;
+    atomicMin(&w.islandOf[la > lb ? la : lb], la < lb ? la : lb);
 }
 
 __global__ void k_island_union(WorldView w) {
@@ -662,20 +660,23 @@ __global__ void k_island_mark(WorldView w) {
 
 // Constraint set of the step: island contacts of awake islands. Contacts
 // leaving the set give their colour back.
-__device__ inline void markConstraintOne(const WorldView& w, Counters* cnt, int c, int bA, int bB) {
+// Returns whether the constraint has no colour yet.
+__device__ inline bool markConstraintOne(const WorldView& w, int c, int bA, int bB) {
     int flags = w.cflags[c] & ~CF_CONSTRAINT;
     const bool isCons = islandContact(w, c) && ((w.bflags[bA] & BF_ISLAND) || (w.bflags[bB] & BF_ISLAND));
     if (!isCons) releaseColour(w, c, bA, bB);
-    if (isCons) {
-        flags |= CF_CONSTRAINT;
-        if (w.ccolour[c] < 0) atomicAdd(&cnt->remaining, 1);
-    }
+    if (isCons) flags |= CF_CONSTRAINT;
     w.cflags[c] = flags;
+    return isCons && w.ccolour[c] < 0;
 }
 
-__global__ void k_mark_constraints(WorldView w, Counters* cnt) {
+// list: the constraints without a colour (cnt->remaining of them, in no
+// fixed order).
+__global__ void k_mark_constraints(WorldView w, int* list, Counters* cnt) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c < w.nContacts) markConstraintOne(w, cnt, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
+    const bool fresh = c < w.nContacts && markConstraintOne(w, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]]);
+    const int slot = waveAppend(&cnt->remaining, fresh);
+    if (fresh) list[slot] = c;
 }
 
 struct ContactArrays {
@@ -789,6 +790,66 @@ __global__ void k_colour_commit(WorldView w, const unsigned long long* claim, ui
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= w.nContacts || !uncoloured(w, c)) return;
     if (!colourCommitOne(w, claim, tag, c, w.fbody[w.cfA[c]], w.fbody[w.cfB[c]])) atomicAdd(&cnt->roundLeft[round], 1);
+}
+
+// Claim tags of a one-workgroup colouring: base, base + 1, ..., and when they
+// run out the claims are cleared and the tags start over.
+struct ClaimTags {
+    uint32_t base;
+    int count, used;
+    __device__ uint32_t next(unsigned long long* claim, int nb) {
+        if (used == count) {
+            for (int b = threadIdx.x; b < nb; b += blockDim.x) claim[b] = 0ull;
+            __syncthreads();
+            used = 0;
+        }
+        return base + (uint32_t)used++;
+    }
+};
+
+// Colouring rounds by one workgroup over the n contacts id(0), id(1), ...
+// until none is left: every round colours at least one, so they end. `left` is
+// a word in LDS.
+template <typename Id, typename BodyA, typename BodyB>
+__device__ inline void colourByBlock(const WorldView& w, unsigned long long* claim, ClaimTags& tags, int n, Id id,
+                                     BodyA bodyA, BodyB bodyB, int* left, Counters* cnt) {
+    for (int round = 0; n > 0; ++round) {
+        const uint32_t tag = tags.next(claim, w.nBodies);
+        if (threadIdx.x == 0) *left = 0;
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            const int c = id(i);
+            if (uncoloured(w, c)) colourClaimOne(w, claim, tag, c, bodyA(c), bodyB(c));
+        }
+        __syncthreads();
+        for (int i = threadIdx.x; i < n; i += blockDim.x) {
+            const int c = id(i);
+            if (uncoloured(w, c) && !colourCommitOne(w, claim, tag, c, bodyA(c), bodyB(c))) atomicAdd(left, 1);
+        }
+        __syncthreads();
+        const int stay = *left;
+        if (threadIdx.x == 0) cnt->colourRounds = round + 1;
+        __syncthreads();
+        if (stay == 0) break;
+    }
+}
+
+// The colouring of a step's new constraints in one launch: of the table's
+// contacts only those few take part (some hundred in a 10 000-body pile), so a
+// round over the whole table in two launches, twice at least, cost 15 us.
+// More than kColourListMost are left to such rounds (cnt->colourLeft): all at
+// once they are more than one workgroup's work.
+constexpr int kColourListMost = 16384;
+constexpr int kClaimTags = 96;  // claim tags of a one-workgroup colouring
+__global__ void __launch_bounds__(1024)
+    k_colour_list(WorldView w, unsigned long long* claim, uint32_t tagBase, const int* list, Counters* cnt) {
+    __shared__ int left;
+    const int n = cnt->remaining;
+    if (threadIdx.x == 0) cnt->colourLeft = n > kColourListMost ? n : 0;
+    if (n > kColourListMost) return;
+    ClaimTags tags{tagBase, kClaimTags, 0};
+    colourByBlock(
+        w, claim, tags, n, [&](int i) { return list[i]; }, [&](int c) { return w.fbody[w.cfA[c]]; },
+        [&](int c) { return w.fbody[w.cfB[c]]; }, &left, cnt);
 }
 
 // Demotion: a constraint keeps its colour for its life, so when the
@@ -3893,7 +3954,7 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
 // launches with 110 and 210 us of kernel time.
 // ====================================================================
 constexpr int kBlockBodies = 4032;       // body rows in LDS: 63 of the 64 KB a launch may ask for
-constexpr int kBlockConstraints = 8192;  // most constraints (blockSolveFits)
+constexpr int kBlockConstraints = 4096;  // most constraints (blockSolveFits)
 constexpr int kBlockJointed = 4096;      // most constraints, and most joints, with joints
 constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane, whose rows take most of them
 template <bool kJoints>
@@ -4666,6 +4727,30 @@ __global__ void k_grid_reset(int* counts, int* cursor, int n, Counters* cnt) {
     }
 }
 
+// See closeTable. Without contacts there is nothing to compact: the live count
+// is zero.
+__global__ void k_close_table(WorldView w, int* keep, unsigned long long* table, uint32_t hashMask, int* counts,
+                              int* cursor, int nCounts, Counters* cnt) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+    for (long long k = i; k <= (long long)hashMask; k += stride) table[k] = ~0ull;
+    if (i < nCounts) {
+        counts[i] = 0;
+        cursor[i] = 0;
+    }
+    if (i == 0) {
+        cnt->nBig = 0;
+        cnt->nQueries = 0;
+        cnt->nNewPairs = 0;
+        cnt->overflow = 0;
+        if (w.nContacts == 0) cnt->nContacts = 0;
+    }
+    if (i < w.nContacts) keep[i] = (w.cflags[i] & CF_DEAD) ? 0 : 1;
+    if (i < w.nFixtures) {
+        const int b = w.fbody[i];
+        if (islandBody(w, b)) syncFixtureOne(w, i, b);
+    }
+}
+
 // Where queries put the pairs they find. With packBase = n (the proxy
 // count, or the order-key span with `ord`) a pair is stored as lo * n + hi,
 // lo < hi its two fixtures' order keys (`ord`, or the fixture indices when
@@ -4872,8 +4957,8 @@ __global__ void k_append_contacts(WorldView w, const unsigned long long* keys, i
 constexpr int kSmallLanes = 1024;
 constexpr int kSmallBodies = kBlockBodies;   // island labels in LDS
 constexpr int kSmallContacts = 5120;         // contact bodies in LDS (see smallWorldFits)
-constexpr int kSmallNewPairs = 4096;         // new pairs sorted in LDS
-constexpr int kSmallTags = 96;               // claim tags of a step
+constexpr int kSortedNewPairs = 4096;        // new pairs sorted in LDS
+constexpr int kAppendFixtures = 32768;       // move flags that one workgroup clears
 static_assert(kSmallBodies <= 1 << 13, "a packed body index has 13 bits");
 static_assert(sizeof(b2g_manifold) == 4 * sizeof(float4), "a manifold moves as four words of 16 bytes");
 
@@ -4940,42 +5025,17 @@ __global__ void __launch_bounds__(kSmallLanes)
     __syncthreads();
     for (int b = t; b < nb; b += T) islandMarkOne(wl, b);
     __syncthreads();
-    for (int c = t; c < nc; c += T) markConstraintOne(w, cnt, c, bodyA(c), bodyB(c));
+    for (int c = t; c < nc; c += T) (void)markConstraintOne(w, c, bodyA(c), bodyB(c));
     __syncthreads();
-    uint32_t used = 0;
-    auto nextTag = [&]() {
-        if ((int)used == tagCount) {
-            for (int b = t; b < nb; b += T) claim[b] = 0ull;
-            __syncthreads();
-            used = 0;
-        }
-        return tagBase + used++;
-    };
+    ClaimTags tags{tagBase, tagCount, 0};
     for (int r = 0; r < demoteRounds; ++r) {
-        const uint32_t tag = nextTag();
+        const uint32_t tag = tags.next(claim, nb);
         for (int c = t; c < nc; c += T) demoteClaimOne(w, claim, tag, c, bodyA(c), bodyB(c));
         __syncthreads();
         for (int c = t; c < nc; c += T) demoteCommitOne(w, claim, tag, c, bodyA(c), bodyB(c));
         __syncthreads();
     }
-    // Every round colours at least one constraint, so the rounds end.
-    for (int round = 0; nc > 0; ++round) {
-        const uint32_t tag = nextTag();
-        if (t == 0) left = 0;
-        for (int c = t; c < nc; c += T)
-            if (uncoloured(w, c)) colourClaimOne(w, claim, tag, c, bodyA(c), bodyB(c));
-        __syncthreads();
-        for (int c = t; c < nc; c += T)
-            if (uncoloured(w, c) && !colourCommitOne(w, claim, tag, c, bodyA(c), bodyB(c))) atomicAdd(&left, 1);
-        __syncthreads();
-        const int stay = left;
-        if (t == 0) {
-            cnt->roundLeft[min(round, kColourRoundSlots - 1)] = stay;
-            cnt->colourRounds = round + 1;
-        }
-        __syncthreads();
-        if (stay == 0) break;
-    }
+    colourByBlock(w, claim, tags, nc, [&](int i) { return i; }, bodyA, bodyB, &left, cnt);
     // Constraints by order key, in table order within a key: counts, then
     // chunks of T contacts ranked by a ballot per key bit and a count per
     // wavefront.
@@ -5141,15 +5201,15 @@ __global__ void k_small_pairs(WorldView w, GridView g, const unsigned long long*
 
 // The new pairs in key order into the table (a bitonic sort in LDS), the move
 // flags and the forces cleared. Pairs that fit neither the sort nor the table
-// are left to the host (cnt->smallPending), with the move flags as they are.
+// are left to the host (cnt->appendPending), with the move flags as they are.
 __global__ void __launch_bounds__(kSmallLanes)
-    k_small_append(WorldView w, const unsigned long long* newKeys, unsigned long long packBase, int capContacts,
+    k_append_sorted(WorldView w, const unsigned long long* newKeys, unsigned long long packBase, int capContacts,
                    int clearForces, Counters* cnt) {
-    __shared__ unsigned long long keys[kSmallNewPairs];
+    __shared__ unsigned long long keys[kSortedNewPairs];
     const int t = threadIdx.x, T = blockDim.x;
     const int n = cnt->nNewPairs, base = cnt->nContacts;
-    const bool fits = !cnt->overflow && n <= kSmallNewPairs && base + n <= capContacts;
-    if (t == 0) cnt->smallPending = fits ? 0 : 1;
+    const bool fits = !cnt->overflow && n <= kSortedNewPairs && base + n <= capContacts;
+    if (t == 0) cnt->appendPending = fits ? 0 : 1;
     if (!fits) return;
     if (n > 0) {
         int size = 1;
@@ -5174,7 +5234,9 @@ __global__ void __launch_bounds__(kSmallLanes)
             appendContactOne(w, fixtureOf(w, (int)(keys[i] / packBase)), fixtureOf(w, (int)(keys[i] % packBase)),
                              base + i);
     }
-    for (int f = t; f < w.nFixtures; f += T) w.moved[f] = 0;
+    uint4* moved = (uint4*)w.moved;
+    for (int i = t; i < w.nFixtures / 16; i += T) moved[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (int f = (w.nFixtures & ~15) + t; f < w.nFixtures; f += T) w.moved[f] = 0;
     if (clearForces)
         for (int b = t; b < w.nBodies; b += T) w.force[b] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
 }
@@ -6611,6 +6673,7 @@ struct b2g_context {
     int demoteRounds = 1;           // colour demotion rounds per coloured step
     int compactedFrom = -1;  // table length before the last coloured step's compaction (-1: none)
     int colourRoundsNeeded = 0;  // colouring rounds the last coloured step needed
+    int lastNewPairs = 0;        // new pairs of the last broad-phase
     int lastConstraints = 0;
 
     // profiling (HIP events around launches)
@@ -6892,7 +6955,7 @@ void chooseCellSize(b2g_context* ctx, const b2g_fixture_def* defs, int n, const 
     }
 }
 
-int rebuildHash(b2g_context* ctx, bool liveOnDevice = false);
+int rebuildHash(b2g_context* ctx);
 
 // Keeps a third of the contact capacity free ahead of the step.
 int reserveContacts(b2g_context* ctx) {
@@ -6925,6 +6988,21 @@ int readCounters(b2g_context* ctx);
 int profKernelEvents(b2g_context* ctx, hipEvent_t* start, hipEvent_t* stop);
 void profKernel(b2g_context* ctx, int phase, int i);
 
+void pairStats(b2g_context* ctx) {
+    ctx->lastNewPairs = ctx->hcnt->nNewPairs;
+    ctx->stats.newPairs += ctx->hcnt->nNewPairs;
+    ctx->stats.queries = ctx->hcnt->nQueries;
+    ctx->stats.scanned = ctx->hcnt->nScanned;
+}
+
+// The set of live pairs is rebuilt by every broad-phase, so it need not use
+// the whole table: a quarter to half full.
+uint32_t liveHashMask(const b2g_context* ctx) {
+    uint32_t mask = 1023;
+    while ((long long)mask < 2ll * ctx->nContacts) mask = 2 * mask + 1;
+    return std::min(mask, ctx->hashMask);
+}
+
 GridView gridView(const b2g_context* ctx) {
     GridView g;
     g.invCell = 1.0f / ctx->cellSize;
@@ -6940,14 +7018,20 @@ GridView gridView(const b2g_context* ctx) {
     return g;
 }
 
-// liveOnDevice: the contact table was compacted without a readback
-// (compactContacts); the query's readback brings the live count.
-int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
+// closedMask: the step's own broad-phase, after closeTable with that hash mask
+// (the grid cleared, the pair set rebuilt, the live contact count on the
+// device, which the query's readback brings). Its new pairs are sorted and
+// appended by one kernel before that readback, as long as there were few in
+// the last step: 440 pairs of a 10 000-body pile took a sort made for 4096
+// (17 us) and five launches.
+int runBroadphase(b2g_context* ctx, const uint32_t* closedMask = nullptr) {
     hipStream_t s = ctx->stream;
     const int nf = ctx->nFixtures;
     if (ctx->orderSpan > 0 && ctx->orderCount != nf)
         return fail(ctx, B2G_ERR_STATE,
                     "proxy ids cover " + std::to_string(ctx->orderCount) + " of " + std::to_string(nf) + " fixtures");
+    const bool liveOnDevice = closedMask != nullptr;
+    uint32_t hashMask = closedMask ? *closedMask : ctx->hashMask;
     if (nf == 0) {
         if (liveOnDevice) {
             const int rc = readCounters(ctx);
@@ -6957,8 +7041,9 @@ int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
         return B2G_OK;
     }
     GridView g = gridView(ctx);
-    hipLaunchKernelGGL(k_grid_reset, dim3(blocks(ctx->nBuckets + 1)), dim3(256), 0, s, ctx->gCounts, ctx->gCursor,
-                       ctx->nBuckets + 1, ctx->cnt);
+    if (!closedMask)
+        hipLaunchKernelGGL(k_grid_reset, dim3(blocks(ctx->nBuckets + 1)), dim3(256), 0, s, ctx->gCounts, ctx->gCursor,
+                           ctx->nBuckets + 1, ctx->cnt);
     hipLaunchKernelGGL(k_grid_count, dim3(blocks(nf)), dim3(256), 0, s, ctx->fat, ctx->moved, nf,
                        (const uint8_t*)nullptr, g, ctx->cnt);
     LAUNCHCHK(ctx);
@@ -6996,22 +7081,33 @@ int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
         const long long queryThreads = std::min((long long)nf * kQueryLanes, 32768LL * kQueryLanes);
         hipExtLaunchKernelGGL(k_pairs_query, dim3((unsigned)((queryThreads + qb - 1) / qb)), dim3(qb), 0,
                               s, e0, e1, 0, ctx->fat, ctx->moved, nf, g, ctx->view(), true, ctx->hashTable,
-                              ctx->hashMask, sink, ctx->cnt);
+                              hashMask, sink, ctx->cnt);
         if (ctx->profiling)
             hipLaunchKernelGGL(k_count_scanned, dim3(blocks(nf)), dim3(256), 0, s, nf, g, ctx->cnt);
         profKernel(ctx, PH_K_PAIRS_QUERY, pk);
         hipLaunchKernelGGL(k_pairs_wide, dim3(blocks(nf)), dim3(256), 0, s, ctx->fat, ctx->moved, nf, g, ctx->view(),
-                           true, ctx->hashTable, ctx->hashMask, sink, ctx->cnt);
+                           true, ctx->hashTable, hashMask, sink, ctx->cnt);
+        const bool append = liveOnDevice && attempt == 0 && ctx->lastNewPairs <= 3 * kSortedNewPairs / 4 &&
+                            nf <= kAppendFixtures;
+        if (append)
+            hipLaunchKernelGGL(k_append_sorted, dim3(1), dim3(kSmallLanes), 0, s, ctx->view(), ctx->newKeys,
+                               (unsigned long long)packBase, ctx->capContacts, 0, ctx->cnt);
         LAUNCHCHK(ctx);
         HIPCHK(ctx, hipMemcpyAsync(ctx->hcnt, ctx->cnt, sizeof(Counters), hipMemcpyDeviceToHost, s));
         HIPCHK(ctx, hipStreamSynchronize(s));
         if (liveOnDevice && attempt == 0) ctx->nContacts = ctx->hcnt->nContacts;
         nNew = ctx->hcnt->nNewPairs;
+        if (append && !ctx->hcnt->appendPending) {
+            ctx->nContacts += nNew;
+            pairStats(ctx);
+            return B2G_OK;
+        }
         if (!ctx->hcnt->overflow && ctx->nContacts + nNew <= ctx->capContacts) break;
         if (attempt >= 2) return fail(ctx, B2G_ERR_CAPACITY, "contact capacity exceeded in the broad-phase");
         int rc = growContacts(ctx, std::max(2 * ctx->capContacts, ctx->nContacts + nNew + 4096));
         if (rc != B2G_OK) return rc;
         if ((rc = rebuildHash(ctx)) != B2G_OK) return rc;
+        hashMask = ctx->hashMask;
     }
     hipLaunchKernelGGL(k_fill<uint8_t>, dim3(blocks(nf)), dim3(256), 0, s, ctx->moved, nf, (uint8_t)0);
     WorldView w = ctx->view();
@@ -7026,21 +7122,17 @@ int runBroadphase(b2g_context* ctx, bool liveOnDevice = false) {
         LAUNCHCHK(ctx);
         ctx->nContacts += nNew;
     }
-    ctx->stats.newPairs += nNew;
-    ctx->stats.queries = ctx->hcnt->nQueries;
-    ctx->stats.scanned = ctx->hcnt->nScanned;
+    pairStats(ctx);
     return B2G_OK;
 }
 
-// liveOnDevice: ctx->nContacts only bounds the table; the live count is the
-// device's (set by k_compact).
-int rebuildHash(b2g_context* ctx, bool liveOnDevice) {
+int rebuildHash(b2g_context* ctx) {
     hipStream_t s = ctx->stream;
     hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(blocks(ctx->hashCap)), dim3(256), 0, s, ctx->hashTable,
                        ctx->hashCap, ~0ull);
     if (ctx->nContacts > 0)
         hipLaunchKernelGGL(k_hash_insert, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, ctx->view(), ctx->hashTable,
-                           ctx->hashMask, liveOnDevice ? (const Counters*)ctx->cnt : (const Counters*)nullptr);
+                           ctx->hashMask, (const Counters*)nullptr);
     LAUNCHCHK(ctx);
     return B2G_OK;
 }
@@ -7586,47 +7678,33 @@ int solveByGraph(b2g_context* ctx, const WorldView& w, const JointView& jv, cons
 }
 
 // Island labels (each body labelled with the smallest body index of its
-// island) by the schedule's method; all three give the same labels.
-//  0: propagation rounds (two per host check of the change flag) until
-//     none lowers a label; best for a few large islands;
-//  1: one propagation round, then the union-find pass;
-//  2: the union-find pass alone; best for many small islands.
+// island) by the schedule's method; all three give the same labels, and all end
+// in a union-find pass, which needs no readback to know that it is done.
+//  0: propagation rounds first, as many as pay: in a pile's one large island
+//     the union-find pass has its wavefronts fight over the same roots (455 000
+//     contacts: a step of 1.65 ms after one round, 1.32 ms with rounds until
+//     nothing changes), so large tables get three, which leave it little to do;
+//     small ones get one (34 000 contacts 630 -> 600 us, against rounds with
+//     their change flag read back);
+//  1: one propagation round;
+//  2: none; best for many small islands.
 // Joints join islands by the union-find pass in every method.
+constexpr int kPropagateContacts = 65536;
 int labelIslands(b2g_context* ctx, const WorldView& w) {
     hipStream_t s = ctx->stream;
     const int nb = ctx->nBodies, nc = ctx->nContacts;
     const int method = ctx->sched.islands;
-    if (nc > 0 && method == 0) {
-        for (int pass = 0;; ++pass) {
-            // rounds before the checked one: four on the first pass (most
-            // scenes settle within them), one after; a checked round that
-            // lowers no label means the labels are final
-            const int unchecked = pass == 0 ? 3 : 1;
-            for (int r = 0; r < unchecked; ++r) {
-                hipLaunchKernelGGL(k_island_hook, dim3(blocks(nc)), dim3(256), 0, s, w, (int*)nullptr);
-                hipLaunchKernelGGL(k_island_jump, dim3(blocks(nb)), dim3(256), 0, s, w);
-            }
-            hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, s, &ctx->cnt->islandChanged, 1, 0);
-            hipLaunchKernelGGL(k_island_hook, dim3(blocks(nc)), dim3(256), 0, s, w, &ctx->cnt->islandChanged);
-            hipLaunchKernelGGL(k_island_jump, dim3(blocks(nb)), dim3(256), 0, s, w);
-            LAUNCHCHK(ctx);
-            HIPCHK(ctx, hipMemcpyAsync(&ctx->hcnt->islandChanged, &ctx->cnt->islandChanged, sizeof(int),
-                                       hipMemcpyDeviceToHost, s));
-            HIPCHK(ctx, hipStreamSynchronize(s));
-            if (!ctx->hcnt->islandChanged) break;
-            // every round that changes something lowers a label, so this is a safeguard only
-            if (pass >= 1000000) return fail(ctx, B2G_ERR_STATE, "island labelling did not converge");
-        }
-    } else if (nc > 0) {
-        if (method == 1) {
-            hipLaunchKernelGGL(k_island_hook, dim3(blocks(nc)), dim3(256), 0, s, w, (int*)nullptr);
+    if (nc > 0) {
+        const int rounds = method == 0 ? (nc < kPropagateContacts ? 1 : 3) : method == 1 ? 1 : 0;
+        for (int r = 0; r < rounds; ++r) {
+            hipLaunchKernelGGL(k_island_hook, dim3(blocks(nc)), dim3(256), 0, s, w);
             hipLaunchKernelGGL(k_island_jump, dim3(blocks(nb)), dim3(256), 0, s, w);
         }
         hipLaunchKernelGGL(k_island_union, dim3(blocks(nc)), dim3(256), 0, s, w);
     }
     if (ctx->nJoints > 0)
         hipLaunchKernelGGL(k_island_union_joints, dim3(blocks(ctx->nJoints)), dim3(256), 0, s, w, ctx->jview());
-    if (method != 0 || ctx->nJoints > 0) hipLaunchKernelGGL(k_island_jump, dim3(blocks(nb)), dim3(256), 0, s, w);
+    hipLaunchKernelGGL(k_island_jump, dim3(blocks(nb)), dim3(256), 0, s, w);
     LAUNCHCHK(ctx);
     return B2G_OK;
 }
@@ -7743,7 +7821,7 @@ void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView
 // 341 -> 232 us, 4500 401 -> 356 us, but 6600 457 -> 480 us.
 bool smallWorldFits(const b2g_context* ctx, const b2g_step_params* p) {
     return blockSolveFits(ctx, p, ctx->nContacts) && ctx->nFixtures <= kSmallBodies && ctx->nFixtures > 0 &&
-           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && !ctx->profiling && ctx->demoteRounds < kSmallTags &&
+           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && !ctx->profiling && ctx->demoteRounds < kClaimTags &&
            (ctx->orderSpan == 0 || ctx->orderCount == ctx->nFixtures);
 }
 
@@ -7812,6 +7890,14 @@ int stepColouredCollide(b2g_context* ctx, const b2g_step_params* p) {
     return B2G_OK;
 }
 
+// The colouring rounds reported: as many as the last step needed, two at
+// least, and those this step needed if they are more.
+void roundStats(b2g_context* ctx, int needed) {
+    const int least = std::min(std::max(ctx->colourRoundsNeeded, 2), kColourRoundSlots - 1);
+    ctx->stats.colouringRounds = std::max(least, needed);
+    ctx->colourRoundsNeeded = needed;
+}
+
 // Statistics of the position iterations.
 void positionStats(b2g_context* ctx, int posIters, int nCons) {
     int ran = 0;
@@ -7833,7 +7919,7 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     const int posIters = std::min(p->positionIterations, kMaxPosIters);
     int rc;
     if (ctx->jointsDirty && (rc = recolourJoints(ctx)) != B2G_OK) return rc;
-    if (ctx->claimTag + kSmallTags >= 0xFFFF) {
+    if (ctx->claimTag + kClaimTags >= 0xFFFF) {
         hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, ctx->claim,
                            ctx->nBodies, 0ull);
         ctx->claimTag = 0;
@@ -7843,8 +7929,8 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     jv.h = p->dt;
     const int before = ctx->nContacts;
     hipLaunchKernelGGL(k_small_prepare, dim3(1), dim3(kSmallLanes), 0, s, w, jv, ctx->claim, ctx->claimTag + 1,
-                       kSmallTags, ctx->nContacts > 0 ? ctx->demoteRounds : 0, posIters, ctx->consOrder, ctx->cnt);
-    ctx->claimTag += kSmallTags;
+                       kClaimTags, ctx->nContacts > 0 ? ctx->demoteRounds : 0, posIters, ctx->consOrder, ctx->cnt);
+    ctx->claimTag += kClaimTags;
     launchBlockSolve(ctx, p, w, jv, blockSolveLanes(ctx, ctx->nContacts), ctx->warmStarting, true);
 
     SmallFinish fin;
@@ -7857,11 +7943,7 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     fin.keep = ctx->keep;
     fin.idx = ctx->idx;
     fin.table = ctx->hashTable;
-    // the set of live pairs is rebuilt every step: half full at most here, its
-    // whole size where TOI events go on with it
-    fin.hashMask = 1023;
-    while ((int)fin.hashMask < 2 * ctx->nContacts) fin.hashMask = 2 * fin.hashMask + 1;
-    if (ctx->continuous || fin.hashMask > ctx->hashMask) fin.hashMask = ctx->hashMask;
+    fin.hashMask = liveHashMask(ctx);
     fin.nBuckets = 256;
     while (fin.nBuckets < 2 * ctx->nFixtures) fin.nBuckets *= 2;
     fin.nBuckets = std::min(fin.nBuckets, ctx->nBuckets);
@@ -7873,11 +7955,11 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     const PairSink sink{ctx->newKeys, ctx->capContacts, (unsigned long long)packBase, ordered ? ctx->fixOrder : nullptr};
     hipLaunchKernelGGL(k_small_pairs, dim3(blocks(ctx->nFixtures * kQueryLanes)), dim3(256), 0, s, w, g, ctx->hashTable,
                        fin.hashMask, sink, ctx->cnt);
-    hipLaunchKernelGGL(k_small_append, dim3(1), dim3(kSmallLanes), 0, s, w, ctx->newKeys, (unsigned long long)packBase,
+    hipLaunchKernelGGL(k_append_sorted, dim3(1), dim3(kSmallLanes), 0, s, w, ctx->newKeys, (unsigned long long)packBase,
                        ctx->capContacts, ctx->autoClearForces && !ctx->continuous ? 1 : 0, ctx->cnt);
     LAUNCHCHK(ctx);
     if ((rc = readCounters(ctx)) != B2G_OK) return rc;
-    *forcesCleared = !ctx->hcnt->smallPending && !ctx->continuous;
+    *forcesCleared = !ctx->hcnt->appendPending && !ctx->continuous;
 
     coloursFromKeys(ctx->hcnt->orderCount, ctx->hcnt->colourCount);
     const ColourLayout layout = colourLayout(ctx->hcnt->colourCount, 0, ctx->sched.tailColours);
@@ -7887,25 +7969,48 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     ctx->stats.constraints = layout.nCons;
     ctx->stats.colours = layout.nColours;
     ctx->stats.wideConstraints = wideConstraints(layout);
-    // the rounds the stage kernels would have launched
-    if (before > 0) {
-        const int unchecked =
-            std::min(std::max(ctx->colourRoundsNeeded, kColourRoundsUnchecked), kColourRoundSlots - 1);
-        ctx->stats.colouringRounds = std::max(unchecked, ctx->hcnt->colourRounds);
-        ctx->colourRoundsNeeded = ctx->hcnt->colourRounds;
-    }
+    if (before > 0) roundStats(ctx, ctx->hcnt->colourRounds);
     ctx->nContacts = ctx->hcnt->nContacts;
-    if (ctx->hcnt->smallPending) {
+    if (ctx->hcnt->appendPending) {
         // more new pairs than the LDS sort or the table takes
         if ((rc = rebuildHash(ctx)) != B2G_OK) return rc;
         if ((rc = runBroadphase(ctx)) != B2G_OK) return rc;
     } else {
         ctx->nContacts += ctx->hcnt->nNewPairs;
-        ctx->stats.newPairs += ctx->hcnt->nNewPairs;
-        ctx->stats.queries = ctx->hcnt->nQueries;
-        ctx->stats.scanned = ctx->hcnt->nScanned;
+        pairStats(ctx);
     }
     positionStats(ctx, posIters, layout.nCons);
+    return B2G_OK;
+}
+
+// The end of a step's solve up to the queries: swept fat boxes, the contact
+// table compacted, the set of live pairs and the grid rebuilt. The first of
+// its kernels does everything that waits for nothing: boxes, keep flags, the
+// clearing of the pair set and of the grid.
+int closeTable(b2g_context* ctx, uint32_t hashMask) {
+    hipStream_t s = ctx->stream;
+    const WorldView w = ctx->view();
+    const int nc = ctx->nContacts;
+    const int n = std::max(std::max(nc, ctx->nFixtures), std::max(ctx->nBuckets + 1, 1));
+    int pe = profStart(ctx);
+    hipLaunchKernelGGL(k_close_table, dim3(blocks(n)), dim3(256), 0, s, w, ctx->keep, ctx->hashTable, hashMask,
+                       ctx->gCounts, ctx->gCursor, ctx->nBuckets + 1, ctx->cnt);
+    profEnd(ctx, PH_SYNC, pe);
+    LAUNCHCHK(ctx);
+    ctx->compactedFrom = nc;  // idx[] maps the step's contact indices to the compacted table
+    if (nc == 0) return B2G_OK;
+    pe = profStart(ctx);
+    HIPCHK(ctx, prims_exclusive_sum(ctx->scratch, ctx->scratchBytes, ctx->keep, ctx->idx, nc, s));
+    hipLaunchKernelGGL(k_compact, dim3(blocks(nc)), dim3(256), 0, s, ctx->cur, ctx->alt, ctx->keep, ctx->idx, nc,
+                       ctx->cnt);
+    profEnd(ctx, PH_COMPACT, pe);
+    LAUNCHCHK(ctx);
+    std::swap(ctx->cur, ctx->alt);
+    pe = profStart(ctx);
+    hipLaunchKernelGGL(k_hash_insert, dim3(blocks(nc)), dim3(256), 0, s, ctx->view(), ctx->hashTable, hashMask,
+                       (const Counters*)ctx->cnt);
+    profEnd(ctx, PH_BROADPHASE, pe);
+    LAUNCHCHK(ctx);
     return B2G_OK;
 }
 
@@ -7943,15 +8048,13 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         {
             const int pe = profStart(ctx);
             const int nb = ctx->nBodies;
-            hipLaunchKernelGGL(k_fill<int>, dim3(blocks(nb * std::max(posIters, 1))), dim3(256), 0, s,
-                               ctx->islandMinSep, nb * std::max(posIters, 1), 0);
-            hipLaunchKernelGGL(k_island_init, dim3(blocks(nb)), dim3(256), 0, s, w);
+            hipLaunchKernelGGL(k_island_init, dim3(blocks(nb * std::max(posIters, 1))), dim3(256), 0, s, w, posIters);
             if ((rc = labelIslands(ctx, w)) != B2G_OK) return rc;
             hipLaunchKernelGGL(k_island_roots, dim3(blocks(nb)), dim3(256), 0, s, w);
             hipLaunchKernelGGL(k_island_mark, dim3(blocks(nb)), dim3(256), 0, s, w);
-            hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, s, &ctx->cnt->remaining, 1, 0);
             if (ctx->nContacts > 0)
-                hipLaunchKernelGGL(k_mark_constraints, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w, ctx->cnt);
+                hipLaunchKernelGGL(k_mark_constraints, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w, ctx->idx,
+                                   ctx->cnt);
             profEnd(ctx, PH_ISLANDS, pe);
             LAUNCHCHK(ctx);
         }
@@ -7970,16 +8073,18 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             profEnd(ctx, PH_COLOUR, pe);
             LAUNCHCHK(ctx);
         }
-        // Colour new constraints: rounds are launched without a readback
-        // (a round with nothing left to colour changes nothing), and the count
-        // still uncoloured comes back with the order's counts below.
+        // Colour new constraints in one launch, or, when it finds too many, in
+        // rounds over the table with the count that is left read back.
         int rounds = 0;
-        auto colourRound = [&]() -> int {
-            if (ctx->claimTag >= 0xFFFF) {
+        auto freshTags = [&](int n) {
+            if (ctx->claimTag + n >= 0xFFFF) {
                 hipLaunchKernelGGL(k_fill<unsigned long long>, dim3(blocks(ctx->nBodies)), dim3(256), 0, s,
                                    ctx->claim, ctx->nBodies, 0ull);
                 ctx->claimTag = 0;
             }
+        };
+        auto colourRound = [&]() -> int {
+            freshTags(1);
             const uint32_t tag = ++ctx->claimTag;
             const int slot = std::min(rounds, kColourRoundSlots - 1);
             const int pe = profStart(ctx);
@@ -7992,12 +8097,15 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
             if (++rounds > 100000) return fail(ctx, B2G_ERR_STATE, "colouring did not converge");
             return B2G_OK;
         };
-        // as many unchecked rounds as the last step needed, at least two
-        const int unchecked =
-            std::min(std::max(ctx->colourRoundsNeeded, kColourRoundsUnchecked), kColourRoundSlots - 1);
-        if (ctx->nContacts > 0)
-            for (int r = 0; r < unchecked; ++r)
-                if ((rc = colourRound()) != B2G_OK) return rc;
+        if (ctx->nContacts > 0) {
+            freshTags(kClaimTags);
+            const int pe = profStart(ctx);
+            hipLaunchKernelGGL(k_colour_list, dim3(1), dim3(1024), 0, s, w, ctx->claim, ctx->claimTag + 1, ctx->idx,
+                               ctx->cnt);
+            profEnd(ctx, PH_COLOUR, pe);
+            ctx->claimTag += kClaimTags;
+            LAUNCHCHK(ctx);
+        }
         auto leftAfterLast = [&]() { return ctx->hcnt->roundLeft[std::min(rounds - 1, kColourRoundSlots - 1)]; };
         // Constraint order by colour; in the clustered solve by (cluster or
         // the boundary set, colour), and colourStart then holds the boundary
@@ -8050,21 +8158,15 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         };
         if (ctx->nContacts > 0) {
             if ((rc = order()) != B2G_OK) return rc;
-            if (leftAfterLast() > 0) {
-                // the colouring needed more rounds: finish it, then order again
-                while (leftAfterLast() > 0) {
+            if (ctx->hcnt->colourLeft > 0) {
+                // too many for one workgroup: rounds over the table, then order again
+                do {
                     if ((rc = colourRound()) != B2G_OK) return rc;
                     if ((rc = readCounters(ctx)) != B2G_OK) return rc;
-                }
+                } while (leftAfterLast() > 0);
                 if ((rc = order()) != B2G_OK) return rc;
             }
-            int needed = rounds;
-            for (int r = 0; r < std::min(rounds, kColourRoundSlots); ++r)
-                if (ctx->hcnt->roundLeft[r] == 0) {
-                    needed = r + 1;
-                    break;
-                }
-            ctx->colourRoundsNeeded = needed;
+            roundStats(ctx, rounds > 0 ? rounds : std::max(ctx->hcnt->colourRounds, 1));
             layout = colourLayout(ctx->hcnt->colourCount, clustered ? ctx->hcnt->boundaryStart : 0,
                                   ctx->sched.tailColours);
         }
@@ -8072,7 +8174,6 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         // Trailing colours with at most sched.tailColours constraints each go to
         // one workgroup (tailLaunch); the colours before them get a launch each.
         const int tailBegin = layout.tailBegin;
-        ctx->stats.colouringRounds = rounds;
         memcpy(ctx->lastColourStart, layout.start, sizeof(layout.start));
         ctx->lastConstraints = nCons;
         ctx->stats.constraints = nCons;
@@ -8441,15 +8542,14 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         if (ctx->allowSleep) {
             hipLaunchKernelGGL(k_sleep_apply, dim3(blocks(ctx->nBodies)), dim3(256), 0, s, w, posIters);
         }
-        hipLaunchKernelGGL(k_sync_fixtures, dim3(blocks(ctx->nFixtures)), dim3(256), 0, s, w);
         profEnd(ctx, PH_SYNC, pe);
         LAUNCHCHK(ctx);
         // Broad-phase against the compacted contact set (its readback brings
         // the live count).
-        if ((rc = compactContacts(ctx)) != B2G_OK) return rc;
+        const uint32_t hashMask = liveHashMask(ctx);
+        if ((rc = closeTable(ctx, hashMask)) != B2G_OK) return rc;
         pe = profStart(ctx);
-        if ((rc = rebuildHash(ctx, true)) != B2G_OK) return rc;
-        if ((rc = runBroadphase(ctx, true)) != B2G_OK) return rc;
+        if ((rc = runBroadphase(ctx, &hashMask)) != B2G_OK) return rc;
         profEnd(ctx, PH_BROADPHASE, pe);
         positionStats(ctx, posIters, nCons);
         if (ctx->hcnt->barrierAbort)
