@@ -5381,61 +5381,75 @@ __global__ void k_collide_compute(WorldView w, RefView r) {
     r.tmpMan[c] = m;
 }
 
-// Sequential commit in the reference's list order: activity is read as
-// earlier contacts' wake-ups leave it.
-__global__ void k_collide_serial(WorldView w, RefView r, Counters* cnt) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    for (int c = w.nContacts - 1; c >= 0; --c) {
-        int flags = w.cflags[c] & ~CF_UPDATED;
-        const int fA = w.cfA[c], fB = w.cfB[c];
-        const int bA = w.fbody[fA], bB = w.fbody[fB];
-        const bool destroyWake = w.cman[c].pointCount > 0 && !sensorOf(w, fA) && !sensorOf(w, fB);
-        if (removedFixture(w, fA) || removedFixture(w, fB) || (flags & CF_DESTROY)) {
-            if (flags & CF_TOUCHING) cnt->endEvents++;
-            w.cflags[c] = flags | CF_DEAD;
-            continue;
-        }
-        if (flags & CF_FILTER) {
-            const bool dynAny = w.btype[bA] == BT_DYNAMIC || w.btype[bB] == BT_DYNAMIC;
-            if (!dynAny || jointKeepsApart(w, bA, bB) || !filterPass(w, fA, fB)) {
-                if (flags & CF_TOUCHING) cnt->endEvents++;
-                if (destroyWake) { wakeBody(w, bA); wakeBody(w, bB); }
-                w.cflags[c] = flags | CF_DEAD;
-                continue;
-            }
-            flags &= ~CF_FILTER;
-        }
-        const bool activeA = (w.bflags[bA] & BF_AWAKE) && w.btype[bA] != BT_STATIC;
-        const bool activeB = (w.bflags[bB] & BF_AWAKE) && w.btype[bB] != BT_STATIC;
-        if (!activeA && !activeB) {
-            w.cflags[c] = flags;
-            continue;
-        }
-        if (!r.overlap[c]) {
-            if (flags & CF_TOUCHING) cnt->endEvents++;
+// b2ContactManager::Collide's step for one contact, its narrowphase done ahead.
+__device__ inline void commitContact(const WorldView& w, const RefView& r, Counters* cnt, int c) {
+    int flags = w.cflags[c] & ~CF_UPDATED;
+    const int fA = w.cfA[c], fB = w.cfB[c];
+    const int bA = w.fbody[fA], bB = w.fbody[fB];
+    const bool destroyWake = w.cman[c].pointCount > 0 && !sensorOf(w, fA) && !sensorOf(w, fB);
+    if (removedFixture(w, fA) || removedFixture(w, fB) || (flags & CF_DESTROY)) {
+        if (flags & CF_TOUCHING) atomicAdd(&cnt->endEvents, 1);
+        w.cflags[c] = flags | CF_DEAD;
+        return;
+    }
+    if (flags & CF_FILTER) {
+        const bool dynAny = w.btype[bA] == BT_DYNAMIC || w.btype[bB] == BT_DYNAMIC;
+        if (!dynAny || jointKeepsApart(w, bA, bB) || !filterPass(w, fA, fB)) {
+            if (flags & CF_TOUCHING) atomicAdd(&cnt->endEvents, 1);
             if (destroyWake) { wakeBody(w, bA); wakeBody(w, bB); }
             w.cflags[c] = flags | CF_DEAD;
-            continue;
+            return;
         }
-        if (sensorOf(w, fA) || sensorOf(w, fB)) {
-            sensorFinish(w, cnt, c, flags, r.overlap[c] == 3);
-            continue;
-        }
-        const b2g_manifold old = w.cman[c];
-        b2g_manifold m = r.tmpMan[c];
-        const bool wasTouching = (flags & CF_TOUCHING) != 0;
-        const bool touching = m.pointCount > 0;
-        carryImpulses(m, old);
-        if (touching != wasTouching) { wakeBody(w, bA); wakeBody(w, bB); }
-        flags |= CF_ENABLED | CF_UPDATED;
-        if (touching) flags |= CF_TOUCHING;
-        else flags &= ~CF_TOUCHING;
-        if (wasTouching) flags |= CF_WAS_TOUCHING;
-        else flags &= ~CF_WAS_TOUCHING;
-        if (!wasTouching && touching) cnt->beginEvents++;
-        if (wasTouching && !touching) cnt->endEvents++;
-        w.cman[c] = m;
+        flags &= ~CF_FILTER;
+    }
+    const bool activeA = (w.bflags[bA] & BF_AWAKE) && w.btype[bA] != BT_STATIC;
+    const bool activeB = (w.bflags[bB] & BF_AWAKE) && w.btype[bB] != BT_STATIC;
+    if (!activeA && !activeB) {
         w.cflags[c] = flags;
+        return;
+    }
+    if (!r.overlap[c]) {
+        if (flags & CF_TOUCHING) atomicAdd(&cnt->endEvents, 1);
+        if (destroyWake) { wakeBody(w, bA); wakeBody(w, bB); }
+        w.cflags[c] = flags | CF_DEAD;
+        return;
+    }
+    if (sensorOf(w, fA) || sensorOf(w, fB)) {
+        sensorFinish(w, cnt, c, flags, r.overlap[c] == 3);
+        return;
+    }
+    const b2g_manifold old = w.cman[c];
+    b2g_manifold m = r.tmpMan[c];
+    const bool wasTouching = (flags & CF_TOUCHING) != 0;
+    const bool touching = m.pointCount > 0;
+    carryImpulses(m, old);
+    if (touching != wasTouching) { wakeBody(w, bA); wakeBody(w, bB); }
+    flags |= CF_ENABLED | CF_UPDATED;
+    if (touching) flags |= CF_TOUCHING;
+    else flags &= ~CF_TOUCHING;
+    if (wasTouching) flags |= CF_WAS_TOUCHING;
+    else flags &= ~CF_WAS_TOUCHING;
+    if (!wasTouching && touching) atomicAdd(&cnt->beginEvents, 1);
+    if (wasTouching && !touching) atomicAdd(&cnt->endEvents, 1);
+    w.cman[c] = m;
+    w.cflags[c] = flags;
+}
+
+// The contacts in the reference's list order: activity is read as earlier
+// contacts' wake-ups leave it. While no body sleeps there is none to change,
+// and the contacts are committed in parallel (210 contacts: 290 us on one
+// lane, 5.3 us).
+__global__ void __launch_bounds__(512) k_collide_commit(WorldView w, RefView r, Counters* cnt) {
+    __shared__ int asleep;
+    if (threadIdx.x == 0) asleep = 0;
+    __syncthreads();
+    for (int b = threadIdx.x; b < w.nBodies; b += blockDim.x)
+        if (w.btype[b] != BT_STATIC && !(w.bflags[b] & BF_AWAKE)) asleep = 1;
+    __syncthreads();
+    if (!asleep) {
+        for (int c = threadIdx.x; c < w.nContacts; c += blockDim.x) commitContact(w, r, cnt, c);
+    } else if (threadIdx.x == 0) {
+        for (int c = w.nContacts - 1; c >= 0; --c) commitContact(w, r, cnt, c);
     }
 }
 
@@ -5511,6 +5525,103 @@ __global__ void k_edge_extract(RefView r, int n) {
 
 // Island search of b2World::Solve (REF/Dynamics/b2World.cpp:429-539), one
 // thread: contact edges, then joint edges to active bodies.
+// The search of a world that fits in LDS: the edges with their other bodies,
+// the body flags and the visited marks, so that the one lane that searches
+// waits for LDS only (79 bodies, 210 contacts: 181 us over global memory,
+// 61 us). What the search does to bodies and contacts is applied after
+// it by all lanes.
+constexpr int kDfsBodies = 2048;
+constexpr int kDfsEdges = 6144;
+constexpr int kDfsMarks = 8192;  // contacts, and joints
+__global__ void __launch_bounds__(256) k_dfs_small(WorldView w, JointView jv, RefView r, int nEdges, Counters* cnt) {
+    __shared__ int edge[kDfsEdges];             // contact c, or ~j
+    __shared__ uint16_t otherBody[kDfsEdges];
+    __shared__ uint16_t start[kDfsBodies + 1];
+    __shared__ uint16_t stack[kDfsBodies], statics[kDfsBodies];
+    __shared__ uint8_t mark[kDfsBodies];
+    __shared__ unsigned seenContact[kDfsMarks / 32], seenJoint[kDfsMarks / 32];
+    enum : uint8_t { AWAKE = 1, ACTIVE = 2, STATIC = 4, SEEN = 8, MEMBER = 16, WOKEN = 32 };
+    const int t = threadIdx.x, T = blockDim.x;
+    for (int b = t; b < w.nBodies; b += T) {
+        const int f = w.bflags[b];
+        mark[b] = (uint8_t)(((f & BF_AWAKE) ? AWAKE : 0) | ((f & BF_ACTIVE) ? ACTIVE : 0) |
+                            (w.btype[b] == BT_STATIC ? STATIC : 0));
+    }
+    for (int b = t; b <= w.nBodies; b += T) start[b] = (uint16_t)r.edgeStart[b];
+    for (int i = t; i < kDfsMarks / 32; i += T) seenContact[i] = seenJoint[i] = 0u;
+    __syncthreads();
+    for (int b = t; b < w.nBodies; b += T) {
+        for (int e = start[b]; e < start[b + 1]; ++e) {
+            const int c = r.edgeContact[e];
+            int x, y;
+            if (c < 0) {
+                const int2 jb = jv.bodies[~c];
+                x = jb.x;
+                y = jb.y;
+            } else {
+                x = w.fbody[w.cfA[c]];
+                y = w.fbody[w.cfB[c]];
+            }
+            edge[e] = c;
+            otherBody[e] = (uint16_t)(x == b ? y : x);
+        }
+    }
+    __syncthreads();
+    if (t == 0) {
+        int nI = 0, nb = 0, nc = 0, nj = 0;
+        for (int seed = w.nBodies - 1; seed >= 0; --seed) {
+            if ((mark[seed] & (AWAKE | ACTIVE | STATIC | SEEN)) != (AWAKE | ACTIVE)) continue;
+            const int bStart = nb, cStart = nc, jStart = nj;
+            int sp = 0, ns = 0;
+            stack[sp++] = (uint16_t)seed;
+            mark[seed] |= SEEN;
+            while (sp > 0) {
+                const int b = stack[--sp];
+                r.islandBodies[nb++] = b;
+                uint8_t m = mark[b];
+                if (!(m & AWAKE)) m |= AWAKE | WOKEN;
+                if (m & STATIC) {
+                    mark[b] = m;
+                    statics[ns++] = (uint16_t)b;
+                    continue;
+                }
+                mark[b] = m | MEMBER;
+                for (int e = start[b]; e < start[b + 1]; ++e) {
+                    const int c = edge[e];
+                    const int other = otherBody[e];
+                    if (c < 0) {
+                        const int j = ~c;
+                        if ((seenJoint[j >> 5] >> (j & 31)) & 1u) continue;
+                        if (!(mark[other] & ACTIVE)) continue;
+                        r.islandJoints[nj++] = j;
+                        seenJoint[j >> 5] |= 1u << (j & 31);
+                    } else {
+                        if ((seenContact[c >> 5] >> (c & 31)) & 1u) continue;
+                        r.islandContacts[nc++] = c;
+                        seenContact[c >> 5] |= 1u << (c & 31);
+                    }
+                    if (mark[other] & SEEN) continue;
+                    stack[sp++] = (uint16_t)other;
+                    mark[other] |= SEEN;
+                }
+            }
+            r.islandJointRange[nI] = make_int2(jStart, nj - jStart);
+            r.islandRange[nI++] = make_int4(bStart, nb - bStart, cStart, nc - cStart);
+            for (int i = 0; i < ns; ++i) mark[statics[i]] &= (uint8_t)~SEEN;
+        }
+        cnt->nIslands = nI;
+        cnt->nConstraints = nc;
+    }
+    __syncthreads();
+    for (int b = t; b < w.nBodies; b += T) {
+        if (mark[b] & WOKEN) w.gsleep[b].y = 0.0f;
+        if (mark[b] & (WOKEN | MEMBER))
+            w.bflags[b] |= ((mark[b] & WOKEN) ? BF_AWAKE : 0) | ((mark[b] & MEMBER) ? BF_ISLAND : 0);
+    }
+    for (int c = t; c < w.nContacts; c += T)
+        if ((seenContact[c >> 5] >> (c & 31)) & 1u) w.cflags[c] |= CF_CONSTRAINT;
+}
+
 __global__ void k_dfs(WorldView w, JointView jv, RefView r, Counters* cnt) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     int nI = 0, nb = 0, nc = 0, nj = 0;
@@ -5567,59 +5678,204 @@ __global__ void k_dfs(WorldView w, JointView jv, RefView r, Counters* cnt) {
     cnt->nConstraints = nc;
 }
 
-// One wavefront per island: parallel per-body and per-constraint set-up,
-// the sequential passes of b2ContactSolver on lane 0.
+// The contact constraints of an island in levels: a constraint's level is one
+// above the highest of the earlier constraints it shares a dynamic body with.
+// Constraints of a level share none, and whatever one of them reads was
+// written by lower levels, so solving level after level gives each constraint
+// the inputs that the reference's order gives it, and the results are those of
+// one after another bit for bit, with as many lanes as a level has
+// constraints. In every round the constraints that are the first left on both
+// of their bodies form the next level; `first` holds, per body, the level
+// counted down above the lowest index, so that a later round's values replace
+// an earlier round's without clearing.
+constexpr int kLevelBodies = 2048;       // bodies of the world, 16 B of LDS each
+constexpr int kLevelConstraints = 2048;  // constraints of the island: 32 a lane
+constexpr int kLevelRows = 4;            // constraints a lane holds in registers
+struct Levels {
+    unsigned first[kLevelBodies];
+    uint16_t perm[kLevelConstraints];    // constraints by level
+    uint16_t start[kLevelConstraints + 1];
+    int placed;
+};
+
+__device__ inline int levelsOf(Levels& l, const ConView& cv, int k0, int n, const int* bodies, int nBodies) {
+    const int t = threadIdx.x, T = blockDim.x;
+    for (int i = t; i < nBodies; i += T) l.first[bodies[i]] = 0xFFFFFFFFu;
+    if (t == 0) l.placed = 0;
+    __syncthreads();
+    unsigned done = 0u;  // bit i: constraint t + i * T is placed
+    int level = 0;
+    for (;; ++level) {
+        const unsigned above = (unsigned)(0xFFFF - level) << 16;
+        for (int k = t, i = 0; k < n; k += T, ++i) {
+            if ((done >> i) & 1u) continue;
+            const int2 b = cv.bodies[k0 + k];
+            const int info = cv.info[k0 + k];
+            if (info & 16) atomicMin(&l.first[b.x], above | (unsigned)k);
+            if (info & 32) atomicMin(&l.first[b.y], above | (unsigned)k);
+        }
+        __syncthreads();
+        const int placed = l.placed;
+        if (t == 0) l.start[level] = (uint16_t)placed;
+        if (placed == n) break;
+        __syncthreads();
+        for (int k = t, i = 0; k < n; k += T, ++i) {
+            if ((done >> i) & 1u) continue;
+            const int2 b = cv.bodies[k0 + k];
+            const int info = cv.info[k0 + k];
+            if ((info & 16) && l.first[b.x] != (above | (unsigned)k)) continue;
+            if ((info & 32) && l.first[b.y] != (above | (unsigned)k)) continue;
+            done |= 1u << i;
+            l.perm[atomicAdd(&l.placed, 1)] = (uint16_t)k;
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+    return level;
+}
+
+// One wavefront per island: parallel per-body and per-constraint set-up, the
+// passes of b2ContactSolver over the contact constraints level by level (or,
+// beyond the levels' tables, one after another on lane 0), the joints on lane
+// 0 in order.
 // Joints as b2Island::Solve orders them (REF/Dynamics/b2Island.cpp:246-328):
 // their InitVelocityConstraints after the contact warm start, each velocity
 // iteration joints then contacts, each position iteration contacts then
 // joints, and the early exit when both are within tolerance.
-__global__ void k_island_solve(WorldView w, ConView cv, JointView jv, RefView r, V2 gravity, float h, float dtRatio,
-                               int warm, int velIters, int posIters, int allowSleep, Counters* cnt) {
+// Bound by the chain: a pyramid of 78 boxes has 144 contacts in 97 levels, and
+// a pass cannot start before the last one's end reached its first bodies. So
+// what counts is the time from one level to the next: a constraint from
+// memory took 1.1 us on lane 0 (1594 us for its 12 passes), levels of them
+// 1294 us, with the rows in registers and the bodies in LDS 1004 us. One
+// wavefront, so that a level's end costs nothing; four, each constraint going
+// ahead as soon as counts of its two bodies said so, took 1173 us.
+__global__ void __launch_bounds__(64)
+    k_island_solve(WorldView w, ConView cv, JointView jv, RefView r, V2 gravity, float h, float dtRatio, int warm,
+                   int velIters, int posIters, int allowSleep, Counters* cnt) {
+    __shared__ Levels levels;
+    __shared__ float4 rows[kLevelBodies];  // velocities, then positions, of the bodies
     const int4 rg = r.islandRange[blockIdx.x];
     const int2 jr = r.islandJointRange[blockIdx.x];
     const int* joints = r.islandJoints + jr.x;
     const int tid = threadIdx.x, nt = blockDim.x;
     const int* bodies = r.islandBodies + rg.x;
-    const int k0 = rg.z, k1 = rg.z + rg.w;
-    for (int i = tid; i < rg.y; i += nt) integrateVelocityOne(w, bodies[i], gravity, h);
-    __syncthreads();
-    const FreshView noFresh{nullptr, nullptr, nullptr};
-    for (int k = k0 + tid; k < k1; k += nt)
-        countPoints(cnt, initConstraintOne(w, cv, k, r.islandContacts[k], dtRatio, warm, noFresh));
-    __syncthreads();
-    if (tid == 0) {
-        if (warm)
-            for (int k = k0; k < k1; ++k) warmStartOne(w, cv, k);
-        for (int i = 0; i < jr.y; ++i) jointInitOne(w, jv, joints[i], dtRatio, warm);
-        for (int it = 0; it < velIters; ++it) {
-            for (int i = 0; i < jr.y; ++i) jointSolveVelocityOne(w, jv, joints[i], h);
-            for (int k = k0; k < k1; ++k) solveVelocityOne(w, cv, k);
-        }
+    const int k0 = rg.z, n = rg.w;
+    // A gear joint reaches bodies of its two joints, which need not be in the
+    // island; its rows stay in memory.
+    bool gear = false;
+    for (int i = tid; i < jr.y; i += nt) gear = gear || jointType(jv.flags[joints[i]]) == JT_GEAR;
+    const bool byLevel = n <= kLevelConstraints && w.nBodies <= kLevelBodies && !__any(gear);
+    WorldView wl = w;  // the bodies' rows in LDS for the functions that take a world
+    if (byLevel) wl.vel = rows;
+    for (int i = tid; i < rg.y; i += nt) {
+        if (byLevel) rows[bodies[i]] = w.vel[bodies[i]];
+        integrateVelocityOne(wl, bodies[i], gravity, h);
     }
     __syncthreads();
-    for (int k = k0 + tid; k < k1; k += nt) storeImpulsesOne(w, cv, k);
-    for (int i = tid; i < rg.y; i += nt)
-        if (w.btype[bodies[i]] != BT_STATIC) integratePositionOne(w, bodies[i], h);
+    for (int k = k0 + tid; k < k0 + n; k += nt)
+        countPoints(cnt, initConstraintOne(wl, cv, k, r.islandContacts[k], dtRatio, warm, FreshView{}));
     __syncthreads();
-    __shared__ int solved;
+    const int nLevels = byLevel ? levelsOf(levels, cv, k0, n, bodies, rg.y) : 0;
+    constexpr int R = kLevelRows;
+    const int held = byLevel ? min(n, R * nt) : 0;
+    VelRow row[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        row[i].info = 0;
+        if (tid + i * nt < held) row[i] = loadVelRow(cv, k0 + levels.perm[tid + i * nt]);
+    }
+    // reg(row) over the constraints in registers, mem(k) over the others.
+    auto contacts = [&](auto reg, auto mem) {
+        if (!byLevel && tid == 0)
+            for (int k = k0; k < k0 + n; ++k) mem(k);
+        for (int l = 0; l < nLevels; ++l) {
+            const int l0 = levels.start[l], l1 = levels.start[l + 1];
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                const int at = tid + i * nt;
+                if (at >= l0 && at < min(l1, held)) reg(i);
+            }
+            for (int at = max(l0, held) + tid; at < l1; at += nt) mem(k0 + levels.perm[at]);
+            __syncthreads();
+        }
+        __syncthreads();
+    };
+    auto keep = [&](int info, int2 b, const float4& x, const float4& y) {
+        if (info & 16) rows[b.x] = x;
+        if (info & 32) rows[b.y] = y;
+    };
+    if (warm)
+        contacts(
+            [&](int i) {
+                float4 va = rows[row[i].bodies.x], vb = rows[row[i].bodies.y];
+                warmStartRow(row[i].info, row[i].mass, row[i].normal, row[i].imp, row[i].r0, row[i].r1, va, vb);
+                keep(row[i].info, row[i].bodies, va, vb);
+            },
+            [&](int k) { warmStartOne(wl, cv, k); });
+    if (tid == 0)
+        for (int i = 0; i < jr.y; ++i) jointInitOne(wl, jv, joints[i], dtRatio, warm);
+    __syncthreads();
+    for (int it = 0; it < velIters; ++it) {
+        if (tid == 0)
+            for (int i = 0; i < jr.y; ++i) jointSolveVelocityOne(wl, jv, joints[i], h);
+        __syncthreads();
+        contacts(
+            [&](int i) {
+                float4 va = rows[row[i].bodies.x], vb = rows[row[i].bodies.y];
+                solveVelocityRow(row[i], va, vb);
+                keep(row[i].info, row[i].bodies, va, vb);
+            },
+            [&](int k) { solveVelocityOne(wl, cv, k); });
+    }
+    PosRow prow[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        if (tid + i * nt >= held) continue;
+        const int k = k0 + levels.perm[tid + i * nt];
+        storeImpulsesTo(w, cv.contact[k], row[i].info & 3, row[i].imp);
+        prow[i] = loadPosRow(cv, k);
+    }
+    for (int at = held + tid; at < n; at += nt) storeImpulsesOne(w, cv, k0 + (byLevel ? levels.perm[at] : at));
+    // A body's row in LDS goes from velocity to position in its own lane.
+    for (int i = tid; i < rg.y; i += nt) {
+        const int b = bodies[i];
+        if (w.btype[b] != BT_STATIC) {
+            integratePositionOne(wl, b, h);
+            if (byLevel) w.vel[b] = rows[b];
+        }
+        if (byLevel) rows[b] = w.pos[b];
+    }
+    wl = w;
+    if (byLevel) wl.pos = rows;
+    __syncthreads();
     __shared__ int minSleep;
-    if (tid == 0) {
-        solved = 0;
-        minSleep = encodeOrdered(FLT_MAX);
-        for (int it = 0; it < posIters; ++it) {
-            float minSep = 0.0f;
-            for (int k = k0; k < k1; ++k) minSep = fminB(minSep, solvePositionOne(w, cv, k));
-            bool jointsOkay = true;
+    __shared__ int jointsOkay;
+    if (tid == 0) minSleep = encodeOrdered(FLT_MAX);
+    bool solved = false;
+    for (int it = 0; it < posIters && !solved; ++it) {
+        float minSep = 0.0f;
+        contacts(
+            [&](int i) {
+                float4 pA = rows[prow[i].bodies.x], pB = rows[prow[i].bodies.y];
+                minSep = fminB(minSep, solvePositionRow(prow[i], pA, pB));
+                keep(prow[i].info, prow[i].bodies, pA, pB);
+            },
+            [&](int k) { minSep = fminB(minSep, solvePositionOne(wl, cv, k)); });
+        if (tid == 0) {
+            bool okay = true;
             for (int i = 0; i < jr.y; ++i) {
-                const bool ok = jointPositionCore(w, jv, joints[i], jv.bodies[joints[i]]);
-                jointsOkay = jointsOkay && ok;
+                const bool ok = jointPositionCore(wl, jv, joints[i], jv.bodies[joints[i]]);
+                okay = okay && ok;
             }
-            if (minSep >= -3.0f * kLinearSlop && jointsOkay) {
-                solved = 1;
-                break;
-            }
+            jointsOkay = okay ? 1 : 0;
         }
+        __syncthreads();
+        solved = __all(minSep >= -3.0f * kLinearSlop) && jointsOkay != 0;
+        __syncthreads();
     }
+    if (byLevel)
+        for (int i = tid; i < rg.y; i += nt)
+            if (w.btype[bodies[i]] != BT_STATIC) w.pos[bodies[i]] = rows[bodies[i]];
     __syncthreads();
     for (int i = tid; i < rg.y; i += nt)
         if (w.btype[bodies[i]] != BT_STATIC) syncTransformOne(w, bodies[i]);
@@ -8818,9 +9074,8 @@ int stepReferenceCollide(b2g_context* ctx, const b2g_step_params* p) {
     if ((rc = reserveContacts(ctx)) != B2G_OK) return rc;
     if ((rc = ensureRefBuffers(ctx)) != B2G_OK) return rc;
     memset(&ctx->stats, 0, sizeof(ctx->stats));
-    Counters zero;
-    memset(&zero, 0, sizeof(zero));
-    HIPCHK(ctx, hipMemcpyAsync(ctx->cnt, &zero, sizeof(Counters), hipMemcpyHostToDevice, s));
+    constexpr int words = sizeof(Counters) / sizeof(int);
+    hipLaunchKernelGGL(k_fill<int>, dim3(blocks(words)), dim3(256), 0, s, (int*)ctx->cnt, words, 0);
     if (ctx->newFixture) {
         if ((rc = rebuildHash(ctx)) != B2G_OK) return rc;
         if ((rc = runBroadphase(ctx)) != B2G_OK) return rc;
@@ -8835,7 +9090,7 @@ int stepReferenceCollide(b2g_context* ctx, const b2g_step_params* p) {
                                        hipMemcpyDeviceToDevice, s));
         }
         hipLaunchKernelGGL(k_collide_compute, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w, r);
-        hipLaunchKernelGGL(k_collide_serial, dim3(1), dim3(64), 0, s, w, r, ctx->cnt);
+        hipLaunchKernelGGL(k_collide_commit, dim3(1), dim3(512), 0, s, w, r, ctx->cnt);
         LAUNCHCHK(ctx);
     }
     return B2G_OK;
@@ -8886,7 +9141,10 @@ int stepReferenceSolve(b2g_context* ctx, const b2g_step_params* p) {
             HIPCHK(ctx, prims_sort_keys_u64(ctx->scratch, ctx->scratchBytes, r.edgeKeys, r.edgeSorted, nEdges, s));
             hipLaunchKernelGGL(k_edge_extract, dim3(blocks(nEdges)), dim3(256), 0, s, r, nEdges);
         }
-        hipLaunchKernelGGL(k_dfs, dim3(1), dim3(64), 0, s, w, jv, r, ctx->cnt);
+        if (nb <= kDfsBodies && nEdges <= kDfsEdges && nc <= kDfsMarks && nj <= kDfsMarks)
+            hipLaunchKernelGGL(k_dfs_small, dim3(1), dim3(256), 0, s, w, jv, r, nEdges, ctx->cnt);
+        else
+            hipLaunchKernelGGL(k_dfs, dim3(1), dim3(64), 0, s, w, jv, r, ctx->cnt);
         LAUNCHCHK(ctx);
         if ((rc = readCounters(ctx)) != B2G_OK) return rc;
         const int nIslands = ctx->hcnt->nIslands;

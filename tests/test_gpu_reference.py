@@ -188,3 +188,32 @@ def test_coloured_mode_pyramid_sleeps(gpu, orc):
     d = np.hypot(gb[1:, E.CX] - ob[1:, E.CX], gb[1:, E.CY] - ob[1:, E.CY])
     assert d.max() < 0.1
     g.close(); o.close()
+
+
+@pytest.mark.parametrize("kind,n,seed,steps,vel,pos", [
+    ("pyramid", 15, 0, 30, 8, 3),      # 225 constraints in an island: in the lanes' registers
+    ("pyramid", 20, 0, 20, 8, 3),      # 400: some read from memory in every pass
+    ("pyramid", 44, 0, 6, 4, 2),       # 1936, the last that the tables hold
+    ("pyramid", 46, 0, 6, 4, 2),       # 2116: beyond the tables, one after another
+    ("pyramid", 12, 0, 40, 1, 1),
+    ("pyramid", 12, 0, 40, 3, 20),
+    ("pyramid", 8, 0, 40, 0, 0),
+    ("pile", 2030, 4, 6, 4, 2),        # the largest world with its rows on the compute unit
+    ("pile", 2060, 4, 6, 4, 2),        # and one beyond it
+    ("terrain", 400, 3, 60, 8, 3),     # many islands
+])
+def test_reference_levels_bitexact(gpu, orc, wide_trig, kind, n, seed, steps, vel, pos):
+    """Sizes around where an island's solve in levels changes its layout."""
+    print(f"case: {kind} {n}, {vel} velocity and {pos} position iterations, reference order", flush=True)
+    g = gpu.world(kind, n, seed, sleep=True)
+    g.set_mode(REFERENCE)
+    o = orc.world(kind, n, seed, sleep=True)
+    for s in range(steps):
+        g.step(1, vel=vel, pos=pos)
+        o.step(1, vel=vel, pos=pos)
+        if s % 10 == 9 or s == steps - 1:
+            assert np.array_equal(_canon(g.bodies()[:, :11]), _canon(o.bodies()[:, :11])), f"step {s + 1}"
+    _, gman = E.contact_table(*g.contacts())
+    _, oman = E.contact_table(*o.contacts())
+    assert np.array_equal(E.manifold_bits(gman), E.manifold_bits(oman))
+    g.close(); o.close()
