@@ -1542,7 +1542,16 @@ __device__ inline PosRow loadPosRow(const ConView& cv, int k) {
 // b2ContactSolver::SolvePositionConstraints with b2PositionSolverManifold,
 // REF/Dynamics/Contacts/b2ContactSolver.cpp:614-744, one constraint: the
 // bodies' positions are passed in and returned (w = 0).
-__device__ inline float solvePositionRow(const PosRow& r, float4& pA, float4& pB) {
+// With kOneLane, where one lane of the wavefront solves at a time, a rotation is
+// only computed again when its angle has changed (`known` holds the two between
+// calls).
+struct RotPair {
+    Rot a, b;
+    unsigned angleA, angleB;  // bits
+};
+template <bool kOneLane = false>
+__device__ inline float solvePositionRow(const PosRow& r, float4& pA, float4& pB, float baumgarte = kBaumgarte,
+                                         RotPair* known = nullptr) {
     const float mA = r.mass.x, iA = r.mass.y, mB = r.mass.z, iB = r.mass.w;
     const int pc = (r.info >> 2) & 3;
     const int type = (r.info >> 8) & 3;
@@ -1559,7 +1568,20 @@ __device__ inline float solvePositionRow(const PosRow& r, float4& pA, float4& pB
 #pragma clang loop unroll(disable)
     for (int j = 0; j < pc; ++j) {
         Xf xfA, xfB;
-        rotOf2(aA, aB, xfA.q, xfB.q);
+        if constexpr (kOneLane) {
+            if (known->angleA != __float_as_uint(aA)) {
+                known->a = rotOf(aA);
+                known->angleA = __float_as_uint(aA);
+            }
+            if (known->angleB != __float_as_uint(aB)) {
+                known->b = rotOf(aB);
+                known->angleB = __float_as_uint(aB);
+            }
+            xfA.q = known->a;
+            xfB.q = known->b;
+        } else {
+            rotOf2(aA, aB, xfA.q, xfB.q);
+        }
         xfA.p = cA - mul(xfA.q, mk(r.lc.x, r.lc.y));
         xfB.p = cB - mul(xfB.q, mk(r.lc.z, r.lc.w));
         Xf xf1, xf2;
@@ -1585,7 +1607,7 @@ __device__ inline float solvePositionRow(const PosRow& r, float4& pA, float4& pB
         const V2 rA = point - cA;
         const V2 rB = point - cB;
         minSep = fminB(minSep, separation);
-        const float C = clampB(kBaumgarte * (separation + kLinearSlop), -kMaxLinearCorrection, 0.0f);
+        const float C = clampB(baumgarte * (separation + kLinearSlop), -kMaxLinearCorrection, 0.0f);
         const float rnA = cross(rA, normal);
         const float rnB = cross(rB, normal);
         const float Kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
@@ -5954,7 +5976,7 @@ __global__ void k_distance_batch(const b2g_shape* a, const b2g_transform* xfA, c
     out[2 * i + 1] = (float)cache.count;
 }
 
-__global__ void k_toi_batch(const b2g_shape* a, const b2g_sweep* sa, const b2g_shape* b, const b2g_sweep* sb, int n,
+__global__ void __launch_bounds__(64) k_toi_batch(const b2g_shape* a, const b2g_sweep* sa, const b2g_shape* b, const b2g_sweep* sb, int n,
                             float tMax, int32_t* state, float* t) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
@@ -6069,8 +6091,8 @@ __global__ void k_penetration(WorldView w, double* acc, int* npts, unsigned long
 // 385-515) solved for the rest of the step, fixtures synchronised and new
 // pairs found. Times of impact are computed in parallel when every pending
 // contact's bodies share a sweep start (always on the first scan of a
-// step); otherwise in list order by one lane, since aligning two sweeps
-// moves the later-starting one for the contacts that follow.
+// step); otherwise the sweeps are aligned in list order first, since aligning
+// two moves the earlier-starting one for the contacts that follow.
 // ====================================================================
 constexpr int kToiGatherCap = 2048;  // edges of the TOI pair sorted in LDS
 constexpr int kToiMovedCap = 256;    // proxies one event may move before the grid broad-phase takes over
@@ -6147,16 +6169,6 @@ __device__ inline void advanceBodyTo(const WorldView& w, int b, float alpha) {
     syncTransformOne(w, b);
 }
 
-// The two sweeps of a contact brought to a common start: the one that
-// starts earlier is advanced (and stays advanced), REF/Dynamics/b2World.cpp:
-// 645-660.
-__device__ inline void alignSweeps(const WorldView& w, int c) {
-    const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
-    const float alphaA = w.pos0[bA].w, alphaB = w.pos0[bB].w;
-    if (alphaA < alphaB) advanceSweepStart(w, bA, alphaB);
-    else if (alphaB < alphaA) advanceSweepStart(w, bB, alphaA);
-}
-
 // TOI of a contact over the rest of the step from aligned sweeps,
 // REF/Dynamics/b2World.cpp:662-689.
 __device__ inline float toiFromSweeps(const WorldView& w, int c, const Sweep& sA, const Sweep& sB) {
@@ -6190,73 +6202,6 @@ __device__ inline void toiUpdateContact(const WorldView& w, int c) {
     w.cflags[c] = flags;
 }
 
-// b2ContactSolver::SolveTOIPositionConstraints, REF/Dynamics/Contacts/
-// b2ContactSolver.cpp:753-841, one constraint: only the TOI pair moves.
-__device__ inline float solveTOIPositionOne(const WorldView& w, const ConView& cv, int k, int toiA, int toiB) {
-    const int2 bi = cv.bodies[k];
-    const float4 ms = cv.mass[k];
-    const bool movesA = bi.x == toiA || bi.x == toiB, movesB = bi.y == toiA || bi.y == toiB;
-    const float mA = movesA ? ms.x : 0.0f, iA = movesA ? ms.y : 0.0f;
-    const float mB = movesB ? ms.z : 0.0f, iB = movesB ? ms.w : 0.0f;
-    const int info = cv.info[k];
-    const int pc = (info >> 2) & 3;
-    const int type = (info >> 8) & 3;
-    const float4 lc = cv.lc[k];
-    const V2 lcA = mk(lc.x, lc.y), lcB = mk(lc.z, lc.w);
-    const float4 lp = cv.lp[k];
-    const float4 lnp = cv.lnp[k];
-    const float2 rad = cv.rad[k];
-    const float4 pA = w.pos[bi.x], pB = w.pos[bi.y];
-    V2 cA = mk(pA.x, pA.y), cB = mk(pB.x, pB.y);
-    float aA = pA.z, aB = pB.z;
-    float minSep = 0.0f;
-    for (int j = 0; j < pc; ++j) {
-        Xf xfA, xfB;
-        rotOf2(aA, aB, xfA.q, xfB.q);
-        xfA.p = cA - mul(xfA.q, lcA);
-        xfB.p = cB - mul(xfB.q, lcB);
-        V2 normal, point;
-        float separation;
-        if (type == B2G_MANIFOLD_CIRCLES) {
-            const V2 pointA = mul(xfA, mk(lnp.z, lnp.w));
-            const V2 pointB = mul(xfB, mk(lp.x, lp.y));
-            normal = pointB - pointA;
-            normalizeV(normal);
-            point = 0.5f * (pointA + pointB);
-            separation = dot(pointB - pointA, normal) - rad.x - rad.y;
-        } else if (type == B2G_MANIFOLD_FACE_A) {
-            normal = mul(xfA.q, mk(lnp.x, lnp.y));
-            const V2 planePoint = mul(xfA, mk(lnp.z, lnp.w));
-            const V2 clipPoint = mul(xfB, j == 0 ? mk(lp.x, lp.y) : mk(lp.z, lp.w));
-            separation = dot(clipPoint - planePoint, normal) - rad.x - rad.y;
-            point = clipPoint;
-        } else {
-            normal = mul(xfB.q, mk(lnp.x, lnp.y));
-            const V2 planePoint = mul(xfB, mk(lnp.z, lnp.w));
-            const V2 clipPoint = mul(xfA, j == 0 ? mk(lp.x, lp.y) : mk(lp.z, lp.w));
-            separation = dot(clipPoint - planePoint, normal) - rad.x - rad.y;
-            point = clipPoint;
-            normal = -normal;
-        }
-        const V2 rA = point - cA;
-        const V2 rB = point - cB;
-        minSep = fminB(minSep, separation);
-        const float C = clampB(kToiBaumgarte * (separation + kLinearSlop), -kMaxLinearCorrection, 0.0f);
-        const float rnA = cross(rA, normal);
-        const float rnB = cross(rB, normal);
-        const float Kn = mA + mB + iA * rnA * rnA + iB * rnB * rnB;
-        const float impulse = Kn > 0.0f ? -C / Kn : 0.0f;
-        const V2 P = impulse * normal;
-        cA -= mA * P;
-        aA -= iA * cross(rA, P);
-        cB += mB * P;
-        aB += iB * cross(rB, P);
-    }
-    if (movesA) w.pos[bi.x] = make_float4(cA.x, cA.y, aA, 0.0f);
-    if (movesB) w.pos[bi.y] = make_float4(cB.x, cB.y, aB, 0.0f);
-    return minSep;
-}
-
 // Start of a TOI pass after a completed step: island flags off, sweeps
 // start at 0, cached TOIs dropped.
 __global__ void k_toi_reset_bodies(WorldView w) {
@@ -6288,67 +6233,129 @@ __device__ inline void toiResetEvent(ToiState* st) {
 }
 
 // Contacts whose TOI the scan computes, and whether their sweeps need aligning.
+__device__ inline bool sweepsDiffer(const WorldView& w, int c) {
+    return w.pos0[w.fbody[w.cfA[c]]].w != w.pos0[w.fbody[w.cfB[c]]].w;
+}
 __global__ void k_toi_classify(WorldView w, int* pending, ToiState* st) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= st->live || st->halt) return;
     const bool p = toiPending(w, c, w.cflags[c]);
     pending[c] = p ? 1 : 0;
-    if (p && w.pos0[w.fbody[w.cfA[c]]].w != w.pos0[w.fbody[w.cfB[c]]].w) atomicOr(&st->mismatch, 1);
+    if (p && sweepsDiffer(w, c)) atomicOr(&st->mismatch, 1);
 }
 
-
-// Otherwise the alignments run in list order on one lane, since an advance
-// moves a body for the contacts after it, and each contact keeps the two
-// sweeps it saw; the TOIs then run in parallel from those.
-__global__ void k_toi_align_serial(WorldView w, const int* pending, const ToiState* st, Sweep* seen) {
-    if (blockIdx.x != 0 || threadIdx.x != 0 || st->halt || !st->mismatch) return;
-    for (int c = st->live - 1; c >= 0; --c) {
-        if (!pending[c]) continue;
-        alignSweeps(w, c);
-        seen[2 * c] = sweepOf(w, w.fbody[w.cfA[c]]);
-        seen[2 * c + 1] = sweepOf(w, w.fbody[w.cfB[c]]);
+// Otherwise the alignments run in list order, since an advance moves a body
+// for the contacts after it, and each contact keeps the two sweeps it saw;
+// the TOIs then run in parallel from those. One wavefront, 64 contacts at a
+// time with their sweeps in registers: the first contact whose sweeps start at
+// different times has the one that starts earlier advanced (and it stays
+// advanced, REF/Dynamics/b2World.cpp:645-660), and the later ones on that body
+// take it over. The chain is as long as the advances are many and not as the
+// list is long (99 bodies, 69 events: 80 us an event on one lane, 14 us
+// with the sweeps read again after every advance, about 5 us so).
+template <class Pending>
+__device__ inline void toiAlignOrdered(const WorldView& w, int live, Sweep* seen, Pending pending) {
+    const int lane = threadIdx.x & 63;
+    for (int top = live - 1; top >= 0; top -= 64) {
+        const int c = top - lane;
+        bool mine = c >= 0 && pending(c);
+        if (!__any(mine)) continue;
+        const int bA = mine ? w.fbody[w.cfA[c]] : -1, bB = mine ? w.fbody[w.cfB[c]] : -1;
+        Sweep sA{}, sB{};
+        if (mine) {
+            sA = sweepOf(w, bA);
+            sB = sweepOf(w, bB);
+        }
+        bool left = mine;
+        for (;;) {
+            const unsigned long long differ = __ballot(left && (sA.alpha0 < sB.alpha0 || sB.alpha0 < sA.alpha0));
+            if (!differ) break;
+            const int first = __ffsll((long long)differ) - 1;
+            left = left && lane > first;
+            int moved = 0;
+            Sweep to{};
+            if (lane == first) {
+                const bool isA = sA.alpha0 < sB.alpha0;
+                moved = isA ? bA : bB;
+                to = isA ? sA : sB;
+                sweepAdvance(to, isA ? sB.alpha0 : sA.alpha0);
+                if (isA) sA = to;
+                else sB = to;
+                w.pos0[moved] = make_float4(to.c0.x, to.c0.y, to.a0, to.alpha0);
+            }
+            moved = __shfl(moved, first);
+            to.c0.x = __shfl(to.c0.x, first);
+            to.c0.y = __shfl(to.c0.y, first);
+            to.a0 = __shfl(to.a0, first);
+            to.alpha0 = __shfl(to.alpha0, first);
+            auto follow = [&](Sweep& sw) {
+                sw.c0 = to.c0;
+                sw.a0 = to.a0;
+                sw.alpha0 = to.alpha0;
+            };
+            if (left && bA == moved) follow(sA);
+            if (left && bB == moved) follow(sB);
+        }
+        if (mine) {
+            seen[2 * c] = sA;
+            seen[2 * c + 1] = sB;
+        }
+        __threadfence_block();
     }
+}
+__global__ void __launch_bounds__(64) k_toi_align(WorldView w, const int* pending, const ToiState* st, Sweep* seen) {
+    if (st->halt || !st->mismatch) return;
+    toiAlignOrdered(w, st->live, seen, [&](int c) { return pending[c] != 0; });
 }
 
 // One lane per pending contact: from the current sweeps when every pending
 // pair's sweeps already start together (each TOI then depends on its own two
 // bodies only), else from the sweeps the list-order alignment recorded.
-__global__ void k_toi_compute(WorldView w, const int* pending, const ToiState* st, const Sweep* seen) {
+__device__ inline void toiComputeOne(const WorldView& w, int c, bool mismatch, const Sweep* seen) {
+    Sweep sA, sB;
+    if (mismatch) {
+        sA = seen[2 * c];
+        sB = seen[2 * c + 1];
+    } else {
+        sA = sweepOf(w, w.fbody[w.cfA[c]]);
+        sB = sweepOf(w, w.fbody[w.cfB[c]]);
+    }
+    w.ctoi[c] = toiFromSweeps(w, c, sA, sB);
+    w.cflags[c] |= CF_TOI;
+}
+__global__ void __launch_bounds__(64) k_toi_compute(WorldView w, const int* pending, const ToiState* st,
+                                                    const Sweep* seen) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= st->live || st->halt || !pending[c]) return;
-    if (st->mismatch) {
-        w.ctoi[c] = toiFromSweeps(w, c, seen[2 * c], seen[2 * c + 1]);
-    } else {
-        const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
-        w.ctoi[c] = toiFromSweeps(w, c, sweepOf(w, bA), sweepOf(w, bB));
-    }
-    w.cflags[c] |= CF_TOI;
+    toiComputeOne(w, c, st->mismatch != 0, seen);
 }
 
 // Earliest cached TOI below 1, first in list order among equal times.
-__global__ void k_toi_min(WorldView w, ToiState* st) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (st->halt) return;
-    unsigned long long key = ~0ull;
-    if (c < st->live) {
-        const int flags = w.cflags[c];
-        if ((flags & CF_ENABLED) && (flags & CF_TOI) && w.ctoiCount[c] <= kMaxSubSteps) {
-            const float alpha = w.ctoi[c];
-            if (alpha < 1.0f)
-                key = ((unsigned long long)__float_as_uint(alpha) << 32) | (unsigned)(st->live - 1 - c);
-        }
-    }
+__device__ inline unsigned long long toiKey(const WorldView& w, int c, int live) {
+    const int flags = w.cflags[c];
+    if (!(flags & CF_ENABLED) || !(flags & CF_TOI) || w.ctoiCount[c] > kMaxSubSteps) return ~0ull;
+    const float alpha = w.ctoi[c];
+    if (!(alpha < 1.0f)) return ~0ull;
+    return ((unsigned long long)__float_as_uint(alpha) << 32) | (unsigned)(live - 1 - c);
+}
+// The least key of a wavefront, on its first lane.
+__device__ inline unsigned long long toiWaveMin(unsigned long long key) {
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_down(key, off);
         key = o < key ? o : key;
     }
+    return key;
+}
+__global__ void k_toi_min(WorldView w, ToiState* st) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (st->halt) return;
+    const unsigned long long key = toiWaveMin(c < st->live ? toiKey(w, c, st->live) : ~0ull);
     if ((threadIdx.x & 63) == 0 && key != ~0ull) atomicMin(&st->minKey, key);
 }
 
 // The event's TOI pair: advance both bodies, update the contact; an island
 // starts when it touches.
-__global__ void k_toi_event(WorldView w, ToiState* st) {
-    if (blockIdx.x != 0 || threadIdx.x != 0 || st->halt) return;
+__device__ inline void toiStartEvent(const WorldView& w, ToiState* st) {
     const unsigned long long key = st->minKey;
     const float alpha = key == ~0ull ? 1.0f : __uint_as_float((unsigned)(key >> 32));
     if (key == ~0ull || 1.0f - 10.0f * FLT_EPSILON < alpha) {
@@ -6394,14 +6401,16 @@ __global__ void k_toi_event(WorldView w, ToiState* st) {
     st->active = 1;
     st->events += 1;
 }
+__global__ void k_toi_event(WorldView w, ToiState* st) {
+    if (blockIdx.x != 0 || threadIdx.x != 0 || st->halt) return;
+    toiStartEvent(w, st);
+}
 
 // Contact edges of the TOI pair's dynamic bodies, keyed for list order:
 // (0 for A / 1 for B) << 62 | list position << 11 | gather slot.
 constexpr int kGatherSlotBits = 11;
 static_assert((1 << kGatherSlotBits) >= kToiGatherCap, "gather slot field");
-__global__ void k_toi_gather(WorldView w, ToiState* st, unsigned long long* gather) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= st->live || st->halt || !st->active) return;
+__device__ inline void toiGatherOne(const WorldView& w, ToiState* st, unsigned long long* gather, int c) {
     const int x = w.fbody[w.cfA[c]], y = w.fbody[w.cfB[c]];
     const unsigned pos = (unsigned)(st->live - 1 - c);
     for (int k = 0; k < 2; ++k) {
@@ -6411,6 +6420,11 @@ __global__ void k_toi_gather(WorldView w, ToiState* st, unsigned long long* gath
         if (slot < kToiGatherCap)
             gather[slot] = ((unsigned long long)k << 62) | ((unsigned long long)pos << kGatherSlotBits) | (unsigned)slot;
     }
+}
+__global__ void k_toi_gather(WorldView w, ToiState* st, unsigned long long* gather) {
+    const int c = blockIdx.x * blockDim.x + threadIdx.x;
+    if (c >= st->live || st->halt || !st->active) return;
+    toiGatherOne(w, st, gather, c);
 }
 
 // One contact edge of the island search (REF/Dynamics/b2World.cpp:760-843).
@@ -6445,11 +6459,8 @@ __device__ inline void toiVisitEdge(const WorldView& w, ToiState* st, int body, 
 // (kept if its contact touches, else restored, so a later edge of the same
 // body sees the same advance again); a contact met twice (between the two
 // TOI bodies) is not touching at either visit or is skipped at the second.
-__global__ void k_toi_prep(WorldView w, ToiState* st, const unsigned long long* gather, b2g_manifold* man,
-                           int* touching) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (st->halt || !st->active || i >= st->nGather || i >= kToiGatherCap) return;
-    const unsigned long long key = gather[i];
+__device__ inline void toiPrepOne(const WorldView& w, const ToiState* st, unsigned long long key, b2g_manifold* man,
+                                  int* touching) {
     const int k = (int)(key >> 62);
     const int pos = (int)((key >> kGatherSlotBits) & ((1ull << 51) - 1));
     const int c = st->live - 1 - pos;
@@ -6477,6 +6488,12 @@ __global__ void k_toi_prep(WorldView w, ToiState* st, const unsigned long long* 
     const int slot = (int)(key & ((1u << kGatherSlotBits) - 1));
     man[slot] = m;
     touching[slot] = m.pointCount > 0 ? 1 : 0;
+}
+__global__ void k_toi_prep(WorldView w, ToiState* st, const unsigned long long* gather, b2g_manifold* man,
+                           int* touching) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (st->halt || !st->active || i >= st->nGather || i >= kToiGatherCap) return;
+    toiPrepOne(w, st, gather[i], man, touching);
 }
 
 // One edge of the island search with its narrowphase done ahead: commits
@@ -6509,19 +6526,83 @@ __device__ inline void toiCommitEdge(const WorldView& w, ToiState* st, int body,
     st->bodies[st->nBodies++] = other;
 }
 
+// The commits of up to 64 edges, lane i the i-th in list order (`key`), by one
+// wavefront. What an edge's commit depends on is known before any of them: its
+// contact is in the island already only if it is the TOI contact or was met
+// from the other TOI body (and then a second visit changes nothing), its other
+// body only as one of the TOI pair, or through an earlier edge. An edge is
+// visited while the island has room for a contact.
+__device__ inline void toiCommitWave(const WorldView& w, ToiState* st, unsigned long long key, bool mine,
+                                     const b2g_manifold* man, const int* touching) {
+    const int lane = threadIdx.x & 63;
+    const unsigned long long before = (1ull << lane) - 1ull;
+    const int bA = st->bodyA, bB = st->bodyB;
+    const int k = (int)(key >> 62);
+    const int c = mine ? st->live - 1 - (int)((key >> kGatherSlotBits) & ((1ull << 51) - 1)) : 0;
+    const int slot = mine ? (int)(key & ((1u << kGatherSlotBits) - 1)) : 0;
+    const int fA = mine ? w.cfA[c] : 0, fB = mine ? w.cfB[c] : 0;
+    const int x = mine ? w.fbody[fA] : 0, y = mine ? w.fbody[fB] : 0;
+    const int body = k == 0 ? bA : bB;
+    const int other = x == body ? y : x;
+    int flags = mine ? w.cflags[c] : 0;
+    const bool inIsland = mine && (w.bflags[other] & BF_ISLAND) != 0;
+    bool visit = mine && !(flags & CF_ISLAND) && !(k == 1 && other == bA && w.btype[bA] == BT_DYNAMIC) &&
+                 !(w.btype[other] == BT_DYNAMIC && !(w.bflags[body] & BF_BULLET) && !(w.bflags[other] & BF_BULLET)) &&
+                 !sensorOf(w, fA) && !sensorOf(w, fB);
+    bool touch = visit && touching[slot] != 0;
+    const int at = st->nContacts + __popcll(__ballot(touch) & before);
+    visit = visit && at < kMaxTOIContacts;
+    touch = touch && at < kMaxTOIContacts;
+    if (visit) {
+        flags |= CF_ENABLED;
+        if (touch != ((flags & CF_TOUCHING) != 0)) {
+            wakeBody(w, x);
+            wakeBody(w, y);
+        }
+        w.cman[c] = man[slot];
+        w.cflags[c] = touch ? flags | CF_TOUCHING | CF_ISLAND : flags & ~CF_TOUCHING;
+        if (!touch) syncTransformOne(w, other);  // the restored sweep's transform
+    }
+    __threadfence_block();
+    bool joins = touch && !inIsland;
+    for (unsigned long long m = __ballot(joins); m; m &= m - 1) {
+        const int j = __ffsll((long long)m) - 1;
+        if (__shfl(other, j) == other && lane > j) joins = false;
+    }
+    const unsigned long long joined = __ballot(joins), touched = __ballot(touch);
+    if (touch) st->contacts[at] = c;
+    if (joins) {
+        advanceBodyTo(w, other, st->alpha);
+        atomicOr(&w.bflags[other], BF_ISLAND);
+        if (w.btype[other] != BT_STATIC) wakeBody(w, other);
+        st->bodies[st->nBodies + __popcll(joined & before)] = other;
+    }
+    __threadfence_block();
+    if (lane == 0) {
+        st->nContacts += __popcll(touched);
+        st->nBodies += __popcll(joined);
+    }
+    __threadfence_block();
+}
+
 // Island search over the TOI pair's edges in list order, then
-// b2Island::SolveTOI on lane 0 (Gauss-Seidel order is the island's).
-__global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, ToiState* st,
-                                                    const unsigned long long* gather, const b2g_manifold* man,
-                                                    const int* touching, float dt, int velIters) {
-    __shared__ unsigned long long keys[kToiGatherCap];
-    if (st->halt || !st->active) return;
+// b2Island::SolveTOI, by one wavefront (the sort of many edges by the
+// workgroup). Every constraint of the island is on one of the TOI pair, so
+// they are solved one after another, in the island's order; each has a lane
+// that holds its row in registers, and the bodies are in LDS. Bound by that
+// chain: up to 20 position and the velocity passes over a few constraints
+// (99 bodies, 69 events: 101 us an event on one lane with rows in memory,
+// 36 to 50 us so: 0.55 us a constraint and pass).
+constexpr int kToiIslandBodies = 2 * kMaxTOIContacts;  // the island's room: one a lane
+static_assert(kToiIslandBodies <= 64 && kMaxTOIContacts <= 64, "a lane per body and constraint");
+__device__ inline void toiSolveIsland(const WorldView& w, const ConView& cv, ToiState* st, unsigned long long* keys,
+                                      float4* rows, const b2g_manifold* man, const int* touching, float dt,
+                                      int velIters) {
     const int n = st->nGather;
-    const bool sorted = n <= kToiGatherCap;
-    if (sorted) {
+    if (n > 64 && n <= kToiGatherCap) {
         int size = 1;
         while (size < n) size <<= 1;
-        for (int i = threadIdx.x; i < size; i += blockDim.x) keys[i] = i < n ? gather[i] : ~0ull;
+        for (int i = n + threadIdx.x; i < size; i += blockDim.x) keys[i] = ~0ull;
         __syncthreads();
         for (int k = 2; k <= size; k <<= 1) {
             for (int j = k >> 1; j > 0; j >>= 1) {
@@ -6540,10 +6621,19 @@ __global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, Toi
             }
         }
     }
-    if (threadIdx.x != 0) return;
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
     const int bA = st->bodyA, bB = st->bodyB;
     const int nc = st->live;
-    if (sorted) {
+    if (n <= 64) {
+        const unsigned long long key = lane < n ? keys[lane] : ~0ull;
+        int rank = 0;
+        for (int j = 0; j < n; ++j) rank += keys[j] < key ? 1 : 0;
+        __threadfence_block();
+        if (lane < n) keys[rank] = key;
+        __threadfence_block();
+        toiCommitWave(w, st, lane < n ? keys[lane] : 0ull, lane < n, man, touching);
+    } else if (lane == 0 && n <= kToiGatherCap) {
         for (int i = 0; i < n; ++i) {
             if (st->nBodies == 2 * kMaxTOIContacts || st->nContacts == kMaxTOIContacts) break;
             const unsigned long long key = keys[i];
@@ -6552,7 +6642,7 @@ __global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, Toi
             const int slot = (int)(key & ((1u << kGatherSlotBits) - 1));
             toiCommitEdge(w, st, k == 0 ? bA : bB, c, man[slot], touching[slot] != 0);
         }
-    } else {
+    } else if (lane == 0) {
         // more edges than the sort holds: walk the list once per body
         for (int k = 0; k < 2; ++k) {
             const int body = k == 0 ? bA : bB;
@@ -6564,34 +6654,95 @@ __global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, Toi
             }
         }
     }
+    __threadfence_block();
     // b2Island::SolveTOI
-    const FreshView noFresh{nullptr, nullptr, nullptr, 0};
-    const int ncons = st->nContacts;
-    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, noFresh);
+    const int ncons = st->nContacts, nbody = st->nBodies;
+    const int myBody = lane < nbody ? st->bodies[lane] : 0;
+    if (lane < nbody) rows[lane] = w.pos[myBody];
+    if (lane < ncons) initConstraintOne(w, cv, lane, st->contacts[lane], 1.0f, 0, FreshView{});
+    __threadfence_block();
+    PosRow p{};
+    int slotA = 0, slotB = 0;
+    if (lane < ncons) {
+        p = loadPosRow(cv, lane);
+        for (int i = 0; i < nbody; ++i) {
+            const int b = st->bodies[i];
+            if (b == p.bodies.x) slotA = i;
+            if (b == p.bodies.y) slotB = i;
+        }
+        // b2ContactSolver::SolveTOIPositionConstraints, REF/Dynamics/Contacts/
+        // b2ContactSolver.cpp:753-841: only the TOI pair moves.
+        if (slotA > 1) p.mass.x = p.mass.y = 0.0f;
+        if (slotB > 1) p.mass.z = p.mass.w = 0.0f;
+    }
+    RotPair known{};
+    if (lane < ncons) {
+        known.angleA = __float_as_uint(rows[slotA].z);
+        known.angleB = __float_as_uint(rows[slotB].z);
+        rotOf2(rows[slotA].z, rows[slotB].z, known.a, known.b);
+    }
     for (int it = 0; it < 20; ++it) {
         float minSep = 0.0f;
-        for (int k = 0; k < ncons; ++k) minSep = fminB(minSep, solveTOIPositionOne(w, cv, k, bA, bB));
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < ncons; ++k) {
+            float sep = 0.0f;
+            if (lane == k) {
+                float4 pA = rows[slotA], pB = rows[slotB];
+                sep = solvePositionRow<true>(p, pA, pB, kToiBaumgarte, &known);
+                if (slotA <= 1) rows[slotA] = pA;
+                if (slotB <= 1) rows[slotB] = pB;
+            }
+            minSep = fminB(minSep, __shfl(sep, k));
+            __threadfence_block();
+        }
         if (minSep >= -1.5f * kLinearSlop) break;
     }
-    const float4 pa = w.pos[bA], pb = w.pos[bB];
-    w.pos0[bA] = make_float4(pa.x, pa.y, pa.z, w.pos0[bA].w);
-    w.pos0[bB] = make_float4(pb.x, pb.y, pb.z, w.pos0[bB].w);
-    for (int k = 0; k < ncons; ++k) initConstraintOne(w, cv, k, st->contacts[k], 1.0f, 0, noFresh);
-    for (int it = 0; it < velIters; ++it)
-        for (int k = 0; k < ncons; ++k) solveVelocityOne(w, cv, k);
-    const float h = (1.0f - st->alpha) * dt;
-    for (int i = 0; i < st->nBodies; ++i) {
-        const int b = st->bodies[i];
-        integratePositionOne(w, b, h);
-        syncTransformOne(w, b);
+    if (lane < 2) {
+        w.pos[myBody] = rows[lane];
+        w.pos0[myBody] = make_float4(rows[lane].x, rows[lane].y, rows[lane].z, w.pos0[myBody].w);
     }
+    __threadfence_block();
+    VelRow v{};
+    if (lane < ncons) {
+        initConstraintOne(w, cv, lane, st->contacts[lane], 1.0f, 0, FreshView{});
+        v = loadVelRow(cv, lane);
+    }
+    __threadfence_block();
+    if (lane < nbody) rows[lane] = w.vel[myBody];
+    __threadfence_block();
+    for (int it = 0; it < velIters; ++it) {
+#pragma clang loop unroll(disable)
+        for (int k = 0; k < ncons; ++k) {
+            if (lane == k) {
+                float4 va = rows[slotA], vb = rows[slotB];
+                solveVelocityRow(v, va, vb);
+                if (v.info & 16) rows[slotA] = va;
+                if (v.info & 32) rows[slotB] = vb;
+            }
+            __threadfence_block();
+        }
+    }
+    const float h = (1.0f - st->alpha) * dt;
+    if (lane < nbody) {
+        w.vel[myBody] = rows[lane];
+        integratePositionOne(w, myBody, h);
+        syncTransformOne(w, myBody);
+    }
+}
+__global__ __launch_bounds__(256) void k_toi_island(WorldView w, ConView cv, ToiState* st,
+                                                    const unsigned long long* gather, const b2g_manifold* man,
+                                                    const int* touching, float dt, int velIters) {
+    __shared__ unsigned long long keys[kToiGatherCap];
+    __shared__ float4 rows[kToiIslandBodies];
+    if (st->halt || !st->active) return;
+    for (int i = threadIdx.x; i < min(st->nGather, kToiGatherCap); i += blockDim.x) keys[i] = gather[i];
+    __syncthreads();
+    toiSolveIsland(w, cv, st, keys, rows, man, touching, dt, velIters);
 }
 
 // Fixtures of the island's dynamic bodies to their swept boxes, and the
 // cached TOIs and island marks of every contact on such a body dropped.
-__global__ void k_toi_displaced(WorldView w, ToiState* st) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (st->halt || !st->active) return;
+__device__ inline void toiDisplacedOne(const WorldView& w, ToiState* st, int i) {
     if (i < w.nFixtures) {
         const int b = w.fbody[i];
         if ((w.bflags[b] & BF_ISLAND) && w.btype[b] == BT_DYNAMIC && syncFixtureOne(w, i, b)) {
@@ -6606,13 +6757,16 @@ __global__ void k_toi_displaced(WorldView w, ToiState* st) {
         if (hit) w.cflags[i] &= ~(CF_TOI | CF_ISLAND);
     }
 }
+__global__ void k_toi_displaced(WorldView w, ToiState* st) {
+    if (st->halt || !st->active) return;
+    toiDisplacedOne(w, st, blockIdx.x * blockDim.x + threadIdx.x);
+}
 
 // b2BroadPhase::UpdatePairs for the event's moved proxies only: every proxy
 // whose fat box overlaps a moved one's, a pair of two moved proxies found by
 // the lower id's thread, filtered as AddPair filters.
-__global__ void k_toi_pairs(WorldView w, ToiState* st, const unsigned long long* table, uint32_t hmask) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= w.nFixtures || st->halt || !st->active) return;
+__device__ inline void toiPairsOne(const WorldView& w, ToiState* st, const unsigned long long* table, uint32_t hmask,
+                                   int f) {
     const int nm = st->nMoved;
     if (nm == 0 || nm > kToiMovedCap) return;
     const float4 ff = w.fat[f];
@@ -6628,15 +6782,18 @@ __global__ void k_toi_pairs(WorldView w, ToiState* st, const unsigned long long*
         if (slot < kToiNewCap) st->newKeys[slot] = pairKey(orderOf(w, a), orderOf(w, b));
     }
 }
+__global__ void k_toi_pairs(WorldView w, ToiState* st, const unsigned long long* table, uint32_t hmask) {
+    const int f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= w.nFixtures || st->halt || !st->active) return;
+    toiPairsOne(w, st, table, hmask, f);
+}
 
 // New contacts of the event in pair order (sorted keys, as the reference
 // sorts its pair buffer), appended to the table and its hash; the moved
 // flags cleared. Lists that overflowed leave everything to the host's grid
 // broad-phase instead.
-__global__ __launch_bounds__(256) void k_toi_append(WorldView w, ToiState* st, unsigned long long* table,
-                                                   uint32_t hmask, int capContacts, int subStepping) {
-    __shared__ unsigned long long keys[kToiNewCap];
-    if (st->halt) return;
+__device__ inline void toiAppend(const WorldView& w, ToiState* st, unsigned long long* keys,
+                                 unsigned long long* table, uint32_t hmask, int capContacts, int subStepping) {
     if (!st->active) {
         __syncthreads();
         if (threadIdx.x == 0) toiResetEvent(st);
@@ -6694,6 +6851,109 @@ __global__ __launch_bounds__(256) void k_toi_append(WorldView w, ToiState* st, u
             st->subStop = 1;
             st->halt = 1;
         }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_toi_append(WorldView w, ToiState* st, unsigned long long* table,
+                                                   uint32_t hmask, int capContacts, int subStepping) {
+    __shared__ unsigned long long keys[kToiNewCap];
+    if (st->halt) return;
+    toiAppend(w, st, keys, table, hmask, capContacts, subStepping);
+}
+
+// The events of a small world one after another in one workgroup: each of
+// them is a chain of eleven stages over a few hundred contacts, and as
+// launches of their own the stages take 4.5 us each however little they do.
+// A step with its events, this kernel against launches for each stage: 344
+// against 501 us (terrain, 589 contacts, 3 events), 636 against 809 us (2880
+// contacts, 6 events), 5.3 against 5.8 ms (bullets, 474 contacts, 36 events);
+// beyond the lists' 4096 contacts the two are equal. A launch does up to
+// `most` events; new pairs that take the table past the lists end it.
+constexpr int kToiSmallContacts = 4096;
+constexpr int kToiSmallFixtures = 4096;
+constexpr int kToiSmallEvents = 64;  // events of a launch
+constexpr int kToiSmallScan = 1024;  // contacts whose first scan stays in the workgroup
+__global__ void __launch_bounds__(256)
+    k_toi_events(WorldView w, ConView cv, ToiState* global, Sweep* seen, b2g_manifold* man, int* touching,
+                 unsigned long long* table, uint32_t hmask, int capContacts, int subStepping, float dt, int velIters,
+                 int most) {
+    __shared__ ToiState state;
+    __shared__ unsigned long long keys[kToiGatherCap];
+    __shared__ float4 rows[kToiIslandBodies];
+    __shared__ unsigned pendingBits[kToiSmallContacts / 32];
+    __shared__ uint16_t pendingList[kToiSmallContacts];
+    __shared__ int nPending;
+    static_assert(kToiGatherCap >= kToiNewCap, "the new pairs' sort uses the same keys");
+    ToiState* st = &state;
+    const int t = threadIdx.x, T = blockDim.x;
+    if (t == 0) {
+        st->done = global->done;
+        st->events = global->events;
+        st->live = global->live;
+        st->added = global->added;
+        st->halt = global->halt;
+        st->subStop = global->subStop;
+        toiResetEvent(st);
+    }
+    __syncthreads();
+    for (int e = 0; e < most && !st->halt && st->live <= kToiSmallContacts; ++e) {
+        const int live = st->live;
+        for (int i = t; i < (live + 31) / 32; i += T) pendingBits[i] = 0u;
+        if (t == 0) nPending = 0;
+        __syncthreads();
+        for (int c = t; c < live; c += T) {
+            if (!toiPending(w, c, w.cflags[c])) continue;
+            pendingList[atomicAdd(&nPending, 1)] = (uint16_t)c;
+            atomicOr(&pendingBits[c >> 5], 1u << (c & 31));
+            if (sweepsDiffer(w, c)) st->mismatch = 1;
+        }
+        __syncthreads();
+        if (st->mismatch) {
+            if (t < 64)
+                toiAlignOrdered(w, live, seen, [&](int c) { return (pendingBits[c >> 5] >> (c & 31)) & 1u; });
+            __syncthreads();
+        }
+        // spread over the wavefronts: each waits for its slowest lane
+        for (int i = (t & 63) * (T / 64) + (t >> 6); i < nPending; i += T)
+            toiComputeOne(w, pendingList[i], st->mismatch != 0, seen);
+        __syncthreads();
+        unsigned long long key = ~0ull;
+        for (int c = t; c < live; c += T) {
+            const unsigned long long k = toiKey(w, c, live);
+            key = k < key ? k : key;
+        }
+        key = toiWaveMin(key);
+        if ((t & 63) == 0 && key != ~0ull) atomicMin(&st->minKey, key);
+        __syncthreads();
+        if (t == 0) toiStartEvent(w, st);
+        __syncthreads();
+        if (st->active) {
+            for (int c = t; c < live; c += T) toiGatherOne(w, st, keys, c);
+            __syncthreads();
+            for (int i = t; i < min(st->nGather, kToiGatherCap); i += T) toiPrepOne(w, st, keys[i], man, touching);
+            __syncthreads();
+            toiSolveIsland(w, cv, st, keys, rows, man, touching, dt, velIters);
+            __syncthreads();
+            for (int i = t; i < max(live, w.nFixtures); i += T) toiDisplacedOne(w, st, i);
+            __syncthreads();
+            for (int f = t; f < w.nFixtures; f += T) toiPairsOne(w, st, table, hmask, f);
+            __syncthreads();
+        }
+        const int halted = st->halt;
+        __syncthreads();
+        if (!halted) toiAppend(w, st, keys, table, hmask, capContacts, subStepping);
+        __syncthreads();
+    }
+    if (t == 0) {
+        global->done = st->done;
+        global->events = st->events;
+        global->live = st->live;
+        global->added = st->added;
+        global->halt = st->halt;
+        global->subStop = st->subStop;
+        global->fallback = st->fallback;
+        global->nMoved = st->nMoved;
+        global->nNew = st->nNew;
     }
 }
 
@@ -8954,7 +9214,8 @@ __global__ void k_toi_resume(ToiState* st, int live) {
 }
 
 // b2World::SolveTOI, REF/Dynamics/b2World.cpp:579-897. The events run on the
-// device, one launch sequence each, in batches that grow geometrically;
+// device: a small world's in one kernel (k_toi_events), a larger one's with one
+// launch sequence each, in batches that grow geometrically;
 // every kernel of an event does nothing once the pass has halted (no event
 // left, a list overflowed, or the sub-step is over), and the host reads one
 // small record per batch. The contact count lives on the device during the
@@ -8986,6 +9247,7 @@ int solveTOI(b2g_context* ctx, const b2g_step_params* p) {
     LAUNCHCHK(ctx);
     const int pe = profStart(ctx);
     int batch = 1;
+    bool first = true;
     for (;;) {
         // every event raises some contact's TOI count or disables it, so a
         // pass ends within kMaxSubSteps + 1 events per contact
@@ -8998,9 +9260,24 @@ int solveTOI(b2g_context* ctx, const b2g_step_params* p) {
         }
         const WorldView w = ctx->view();
         const int cap = ctx->capContacts;
-        for (int e = 0; e < batch; ++e) {
+        const bool small = ctx->nContacts <= kToiSmallContacts && ctx->nFixtures <= kToiSmallFixtures &&
+                           ctx->sched.tailColours != 0;
+        // The pass's first scan is of all contacts, and their sweeps start
+        // together: in a larger world the chip does it. (At 589 contacts, 100 of
+        // them pending, two launches cost 18 us more than they save.)
+        if (small && first && ctx->stepComplete && ctx->nContacts > kToiSmallScan) {
+            hipLaunchKernelGGL(k_toi_classify, dim3(blocks(ctx->nContacts)), dim3(256), 0, s, w, ctx->keep, st);
+            hipLaunchKernelGGL(k_toi_compute, dim3(blocks(ctx->nContacts, 64)), dim3(64), 0, s, w, ctx->keep, st,
+                               ctx->toiSeen);
+        }
+        first = false;
+        if (small)
+            hipLaunchKernelGGL(k_toi_events, dim3(1), dim3(256), 0, s, w, ctx->toiCv, st, ctx->toiSeen, ctx->toiMan,
+                               ctx->toiTouch, ctx->hashTable, ctx->hashMask, cap, ctx->subStepping ? 1 : 0, p->dt,
+                               p->velocityIterations, kToiSmallEvents);
+        for (int e = 0; e < batch && !small; ++e) {
             hipLaunchKernelGGL(k_toi_classify, dim3(blocks(cap)), dim3(256), 0, s, w, ctx->keep, st);
-            hipLaunchKernelGGL(k_toi_align_serial, dim3(1), dim3(64), 0, s, w, ctx->keep, st, ctx->toiSeen);
+            hipLaunchKernelGGL(k_toi_align, dim3(1), dim3(64), 0, s, w, ctx->keep, st, ctx->toiSeen);
             hipLaunchKernelGGL(k_toi_compute, dim3(blocks(cap, 64)), dim3(64), 0, s, w, ctx->keep, st, ctx->toiSeen);
             hipLaunchKernelGGL(k_toi_min, dim3(blocks(cap)), dim3(256), 0, s, w, st);
             hipLaunchKernelGGL(k_toi_event, dim3(1), dim3(64), 0, s, w, st);

@@ -82,7 +82,8 @@ def test_equals_a_launch_per_colour(gpu, kind, n, seed, steps, sleep, vel, pos):
 
 
 @pytest.mark.parametrize("kind, n, ccd", [("terrain", 60, True), ("bullets", 40, True), ("sensors", 30, False),
-                                          ("oneway", 6, True)])
+                                          ("oneway", 6, True), ("bullets", 130, True), ("terrain", 250, True),
+                                          ("plank", 100, True), ("world", 700, True), ("world", 2300, True)])
 def test_with_events_and_sensors(gpu, kind, n, ccd):
     same(run(gpu.world(kind, n, 2, ccd=ccd), False, 60), run(gpu.world(kind, n, 2, ccd=ccd), True, 60))
 
