@@ -10714,9 +10714,8 @@ int b2g_mlp_train(b2g_context* ctx, int epochs, int batch, float lr, uint32_t se
             const int count = std::min(batch, n - first);
             hipEvent_t e0, e1;
             const int pk = profKernelEvents(ctx, &e0, &e1);
-            HIPCHK(ctx, mlpGradient(net, ctx->logFeat, ctx->logTarget, order, first, count, s, e0, e1));
+            HIPCHK(ctx, mlpTrainStep(net, ctx->logFeat, ctx->logTarget, order, first, count, lr, s, e0, e1));
             profKernel(ctx, PH_K_MLP_GRAD, pk);
-            HIPCHK(ctx, mlpAdam(net, lr, s));
         }
         float l = 0.0f;
         HIPCHK(ctx, hipMemcpyAsync(&l, net.loss, sizeof(float), hipMemcpyDeviceToHost, s));

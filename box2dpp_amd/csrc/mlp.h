@@ -44,7 +44,7 @@ constexpr int kNormXMean = 0, kNormXInv = 16, kNormYMean = 32, kNormYStd = 34, k
 
 struct Net {
     float* params = nullptr;  // kParams, FP32 master weights
-    float* grad = nullptr;    // kParams, accumulated by mlpGradient, cleared by mlpAdam
+    float* grad = nullptr;    // kParams, accumulated by mlpGradient, cleared by mlpTrainStep
     float* m = nullptr;       // Adam first moment
     float* v = nullptr;       // Adam second moment
     uint16_t* wh = nullptr;   // hTotal BF16 weights
@@ -68,8 +68,10 @@ hipError_t mlpForward(const Net& n, const float* x, int count, float* y, hipStre
 // standardised targets, N = count, and adds L to *n.loss.
 hipError_t mlpGradient(const Net& n, const float* x, const float* t, const int* order, int first, int count,
                        hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
-// One Adam step from n.grad (then cleared); refreshes the BF16 image.
-hipError_t mlpAdam(Net& n, float lr, hipStream_t s);
+// One training step: the gradient as above, and an Adam step from n.grad with
+// it (then cleared), which refreshes the BF16 image.
+hipError_t mlpTrainStep(Net& n, const float* x, const float* t, const int* order, int first, int count, float lr,
+                        hipStream_t s, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // Impulses for the candidate contact points of the step: rows of feat
 // (count x 16) through the network, clamped to the friction cone, written
 // into the constraint impulses imp[ref[i] >> 1] component (ref[i] & 1). With

@@ -87,22 +87,26 @@ __device__ inline Cdf gaussCdf(float x) {
     r.pdf = 0.39894228040143268f * e;
     return r;
 }
-__device__ inline float gelu(float x) { return x * gaussCdf(x).cdf; }
-__device__ inline float geluGrad(float x) {
+// The value, and the derivative for the backward pass: one exponential and one
+// reciprocal for both.
+__device__ inline float gelu(float x, float& grad) {
     const Cdf c = gaussCdf(x);
-    return c.cdf + x * c.pdf;
+    grad = c.cdf + x * c.pdf;
+    return x * c.cdf;
 }
 
 struct Smem {
-    uint16_t w[hTotal];
+    alignas(16) uint16_t w[hTotal];
     float b[kBiasCount];   // b1 | b2 | b3 | b4 (padded)
     float norm[kNorm];
 };
 
 __device__ inline void loadSmem(Smem& S, const uint16_t* wh, const float* params, const float* norm) {
-    const uint32_t* src = (const uint32_t*)wh;
-    uint32_t* dst = (uint32_t*)S.w;
-    for (int i = threadIdx.x; i < hTotal / 2; i += blockDim.x) dst[i] = src[i];
+    static_assert(hTotal % 8 == 0, "16-byte copies");
+    const uint4* src = (const uint4*)wh;
+    uint4* dst = (uint4*)S.w;
+#pragma unroll 5
+    for (int i = threadIdx.x; i < hTotal / 8; i += blockDim.x) dst[i] = src[i];
     for (int i = threadIdx.x; i < kHidden; i += blockDim.x) {
         S.b[i] = params[kB1 + i];
         S.b[kHidden + i] = params[kB2 + i];
@@ -142,18 +146,21 @@ __device__ inline f32x4 product64(const Smem& S, int wOff, int ldw, int mt, cons
     return acc;
 }
 
-// Hidden layer: acc[mt] = W[16mt + c][.] x in + bias; the 16-feature input
-// layer with one 16x16x16 product, the 64-feature ones with product64.
+// Hidden layer: W[16mt + c][.] x in + bias, its GELU in a and the GELU's
+// derivative in dz; the 16-feature input layer with one 16x16x16 product, the
+// 64-feature ones with product64.
 template <int KT>
-__device__ inline void hiddenLayer(const Smem& S, int wOff, int ldw, int bOff, const bf16x4* in, f32x4* z,
+__device__ inline void hiddenLayer(const Smem& S, int wOff, int ldw, int bOff, const bf16x4* in, f32x4* dz,
                                    bf16x4* a, int g, int c) {
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
         f32x4 acc = biasTile(S, bOff + 16 * mt, g);
         if (KT == 1) acc = mfma(frag(&S.w[wOff + (16 * mt + c) * ldw + 4 * g]), in[0], acc);
         else acc = product64(S, wOff, ldw, mt, in, acc, g, c);
-        z[mt] = acc;
-        a[mt] = pack4(gelu(acc[0]), gelu(acc[1]), gelu(acc[2]), gelu(acc[3]));
+        float d[4], v[4];
+        for (int j = 0; j < 4; ++j) v[j] = gelu(acc[j], d[j]);
+        for (int j = 0; j < 4; ++j) dz[mt][j] = d[j];
+        a[mt] = pack4(v[0], v[1], v[2], v[3]);
     }
 }
 
@@ -215,7 +222,8 @@ __global__ __launch_bounds__(kThreads) void k_mlp_infer(const uint16_t* wh, cons
 
 // ------------------------------------------------------------ training
 // Per-wave 16x16 transpose through LDS: in holds rows 4g..4g+3 of column c;
-// the result holds row c, columns 4g..4g+3, as BF16.
+// the result holds row c, columns 4g..4g+3, as BF16. For the output layer's
+// gradient, where an infinite target must not reach the other output.
 __device__ inline bf16x4 transposeF(float (*T)[17], f32x4 d, int g, int c) {
     for (int j = 0; j < 4; ++j) T[4 * g + j][c] = d[j];
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -225,18 +233,21 @@ __device__ inline bf16x4 transposeF(float (*T)[17], f32x4 d, int g, int c) {
     __builtin_amdgcn_wave_barrier();
     return r;
 }
-__device__ inline bf16x4 transposeH(uint16_t (*T)[18], bf16x4 d, int g, int c) {
-    for (int j = 0; j < 4; ++j) T[4 * g + j][c] = (uint16_t)d[j];
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    bf16x4 r;
-    for (int j = 0; j < 4; ++j) r[j] = (short)T[c][4 * g + j];
-    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    return r;
-}
-
 __device__ inline bf16x4 packTile(f32x4 d) { return pack4(d[0], d[1], d[2], d[3]); }
+
+// The same transpose on the matrix cores: read as an A operand, rows 4g..4g+3
+// of column c are the transposed matrix, and its product with the identity
+// has it in the accumulator's layout. Every sum is one value and zeros, so
+// nothing is rounded; 25 of them a tile are 25 products instead of 25 trips
+// to LDS of four writes and four reads.
+__device__ inline bf16x4 identityTile(int g, int c) {
+    return pack4(4 * g == c ? 1.0f : 0.0f, 4 * g + 1 == c ? 1.0f : 0.0f, 4 * g + 2 == c ? 1.0f : 0.0f,
+                 4 * g + 3 == c ? 1.0f : 0.0f);
+}
+__device__ inline bf16x4 transpose(bf16x4 d, bf16x4 identity) {
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    return packTile(mfma(d, identity, zero));
+}
 
 // Sum over the 16 lanes that share g (lanes 16g..16g+15).
 __device__ inline float groupSum16(float v) {
@@ -254,15 +265,13 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
     __shared__ float red[kParams];
     __shared__ float lossShared;
     __shared__ float tf[kWaves][16][17];
-    __shared__ uint16_t th[kWaves][16][18];
     loadSmem(S, wh, params, norm);
-    for (int i = threadIdx.x; i < kParams; i += blockDim.x) red[i] = 0.0f;
     if (threadIdx.x == 0) lossShared = 0.0f;
     __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, c = lane & 15;
     float (*TF)[17] = tf[wave];
-    uint16_t (*TH)[18] = th[wave];
+    const bf16x4 ident = identityTile(g, c);
 
     f32x4 gW1[4], gW2[4][4], gW3[4][4], gW4[4];
     float gb1[4][4], gb2[4][4], gb3[4][4], gb4[4];
@@ -283,9 +292,9 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
         const int local = t * 16 + c;
         const bool valid = local < count;
         const long long s = valid ? (order ? (long long)order[first + local] : (long long)first + local) : 0;
-        // forward, keeping pre-activations and activations
+        // forward, keeping activations and their derivatives
         bf16x4 x0[1] = {inputFrag(S, x, s, valid, g)};
-        f32x4 z1[4], z2[4], z3[4];
+        f32x4 z1[4], z2[4], z3[4];  // the GELUs' derivatives
         bf16x4 a1[4], a2[4], a3[4];
         hiddenLayer<1>(S, hW1, kIn, 0, x0, z1, a1, g, c);
         hiddenLayer<4>(S, hW2, kHidden, kHidden, a1, z2, a2, g, c);
@@ -305,7 +314,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
         {
             const bf16x4 dT = transposeF(TF, d4, g, c);
 #pragma unroll
-            for (int ni = 0; ni < 4; ++ni) gW4[ni] = mfma(dT, transposeH(TH, a3[ni], g, c), gW4[ni]);
+            for (int ni = 0; ni < 4; ++ni) gW4[ni] = mfma(dT, transpose(a3[ni], ident), gW4[ni]);
             for (int j = 0; j < 4; ++j) gb4[j] += d4[j];
         }
         f32x4 d3[4];
@@ -314,114 +323,93 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
                 f32x4 acc = mfma(frag(&S.w[hW4t + (16 * mt + c) * kOutPad + 4 * g]), dB, zero4);
-                for (int j = 0; j < 4; ++j) acc[j] *= geluGrad(z3[mt][j]);
+                for (int j = 0; j < 4; ++j) acc[j] *= z3[mt][j];
                 d3[mt] = acc;
             }
         }
         // layer 3
         {
             bf16x4 hT[4], dB[4];
-            for (int ni = 0; ni < 4; ++ni) hT[ni] = transposeH(TH, a2[ni], g, c);
+            for (int ni = 0; ni < 4; ++ni) hT[ni] = transpose(a2[ni], ident);
 #pragma unroll
             for (int mo = 0; mo < 4; ++mo) {
-                const bf16x4 dT = transposeF(TF, d3[mo], g, c);
+                dB[mo] = packTile(d3[mo]);
+                const bf16x4 dT = transpose(dB[mo], ident);
 #pragma unroll
                 for (int ni = 0; ni < 4; ++ni) gW3[mo][ni] = mfma(dT, hT[ni], gW3[mo][ni]);
                 for (int j = 0; j < 4; ++j) gb3[mo][j] += d3[mo][j];
-                dB[mo] = packTile(d3[mo]);
             }
             f32x4 d2[4];
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
                 f32x4 acc = product64(S, hW3t, kHidden, mt, dB, zero4, g, c);
-                for (int j = 0; j < 4; ++j) acc[j] *= geluGrad(z2[mt][j]);
+                for (int j = 0; j < 4; ++j) acc[j] *= z2[mt][j];
                 d2[mt] = acc;
             }
             // layer 2
-            for (int ni = 0; ni < 4; ++ni) hT[ni] = transposeH(TH, a1[ni], g, c);
+            for (int ni = 0; ni < 4; ++ni) hT[ni] = transpose(a1[ni], ident);
 #pragma unroll
             for (int mo = 0; mo < 4; ++mo) {
-                const bf16x4 dT = transposeF(TF, d2[mo], g, c);
+                dB[mo] = packTile(d2[mo]);
+                const bf16x4 dT = transpose(dB[mo], ident);
 #pragma unroll
                 for (int ni = 0; ni < 4; ++ni) gW2[mo][ni] = mfma(dT, hT[ni], gW2[mo][ni]);
                 for (int j = 0; j < 4; ++j) gb2[mo][j] += d2[mo][j];
-                dB[mo] = packTile(d2[mo]);
             }
             // layer 1
-            const bf16x4 xT = transposeH(TH, x0[0], g, c);
+            const bf16x4 xT = transpose(x0[0], ident);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
                 f32x4 acc = product64(S, hW2t, kHidden, mt, dB, zero4, g, c);
-                for (int j = 0; j < 4; ++j) acc[j] *= geluGrad(z1[mt][j]);
-                const bf16x4 dT = transposeF(TF, acc, g, c);
+                for (int j = 0; j < 4; ++j) acc[j] *= z1[mt][j];
+                const bf16x4 dT = transpose(packTile(acc), ident);
                 gW1[mt] = mfma(dT, xT, gW1[mt]);
                 for (int j = 0; j < 4; ++j) gb1[mt][j] += acc[j];
             }
         }
     }
-    // Reduce the four wavefronts in LDS, one wavefront after another (each
-    // lane owns distinct entries, so plain read-add-writes): accumulator
-    // element j of tile (mo, ni) is dW[16mo + 4g + j][16ni + c]. Then the
-    // workgroup's sums go to its row of `partial`, which k_mlp_reduce adds up
-    // in a fixed order: the gradient does not depend on the schedule.
+    // Reduce the four wavefronts in LDS: in each of four turns a wavefront adds
+    // one quarter of its sums, a different one each, so that all four work at
+    // once (each lane owns distinct entries, so plain read-add-writes, the first
+    // turn's a write): accumulator element j of tile (mo, ni) is
+    // dW[16mo + 4g + j][16ni + c]. Then the workgroup's sums go to its row of
+    // `partial`, which k_mlp_reduce adds up in a fixed order: the gradient does
+    // not depend on the schedule.
     float l = loss;
     for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off);
-    for (int wv = 0; wv < kWaves; ++wv) {
-        if (wave == wv) {
-            for (int mo = 0; mo < 4; ++mo)
-                for (int j = 0; j < 4; ++j) {
-                    const int o = 16 * mo + 4 * g + j;
-                    red[kW1 + o * kIn + c] += gW1[mo][j];
-                    for (int ni = 0; ni < 4; ++ni) {
-                        red[kW2 + o * kHidden + 16 * ni + c] += gW2[mo][ni][j];
-                        red[kW3 + o * kHidden + 16 * ni + c] += gW3[mo][ni][j];
-                    }
-                }
-            for (int ni = 0; ni < 4; ++ni)
-                for (int j = 0; j < 4; ++j) red[kW4 + (4 * g + j) * kHidden + 16 * ni + c] += gW4[ni][j];
-            for (int mt = 0; mt < 4; ++mt)
-                for (int j = 0; j < 4; ++j) {
-                    const float s1 = groupSum16(gb1[mt][j]), s2 = groupSum16(gb2[mt][j]), s3 = groupSum16(gb3[mt][j]);
-                    if (c == 0) {
-                        red[kB1 + 16 * mt + 4 * g + j] += s1;
-                        red[kB2 + 16 * mt + 4 * g + j] += s2;
-                        red[kB3 + 16 * mt + 4 * g + j] += s3;
-                    }
-                }
+#pragma clang loop unroll(disable)
+    for (int turn = 0; turn < kWaves; ++turn) {
+        auto add = [&](int i, float v) { red[i] = turn == 0 ? v : red[i] + v; };
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (((wave + turn) & 3) != q) continue;
             for (int j = 0; j < 4; ++j) {
-                const float s4 = groupSum16(gb4[j]);
-                if (c == 0) red[kB4 + 4 * g + j] += s4;
+                const int o = 16 * q + 4 * g + j;
+                add(kW1 + o * kIn + c, gW1[q][j]);
+                for (int ni = 0; ni < 4; ++ni) {
+                    add(kW2 + o * kHidden + 16 * ni + c, gW2[q][ni][j]);
+                    add(kW3 + o * kHidden + 16 * ni + c, gW3[q][ni][j]);
+                }
+                add(kW4 + (4 * g + j) * kHidden + 16 * q + c, gW4[q][j]);
+                const float s1 = groupSum16(gb1[q][j]), s2 = groupSum16(gb2[q][j]), s3 = groupSum16(gb3[q][j]);
+                if (c == 0) {
+                    add(kB1 + o, s1);
+                    add(kB2 + o, s2);
+                    add(kB3 + o, s3);
+                }
             }
-            if (lane == 0) lossShared += l;
+            if (q == 0)
+                for (int j = 0; j < 4; ++j) {
+                    const float s4 = groupSum16(gb4[j]);
+                    if (c == 0) add(kB4 + 4 * g + j, s4);
+                }
         }
+        if (lane == 0 && wave == turn) lossShared += l;
         __syncthreads();
     }
     float* row = partial + (size_t)blockIdx.x * (kParams + 1);
     for (int i = threadIdx.x; i < kParams; i += blockDim.x) row[i] = red[i];
     if (threadIdx.x == 0) row[kParams] = lossShared;
-}
-
-// Sum of the workgroups' rows added to the gradient and the loss, in a
-// fixed order: a workgroup takes kReduceCols consecutive entries; its
-// kReduceSplit lane groups each sum every kReduceSplit-th row in row order
-// (coalesced across the entries), then the groups' sums are added in group
-// order.
-constexpr int kReduceCols = 64, kReduceSplit = 4;
-__global__ __launch_bounds__(kReduceCols * kReduceSplit) void k_mlp_reduce(const float* partial, int rows,
-                                                                            float* grad, float* loss) {
-    __shared__ float part[kReduceSplit][kReduceCols];
-    const int col = threadIdx.x % kReduceCols, grp = threadIdx.x / kReduceCols;
-    const int i = blockIdx.x * kReduceCols + col;
-    float acc = 0.0f;
-    if (i <= kParams)
-        for (int r = grp; r < rows; r += kReduceSplit) acc += partial[(size_t)r * (kParams + 1) + i];
-    part[grp][col] = acc;
-    __syncthreads();
-    if (grp != 0 || i > kParams) return;
-    float sum = part[0][col];
-    for (int k = 1; k < kReduceSplit; ++k) sum += part[k][col];
-    if (i < kParams) grad[i] += sum;
-    else *loss += sum;
 }
 
 // BF16 image entries of parameter i (weights only; biases stay FP32).
@@ -449,18 +437,53 @@ __global__ void k_mlp_image(const float* params, uint16_t* wh) {
     if (i < kParams) writeImage(wh, i, params[i]);
 }
 
-__global__ void k_mlp_adam(float* params, float* grad, float* m, float* v, uint16_t* wh, float lr, float c1, float c2) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= kParams) return;
-    const float gi = grad[i];
-    grad[i] = 0.0f;
-    const float mi = 0.9f * m[i] + 0.1f * gi;
-    const float vi = 0.999f * v[i] + 0.001f * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    const float p = params[i] - lr * (mi * c1) / (sqrtf(vi * c2) + 1e-8f);
-    params[i] = p;
-    writeImage(wh, i, p);
+struct AdamState {
+    float *params, *m, *v;
+    uint16_t* wh;
+    float lr, c1, c2;
+};
+__device__ inline void adamOne(const AdamState& a, int i, float gi) {
+    const float mi = 0.9f * a.m[i] + 0.1f * gi;
+    const float vi = 0.999f * a.v[i] + 0.001f * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    const float p = a.params[i] - a.lr * (mi * a.c1) / (sqrtf(vi * a.c2) + 1e-8f);
+    a.params[i] = p;
+    writeImage(a.wh, i, p);
+}
+
+// Sum of the workgroups' rows added to the gradient and the loss, in a
+// fixed order: a workgroup takes kReduceCols consecutive entries; its
+// kReduceSplit lane groups each sum every kReduceSplit-th row in row order
+// (coalesced across the entries), then the groups' sums are added in group
+// order. In training the entries' Adam step follows in the same lanes.
+// Bound by the trips for the rows (10.7 MB at 256 rows): REDUCE_FIGURES
+constexpr int kReduceCols = 64, kReduceSplit = 16;
+template <bool kAdam>
+__global__ __launch_bounds__(kReduceCols * kReduceSplit) void k_mlp_reduce(const float* partial, int rows,
+                                                                            float* grad, float* loss, AdamState adam) {
+    __shared__ float part[kReduceSplit][kReduceCols];
+    const int col = threadIdx.x % kReduceCols, grp = threadIdx.x / kReduceCols;
+    const int i = blockIdx.x * kReduceCols + col;
+    float acc = 0.0f;
+    if (i <= kParams) {
+#pragma unroll 8
+        for (int r = grp; r < rows; r += kReduceSplit) acc += partial[(size_t)r * (kParams + 1) + i];
+    }
+    part[grp][col] = acc;
+    __syncthreads();
+    if (grp != 0 || i > kParams) return;
+    float sum = part[0][col];
+#pragma unroll
+    for (int k = 1; k < kReduceSplit; ++k) sum += part[k][col];
+    if (i == kParams) {
+        *loss += sum;
+    } else if (kAdam) {
+        adamOne(adam, i, grad[i] + sum);
+        grad[i] = 0.0f;
+    } else {
+        grad[i] += sum;
+    }
 }
 
 int gridFor(int count) {
@@ -525,9 +548,9 @@ hipError_t mlpPredictImpulses(const Net& n, const float* feat, const int* ref, c
     return hipGetLastError();
 }
 
-hipError_t mlpGradient(const Net& n, const float* x, const float* t, const int* order, int first, int count,
-                       hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
-    if (count <= 0) return hipSuccess;
+namespace {
+int launchGrad(const Net& n, const float* x, const float* t, const int* order, int first, int count, hipStream_t s,
+               hipEvent_t e0, hipEvent_t e1) {
     // one workgroup per CU at most (the kernel's LDS allows one), each
     // wavefront taking as many 16-sample tiles as needed
     const int tiles = (count + 15) / 16;
@@ -536,17 +559,30 @@ hipError_t mlpGradient(const Net& n, const float* x, const float* t, const int* 
     if (grid < 1) grid = 1;
     hipExtLaunchKernelGGL(k_mlp_grad, dim3(grid), dim3(kThreads), 0, s, e0, e1, 0, n.wh, n.params, n.norm, x, t,
                           order, first, count, 1.0f / (float)count, n.partial);
-    hipLaunchKernelGGL(k_mlp_reduce, dim3((kParams + 1 + kReduceCols - 1) / kReduceCols),
-                       dim3(kReduceCols * kReduceSplit), 0, s, n.partial, grid, n.grad, n.loss);
+    return grid;
+}
+constexpr int kReduceGrid = (kParams + 1 + kReduceCols - 1) / kReduceCols;
+}  // namespace
+
+hipError_t mlpGradient(const Net& n, const float* x, const float* t, const int* order, int first, int count,
+                       hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+    if (count <= 0) return hipSuccess;
+    const int grid = launchGrad(n, x, t, order, first, count, s, e0, e1);
+    hipLaunchKernelGGL(k_mlp_reduce<false>, dim3(kReduceGrid), dim3(kReduceCols * kReduceSplit), 0, s, n.partial, grid,
+                       n.grad, n.loss, AdamState{});
     return hipGetLastError();
 }
 
-hipError_t mlpAdam(Net& n, float lr, hipStream_t s) {
+hipError_t mlpTrainStep(Net& n, const float* x, const float* t, const int* order, int first, int count, float lr,
+                        hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+    if (count <= 0) return hipSuccess;
+    const int grid = launchGrad(n, x, t, order, first, count, s, e0, e1);
     ++n.adamStep;
     const double c1 = 1.0 / (1.0 - pow(0.9, n.adamStep));
     const double c2 = 1.0 / (1.0 - pow(0.999, n.adamStep));
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kParams + 255) / 256), dim3(256), 0, s, n.params, n.grad, n.m, n.v, n.wh, lr,
-                       (float)c1, (float)c2);
+    const AdamState adam{n.params, n.m, n.v, n.wh, lr, (float)c1, (float)c2};
+    hipLaunchKernelGGL(k_mlp_reduce<true>, dim3(kReduceGrid), dim3(kReduceCols * kReduceSplit), 0, s, n.partial, grid,
+                       n.grad, n.loss, adam);
     return hipGetLastError();
 }
 
