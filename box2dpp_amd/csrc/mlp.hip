@@ -95,8 +95,23 @@ __device__ inline float gelu(float x, float& grad) {
     return x * c.cdf;
 }
 
+// The weights in LDS. A wavefront reads 8 bytes of four neighbouring places in
+// each of 16 rows at once: with rows of 64 entries, 32 banks, eight of the rows
+// meet in the same banks; 72 entries spread the 16 rows over all 64 banks.
+constexpr int kLd = kHidden + 8;  // row stride of the 64-column matrices
+constexpr int sW1 = 0;
+constexpr int sW2 = sW1 + kHidden * kIn;
+constexpr int sW3 = sW2 + kHidden * kLd;
+constexpr int sW4 = sW3 + kHidden * kLd;
+constexpr int sW2t = sW4 + kOutPad * kLd;
+constexpr int sW3t = sW2t + kHidden * kLd;
+constexpr int sW4t = sW3t + kHidden * kLd;
+constexpr int sTotal = sW4t + kHidden * kOutPad;
+static_assert(hW2 == hW1 + kHidden * kIn && hW4t == hW2 + (4 * kHidden + kOutPad) * kHidden,
+              "the 64-column matrices lie between the two 16-column ones");
+
 struct Smem {
-    alignas(16) uint16_t w[hTotal];
+    alignas(16) uint16_t w[sTotal];
     float b[kBiasCount];   // b1 | b2 | b3 | b4 (padded)
     float norm[kNorm];
 };
@@ -104,9 +119,12 @@ struct Smem {
 __device__ inline void loadSmem(Smem& S, const uint16_t* wh, const float* params, const float* norm) {
     static_assert(hTotal % 8 == 0, "16-byte copies");
     const uint4* src = (const uint4*)wh;
-    uint4* dst = (uint4*)S.w;
 #pragma unroll 5
-    for (int i = threadIdx.x; i < hTotal / 8; i += blockDim.x) dst[i] = src[i];
+    for (int i = threadIdx.x; i < hTotal / 8; i += blockDim.x) {
+        const int e = 8 * i, row = (e - hW2) / kHidden;
+        const int at = e < hW2 ? e : e < hW4t ? sW2 + row * kLd + (e - hW2) % kHidden : sW4t + e - hW4t;
+        *(uint4*)&S.w[at] = src[i];
+    }
     for (int i = threadIdx.x; i < kHidden; i += blockDim.x) {
         S.b[i] = params[kB1 + i];
         S.b[kHidden + i] = params[kB2 + i];
@@ -116,11 +134,10 @@ __device__ inline void loadSmem(Smem& S, const uint16_t* wh, const float* params
     for (int i = threadIdx.x; i < kNorm; i += blockDim.x) S.norm[i] = norm[i];
 }
 
-// Input fragment of sample s (features 4g..4g+3), standardised; zero when
+// Input fragment of a sample (v its features 4g..4g+3), standardised; zero when
 // the sample is out of range.
-__device__ inline bf16x4 inputFrag(const Smem& S, const float* x, long long s, bool valid, int g) {
+__device__ inline bf16x4 inputFrag(const Smem& S, const float4& v, bool valid, int g) {
     if (!valid) return pack4(0.0f, 0.0f, 0.0f, 0.0f);
-    const float4 v = *(const float4*)(x + s * kIn + 4 * g);
     const int f = 4 * g;
     return pack4((v.x - S.norm[kNormXMean + f]) * S.norm[kNormXInv + f],
                  (v.y - S.norm[kNormXMean + f + 1]) * S.norm[kNormXInv + f + 1],
@@ -165,7 +182,7 @@ __device__ inline void hiddenLayer(const Smem& S, int wOff, int ldw, int bOff, c
 }
 
 __device__ inline f32x4 outputLayer(const Smem& S, const bf16x4* a3, int g, int c) {
-    return product64(S, hW4, kHidden, 0, a3, biasTile(S, 3 * kHidden, g), g, c);
+    return product64(S, sW4, kLd, 0, a3, biasTile(S, 3 * kHidden, g), g, c);
 }
 
 // ------------------------------------------------------------ inference
@@ -187,12 +204,13 @@ __global__ __launch_bounds__(kThreads) void k_mlp_infer(const uint16_t* wh, cons
     for (int t = blockIdx.x * kWaves + wave; t < tiles; t += gridDim.x * kWaves) {
         const long long s = (long long)t * 16 + c;
         const bool valid = s < n;
-        bf16x4 x0[1] = {inputFrag(S, x, s, valid, g)};
+        const float4 xv = valid ? *(const float4*)(x + s * kIn + 4 * g) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        bf16x4 x0[1] = {inputFrag(S, xv, valid, g)};
         f32x4 z[4];
         bf16x4 a1[4], a2[4], a3[4];
-        hiddenLayer<1>(S, hW1, kIn, 0, x0, z, a1, g, c);
-        hiddenLayer<4>(S, hW2, kHidden, kHidden, a1, z, a2, g, c);
-        hiddenLayer<4>(S, hW3, kHidden, 2 * kHidden, a2, z, a3, g, c);
+        hiddenLayer<1>(S, sW1, kIn, 0, x0, z, a1, g, c);
+        hiddenLayer<4>(S, sW2, kLd, kHidden, a1, z, a2, g, c);
+        hiddenLayer<4>(S, sW3, kLd, 2 * kHidden, a2, z, a3, g, c);
         const f32x4 o = outputLayer(S, a3, g, c);
         if (g == 0 && valid) {
             const float y0 = o[0] * S.norm[kNormYStd] + S.norm[kNormYMean];
@@ -249,20 +267,55 @@ __device__ inline bf16x4 transpose(bf16x4 d, bf16x4 identity) {
     return packTile(mfma(d, identity, zero));
 }
 
-// Sum over the 16 lanes that share g (lanes 16g..16g+15).
+// Sum over the 16 lanes that share g (lanes 16g..16g+15): neighbours, pairs,
+// then the mirrored halves, in data-parallel moves instead of trips to LDS.
+template <int kMove>
+__device__ inline float moved(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kMove, 0xF, 0xF, true));
+}
 __device__ inline float groupSum16(float v) {
-    v += __shfl_xor(v, 1);
-    v += __shfl_xor(v, 2);
-    v += __shfl_xor(v, 4);
-    v += __shfl_xor(v, 8);
+    v += moved<0xB1>(v);   // lanes 1, 0, 3, 2
+    v += moved<0x4E>(v);   // lanes 2, 3, 0, 1
+    v += moved<0x141>(v);  // half rows mirrored
+    v += moved<0x140>(v);  // rows mirrored
     return v;
 }
 
+// A workgroup's sums in LDS: like the parameter vector, with row strides at
+// which the four rows that a wavefront adds to at once are 16 banks apart.
+constexpr int kRedIn = kIn + 4, kRedLd = kHidden + 4;
+constexpr int rB1 = kHidden * kRedIn;
+constexpr int rW2 = rB1 + kHidden;
+constexpr int rB2 = rW2 + kHidden * kRedLd;
+constexpr int rW3 = rB2 + kHidden;
+constexpr int rB3 = rW3 + kHidden * kRedLd;
+constexpr int rW4 = rB3 + kHidden;
+constexpr int rB4 = rW4 + kOutPad * kRedLd;
+constexpr int rTotal = rB4 + kOutPad;
+__device__ inline int redAt(int i) {
+    auto row = [](int j, int width, int ld) { return j / width * ld + j % width; };
+    if (i < kB1) return row(i, kIn, kRedIn);
+    if (i < kW2) return rB1 + i - kB1;
+    if (i < kB2) return rW2 + row(i - kW2, kHidden, kRedLd);
+    if (i < kW3) return rB2 + i - kB2;
+    if (i < kB3) return rW3 + row(i - kW3, kHidden, kRedLd);
+    if (i < kW4) return rB3 + i - kB3;
+    if (i < kB4) return rW4 + row(i - kW4, kHidden, kRedLd);
+    return rB4 + i - kB4;
+}
+
+// Bound by its one wavefront per SIMD (its sums are half the registers): the
+// instructions of a tile one after another, and by what it does once: of 52 us
+// for 65536 samples, four tiles a wavefront, the tiles take about 40 us and the
+// sums' reduction most of the rest. 89 us with transposes through LDS, the
+// GELU's exponential computed again for its derivative and one wavefront
+// reducing at a time; 63 us with rows of 64 entries in LDS. Reading a tile's
+// samples while the one before is worked on: 53 us.
 __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const float* params, const float* norm,
                                                        const float* x, const float* tgt, const int* order, int first,
                                                        int count, float invN, float* partial) {
     __shared__ Smem S;
-    __shared__ float red[kParams];
+    __shared__ float red[rTotal];
     __shared__ float lossShared;
     __shared__ float tf[kWaves][16][17];
     loadSmem(S, wh, params, norm);
@@ -289,22 +342,24 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
     float loss = 0.0f;
     const int tiles = (count + 15) / 16;
     for (int t = blockIdx.x * kWaves + wave; t < tiles; t += gridDim.x * kWaves) {
-        const int local = t * 16 + c;
+        const long long local = (long long)t * 16 + c;
         const bool valid = local < count;
-        const long long s = valid ? (order ? (long long)order[first + local] : (long long)first + local) : 0;
+        const long long s = valid ? (order ? (long long)order[first + local] : first + local) : 0;
+        const float4 xv = *(const float4*)(x + s * kIn + 4 * g);
+        const float2 tv = *(const float2*)(tgt + 2 * s);
         // forward, keeping activations and their derivatives
-        bf16x4 x0[1] = {inputFrag(S, x, s, valid, g)};
+        bf16x4 x0[1] = {inputFrag(S, xv, valid, g)};
         f32x4 z1[4], z2[4], z3[4];  // the GELUs' derivatives
         bf16x4 a1[4], a2[4], a3[4];
-        hiddenLayer<1>(S, hW1, kIn, 0, x0, z1, a1, g, c);
-        hiddenLayer<4>(S, hW2, kHidden, kHidden, a1, z2, a2, g, c);
-        hiddenLayer<4>(S, hW3, kHidden, 2 * kHidden, a2, z3, a3, g, c);
+        hiddenLayer<1>(S, sW1, kIn, 0, x0, z1, a1, g, c);
+        hiddenLayer<4>(S, sW2, kLd, kHidden, a1, z2, a2, g, c);
+        hiddenLayer<4>(S, sW3, kLd, 2 * kHidden, a2, z3, a3, g, c);
         const f32x4 o = outputLayer(S, a3, g, c);
         // dL/dy on standardised targets (rows 0, 1 of the output tile are in lanes g == 0)
         f32x4 d4 = zero4;
         if (g == 0 && valid) {
-            const float t0 = (tgt[2 * s] - S.norm[kNormYMean]) / S.norm[kNormYStd];
-            const float t1 = (tgt[2 * s + 1] - S.norm[kNormYMean + 1]) / S.norm[kNormYStd + 1];
+            const float t0 = (tv.x - S.norm[kNormYMean]) / S.norm[kNormYStd];
+            const float t1 = (tv.y - S.norm[kNormYMean + 1]) / S.norm[kNormYStd + 1];
             const float e0 = o[0] - t0, e1 = o[1] - t1;
             loss += 0.5f * (e0 * e0 + e1 * e1) * invN;
             d4[0] = e0 * invN;
@@ -322,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
             const bf16x4 dB = packTile(d4);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
-                f32x4 acc = mfma(frag(&S.w[hW4t + (16 * mt + c) * kOutPad + 4 * g]), dB, zero4);
+                f32x4 acc = mfma(frag(&S.w[sW4t + (16 * mt + c) * kOutPad + 4 * g]), dB, zero4);
                 for (int j = 0; j < 4; ++j) acc[j] *= z3[mt][j];
                 d3[mt] = acc;
             }
@@ -342,7 +397,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
             f32x4 d2[4];
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
-                f32x4 acc = product64(S, hW3t, kHidden, mt, dB, zero4, g, c);
+                f32x4 acc = product64(S, sW3t, kLd, mt, dB, zero4, g, c);
                 for (int j = 0; j < 4; ++j) acc[j] *= z2[mt][j];
                 d2[mt] = acc;
             }
@@ -360,7 +415,7 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
             const bf16x4 xT = transpose(x0[0], ident);
 #pragma unroll
             for (int mt = 0; mt < 4; ++mt) {
-                f32x4 acc = product64(S, hW2t, kHidden, mt, dB, zero4, g, c);
+                f32x4 acc = product64(S, sW2t, kLd, mt, dB, zero4, g, c);
                 for (int j = 0; j < 4; ++j) acc[j] *= z1[mt][j];
                 const bf16x4 dT = transpose(packTile(acc), ident);
                 gW1[mt] = mfma(dT, xT, gW1[mt]);
@@ -385,30 +440,30 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
             if (((wave + turn) & 3) != q) continue;
             for (int j = 0; j < 4; ++j) {
                 const int o = 16 * q + 4 * g + j;
-                add(kW1 + o * kIn + c, gW1[q][j]);
+                add(o * kRedIn + c, gW1[q][j]);
                 for (int ni = 0; ni < 4; ++ni) {
-                    add(kW2 + o * kHidden + 16 * ni + c, gW2[q][ni][j]);
-                    add(kW3 + o * kHidden + 16 * ni + c, gW3[q][ni][j]);
+                    add(rW2 + o * kRedLd + 16 * ni + c, gW2[q][ni][j]);
+                    add(rW3 + o * kRedLd + 16 * ni + c, gW3[q][ni][j]);
                 }
-                add(kW4 + (4 * g + j) * kHidden + 16 * q + c, gW4[q][j]);
+                add(rW4 + (4 * g + j) * kRedLd + 16 * q + c, gW4[q][j]);
                 const float s1 = groupSum16(gb1[q][j]), s2 = groupSum16(gb2[q][j]), s3 = groupSum16(gb3[q][j]);
                 if (c == 0) {
-                    add(kB1 + o, s1);
-                    add(kB2 + o, s2);
-                    add(kB3 + o, s3);
+                    add(rB1 + o, s1);
+                    add(rB2 + o, s2);
+                    add(rB3 + o, s3);
                 }
             }
             if (q == 0)
                 for (int j = 0; j < 4; ++j) {
                     const float s4 = groupSum16(gb4[j]);
-                    if (c == 0) add(kB4 + 4 * g + j, s4);
+                    if (c == 0) add(rB4 + 4 * g + j, s4);
                 }
         }
         if (lane == 0 && wave == turn) lossShared += l;
         __syncthreads();
     }
     float* row = partial + (size_t)blockIdx.x * (kParams + 1);
-    for (int i = threadIdx.x; i < kParams; i += blockDim.x) row[i] = red[i];
+    for (int i = threadIdx.x; i < kParams; i += blockDim.x) row[i] = red[redAt(i)];
     if (threadIdx.x == 0) row[kParams] = lossShared;
 }
 
@@ -457,7 +512,9 @@ __device__ inline void adamOne(const AdamState& a, int i, float gi) {
 // kReduceSplit lane groups each sum every kReduceSplit-th row in row order
 // (coalesced across the entries), then the groups' sums are added in group
 // order. In training the entries' Adam step follows in the same lanes.
-// Bound by the trips for the rows (10.7 MB at 256 rows): REDUCE_FIGURES
+// Bound by the trips for the rows (10.7 MB at 256 rows): 18 us with four groups
+// and a load at a time, 4.2 us so, 5.1 us with the Adam step, which took 4.9 us
+// as a launch of its own.
 constexpr int kReduceCols = 64, kReduceSplit = 16;
 template <bool kAdam>
 __global__ __launch_bounds__(kReduceCols * kReduceSplit) void k_mlp_reduce(const float* partial, int rows,
