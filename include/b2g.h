@@ -696,8 +696,8 @@ int b2g_set_body_worlds(b2g_context* ctx, int first, int count, const int32_t* w
  * same results bit for bit. No counterpart in the reference (its step is
  * single-threaded). */
 typedef struct b2g_schedule {
-    int32_t islands;       /* island labelling: 0 label-propagation rounds, 1 one round
-                              then union-find, 2 union-find */
+    int32_t islands;       /* island labelling by union-find after: 0 label-propagation
+                              rounds by the world's size, 1 one round, 2 none */
     int32_t collideOrder;  /* 0 contact-table order, 1 grouped by shape-pair class,
                               2 table order with polygon pairs by eight-lane tiles */
     int32_t solverBlock;   /* workgroup size of the per-colour solver kernels */
@@ -705,7 +705,8 @@ typedef struct b2g_schedule {
     int32_t queryBlock;    /* workgroup size of the broad-phase query */
     int32_t tailColours;   /* trailing colours of at most this many constraints are
                               solved by one 1024-lane workgroup, colour after colour
-                              (0: every colour its own launch) */
+                              (0: every colour its own launch, and small worlds run
+                              stage by stage as large ones do) */
     int32_t clusterBodies; /* clustered solve: awake bodies are grouped into clusters of
                               this many (a power of two, 64-2048) by the Morton order of
                               their positions; constraints inside a cluster are solved by
