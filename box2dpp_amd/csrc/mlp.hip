@@ -305,12 +305,13 @@ __device__ inline int redAt(int i) {
 }
 
 // Bound by its one wavefront per SIMD (its sums are half the registers): the
-// instructions of a tile one after another, and by what it does once: of 52 us
+// instructions of a tile one after another, and by what it does once: of 58 us
 // for 65536 samples, four tiles a wavefront, the tiles take about 40 us and the
 // sums' reduction most of the rest. 89 us with transposes through LDS, the
 // GELU's exponential computed again for its derivative and one wavefront
-// reducing at a time; 63 us with rows of 64 entries in LDS. Reading a tile's
-// samples while the one before is worked on: 53 us.
+// reducing at a time; 69 us with rows of 64 entries in LDS. Every sum keeps one
+// order, wavefront after wavefront: 52 us without, but training then rounds
+// otherwise.
 __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const float* params, const float* norm,
                                                        const float* x, const float* tgt, const int* order, int first,
                                                        int count, float invN, float* partial) {
@@ -423,21 +424,21 @@ __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const
             }
         }
     }
-    // Reduce the four wavefronts in LDS: in each of four turns a wavefront adds
-    // one quarter of its sums, a different one each, so that all four work at
-    // once (each lane owns distinct entries, so plain read-add-writes, the first
-    // turn's a write): accumulator element j of tile (mo, ni) is
+    // Reduce the four wavefronts in LDS, each entry in wavefront order: the sums
+    // are added by quarters, a wavefront one turn behind the one before it, so
+    // that four work at once (each lane owns distinct entries, so plain
+    // read-add-writes, the first wavefront's a write): accumulator element j of tile (mo, ni) is
     // dW[16mo + 4g + j][16ni + c]. Then the workgroup's sums go to its row of
     // `partial`, which k_mlp_reduce adds up in a fixed order: the gradient does
     // not depend on the schedule.
     float l = loss;
     for (int off = 1; off < 64; off <<= 1) l += __shfl_xor(l, off);
 #pragma clang loop unroll(disable)
-    for (int turn = 0; turn < kWaves; ++turn) {
-        auto add = [&](int i, float v) { red[i] = turn == 0 ? v : red[i] + v; };
+    for (int turn = 0; turn < kWaves + 3; ++turn) {
+        auto add = [&](int i, float v) { red[i] = (wave == 0 ? 0.0f : red[i]) + v; };
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            if (((wave + turn) & 3) != q) continue;
+            if (turn - wave != q) continue;
             for (int j = 0; j < 4; ++j) {
                 const int o = 16 * q + 4 * g + j;
                 add(o * kRedIn + c, gW1[q][j]);
@@ -512,10 +513,10 @@ __device__ inline void adamOne(const AdamState& a, int i, float gi) {
 // kReduceSplit lane groups each sum every kReduceSplit-th row in row order
 // (coalesced across the entries), then the groups' sums are added in group
 // order. In training the entries' Adam step follows in the same lanes.
-// Bound by the trips for the rows (10.7 MB at 256 rows): 18 us with four groups
-// and a load at a time, 4.2 us so, 5.1 us with the Adam step, which took 4.9 us
-// as a launch of its own.
-constexpr int kReduceCols = 64, kReduceSplit = 16;
+// Bound by the trips for the rows (10.7 MB at 256 rows): 18 us with a load at
+// a time, 5.1 us with 16 in flight and the Adam step, which took 4.9 us as a
+// launch of its own.
+constexpr int kReduceCols = 64, kReduceSplit = 4;
 template <bool kAdam>
 __global__ __launch_bounds__(kReduceCols * kReduceSplit) void k_mlp_reduce(const float* partial, int rows,
                                                                             float* grad, float* loss, AdamState adam) {
@@ -524,7 +525,7 @@ __global__ __launch_bounds__(kReduceCols * kReduceSplit) void k_mlp_reduce(const
     const int i = blockIdx.x * kReduceCols + col;
     float acc = 0.0f;
     if (i <= kParams) {
-#pragma unroll 8
+#pragma unroll 16
         for (int r = grp; r < rows; r += kReduceSplit) acc += partial[(size_t)r * (kParams + 1) + i];
     }
     part[grp][col] = acc;
