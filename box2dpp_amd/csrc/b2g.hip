@@ -4116,10 +4116,10 @@ __global__ void __launch_bounds__(kBlockLanes)
     }
     for (int k = held + t; k < nCons; k += T) storeImpulsesOne(w, cv, k);
     for (int b = t; b < nb; b += T) {
-        if (islandBody(w, b)) {
-            integratePositionOne(wl, b, p.h);
-            w.vel[b] = rows[b];
-        }
+        // (a gear joint may have moved a body of its two joints that is in no
+        // island: an inactive one)
+        if (islandBody(w, b)) integratePositionOne(wl, b, p.h);
+        if (kJoints || islandBody(w, b)) w.vel[b] = rows[b];
         rows[b] = w.pos[b];
     }
     wl = w;
@@ -4160,11 +4160,10 @@ __global__ void __launch_bounds__(kBlockLanes)
         recordMinSep(cnt, it, 0, lowest);
         jointColours([&](int j) { jointSolvePositionOne(wl, jv, j, it); });
     }
-    for (int b = t; b < nb; b += T)
-        if (islandBody(w, b)) {
-            w.pos[b] = rows[b];
-            syncTransformOne(w, b);
-        }
+    for (int b = t; b < nb; b += T) {
+        if (kJoints || islandBody(w, b)) w.pos[b] = rows[b];
+        if (islandBody(w, b)) syncTransformOne(w, b);
+    }
 }
 
 // ====================================================================
@@ -8266,10 +8265,11 @@ int wideConstraints(const ColourLayout& l) {
 // asks for another way of running them (captured, clustered, one-launch or
 // per-colour solve: tailColours 0). Settled piles, a step per colour against
 // the block solve: 433 constraints 357 -> 297 us, 2868 463 -> 401 us, 6010
-// 624 -> 521 us, 8145 672 -> 600 us; beyond its registers the one compute
-// unit is left behind by the whole chip somewhere above that. With joints,
-// whose passes read memory: 1558 constraints and 620 joints 597 -> 501 us,
-// 3607 703 -> 643 us, but 4831 689 -> 718 us.
+// 624 -> 521 us, 8145 672 -> 600 us. The line to the team solve lies where the
+// two meet: 460 us for either at 4289 constraints, 538 against 438 to 472 us
+// at 8145. With joints, which the team solve does not take and whose passes
+// read memory: 1558 constraints and 620 joints 597 -> 501 us, 3607 703 ->
+// 643 us, but 4831 689 -> 718 us.
 bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
     if (ctx->nBodies > kBlockBodies || constraints > kBlockConstraints) return false;
     if (ctx->nJoints > 0 && (constraints > kBlockJointed || ctx->nJoints > kBlockJointed)) return false;
