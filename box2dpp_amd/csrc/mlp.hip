@@ -309,9 +309,9 @@ __device__ inline int redAt(int i) {
 // for 65536 samples, four tiles a wavefront, the tiles take about 40 us and the
 // sums' reduction most of the rest. 89 us with transposes through LDS, the
 // GELU's exponential computed again for its derivative and one wavefront
-// reducing at a time; 69 us with rows of 64 entries in LDS. Every sum keeps one
-// order, wavefront after wavefront: 52 us without, but training then rounds
-// otherwise.
+// reducing at a time. Every sum keeps one order, wavefront after wavefront: 52 us
+// without, but training then rounds otherwise (and that 63 us with rows of 64
+// entries in LDS).
 __global__ __launch_bounds__(kThreads) void k_mlp_grad(const uint16_t* wh, const float* params, const float* norm,
                                                        const float* x, const float* tgt, const int* order, int first,
                                                        int count, float invN, float* partial) {
