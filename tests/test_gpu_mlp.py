@@ -105,6 +105,38 @@ def test_gradient_is_deterministic(lib, ctx):
     assert all(np.array_equal(o[0], out[0][0]) and o[1] == out[0][1] for o in out)
 
 
+@pytest.mark.parametrize("n, sample", [(16, 3), (777, 776), (40000, 20000)])
+@pytest.mark.parametrize("target", [np.inf, -np.inf])
+def test_gradient_of_an_infinite_target(lib, ctx, n, sample, target):
+    """One infinite target makes infinite, not undefined, every gradient entry
+    that it reaches, and leaves the other output's as they are: where all
+    weights, biases and inputs are positive no sum meets infinities of both
+    signs, and the oracle's entries say which are infinite and with what sign.
+    Sizes: one tile, a ragged last tile, several tiles a wavefront."""
+    rng = np.random.default_rng(31)
+    p = M.random_params(rng, norm=False)
+    for k in M.WEIGHTS:
+        p[k] = np.abs(p[k]) / 8
+    _set(lib, ctx, p)
+    x, t = _inputs(rng, n)
+    x = np.abs(x) + np.float32(0.125)
+    t[sample, 0] = target
+    g = np.zeros(1, M.PARAMS_DTYPE)
+    loss = ctypes.c_double()
+    E.b2g_check(lib, ctx, lib.b2g_mlp_gradient(ctx, E.ptr(x), E.ptr(t), n, E.ptr(g), ctypes.byref(loss)))
+    with np.errstate(invalid="ignore"):
+        _, want = M.loss_and_grad(p, x, t, emulate=True)
+    assert np.isposinf(loss.value)
+    for k in M.WEIGHTS:
+        got = g[0][k].astype(np.float64).reshape(M.SHAPES[k])
+        assert not np.isnan(want[k]).any() and np.array_equal(np.isfinite(want[k]), np.isfinite(got)), k
+        assert np.array_equal(want[k][np.isinf(want[k])], got[np.isinf(want[k])]), k
+    # the other output's sums, within the bound of test_gradient_matches_oracle
+    for k in ("W4", "b4"):
+        got, ek = g[0][k].astype(np.float64).reshape(M.SHAPES[k])[1], want[k][1]
+        assert np.linalg.norm(got - ek) < 3e-3 * np.linalg.norm(ek), k
+
+
 def test_adam_training_fits_a_smooth_map(lib, gpu):
     """Log fresh points from a pile, then train: the loss falls well below
     the loss of predicting the mean."""
