@@ -836,9 +836,11 @@ __device__ inline void colourByBlock(const WorldView& w, unsigned long long* cla
 // The colouring of a step's new constraints in one launch: of the table's
 // contacts only those few take part (some hundred in a 10 000-body pile), so a
 // round over the whole table in two launches, twice at least, cost 15 us.
-// More than kColourListMost are left to such rounds (cnt->colourLeft): all at
-// once they are more than one workgroup's work.
-constexpr int kColourListMost = 16384;
+// More than kColourListMost are left to such rounds (cnt->colourLeft): a whole
+// pile that becomes new at once takes some 15 rounds, each over the whole list.
+// That step with 3400 new constraints 569 us by the list and 671 us by rounds,
+// 5700 778 and 762, 8900 1059 and 792, 16 400 1669 and 924.
+constexpr int kColourListMost = 5120;
 constexpr int kClaimTags = 96;  // claim tags of a one-workgroup colouring
 __global__ void __launch_bounds__(1024)
     k_colour_list(WorldView w, unsigned long long* claim, uint32_t tagBase, const int* list, Counters* cnt) {

@@ -10,6 +10,8 @@ body in more contacts than there are colours (the overflow colour), islands
 that sleep, contacts that end, sub-worlds, few iterations. Larger worlds go to
 the team solve (the workgroups of one XCD with a barrier between colours).
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -117,5 +119,44 @@ def test_many_new_pairs_at_once(gpu):
             pairs = max(pairs, int(w.stats()["newPairs"]))
         assert pairs > 4096
         states += run(w, False, 90)
+        out.append(states)
+    same(*out)
+
+
+@pytest.mark.parametrize("n", [1200, 2500, 3100, 6000])
+def test_all_constraints_new_at_once(gpu, n):
+    """A pile taken apart and put back: its constraints are all new in one
+    step. Sizes for each way of colouring them: in the small world's kernel,
+    from the list by one workgroup (5120 at most), and by rounds over the
+    table."""
+    lib = E.b2g_lib()
+    out = []
+    for per_colour in (False, True):
+        w = gpu.world("world", n, 7, sleep=False)
+        if per_colour:
+            a_launch_per_colour(w)
+        w.step(500)
+        ctx = w.device_context()
+        here = np.zeros(n + 1, BODY)
+        E.b2g_check(lib, ctx, lib.b2g_get_bodies(ctx, 0, n + 1, E.ptr(here)))
+        apart = here.copy()
+        for k in ("c", "c0", "xf"):
+            apart[k][here["type"] == 2, :2] *= np.float32(4.0)
+        settled = int(w.stats()["constraints"])
+        E.b2g_check(lib, ctx, lib.b2g_set_bodies(ctx, 0, n + 1, E.ptr(apart)))
+        w.step(2)
+        assert w.stats()["constraints"] < settled // 4
+        E.b2g_check(lib, ctx, lib.b2g_set_bodies(ctx, 0, n + 1, E.ptr(here)))
+        states, most = [], 0
+        for _ in range(4):
+            w.step(1)
+            states.append(state(w))
+            most = max(most, int(w.stats()["constraints"]))
+            conflicts, mask = ctypes.c_int(-1), ctypes.c_int(-1)
+            E.b2g_check(lib, ctx, lib.b2g_check_colouring(ctx, ctypes.byref(conflicts), ctypes.byref(mask)))
+            assert conflicts.value == 0 and mask.value == 0
+        assert most > 0.9 * settled
+        assert (n < 2000) or (most <= 5120) == (n < 3000)
+        w.close()
         out.append(states)
     same(*out)
