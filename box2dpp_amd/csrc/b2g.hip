@@ -4981,7 +4981,8 @@ constexpr int kSmallLanes = 1024;
 constexpr int kSmallBodies = kBlockBodies;   // island labels in LDS
 constexpr int kSmallContacts = 5120;         // contact bodies in LDS (see smallWorldFits)
 constexpr int kSortedNewPairs = 4096;        // new pairs sorted in LDS
-constexpr int kAppendFixtures = 32768;       // move flags that one workgroup clears
+constexpr int kAppendPairs = 768;            // see runBroadphase
+constexpr int kAppendFixtures = 65536;       // move flags that one workgroup clears
 static_assert(kSmallBodies <= 1 << 13, "a packed body index has 13 bits");
 static_assert(sizeof(b2g_manifold) == 4 * sizeof(float4), "a manifold moves as four words of 16 bytes");
 
@@ -7539,8 +7540,11 @@ GridView gridView(const b2g_context* ctx) {
 // (the grid cleared, the pair set rebuilt, the live contact count on the
 // device, which the query's readback brings). Its new pairs are sorted and
 // appended by one kernel before that readback, as long as there were few in
-// the last step: 440 pairs of a 10 000-body pile took a sort made for 4096
-// (17 us) and five launches.
+// the last step: up to 512 of them a step gets 8 to 17 us shorter than with a
+// sort made for 4096 (17 us) and three launches, at 512 to 1024 the two are
+// equal, at 1024 to 2048 it gets 13 to 25 us longer and beyond that 44 to 63
+// (falling piles of 9973 to 60 000 bodies; the number of move flags makes no
+// difference up to there).
 int runBroadphase(b2g_context* ctx, const uint32_t* closedMask = nullptr) {
     hipStream_t s = ctx->stream;
     const int nf = ctx->nFixtures;
@@ -7604,7 +7608,7 @@ int runBroadphase(b2g_context* ctx, const uint32_t* closedMask = nullptr) {
         profKernel(ctx, PH_K_PAIRS_QUERY, pk);
         hipLaunchKernelGGL(k_pairs_wide, dim3(blocks(nf)), dim3(256), 0, s, ctx->fat, ctx->moved, nf, g, ctx->view(),
                            true, ctx->hashTable, hashMask, sink, ctx->cnt);
-        const bool append = liveOnDevice && attempt == 0 && ctx->lastNewPairs <= 3 * kSortedNewPairs / 4 &&
+        const bool append = liveOnDevice && attempt == 0 && ctx->lastNewPairs <= kAppendPairs &&
                             nf <= kAppendFixtures;
         if (append)
             hipLaunchKernelGGL(k_append_sorted, dim3(1), dim3(kSmallLanes), 0, s, ctx->view(), ctx->newKeys,

@@ -246,3 +246,37 @@ def test_resumed_after_destruction_matches_oracle(gpu, orc, wide_trig):
     finally:
         lib.b2g_destroy(b)
         o.close()
+
+
+@pytest.mark.parametrize("n", [9000, 20000])
+def test_new_pairs_sorted_either_way(gpu, n):
+    """New pairs are sorted and appended by one workgroup when the last step
+    had few (768), else by the general sort. A restored context has no last
+    step, so its first step takes the one way where the original takes the
+    other: the tables stay equal."""
+    lib = E.b2g_lib()
+    w = gpu.world("world", n, 5, sleep=False)
+    ctx, p = w.device_context(), _params()
+    seen = 0
+    w.step(150)
+    for _ in range(300):
+        w.step(1)
+        if not 1000 < w.stats()["newPairs"] < 3500:
+            continue
+        buf = _snapshot(lib, ctx)
+        c = _fresh(lib)
+        E.b2g_check(lib, c, lib.b2g_restore(c, E.ptr(buf), ctypes.c_size_t(buf.size)))
+        E.b2g_check(lib, ctx, lib.b2g_step(ctx, E.ptr(p)))
+        E.b2g_check(lib, c, lib.b2g_step(c, E.ptr(p)))
+        st = np.zeros(1, E.STATS)
+        E.b2g_check(lib, c, lib.b2g_get_stats(c, E.ptr(st)))
+        assert st[0]["newPairs"] > 0
+        for a, b in zip(_state(lib, ctx), _state(lib, c)):
+            assert np.array_equal(a, b)
+        assert np.array_equal(_bodies(lib, ctx, n + 1), _bodies(lib, c, n + 1))
+        lib.b2g_destroy(c)
+        seen += 1
+        if seen == 3:
+            break
+    assert seen == 3
+    w.close()
