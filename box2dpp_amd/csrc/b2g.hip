@@ -5017,11 +5017,12 @@ __global__ void __launch_bounds__(kSmallLanes)
     __shared__ uint32_t ends[kSmallContacts];  // bodies A, B of each contact, 13 bits each
     __shared__ int hist[kSmallLanes / 64][kOrderKeys];
     __shared__ int next[kOrderKeys];           // where the next constraint of a key goes
-    __shared__ int left;
+    __shared__ int left, fresh;
     const int t = threadIdx.x, T = blockDim.x;
     const int nb = w.nBodies, nc = w.nContacts;
     WorldView wl = w;
     wl.islandOf = label;
+    if (t == 0) fresh = 0;
     auto bodyA = [&](int c) { return (int)(ends[c] & 0x1FFFu); };
     auto bodyB = [&](int c) { return (int)(ends[c] >> 13); };
     for (int c = t; c < nc; c += T) {
@@ -5049,7 +5050,8 @@ __global__ void __launch_bounds__(kSmallLanes)
     __syncthreads();
     for (int b = t; b < nb; b += T) islandMarkOne(wl, b);
     __syncthreads();
-    for (int c = t; c < nc; c += T) (void)markConstraintOne(w, c, bodyA(c), bodyB(c));
+    for (int c = t; c < nc; c += T)
+        if (markConstraintOne(w, c, bodyA(c), bodyB(c))) fresh = 1;
     __syncthreads();
     ClaimTags tags{tagBase, tagCount, 0};
     for (int r = 0; r < demoteRounds; ++r) {
@@ -5059,7 +5061,7 @@ __global__ void __launch_bounds__(kSmallLanes)
         for (int c = t; c < nc; c += T) demoteCommitOne(w, claim, tag, c, bodyA(c), bodyB(c));
         __syncthreads();
     }
-    colourByBlock(w, claim, tags, nc, [&](int i) { return i; }, bodyA, bodyB, &left, cnt);
+    colourByBlock(w, claim, tags, fresh ? nc : 0, [&](int i) { return i; }, bodyA, bodyB, &left, cnt);
     // Constraints by order key, in table order within a key: counts, then
     // chunks of T contacts ranked by a ballot per key bit and a count per
     // wavefront.
@@ -7190,7 +7192,6 @@ struct b2g_context {
     int lastColourStart[kColourSlots + 1] = {};  // colour ranges of the last coloured step
     int demoteRounds = 1;           // colour demotion rounds per coloured step
     int compactedFrom = -1;  // table length before the last coloured step's compaction (-1: none)
-    int colourRoundsNeeded = 0;  // colouring rounds the last coloured step needed
     int lastNewPairs = 0;        // new pairs of the last broad-phase
     int lastConstraints = 0;
 
@@ -8412,14 +8413,6 @@ int stepColouredCollide(b2g_context* ctx, const b2g_step_params* p) {
     return B2G_OK;
 }
 
-// The colouring rounds reported: as many as the last step needed, two at
-// least, and those this step needed if they are more.
-void roundStats(b2g_context* ctx, int needed) {
-    const int least = std::min(std::max(ctx->colourRoundsNeeded, 2), kColourRoundSlots - 1);
-    ctx->stats.colouringRounds = std::max(least, needed);
-    ctx->colourRoundsNeeded = needed;
-}
-
 // Statistics of the position iterations.
 void positionStats(b2g_context* ctx, int posIters, int nCons) {
     int ran = 0;
@@ -8490,8 +8483,7 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     ctx->compactedFrom = before;
     ctx->stats.constraints = layout.nCons;
     ctx->stats.colours = layout.nColours;
-    ctx->stats.wideConstraints = wideConstraints(layout);
-    if (before > 0) roundStats(ctx, ctx->hcnt->colourRounds);
+    ctx->stats.colouringRounds = ctx->hcnt->colourRounds;
     ctx->nContacts = ctx->hcnt->nContacts;
     if (ctx->hcnt->appendPending) {
         // more new pairs than the LDS sort or the table takes
@@ -8688,7 +8680,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
                 } while (leftAfterLast() > 0);
                 if ((rc = order()) != B2G_OK) return rc;
             }
-            roundStats(ctx, rounds > 0 ? rounds : std::max(ctx->hcnt->colourRounds, 1));
+            ctx->stats.colouringRounds = rounds > 0 ? rounds : ctx->hcnt->colourRounds;
             layout = colourLayout(ctx->hcnt->colourCount, clustered ? ctx->hcnt->boundaryStart : 0,
                                   ctx->sched.tailColours);
         }
@@ -8748,7 +8740,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         ctx->stats.residual = -1.0f;
         const int sb = ctx->sched.solverBlock;
         auto sgrid = [sb](int n) { return dim3((unsigned)((n + sb - 1) / sb)); };
-        ctx->stats.wideConstraints = wideConstraints(layout);
+        ctx->stats.wideConstraints = block || team ? 0 : wideConstraints(layout);
         ColourRanges ranges;
         memcpy(ranges.s, colourStart, sizeof(ranges.s));
         auto perColour = [&](int phase, auto kernelLaunch, auto tailLaunch) {

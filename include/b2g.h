@@ -189,7 +189,7 @@ typedef struct b2g_step_stats {
     int32_t constraints;       /* touching contacts solved this step */
     int32_t points;            /* manifold points of those contacts */
     int32_t colours;
-    int32_t colouringRounds;
+    int32_t colouringRounds;   /* rounds that coloured the step's new constraints (0: none new) */
     int32_t newPairs;          /* contacts created by the broad-phase this step */
     int32_t positionIterations;/* position iterations actually run */
     int32_t beginEvents;       /* BeginContact count this step */
@@ -206,7 +206,8 @@ typedef struct b2g_step_stats {
     int32_t scanned;           /* grid entries and wide proxies those queries examined */
     int32_t wideConstraints;   /* constraints in the colours that get a solver launch
                                   each (not the fused trailing colours, not the
-                                  overflow colour) */
+                                  overflow colour; none where one workgroup or the
+                                  workgroups of one XCD solve the whole island) */
 } b2g_step_stats;
 
 typedef struct b2g_context b2g_context;

@@ -233,3 +233,29 @@ def test_colour_demotion(gpu):
     assert pd <= pp + 0.005, (pd, pp)
     assert abs(kd / kp - 1.0) <= 0.25, (kd, kp)
     plain.close(); dem.close()
+
+
+@pytest.mark.parametrize("kind, n, steps", [("pyramid", 12, 200), ("world", 2000, 300), ("world", 4100, 150)])
+def test_stats_count_what_ran(gpu, kind, n, steps):
+    """colouringRounds counts the rounds that coloured something, and
+    wideConstraints only constraints of colours with a launch of their own: a
+    small world, one for the block solve and one for the team solve against
+    the step by colours."""
+    lib = E.b2g_lib()
+    a, b = gpu.world(kind, n, 3, sleep=False), gpu.world(kind, n, 3, sleep=False)
+    _set(a, (0, 0, 256, 256, 256, 1, 0, 0))
+    _set(b, (0, 0, 256, 256, 256, 0, 0, 0))
+    rounds = []
+    for _ in range(steps):
+        a.step(1)
+        b.step(1)
+        sa, sb = a.stats(), b.stats()
+        assert sa["colouringRounds"] == sb["colouringRounds"]
+        assert sa["wideConstraints"] == 0
+        assert sb["wideConstraints"] == sb["constraints"] - _colour_counts(lib, b)[64]
+        rounds.append(int(sa["colouringRounds"]))
+    assert max(rounds) >= 2
+    if kind == "pyramid":
+        # at rest no constraint is new
+        assert rounds[-50:] == [0] * 50
+    a.close(); b.close()
