@@ -7493,7 +7493,8 @@ enum Phase {
     PH_COLLIDE, PH_COMPACT, PH_COLOUR, PH_ORDER, PH_INTEGRATE_V, PH_INIT, PH_WARM, PH_SOLVE_V, PH_STORE,
     PH_INTEGRATE_X, PH_SOLVE_X, PH_SYNC, PH_BROADPHASE, PH_ISLANDS, PH_LEARNED, PH_K_SOLVE_V, PH_K_SOLVE_X,
     PH_K_MLP_INFER, PH_K_MLP_GRAD, PH_TOI, PH_K_SOLVE_V_CLUSTER, PH_K_SOLVE_X_CLUSTER, PH_K_COLLIDE,
-    PH_K_PAIRS_QUERY, PH_K_SOLVE_PERSIST, PH_COUNT
+    PH_K_PAIRS_QUERY, PH_K_SOLVE_PERSIST, PH_SMALL_PREPARE, PH_SOLVE_ISLAND, PH_SMALL_FINISH, PH_K_SMALL_PREPARE,
+    PH_K_SOLVE_BLOCK, PH_K_SOLVE_TEAM, PH_K_SMALL_FINISH, PH_COUNT
 };
 const char* kPhaseNames[PH_COUNT] = {"collide", "compact", "colour", "order", "integrate_velocities",
                                      "init_constraints", "warm_start", "solve_velocity", "store_impulses",
@@ -7501,7 +7502,9 @@ const char* kPhaseNames[PH_COUNT] = {"collide", "compact", "colour", "order", "i
                                      "fresh_points", "k_solve_velocity", "k_solve_position", "k_mlp_infer",
                                      "k_mlp_grad", "toi", "k_solve_velocity_cluster",
                                      "k_solve_position_cluster", "k_collide", "k_pairs_query",
-                                     "k_solve_persistent"};
+                                     "k_solve_persistent", "small_prepare", "solve_island", "small_finish",
+                                     "k_small_prepare", "k_solve_block", "k_solve_team", "k_small_finish"};
+static_assert(PH_COUNT <= 32, "the profile's arrays");
 
 int readCounters(b2g_context* ctx);
 int profKernelEvents(b2g_context* ctx, hipEvent_t* start, hipEvent_t* stop);
@@ -8304,9 +8307,14 @@ void launchBlockSolve(b2g_context* ctx, const b2g_step_params* p, const WorldVie
     plan.contactWarm = contactWarm ? 1 : 0;
     plan.warm = ctx->warmStarting ? 1 : 0;
     plan.initHere = initHere ? 1 : 0;
-    hipLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(lanes),
-                       sizeof(float4) * (size_t)ctx->nBodies, ctx->stream, w, ctx->cv, jv, (const int*)ctx->consOrder,
-                       plan, ctx->cnt);
+    const int pe = profStart(ctx);
+    hipEvent_t e0, e1;
+    const int pk = profKernelEvents(ctx, &e0, &e1);
+    hipExtLaunchKernelGGL(ctx->nJoints > 0 ? k_solve_block<true> : k_solve_block<false>, dim3(1), dim3(lanes),
+                          sizeof(float4) * (size_t)ctx->nBodies, ctx->stream, e0, e1, 0, w, ctx->cv, jv,
+                          (const int*)ctx->consOrder, plan, ctx->cnt);
+    profKernel(ctx, PH_K_SOLVE_BLOCK, pk);
+    profEnd(ctx, PH_SOLVE_ISLAND, pe);
 }
 
 // Whether a step's solve goes to the team solve (k_solve_team) when the block
@@ -8330,21 +8338,25 @@ void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView
     plan.posIters = std::min(p->positionIterations, kMaxPosIters);
     plan.contactWarm = contactWarm ? 1 : 0;
     plan.wanted = kTeamSize;
-    hipLaunchKernelGGL(constraints <= 4 * kTeamSize * kTeamLanes ? k_solve_team<4> : k_solve_team<8>,
-                       dim3(8 * kTeamSize), dim3(kTeamLanes), 0, ctx->stream, w, ctx->cv, plan, ctx->cnt);
+    const int pe = profStart(ctx);
+    hipEvent_t e0, e1;
+    const int pk = profKernelEvents(ctx, &e0, &e1);
+    hipExtLaunchKernelGGL(constraints <= 4 * kTeamSize * kTeamLanes ? k_solve_team<4> : k_solve_team<8>,
+                          dim3(8 * kTeamSize), dim3(kTeamLanes), 0, ctx->stream, e0, e1, 0, w, ctx->cv, plan, ctx->cnt);
+    profKernel(ctx, PH_K_SOLVE_TEAM, pk);
+    profEnd(ctx, PH_SOLVE_ISLAND, pe);
 }
 
 // Whether the whole step after the narrowphase goes to the small-world kernels:
 // the block solve takes it whatever share of the contacts are constraints, the
 // LDS tables hold the world, and no candidate point has to be gathered for the
-// network. With profiling on the step runs stage by stage, so that the phases
-// keep their times. One compute unit works through a stage where the grid
+// network. One compute unit works through a stage where the grid
 // kernels have the whole chip, so the gain ends with the contacts: settled
 // worlds of 590 contacts 278 -> 129 us a step, 1700 (700-body pile)
 // 341 -> 232 us, 4500 401 -> 356 us, but 6600 457 -> 480 us.
 bool smallWorldFits(const b2g_context* ctx, const b2g_step_params* p) {
     return blockSolveFits(ctx, p, ctx->nContacts) && ctx->nFixtures <= kSmallBodies && ctx->nFixtures > 0 &&
-           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && !ctx->profiling && ctx->demoteRounds < kClaimTags &&
+           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && ctx->demoteRounds < kClaimTags &&
            (ctx->orderSpan == 0 || ctx->orderCount == ctx->nFixtures);
 }
 
@@ -8443,8 +8455,13 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     JointView jv = ctx->jview();
     jv.h = p->dt;
     const int before = ctx->nContacts;
-    hipLaunchKernelGGL(k_small_prepare, dim3(1), dim3(kSmallLanes), 0, s, w, jv, ctx->claim, ctx->claimTag + 1,
-                       kClaimTags, ctx->nContacts > 0 ? ctx->demoteRounds : 0, posIters, ctx->consOrder, ctx->cnt);
+    hipEvent_t e0, e1;
+    int pe = profStart(ctx), pk = profKernelEvents(ctx, &e0, &e1);
+    hipExtLaunchKernelGGL(k_small_prepare, dim3(1), dim3(kSmallLanes), 0, s, e0, e1, 0, w, jv, ctx->claim,
+                          ctx->claimTag + 1, kClaimTags, ctx->nContacts > 0 ? ctx->demoteRounds : 0, posIters,
+                          ctx->consOrder, ctx->cnt);
+    profKernel(ctx, PH_K_SMALL_PREPARE, pk);
+    profEnd(ctx, PH_SMALL_PREPARE, pe);
     ctx->claimTag += kClaimTags;
     launchBlockSolve(ctx, p, w, jv, blockSolveLanes(ctx, ctx->nContacts), ctx->warmStarting, true);
 
@@ -8464,14 +8481,25 @@ int stepSmallSolve(b2g_context* ctx, const b2g_step_params* p, bool* forcesClear
     fin.nBuckets = std::min(fin.nBuckets, ctx->nBuckets);
     GridView g = gridView(ctx);
     g.bucketMask = (uint32_t)(fin.nBuckets - 1);
-    hipLaunchKernelGGL(k_small_finish, dim3(1), dim3(kSmallLanes), 0, s, w, jv, ctx->cur, fin, g, ctx->cnt);
+    pe = profStart(ctx);
+    pk = profKernelEvents(ctx, &e0, &e1);
+    hipExtLaunchKernelGGL(k_small_finish, dim3(1), dim3(kSmallLanes), 0, s, e0, e1, 0, w, jv, ctx->cur, fin, g,
+                          ctx->cnt);
+    profKernel(ctx, PH_K_SMALL_FINISH, pk);
+    profEnd(ctx, PH_SMALL_FINISH, pe);
     const bool ordered = ctx->orderSpan > 0;
     const int packBase = ordered ? ctx->orderSpan : ctx->nFixtures;
     const PairSink sink{ctx->newKeys, ctx->capContacts, (unsigned long long)packBase, ordered ? ctx->fixOrder : nullptr};
-    hipLaunchKernelGGL(k_small_pairs, dim3(blocks(ctx->nFixtures * kQueryLanes)), dim3(256), 0, s, w, g, ctx->hashTable,
-                       fin.hashMask, sink, ctx->cnt);
+    pe = profStart(ctx);
+    pk = profKernelEvents(ctx, &e0, &e1);
+    hipExtLaunchKernelGGL(k_small_pairs, dim3(blocks(ctx->nFixtures * kQueryLanes)), dim3(256), 0, s, e0, e1, 0, w, g,
+                          ctx->hashTable, fin.hashMask, sink, ctx->cnt);
+    if (ctx->profiling)
+        hipLaunchKernelGGL(k_count_scanned, dim3(blocks(ctx->nFixtures)), dim3(256), 0, s, ctx->nFixtures, g, ctx->cnt);
+    profKernel(ctx, PH_K_PAIRS_QUERY, pk);
     hipLaunchKernelGGL(k_append_sorted, dim3(1), dim3(kSmallLanes), 0, s, w, ctx->newKeys, (unsigned long long)packBase,
                        ctx->capContacts, ctx->autoClearForces && !ctx->continuous ? 1 : 0, ctx->cnt);
+    profEnd(ctx, PH_BROADPHASE, pe);
     LAUNCHCHK(ctx);
     if ((rc = readCounters(ctx)) != B2G_OK) return rc;
     *forcesCleared = !ctx->hcnt->appendPending && !ctx->continuous;
@@ -8935,13 +8963,9 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const bool velocityDeferred = persist && !checkResidual && ctx->logCap == 0;
         const bool contactWarm = nCons > 0 && (ctx->warmStarting || usePrediction);
         if (block) {
-            pe = profStart(ctx);
             launchBlockSolve(ctx, p, w, jv, blockLanes, contactWarm, blockInit);
-            profEnd(ctx, PH_SOLVE_V, pe);
         } else if (team) {
-            pe = profStart(ctx);
             launchTeamSolve(ctx, p, w, nCons, contactWarm);
-            profEnd(ctx, PH_SOLVE_V, pe);
         } else if (!persist) {
             startSolve(contactWarm);
             solveVelocity(p->velocityIterations);

@@ -317,7 +317,12 @@ int b2g_joint_drift(b2g_context* ctx, double* out);
 int b2g_energy(b2g_context* ctx, double* out);
 
 /* Per-phase GPU time of the steps run while profiling is on, measured with
- * HIP events on the context's stream around every launch of the phase. */
+ * HIP events on the context's stream around every launch of the phase; rows
+ * named after a kernel ("k_...") hold its own execution time. A world steps
+ * with profiling as it does without: where one launch does the work of several
+ * phases, those stay empty and the launch has a row of its own (solve_island:
+ * the island solve of a small or mid-sized world; small_prepare and
+ * small_finish: a small world's stages before and after it). */
 typedef struct b2g_phase_profile {
     char name[24];
     int32_t launches;

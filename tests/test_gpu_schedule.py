@@ -259,3 +259,40 @@ def test_stats_count_what_ran(gpu, kind, n, steps):
         # at rest no constraint is new
         assert rounds[-50:] == [0] * 50
     a.close(); b.close()
+
+
+PROFILE = np.dtype([("name", "S24"), ("launches", "<i4"), ("pad", "<i4"), ("ms", "<f8")])
+
+
+def _profile(w):
+    lib, ctx = E.b2g_lib(), w.device_context()
+    rows, n = np.zeros(32, PROFILE), ctypes.c_int()
+    E.b2g_check(lib, ctx, lib.b2g_get_profile(ctx, E.ptr(rows), 32, ctypes.byref(n)))
+    return {r["name"].decode(): (int(r["launches"]), float(r["ms"])) for r in rows[:n.value]}
+
+
+@pytest.mark.parametrize("n, launch", [(300, "k_small_prepare"), (300, "k_solve_block"), (300, "k_small_finish"),
+                                       (4100, "k_solve_team"), (3000, "k_solve_block")])
+def test_profile_shows_the_step_that_runs(gpu, n, launch):
+    """Profiling does not change how a world steps: the kernels of its size
+    are in the profile once a step, and the stages that they replace are not."""
+    lib = E.b2g_lib()
+    a, b = gpu.world("world", n, 3, sleep=False), gpu.world("world", n, 3, sleep=False)
+    a.step(150)
+    b.step(150)
+    ctx = a.device_context()
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 1))
+    a.step(10)
+    p = _profile(a)
+    scanned = int(a.stats()["scanned"])
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 0))
+    b.step(10)
+    _same(a, b)
+    assert p[launch][0] == 10 and 0.0 < p[launch][1] < 50.0
+    assert p["k_solve_velocity"][0] == 0 and p["solve_position"][0] == 0 and p["solve_velocity"][0] == 0
+    assert p["solve_island"][0] == 10
+    if n == 300:
+        assert p["small_prepare"][0] == p["small_finish"][0] == 10 and p["islands"][0] == p["colour"][0] == 0
+    assert p["k_collide"][0] == p["k_pairs_query"][0] == 10
+    assert scanned > 0
+    a.close(); b.close()
