@@ -7007,9 +7007,11 @@ inline int blocks(int n, int bs = 256) { return (n + bs - 1) / bs; }
 // ====================================================================
 // Host side
 // ====================================================================
+constexpr int kTailDefault = 1024;  // b2g_schedule.tailColours of a new context
+
 struct b2g_context {
     int device = 0;
-    b2g_schedule sched{0, 0, 256, 256, 256, 1024, 0, 0};
+    b2g_schedule sched{0, 0, 256, 256, 256, kTailDefault, 0, 0};
     hipStream_t stream = nullptr;
     std::string err;
     int cuCount = 0;            // compute units of the device (one-launch solve)
@@ -7193,6 +7195,8 @@ struct b2g_context {
     int demoteRounds = 1;           // colour demotion rounds per coloured step
     int compactedFrom = -1;  // table length before the last coloured step's compaction (-1: none)
     int lastNewPairs = 0;        // new pairs of the last broad-phase
+    bool lastSmall = false;      // the last step ran in the small-world kernels
+    bool lastOneLaunch = false;  // the last step's island solve was one launch (block or team solve)
     int lastConstraints = 0;
 
     // profiling (HIP events around launches)
@@ -8575,6 +8579,8 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         ctx->islandIterCap = posIters;
     }
     const bool small = solves && smallWorldFits(ctx, p);
+    ctx->lastSmall = small;
+    ctx->lastOneLaunch = small;
     bool forcesCleared = false;
     if (ctx->nContacts > 0 && !small) {
         const int pe = profStart(ctx);
@@ -8734,6 +8740,7 @@ int stepColouredSolve(b2g_context* ctx, const b2g_step_params* p) {
         const FreshView fv{wantFresh ? ctx->freshMask : nullptr, ctx->freshNum, ctx->freshAll, ctx->learnedScope};
         const bool block = nCons > 0 && blockSolveFits(ctx, p, nCons);
         const bool team = !block && teamSolveFits(ctx, p, nCons);
+        ctx->lastOneLaunch = block || team;
         const int blockLanes = block ? blockSolveLanes(ctx, nCons) : 0;
         const bool blockInit = block && !wantFresh &&
                                nCons <= blockLanes * (ctx->nJoints > 0 ? kBlockRows<true> : kBlockRows<false>);
@@ -11225,19 +11232,31 @@ int b2g_autotune(b2g_context* ctx, const b2g_step_params* p, int rounds, b2g_sch
         return fail(ctx, B2G_ERR_UNSUPPORTED, "the schedule applies to the coloured step");
     // Each field is judged by the time of the phases it affects, from the
     // events the profiler records on the step stream (dispatch gaps and
-    // host round trips inside a phase included).
+    // host round trips inside a phase included). A field that the kernels of
+    // its trial steps did not all read keeps its value.
+    enum Reach { ALWAYS, NOT_SMALL, PER_COLOUR };
     struct Knob {
         int32_t b2g_schedule::*field;
         std::vector<int> values;
         std::vector<int> phases;
+        Reach reach;
     };
     const Knob knobs[] = {
-        {&b2g_schedule::islands, {0, 1, 2}, {PH_ISLANDS}},
-        {&b2g_schedule::collideOrder, {0, 1, 2}, {PH_COLLIDE}},
-        {&b2g_schedule::solverBlock, {64, 128, 256, 512}, {PH_WARM, PH_SOLVE_V, PH_SOLVE_X}},
-        {&b2g_schedule::collideBlock, {64, 128, 256}, {PH_COLLIDE}},
-        {&b2g_schedule::queryBlock, {64, 128, 256}, {PH_BROADPHASE}},
-        {&b2g_schedule::tailColours, {0, 512, 1024, 2048}, {PH_WARM, PH_SOLVE_V, PH_SOLVE_X}},
+        {&b2g_schedule::islands, {0, 1, 2}, {PH_ISLANDS}, NOT_SMALL},
+        {&b2g_schedule::collideOrder, {0, 1, 2}, {PH_COLLIDE}, ALWAYS},
+        {&b2g_schedule::solverBlock, {64, 128, 256, 512}, {PH_WARM, PH_SOLVE_V, PH_SOLVE_X}, PER_COLOUR},
+        {&b2g_schedule::collideBlock, {64, 128, 256}, {PH_COLLIDE}, ALWAYS},
+        {&b2g_schedule::queryBlock, {64, 128, 256}, {PH_BROADPHASE}, NOT_SMALL},
+        {&b2g_schedule::tailColours, {0, 512, 1024, 2048}, {PH_WARM, PH_SOLVE_V, PH_SOLVE_X}, ALWAYS},
+    };
+    // Whether this world's solve is one launch unless tailColours is 0.
+    auto oneLaunchWorld = [&]() {
+        const int tail = ctx->sched.tailColours;
+        ctx->sched.tailColours = kTailDefault;
+        const bool fits = smallWorldFits(ctx, p) || blockSolveFits(ctx, p, ctx->lastConstraints) ||
+                          teamSolveFits(ctx, p, ctx->lastConstraints);
+        ctx->sched.tailColours = tail;
+        return fits;
     };
     (void)hipSetDevice(ctx->device);
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -11249,24 +11268,53 @@ int b2g_autotune(b2g_context* ctx, const b2g_step_params* p, int rounds, b2g_sch
         savedMs[i] = ctx->profMs[i];
         savedLaunches[i] = ctx->profLaunches[i];
     }
-    ctx->profiling = true;
     ctx->evMarks.clear();
     ctx->evUsed = 0;
     int rc = B2G_OK;
     for (const Knob& k : knobs) {
         const int nv = (int)k.values.size();
+        const int32_t before = ctx->sched.*k.field;
         std::vector<double> total(nv, 0.0);
+        // tailColours 0 turns the one-launch solves off, which moves work
+        // between phases: there the whole step without the profiler's events
+        // decides, and only whether to turn them off.
+        const bool onOff = k.field == &b2g_schedule::tailColours && oneLaunchWorld();
+        int reached = 0, oneLaunch = 0, longest = 0;
+        ctx->profiling = !onOff;
         for (int r = 0; r < rounds && rc == B2G_OK; ++r) {
             for (int j = 0; j < nv && rc == B2G_OK; ++j) {
                 const int i = (j + r) % nv;
                 ctx->sched.*k.field = k.values[i];
                 for (int ph : k.phases) ctx->profMs[ph] = 0.0;
+                (void)hipStreamSynchronize(ctx->stream);
+                const auto t0 = std::chrono::steady_clock::now();
                 rc = b2g_step(ctx, p);
+                (void)hipStreamSynchronize(ctx->stream);
+                const std::chrono::duration<double, std::milli> ms = std::chrono::steady_clock::now() - t0;
+                if (onOff) total[i] += ms.count();
                 profCollect(ctx);
-                for (int ph : k.phases) total[i] += ctx->profMs[ph];
+                for (int ph : k.phases) total[i] += onOff ? 0.0 : ctx->profMs[ph];
+                if (k.reach == ALWAYS || !(k.reach == NOT_SMALL ? ctx->lastSmall : ctx->lastOneLaunch)) ++reached;
+                if (ctx->lastOneLaunch) ++oneLaunch;
+                longest = std::max(longest, ctx->nContacts);
             }
         }
+        ctx->sched.*k.field = before;
         if (rc != B2G_OK) break;
+        if (reached < nv * rounds) continue;
+        if (onOff) {
+            if (oneLaunch != (nv - 1) * rounds) continue;  // the world grew out of it meanwhile
+            const double on = (total[1] + total[2] + total[3]) / 3.0;
+            if (total[0] < on) ctx->sched.tailColours = 0;
+            else if (before == 0) ctx->sched.tailColours = kTailDefault;
+            continue;
+        }
+        // below that table length labelling methods 0 and 1 are one and the same
+        if (k.field == &b2g_schedule::islands && longest < kPropagateContacts)
+            total[0] = total[1] = 0.5 * (total[0] + total[1]);
+        // 0 would also keep the world from the one-launch solves once it is
+        // smaller, so it has to be clearly better
+        if (k.field == &b2g_schedule::tailColours) total[0] *= 1.02;
         ctx->sched.*k.field = k.values[std::min_element(total.begin(), total.end()) - total.begin()];
     }
     ctx->profiling = wasProfiling;

@@ -711,8 +711,10 @@ typedef struct b2g_schedule {
     int32_t queryBlock;    /* workgroup size of the broad-phase query */
     int32_t tailColours;   /* trailing colours of at most this many constraints are
                               solved by one 1024-lane workgroup, colour after colour
-                              (0: every colour its own launch, and small worlds run
-                              stage by stage as large ones do) */
+                              (0: every colour its own launch in worlds of any size:
+                              no solve of a small or mid-sized world in one launch by
+                              a workgroup or the workgroups of one XCD, no small-world
+                              step, and continuous collision stage by stage) */
     int32_t clusterBodies; /* clustered solve: awake bodies are grouped into clusters of
                               this many (a power of two, 64-2048) by the Morton order of
                               their positions; constraints inside a cluster are solved by
@@ -742,7 +744,9 @@ int b2g_get_schedule(b2g_context* ctx, b2g_schedule* s);
  * timing the candidates on real steps of this world (the event time of the
  * phases the field affects, candidates interleaved and their order rotated
  * each of `rounds` rounds), keeps the fastest, and returns the result in
- * *out. The steps advance the world as ordinary steps do; since no choice
+ * *out. Where one launch solves the island (see tailColours), the whole step's
+ * time decides whether that stays on, and fields that its kernels do not read
+ * keep their values. The steps advance the world as ordinary steps do; since no choice
  * changes results, the trajectory is the one the world would have had
  * anyway. (3 + 3 + 4 + 3 + 3 + 4) * rounds steps. */
 int b2g_autotune(b2g_context* ctx, const b2g_step_params* p, int rounds, b2g_schedule* out);

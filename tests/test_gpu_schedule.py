@@ -296,3 +296,55 @@ def test_profile_shows_the_step_that_runs(gpu, n, launch):
     assert p["k_collide"][0] == p["k_pairs_query"][0] == 10
     assert scanned > 0
     a.close(); b.close()
+
+
+def _tuned(w, rounds):
+    out = np.zeros(1, E.SCHEDULE)
+    rc = w.e.lib.b2pp_world_autotune(w.h, ctypes.c_float(1.0 / 60.0), 8, 3, rounds, E.ptr(out))
+    assert rc == 0, w.error()
+    return out[0]
+
+
+@pytest.mark.parametrize("n", [300, 4100])
+def test_autotune_keeps_fields_that_change_nothing(gpu, n):
+    """Worlds whose solve is one launch (by one workgroup, or the workgroups of
+    an XCD): the solver's workgroup size and the length of the fused tail
+    change nothing there, and a small world has no labelling rounds or query
+    kernel of its own either, so the tuner leaves those fields as they are."""
+    w = gpu.world("world", n, 3, sleep=False)
+    w.step(120)
+    _set(w, (2, 0, 64, 256, 128, 300, 0, 0))
+    out = _tuned(w, 1)
+    assert out["solverBlock"] == 64 and out["tailColours"] == 300
+    if n < 4000:
+        assert out["islands"] == 2 and out["queryBlock"] == 128
+    w.close()
+
+
+@pytest.mark.parametrize("n", [40, 300, 4100])
+def test_autotune_finds_the_one_launch_solve(gpu, n):
+    """tailColours 0 turns the one-launch solves of these worlds off; a whole
+    step is a quarter to two thirds shorter with them, so the tuner does not
+    leave the field at 0."""
+    w = gpu.world("world", n, 3, sleep=False)
+    w.step(120)
+    _set(w, (0, 0, 256, 256, 256, 0, 0, 0))
+    assert _tuned(w, 3)["tailColours"] != 0
+    w.close()
+
+
+def test_autotune_profile_and_islands(gpu):
+    """The tuner leaves the caller's profile alone; below 65536 contacts
+    labelling methods 0 and 1 are one and the same, and it takes 0 for them."""
+    lib = E.b2g_lib()
+    w = gpu.world("world", 4500, 3, sleep=False)
+    w.step(120)
+    ctx = w.device_context()
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 1))
+    w.step(5)
+    before = _profile(w)
+    for _ in range(3):
+        assert _tuned(w, 1)["islands"] in (0, 2)
+    assert _profile(w) == before
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 0))
+    w.close()
