@@ -3979,7 +3979,7 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
 // ====================================================================
 constexpr int kBlockBodies = 4032;       // body rows in LDS: 63 of the 64 KB a launch may ask for
 constexpr int kBlockConstraints = 4096;  // most constraints (blockSolveFits)
-constexpr int kBlockJointed = 4096;      // most constraints, and most joints, with joints
+constexpr int kBlockJoints = 4096;       // most joints (chained bodies have about one each)
 constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane, whose rows take most of them
 template <bool kJoints>
 constexpr int kBlockRows = kJoints ? 3 : 4;  // constraint rows a lane holds
@@ -4974,12 +4974,13 @@ __global__ void k_append_contacts(WorldView w, const unsigned long long* keys, i
 // item, so the results are theirs; what differs is that the labels always
 // come from the union-find pass (the same labels), that dead contacts leave
 // the table in place, and that nothing is read back before the end. At 590
-// contacts k_small_prepare takes 13 us and k_small_finish 15 us, at 4500
-// contacts 54 and 64 us: memory latency, a few loads deep per stage.
+// contacts k_small_prepare takes 12 us and k_small_finish 15 us, at 2119
+// contacts 29 and 33 us, at 3900 46 and 60 us: memory latency, a few loads
+// deep per stage.
 // ====================================================================
 constexpr int kSmallLanes = 1024;
 constexpr int kSmallBodies = kBlockBodies;   // island labels in LDS
-constexpr int kSmallContacts = 5120;         // contact bodies in LDS (see smallWorldFits)
+constexpr int kSmallContacts = kBlockConstraints;  // contact bodies in LDS (see smallWorldFits)
 constexpr int kSortedNewPairs = 4096;        // new pairs sorted in LDS
 constexpr int kAppendPairs = 768;            // see runBroadphase
 constexpr int kAppendFixtures = 65536;       // move flags that one workgroup clears
@@ -8286,7 +8287,7 @@ int wideConstraints(const ColourLayout& l) {
 // 643 us, but 4831 689 -> 718 us.
 bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
     if (ctx->nBodies > kBlockBodies || constraints > kBlockConstraints) return false;
-    if (ctx->nJoints > 0 && (constraints > kBlockJointed || ctx->nJoints > kBlockJointed)) return false;
+    if (ctx->nJoints > kBlockJoints) return false;
     if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->sched.clusterBodies > 0 || ctx->graphs)
         return false;
     if (ctx->traceIters > 0 || ctx->logCap > 0) return false;
@@ -8352,15 +8353,15 @@ void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView
 }
 
 // Whether the whole step after the narrowphase goes to the small-world kernels:
-// the block solve takes it whatever share of the contacts are constraints, the
-// LDS tables hold the world, and no candidate point has to be gathered for the
-// network. One compute unit works through a stage where the grid
+// the block solve takes it if every contact is a constraint (kSmallContacts at
+// most, which the LDS tables hold), and no candidate point has to be gathered
+// for the network. One compute unit works through a stage where the grid
 // kernels have the whole chip, so the gain ends with the contacts: settled
-// worlds of 590 contacts 278 -> 129 us a step, 1700 (700-body pile)
-// 341 -> 232 us, 4500 401 -> 356 us, but 6600 457 -> 480 us.
+// piles of 2968 contacts 292 us a step stage by stage and 254 us so, 3438 297
+// and 286, 3902 336 and 328, but 4526 329 and 339, 5098 339 and 366.
 bool smallWorldFits(const b2g_context* ctx, const b2g_step_params* p) {
     return blockSolveFits(ctx, p, ctx->nContacts) && ctx->nFixtures <= kSmallBodies && ctx->nFixtures > 0 &&
-           ctx->nContacts <= kSmallContacts && !p->learnedWarmStart && ctx->demoteRounds < kClaimTags &&
+           !p->learnedWarmStart && ctx->demoteRounds < kClaimTags &&
            (ctx->orderSpan == 0 || ctx->orderCount == ctx->nFixtures);
 }
 
