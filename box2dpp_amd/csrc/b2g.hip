@@ -659,8 +659,8 @@ __global__ void k_island_mark(WorldView w) {
 }
 
 // Constraint set of the step: island contacts of awake islands. Contacts
-// leaving the set give their colour back.
-// Returns whether the constraint has no colour yet.
+// leaving the set give their colour back. Returns whether a constraint has no
+// colour yet.
 __device__ inline bool markConstraintOne(const WorldView& w, int c, int bA, int bB) {
     int flags = w.cflags[c] & ~CF_CONSTRAINT;
     const bool isCons = islandContact(w, c) && ((w.bflags[bA] & BF_ISLAND) || (w.bflags[bB] & BF_ISLAND));
@@ -746,7 +746,6 @@ __device__ inline unsigned long long claimValue(uint32_t tag, const WorldView& w
     return ((unsigned long long)tag << 48) | (0xFFFFFFFFFFFFull - prio);
 }
 
-// Also clears the count of losers that k_colour_commit then takes.
 __device__ inline bool uncoloured(const WorldView& w, int c) {
     return (w.cflags[c] & CF_CONSTRAINT) && w.ccolour[c] < 0;
 }
@@ -758,6 +757,7 @@ __device__ inline void colourClaimOne(const WorldView& w, unsigned long long* cl
     if (w.btype[bB] == BT_DYNAMIC) atomicMax(&claim[bB], v);
 }
 
+// Also clears the count of losers that k_colour_commit then takes.
 __global__ void k_colour_claim(WorldView w, unsigned long long* claim, uint32_t tag, Counters* cnt, int round) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c == 0) cnt->roundLeft[round] = 0;
@@ -5494,7 +5494,7 @@ __global__ void k_edge_count(WorldView w, RefView r, Counters* cnt) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= w.nContacts) return;
     r.cvisited[c] = 0;
-    w.cflags[c] &= ~CF_CONSTRAINT;  // set again for the island contacts by k_dfs
+    w.cflags[c] &= ~CF_CONSTRAINT;  // set again for the island contacts by the search
     if (!islandContact(w, c)) return;
     const int bA = w.fbody[w.cfA[c]], bB = w.fbody[w.cfB[c]];
     if (w.btype[bA] != BT_STATIC) { atomicAdd(&r.edgeCount[bA], 1); atomicAdd(&cnt->nEdges, 1); }
@@ -5550,9 +5550,8 @@ __global__ void k_edge_extract(RefView r, int n) {
     r.edgeContact[i] = low < 0x80000000u ? (int)(0x7FFFFFFFu - low) : ~(int)(0xFFFFFFFFu - low);
 }
 
-// Island search of b2World::Solve (REF/Dynamics/b2World.cpp:429-539), one
-// thread: contact edges, then joint edges to active bodies.
-// The search of a world that fits in LDS: the edges with their other bodies,
+// Island search of b2World::Solve (REF/Dynamics/b2World.cpp:429-539) in a
+// world that fits in LDS: the edges with their other bodies,
 // the body flags and the visited marks, so that the one lane that searches
 // waits for LDS only (79 bodies, 210 contacts: 181 us over global memory,
 // 61 us). What the search does to bodies and contacts is applied after
@@ -5560,7 +5559,7 @@ __global__ void k_edge_extract(RefView r, int n) {
 constexpr int kDfsBodies = 2048;
 constexpr int kDfsEdges = 6144;
 constexpr int kDfsMarks = 8192;  // contacts, and joints
-__global__ void __launch_bounds__(256) k_dfs_small(WorldView w, JointView jv, RefView r, int nEdges, Counters* cnt) {
+__global__ void __launch_bounds__(256) k_dfs_small(WorldView w, JointView jv, RefView r, Counters* cnt) {
     __shared__ int edge[kDfsEdges];             // contact c, or ~j
     __shared__ uint16_t otherBody[kDfsEdges];
     __shared__ uint16_t start[kDfsBodies + 1];
@@ -5649,6 +5648,8 @@ __global__ void __launch_bounds__(256) k_dfs_small(WorldView w, JointView jv, Re
         if ((seenContact[c >> 5] >> (c & 31)) & 1u) w.cflags[c] |= CF_CONSTRAINT;
 }
 
+// The same search over memory, by one thread: contact edges, then joint edges
+// to active bodies.
 __global__ void k_dfs(WorldView w, JointView jv, RefView r, Counters* cnt) {
     if (blockIdx.x != 0 || threadIdx.x != 0) return;
     int nI = 0, nb = 0, nc = 0, nj = 0;
@@ -7598,7 +7599,7 @@ int runBroadphase(b2g_context* ctx, const uint32_t* closedMask = nullptr) {
     const int packBase = ordered ? ctx->orderSpan : nf;
     int nNew = 0;
     for (int attempt = 0;; ++attempt) {
-        if (attempt > 0) {  // k_grid_reset cleared them for the first
+        if (attempt > 0) {  // k_grid_reset or k_close_table cleared them for the first
             hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, s, &ctx->cnt->nNewPairs, 1, 0);
             hipLaunchKernelGGL(k_fill<int>, dim3(1), dim3(64), 0, s, &ctx->cnt->overflow, 1, 0);
         }
@@ -9449,7 +9450,7 @@ int stepReferenceSolve(b2g_context* ctx, const b2g_step_params* p) {
             hipLaunchKernelGGL(k_edge_extract, dim3(blocks(nEdges)), dim3(256), 0, s, r, nEdges);
         }
         if (nb <= kDfsBodies && nEdges <= kDfsEdges && nc <= kDfsMarks && nj <= kDfsMarks)
-            hipLaunchKernelGGL(k_dfs_small, dim3(1), dim3(256), 0, s, w, jv, r, nEdges, ctx->cnt);
+            hipLaunchKernelGGL(k_dfs_small, dim3(1), dim3(256), 0, s, w, jv, r, ctx->cnt);
         else
             hipLaunchKernelGGL(k_dfs, dim3(1), dim3(64), 0, s, w, jv, r, ctx->cnt);
         LAUNCHCHK(ctx);
