@@ -7197,6 +7197,7 @@ struct b2g_context {
     int demoteRounds = 1;           // colour demotion rounds per coloured step
     int compactedFrom = -1;  // table length before the last coloured step's compaction (-1: none)
     int lastNewPairs = 0;        // new pairs of the last broad-phase
+    int teamSize = kTeamSize;    // workgroups the team solve wants
     bool lastSmall = false;      // the last step ran in the small-world kernels
     bool lastOneLaunch = false;  // the last step's island solve was one launch (block or team solve)
     int lastConstraints = 0;
@@ -8343,7 +8344,7 @@ void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView
     plan.velIters = p->velocityIterations;
     plan.posIters = std::min(p->positionIterations, kMaxPosIters);
     plan.contactWarm = contactWarm ? 1 : 0;
-    plan.wanted = kTeamSize;
+    plan.wanted = (unsigned)ctx->teamSize;
     const int pe = profStart(ctx);
     hipEvent_t e0, e1;
     const int pk = profKernelEvents(ctx, &e0, &e1);
@@ -11219,6 +11220,13 @@ int b2g_set_schedule(b2g_context* ctx, const b2g_schedule* sc) {
         sc->persistentSolve < 0 || sc->persistentSolve > 16)
         return fail(ctx, B2G_ERR_ARG, "schedule field out of range");
     ctx->sched = *sc;
+    return B2G_OK;
+}
+
+int b2g_set_team_size(b2g_context* ctx, int workgroups) {
+    if (!ctx) return B2G_ERR_ARG;
+    if (workgroups < 1 || workgroups > kTeamSize) return fail(ctx, B2G_ERR_ARG, "team size out of range");
+    ctx->teamSize = workgroups;
     return B2G_OK;
 }
 

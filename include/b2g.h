@@ -738,6 +738,11 @@ typedef struct b2g_schedule {
    persistentSolve 0 to 16. */
 int b2g_set_schedule(b2g_context* ctx, const b2g_schedule* s);
 int b2g_get_schedule(b2g_context* ctx, b2g_schedule* s);
+/* Workgroups of one XCD that a mid-sized world's island solve waits for, 1 to
+ * 16 (default 16). It starts with those that are there after 20 us, so other
+ * work on the chip makes it slower and changes no result; a program that
+ * leaves it little room can ask for fewer. */
+int b2g_set_team_size(b2g_context* ctx, int workgroups);
 /* Autotuner: picks each schedule field in turn (islands, collideOrder,
  * solverBlock, collideBlock, queryBlock, tailColours; the clustered and the
  * one-launch solve, both measured slower on the piles, are not tried) by

@@ -7,15 +7,22 @@ that lanes hold in registers (1024 with 256 lanes, 2048 with 512; 768 and 1536
 with joints), the largest number of bodies in LDS and one beyond it, worlds
 that start with more new pairs than the LDS sort takes, every joint type, a
 body in more contacts than there are colours (the overflow colour), islands
-that sleep, contacts that end, sub-worlds, few iterations. Larger worlds go to
-the team solve (the workgroups of one XCD with a barrier between colours).
+that sleep, contacts that end, sub-worlds, a learned start, few iterations.
+Larger worlds go to the team solve (the workgroups of one XCD with a barrier
+between colours), with full and with small teams.
 """
 import ctypes
+import os
+import sys
+import threading
 
 import numpy as np
 import pytest
 
 import engines as E
+
+sys.path.insert(0, os.path.join(E.ROOT, "oracle"))
+import mlp_ref as M  # noqa: E402
 
 pytestmark = pytest.mark.gpu
 
@@ -90,10 +97,74 @@ def test_with_events_and_sensors(gpu, kind, n, ccd):
     same(run(gpu.world(kind, n, 2, ccd=ccd), False, 60), run(gpu.world(kind, n, 2, ccd=ccd), True, 60))
 
 
-@pytest.mark.parametrize("kind, n_worlds, n, sleep", [("world", 9, 120, True), ("pendulums", 5, 7, False)])
+@pytest.mark.parametrize("kind, n_worlds, n, sleep", [("world", 9, 120, True), ("pendulums", 5, 7, False),
+                                                      # the team solve, islands that sleep one by one
+                                                      ("world", 20, 263, True), ("world", 20, 263, False)])
 def test_sub_worlds(gpu, kind, n_worlds, n, sleep):
     same(run(E.World.worlds(gpu, kind, n_worlds, n, 4, sleep), False, 240),
          run(E.World.worlds(gpu, kind, n_worlds, n, 4, sleep), True, 240))
+
+
+def learned(w, scope, seed):
+    """A random network's start for every step: impulses of the size of a contact's."""
+    lib, ctx = E.b2g_lib(), w.device_context()
+    p = M.random_params(np.random.default_rng(seed))
+    p["ystd"] = 0.05
+    p["ymean"] = 0.0
+    E.b2g_check(lib, ctx, lib.b2g_mlp_set_params(ctx, E.ptr(np.atleast_1d(p))))
+    E.b2g_check(lib, ctx, lib.b2g_set_learned_scope(ctx, scope, 1))
+    w.set_learned(True, 0.0)
+    return w
+
+
+@pytest.mark.parametrize("scope", [0, 1])
+@pytest.mark.parametrize("n, steps", [(700, 240), (3000, 240), (6000, 300)])
+def test_with_a_learned_start(gpu, n, steps, scope):
+    """The network's impulses reach the rows that the block solve (two sizes)
+    and the team solve hold."""
+    a = learned(gpu.world("world", n, 3, sleep=False), scope, 5)
+    b = learned(gpu.world("world", n, 3, sleep=False), scope, 5)
+    same(run(a, False, steps), run(b, True, steps))
+    plain = gpu.world("world", n, 3, sleep=False)
+    plain.step(60)
+    c = learned(gpu.world("world", n, 3, sleep=False), scope, 5)
+    c.step(60)
+    assert not np.array_equal(plain.bodies(), c.bodies()) and np.isfinite(c.bodies()).all()
+    plain.close(); c.close()
+
+
+@pytest.mark.parametrize("kind, n, team", [("world", 4033, 1), ("world", 9000, 1), ("world", 9000, 3),
+                                           ("world", 13000, 5), ("plank", 4100, 2)])
+def test_small_teams(gpu, kind, n, team):
+    """A team smaller than its constraints need reads those that its lanes
+    cannot hold from memory in every pass, and turns the workgroups away that
+    come once it is complete."""
+    a = gpu.world(kind, n, 8, sleep=False)
+    ctx, lib = a.device_context(), E.b2g_lib()
+    assert lib.b2g_set_team_size(ctx, 0) != 0 and lib.b2g_set_team_size(ctx, 17) != 0
+    E.b2g_check(lib, ctx, lib.b2g_set_team_size(ctx, team))
+    steps = 9 if kind == "plank" else 300
+    same(run(a, False, steps), run(gpu.world(kind, n, 8, sleep=False), True, steps))
+
+
+def test_two_worlds_at_once(gpu):
+    """Two contexts stepped by two threads, whose teams share the chip."""
+    def go(seed, out):
+        w = gpu.world("world", 6000, seed, sleep=False)
+        out.append(run(w, False, 300))
+
+    alone, both = [], [[], []]
+    for seed in (1, 2):
+        out = []
+        go(seed, out)
+        alone.append(out[0])
+    threads = [threading.Thread(target=go, args=(seed, both[seed - 1])) for seed in (1, 2)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    for i in range(2):
+        same(alone[i], both[i][0])
 
 
 def test_many_new_pairs_at_once(gpu):
