@@ -4288,9 +4288,9 @@ __global__ void __launch_bounds__(kTeamLanes) k_solve_team(WorldView w, ConView 
     const int lane = ((int)(threadIdx.x >> 6) * (int)size + (int)rank) * 64 + (int)(threadIdx.x & 63);
     const int lanes = (int)size * kTeamLanes;
     // Constraint lane + r * lanes in row r; those beyond (a team smaller than
-    // wanted) and all of them with an overflow colour, which one lane solves
-    // in order, are read in every pass.
-    const int held = nCons > cs[kOverflowColour] ? 0 : min(nCons, R * lanes);
+    // wanted) are read in every pass. There is no overflow colour
+    // (teamSolveFits).
+    const int held = min(nCons, R * lanes);
     VelRow row[R];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -4299,20 +4299,15 @@ __global__ void __launch_bounds__(kTeamLanes) k_solve_team(WorldView w, ConView 
     // reg(r) over the constraints in registers, mem(k) over the others, colour
     // after colour.
     auto colours = [&](auto reg, auto mem) {
-        for (int c = 0; c < kColourSlots && cs[c] < nCons; ++c) {
+        for (int c = 0; c < kOverflowColour && cs[c] < nCons; ++c) {
             const int b0 = cs[c], b1 = cs[c + 1];
             if (b1 <= b0) continue;
-            if (c == kOverflowColour) {
-                if (lane == 0)
-                    for (int k = b0; k < b1; ++k) mem(k);
-            } else {
 #pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    const int k = lane + r * lanes;
-                    if (k >= b0 && k < min(b1, held)) reg(r);
-                }
-                for (int k = max(b0, held) + lane; k < b1; k += lanes) mem(k);
+            for (int r = 0; r < R; ++r) {
+                const int k = lane + r * lanes;
+                if (k >= b0 && k < min(b1, held)) reg(r);
             }
+            for (int k = max(b0, held) + lane; k < b1; k += lanes) mem(k);
             teamBarrier(cnt, size, phase);
         }
     };
@@ -4351,12 +4346,8 @@ __global__ void __launch_bounds__(kTeamLanes) k_solve_team(WorldView w, ConView 
         const int k = lane + r * lanes;
         if (k < held) storeImpulsesTo(w, cv.contact[k], row[r].info & 3, row[r].imp);
     }
-    for (int c = 0; c < kColourSlots; ++c) {
-        const bool serial = c == kOverflowColour;
-        if (serial && lane != 0) continue;
-        for (int k = max(cs[c], held) + (serial ? 0 : lane); k < cs[c + 1]; k += serial ? 1 : lanes)
-            storeImpulsesOne(w, cv, k);
-    }
+    for (int c = 0; c < kOverflowColour; ++c)
+        for (int k = max(cs[c], held) + lane; k < cs[c + 1]; k += lanes) storeImpulsesOne(w, cv, k);
     for (int b = lane; b < nb; b += lanes) {
         if (!islandBody(w, b)) continue;
         float4 pos = w.pos[b], v = teamRow(w.vel + b);
@@ -8328,9 +8319,14 @@ void launchBlockSolve(b2g_context* ctx, const b2g_step_params* p, const WorldVie
 // solve does not take it. Settled piles, launches per colour against the team:
 // 8355 constraints 630 -> 450 us a step, 12 576 590 -> 500 us, 21 885
 // 633 -> 590 us, 33 886 658 -> 660 us (and 32 batched worlds of 14 700 in all
-// 515 -> 455 us): by then a colour has work enough for the whole chip.
+// 515 -> 455 us): by then a colour has work enough for the whole chip. A body
+// that fills all the colours makes most of them thin, and those are faster
+// fused (planks under 4100 to 5000 boxes, 12 000 to 24 000 constraints of
+// which 130 to 670 have no colour: launches 2.5 to 6.6 ms a step, the team 2.9
+// to 7.6 ms), so the colours of the step's order decide, too.
 bool teamSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
     if (ctx->nJoints > 0 || constraints == 0 || constraints > kTeamConstraints) return false;
+    if (ctx->lastColourStart[kOverflowColour + 1] > ctx->lastColourStart[kOverflowColour]) return false;
     if (ctx->sched.tailColours == 0 || ctx->sched.persistentSolve > 0 || ctx->sched.clusterBodies > 0 || ctx->graphs)
         return false;
     if (ctx->traceIters > 0 || ctx->logCap > 0) return false;

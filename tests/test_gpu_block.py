@@ -31,6 +31,7 @@ BODY = np.dtype([
     ("c", "<f4", 2), ("a", "<f4"), ("rest", "<f4", 12),
 ])
 assert BODY.itemsize == 104
+PROFILE = np.dtype([("name", "S24"), ("launches", "<i4"), ("pad", "<i4"), ("ms", "<f8")])
 
 
 def a_launch_per_colour(w):
@@ -133,18 +134,33 @@ def test_with_a_learned_start(gpu, n, steps, scope):
     plain.close(); c.close()
 
 
-@pytest.mark.parametrize("kind, n, team", [("world", 4033, 1), ("world", 9000, 1), ("world", 9000, 3),
-                                           ("world", 13000, 5), ("plank", 4100, 2)])
-def test_small_teams(gpu, kind, n, team):
+@pytest.mark.parametrize("n, team", [(4033, 1), (9000, 1), (9000, 3), (13000, 5)])
+def test_small_teams(gpu, n, team):
     """A team smaller than its constraints need reads those that its lanes
     cannot hold from memory in every pass, and turns the workgroups away that
     come once it is complete."""
-    a = gpu.world(kind, n, 8, sleep=False)
+    a = gpu.world("world", n, 8, sleep=False)
     ctx, lib = a.device_context(), E.b2g_lib()
     assert lib.b2g_set_team_size(ctx, 0) != 0 and lib.b2g_set_team_size(ctx, 17) != 0
     E.b2g_check(lib, ctx, lib.b2g_set_team_size(ctx, team))
-    steps = 9 if kind == "plank" else 300
-    same(run(a, False, steps), run(gpu.world(kind, n, 8, sleep=False), True, steps))
+    same(run(a, False, 300), run(gpu.world("world", n, 8, sleep=False), True, 300))
+
+
+def test_a_full_set_of_colours_gets_no_team(gpu):
+    """A plank under 4100 boxes fills every colour: its thin ones are faster
+    fused, so the team solve leaves it alone while a pile of the size gets it."""
+    lib = E.b2g_lib()
+    for kind, steps, want in (("plank", 70, 0), ("world", 150, 10)):
+        w = gpu.world(kind, 4100, 3, sleep=False)
+        w.step(steps)
+        ctx = w.device_context()
+        E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 1))
+        w.step(10)
+        assert 4096 < w.stats()["constraints"] < 24576 or kind == "world"
+        rows, n = np.zeros(32, PROFILE), ctypes.c_int()
+        E.b2g_check(lib, ctx, lib.b2g_get_profile(ctx, E.ptr(rows), 32, ctypes.byref(n)))
+        assert {r["name"]: int(r["launches"]) for r in rows}[b"k_solve_team"] == want, kind
+        w.close()
 
 
 def test_two_worlds_at_once(gpu):
