@@ -3979,7 +3979,8 @@ __global__ void __launch_bounds__(kJoints ? kPersistJointBlock : 1024) k_solve_p
 // ====================================================================
 constexpr int kBlockBodies = 4032;       // body rows in LDS: 63 of the 64 KB a launch may ask for
 constexpr int kBlockConstraints = 4096;  // most constraints (blockSolveFits)
-constexpr int kBlockJoints = 4096;       // most joints (chained bodies have about one each)
+constexpr int kBlockJoints = 1536;       // most joints (blockSolveFits)
+constexpr int kSmallIdle = 1536;         // most bodies and joints, a joint counted as three, without contacts
 constexpr int kBlockLanes = 512;         // largest workgroup: 256 VGPRs a lane, whose rows take most of them
 template <bool kJoints>
 constexpr int kBlockRows = kJoints ? 3 : 4;  // constraint rows a lane holds
@@ -8277,7 +8278,10 @@ int wideConstraints(const ColourLayout& l) {
 // two meet: 460 us for either at 4289 constraints, 538 against 438 to 472 us
 // at 8145. With joints, which the team solve does not take and whose passes
 // read memory: 1558 constraints and 620 joints 597 -> 501 us, 3607 703 ->
-// 643 us, but 4831 689 -> 718 us.
+// 643 us, but 4831 689 -> 718 us. A joint costs the workgroup about 0.1 us a
+// step, the chip next to nothing: 1488 joints and 2612 constraints 715 ->
+// 549 us, wheels with 1400 joints and 129 constraints 362 -> 293 us, with
+// 2600 352 -> 451 us, sliding boxes with 1500 joints 241 -> 257 us.
 bool blockSolveFits(const b2g_context* ctx, const b2g_step_params* p, int constraints) {
     if (ctx->nBodies > kBlockBodies || constraints > kBlockConstraints) return false;
     if (ctx->nJoints > kBlockJoints) return false;
@@ -8356,8 +8360,14 @@ void launchTeamSolve(b2g_context* ctx, const b2g_step_params* p, const WorldView
 // for the network. One compute unit works through a stage where the grid
 // kernels have the whole chip, so the gain ends with the contacts: settled
 // piles of 2968 contacts 292 us a step stage by stage and 254 us so, 3438 297
-// and 286, 3902 336 and 328, but 4526 329 and 339, 5098 339 and 366.
+// and 286, 3902 336 and 328, but 4526 329 and 339, 5098 339 and 366. Without
+// any contact the step has only its bodies' and joints' stages and few
+// launches to save: 1400 falling bodies 98 and 90 us, but 2200 98 and 121 us;
+// pendulums of 300 joints 134 and 128 us, of 400 113 and 128 us, of 3000 124
+// and 422 us; hanging chains of 300 joints 144 and 125 us, of 600 155 and
+// 156 us.
 bool smallWorldFits(const b2g_context* ctx, const b2g_step_params* p) {
+    if (ctx->nContacts == 0 && ctx->nBodies + 3 * ctx->nJoints > kSmallIdle) return false;
     return blockSolveFits(ctx, p, ctx->nContacts) && ctx->nFixtures <= kSmallBodies && ctx->nFixtures > 0 &&
            !p->learnedWarmStart && ctx->demoteRounds < kClaimTags &&
            (ctx->orderSpan == 0 || ctx->orderCount == ctx->nFixtures);

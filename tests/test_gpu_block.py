@@ -146,21 +146,44 @@ def test_small_teams(gpu, n, team):
     same(run(a, False, 300), run(gpu.world("world", n, 8, sleep=False), True, 300))
 
 
+def launches(w, steps):
+    """Launches of each kernel that has a row in the profile."""
+    lib, ctx = E.b2g_lib(), w.device_context()
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 1))
+    w.step(steps)
+    rows, n = np.zeros(32, PROFILE), ctypes.c_int()
+    E.b2g_check(lib, ctx, lib.b2g_get_profile(ctx, E.ptr(rows), 32, ctypes.byref(n)))
+    E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 0))
+    return {r["name"].decode(): int(r["launches"]) for r in rows}
+
+
 def test_a_full_set_of_colours_gets_no_team(gpu):
     """A plank under 4100 boxes fills every colour: its thin ones are faster
     fused, so the team solve leaves it alone while a pile of the size gets it."""
-    lib = E.b2g_lib()
     for kind, steps, want in (("plank", 70, 0), ("world", 150, 10)):
         w = gpu.world(kind, 4100, 3, sleep=False)
         w.step(steps)
-        ctx = w.device_context()
-        E.b2g_check(lib, ctx, lib.b2g_set_profiling(ctx, 1))
-        w.step(10)
-        assert 4096 < w.stats()["constraints"] < 24576 or kind == "world"
-        rows, n = np.zeros(32, PROFILE), ctypes.c_int()
-        E.b2g_check(lib, ctx, lib.b2g_get_profile(ctx, E.ptr(rows), 32, ctypes.byref(n)))
-        assert {r["name"]: int(r["launches"]) for r in rows}[b"k_solve_team"] == want, kind
+        assert launches(w, 10)["k_solve_team"] == want, kind
         w.close()
+
+
+@pytest.mark.parametrize("kind, n, before, want", [
+    ("pile", 500, 2, 10), ("pile", 1535, 2, 10), ("pile", 1536, 2, 0), ("pile", 3000, 2, 0), ("pile", 3000, 250, 10),
+    ("pendulums", 100, 2, 10), ("pendulums", 383, 2, 10), ("pendulums", 384, 2, 0), ("pendulums", 3000, 2, 0),
+    ("chains", 100, 2, 10), ("chains", 400, 2, 0), ("welds", 200, 2, 0), ("wheels", 500, 5, 10), ("wheels", 1300, 5, 0),
+])
+def test_what_is_a_small_world(gpu, kind, n, before, want):
+    """Worlds of many joints, or of many bodies and no contact, are slower in
+    one workgroup than stage by stage; either way the steps are the same."""
+    a, b = gpu.world(kind, n, 3, sleep=False), gpu.world(kind, n, 3, sleep=False)
+    a_launch_per_colour(b)
+    a.step(before)
+    b.step(before)
+    contacts = len(a.contacts()[0])
+    assert launches(a, 10)["k_small_prepare"] == want, contacts
+    b.step(10)
+    same([state(a)], [state(b)])
+    a.close(); b.close()
 
 
 def test_two_worlds_at_once(gpu):
