@@ -7917,7 +7917,7 @@ int ensureVelSnap(b2g_context* ctx) {
 
 int ensureMlp(b2g_context* ctx) {
     if (ctx->mlpAllocated) return B2G_OK;
-    HIPCHK(ctx, b2mlp::mlpAlloc(ctx->mlp));
+    HIPCHK(ctx, b2mlp::mlpAlloc(ctx->mlp, ctx->stream));
     ctx->mlpAllocated = true;
     return B2G_OK;
 }

@@ -55,7 +55,8 @@ struct Net {
     bool ready = false;       // parameters set (initialised, trained or loaded)
 };
 
-hipError_t mlpAlloc(Net& n);
+// The arrays, cleared on s (the stream that fills them).
+hipError_t mlpAlloc(Net& n, hipStream_t s);
 void mlpFree(Net& n);
 // BF16 image from the FP32 master weights.
 hipError_t mlpPrepare(const Net& n, hipStream_t s);

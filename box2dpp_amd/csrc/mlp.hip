@@ -577,7 +577,7 @@ int gridFor(int count) {
 
 }  // namespace
 
-hipError_t mlpAlloc(Net& n) {
+hipError_t mlpAlloc(Net& n, hipStream_t s) {
     hipError_t e;
     if ((e = hipMalloc((void**)&n.params, sizeof(float) * kParams)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&n.grad, sizeof(float) * kParams)) != hipSuccess) return e;
@@ -587,13 +587,13 @@ hipError_t mlpAlloc(Net& n) {
     if ((e = hipMalloc((void**)&n.norm, sizeof(float) * kNorm)) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&n.loss, sizeof(float))) != hipSuccess) return e;
     if ((e = hipMalloc((void**)&n.partial, sizeof(float) * kMaxGradBlocks * (kParams + 1))) != hipSuccess) return e;
-    if ((e = hipMemset(n.params, 0, sizeof(float) * kParams)) != hipSuccess) return e;
-    if ((e = hipMemset(n.grad, 0, sizeof(float) * kParams)) != hipSuccess) return e;
-    if ((e = hipMemset(n.m, 0, sizeof(float) * kParams)) != hipSuccess) return e;
-    if ((e = hipMemset(n.v, 0, sizeof(float) * kParams)) != hipSuccess) return e;
-    if ((e = hipMemset(n.wh, 0, sizeof(uint16_t) * hTotal)) != hipSuccess) return e;
-    if ((e = hipMemset(n.norm, 0, sizeof(float) * kNorm)) != hipSuccess) return e;
-    return hipMemset(n.loss, 0, sizeof(float));
+    if ((e = hipMemsetAsync(n.params, 0, sizeof(float) * kParams, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(n.grad, 0, sizeof(float) * kParams, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(n.m, 0, sizeof(float) * kParams, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(n.v, 0, sizeof(float) * kParams, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(n.wh, 0, sizeof(uint16_t) * hTotal, s)) != hipSuccess) return e;
+    if ((e = hipMemsetAsync(n.norm, 0, sizeof(float) * kNorm, s)) != hipSuccess) return e;
+    return hipMemsetAsync(n.loss, 0, sizeof(float), s);
 }
 
 void mlpFree(Net& n) {

@@ -42,6 +42,27 @@ def _inputs(rng, n):
     return x, t
 
 
+def test_a_new_network_waits_for_no_other_stream(lib, ctx):
+    """The network's arrays are cleared on the context's own stream: work that
+    is queued on the process's default stream meanwhile (here some 10 ms of
+    fills) must not let the clearing come after the parameters."""
+    size = 1 << 30
+    buf = ctypes.c_void_p()
+    assert lib.hipMalloc(ctypes.byref(buf), ctypes.c_size_t(size)) == 0
+    try:
+        p = np.atleast_1d(M.random_params(np.random.default_rng(3)))
+        for _ in range(64):
+            assert lib.hipMemsetAsync(buf, 1, ctypes.c_size_t(size), None) == 0
+        E.b2g_check(lib, ctx, lib.b2g_mlp_set_params(ctx, E.ptr(p)))
+        assert lib.hipStreamSynchronize(None) == 0
+        got = np.zeros(1, M.PARAMS_DTYPE)
+        E.b2g_check(lib, ctx, lib.b2g_mlp_get_params(ctx, E.ptr(got)))
+        for k in M.WEIGHTS + ("xmean", "ymean", "ystd"):
+            assert np.array_equal(got[k], p[k]), k
+    finally:
+        lib.hipFree(buf)
+
+
 def test_forward_matches_oracle(lib, ctx):
     rng = np.random.default_rng(11)
     p = M.random_params(rng)
